@@ -135,6 +135,35 @@ __device__ __forceinline__ uint32_t packed_nibble(const uint8_t *k, uint32_t j) 
   return (j & 1) ? (b & 15u) : (b >> 4);
 }
 
+// Packed key bytes as big-endian nibble words: 16 nibbles from nibble s of
+// the key at p (8-byte aligned), first nibble in bits 63..60.  Reads only the
+// aligned 8-byte words that hold nibbles below lim (the caller's bound on
+// valid nibbles, s < lim), so every read stays inside the key's slot.
+__device__ __forceinline__ uint64_t nib_word(const uint8_t *p, uint32_t s, uint32_t lim) {
+  const uint32_t wi = s >> 4, sh = (s & 15u) * 4u;
+  const uint64_t *w = (const uint64_t *)p;
+  uint64_t hi = __builtin_bswap64(w[wi]);
+  if (sh == 0) return hi;
+  uint64_t lo = 16u * (wi + 1) < lim ? __builtin_bswap64(w[wi + 1]) : 0ull;
+  return (hi << sh) | (lo >> (64u - sh));
+}
+
+// Nibbles two packed keys share from nibbles sa and sb on, at most m (16 per
+// step instead of one: a leaf's remainder of ~60 nibbles takes four dependent
+// loads).  la and lb bound the keys' valid nibbles (nib_word).
+__device__ __forceinline__ uint32_t match_nibbles(const uint8_t *pa, uint32_t sa, uint32_t la, const uint8_t *pb,
+                                                  uint32_t sb, uint32_t lb, uint32_t m) {
+  for (uint32_t p = 0; p < m; p += 16) {
+    const uint64_t x = nib_word(pa, sa + p, la) ^ nib_word(pb, sb + p, lb);
+    if (x) {
+      const uint32_t q = p + ((uint32_t)__clzll((long long)x) >> 2);
+      if (q < m) return q;  // nibbles past m do not count
+      return m;
+    }
+  }
+  return m;
+}
+
 __device__ __forceinline__ uint32_t *node_dirty_flag(const Pools &P, ref_t r) {
   uint32_t t = ref_type(r), i = ref_idx(r);
   return t == T_BRANCH ? &P.branch[i].dirty : &P.shrt[i].dirty;

@@ -36,9 +36,41 @@ __device__ __forceinline__ HexKey hex_key(const GetArgs &g, uint32_t i) {
   return k;
 }
 
-__device__ __forceinline__ uint32_t short_nib(const Pools &P, const Short &S, uint32_t rel) {
-  if (S.term && rel + 1 == S.key_len) return kNibbleT;
-  return packed_nibble(P.keys + S.key_off, S.key_start + rel);
+// Bytes [0, c) at p (c <= 8), upper bytes zero; reads only the aligned words
+// that hold them.
+__device__ __forceinline__ uint64_t hex_bytes(const uint8_t *p, uint32_t c) {
+  const uintptr_t a = (uintptr_t)p;
+  const uint32_t sh = (uint32_t)(a & 7);
+  const uint64_t *q = (const uint64_t *)(a - sh);
+  uint64_t v = q[0] >> (8 * sh);
+  if (sh + c > 8) v |= q[1] << (64 - 8 * sh);
+  return c >= 8 ? v : v & ((1ull << (8 * c)) - 1);
+}
+
+// Nibbles [s, s + m) of the packed key at kp (8-byte aligned) against the m
+// hex bytes at h, eight per step (byte by byte, a leaf remainder of ~60
+// nibbles made 60 dependent loads: 95 us for 20,000 reads of a 200,000-key
+// trie, 24 now).  A hex byte above 15 matches nothing.
+__device__ __forceinline__ bool nibbles_equal(const uint8_t *kp, uint32_t s, uint32_t m, const uint8_t *h) {
+  for (uint32_t q = 0; q < m; q += 16) {
+    // a packed word and its 16 hex bytes
+    const uint64_t w = nib_word(kp, s + q, s + m);
+    const uint32_t c = min(16u, m - q);
+    const uint64_t h0 = hex_bytes(h + q, min(8u, c)), h1 = c > 8 ? hex_bytes(h + q + 8, c - 8) : 0ull;
+    if ((h0 | h1) & 0xF0F0F0F0F0F0F0F0ull) return false;
+    // bytes 0x0a 0x0b -> one byte 0xab, big-endian nibble order
+    uint64_t b0 = __builtin_bswap64(h0), b1 = __builtin_bswap64(h1);
+    b0 = (b0 | (b0 >> 4)) & 0x00FF00FF00FF00FFull;
+    b1 = (b1 | (b1 >> 4)) & 0x00FF00FF00FF00FFull;
+    b0 = (b0 | (b0 >> 8)) & 0x0000FFFF0000FFFFull;
+    b1 = (b1 | (b1 >> 8)) & 0x0000FFFF0000FFFFull;
+    b0 = (b0 | (b0 >> 16)) & 0xFFFFFFFFull;
+    b1 = (b1 | (b1 >> 16)) & 0xFFFFFFFFull;
+    uint64_t x = w ^ (b0 << 32 | b1);
+    if (c < 16) x &= ~0ull << (64u - 4u * c);
+    if (x) return false;
+  }
+  return true;
 }
 
 // Walks the key's path; calls visit(ref) for every branch / short node and
@@ -59,11 +91,13 @@ __device__ ref_t walk(const Pools &P, ref_t node, HexKey k, F visit) {
       pos++;
     } else {
       const Short &S = P.shrt[ref_idx(node)];
-      if (k.len - pos < S.key_len) return REF_NULL;
-      for (uint32_t q = 0; q < S.key_len; q++)
-        if (short_nib(P, S, q) != k.k[pos + q]) return REF_NULL;
-      pos += S.key_len;
-      node = S.child;
+      const uint32_t len = S.key_len, term = S.term, real = len - term;
+      const ref_t child = S.child;
+      if (k.len - pos < len) return REF_NULL;
+      if (!nibbles_equal(P.keys + S.key_off, S.key_start, real, k.k + pos)) return REF_NULL;
+      if (term && k.k[pos + real] != kNibbleT) return REF_NULL;
+      pos += len;
+      node = child;
     }
   }
   return REF_NULL;

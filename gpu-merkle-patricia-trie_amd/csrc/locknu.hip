@@ -81,19 +81,6 @@ __device__ __forceinline__ void ver_unlock_obsolete(uint64_t *l) {
   __hip_atomic_fetch_add(l, (uint64_t)3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Packed key bytes as big-endian nibble words: 16 nibbles from nibble s of
-// the key at p (8-byte aligned), first nibble in bits 63..60.  Reads only the
-// aligned 8-byte words that hold nibbles below lim (the caller's bound on
-// valid nibbles, s < lim), so every read stays inside the key's slot.
-__device__ __forceinline__ uint64_t nib_word(const uint8_t *p, uint32_t s, uint32_t lim) {
-  const uint32_t wi = s >> 4, sh = (s & 15u) * 4u;
-  const uint64_t *w = (const uint64_t *)p;
-  uint64_t hi = __builtin_bswap64(w[wi]);
-  if (sh == 0) return hi;
-  uint64_t lo = 16u * (wi + 1) < lim ? __builtin_bswap64(w[wi + 1]) : 0ull;
-  return (hi << sh) | (lo >> (64u - sh));
-}
-
 struct Ctx {
   const uint8_t *kp;  // packed nibbles of the key (8-byte aligned)
   uint32_t len;       // hex length, terminator included
@@ -309,17 +296,7 @@ __device__ __forceinline__ int attempt(const NuArgs &a, const Ctx &c, DirtyStage
       // match the node's key against the key from pos, 16 nibbles per load
       const uint32_t sreal = klen - term, kleft = c.len - 1 - pos;
       const uint32_t mreal = min(sreal, kleft);
-      uint32_t p = 0;
-      while (p < mreal) {
-        uint64_t x = nib_word(sk, kstart + p, kstart + sreal) ^ nib_word(c.kp, pos + p, c.len - 1);
-        const uint32_t cnt = min(16u, mreal - p);
-        if (cnt < 16) x &= ~0ull << (64u - 4u * cnt);
-        if (x) {
-          p += (uint32_t)__clzll((long long)x) >> 2;
-          break;
-        }
-        p += cnt;
-      }
+      uint32_t p = match_nibbles(sk, kstart, kstart + sreal, c.kp, pos, c.len - 1, mreal);
       if (p == mreal && p == sreal && term && p == kleft) p++;  // both at the terminator
       if (p == klen) {
         if (ref_type(child) == T_VALUE) {
@@ -452,15 +429,7 @@ __global__ __launch_bounds__(256) void k_lock_classify(NuArgs a, uint32_t *fresh
     if (term && pos + klen != len) break;
     if (!term && pos + klen == len) break;
     const uint8_t *sk = P.keys + (S.key_off & ~7ull);
-    uint32_t p = 0;
-    while (p < sreal) {
-      uint64_t x = nib_word(sk, S.key_start + p, S.key_start + sreal) ^ nib_word(kp, pos + p, len - 1);
-      const uint32_t cnt = min(16u, sreal - p);
-      if (cnt < 16) x &= ~0ull << (64u - 4u * cnt);
-      if (x) break;
-      p += cnt;
-    }
-    if (p < sreal) break;
+    if (match_nibbles(sk, S.key_start, S.key_start + sreal, kp, pos, len - 1, sreal) < sreal) break;
     pos += klen;
     node = S.child;
   }

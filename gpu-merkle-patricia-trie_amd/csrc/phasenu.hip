@@ -645,15 +645,17 @@ __global__ __launch_bounds__(256) void k_unique(NuArgs a, const uint64_t *sk, co
 
 // --------------------------------------------------- 3. descend + groups --
 
-__global__ __launch_bounds__(256) void k_descend(NuArgs a) {
-  __shared__ ref_t dbuf[kDirtyStage];
-  __shared__ uint32_t dcnt;
-  if (threadIdx.x == 0) dcnt = 0;
-  __syncthreads();
-  DirtyStage ds{dbuf, &dcnt, kDirtyStage};
-  uint32_t i = grid_tid();
-  uint32_t m = a.scal[SC_M_UNIQ];
-  bool active = i < m;
+// One unique key's descent to its stop point.  The dependent loads of a step
+// are one node line and, every 16 nibbles, one key word; a short node's key is
+// compared 16 nibbles per load (nibble by nibble, a leaf remainder of ~60
+// nibbles made 60 dependent byte loads: 139 us for 2,000 keys on a 200,000-key
+// trie, 23 now).
+// Path nodes are marked without atomics: the sorted unique keys that reach a
+// node form one contiguous range, whose first key shares fewer nibbles with
+// its predecessor than the node's start position; that key alone flags and
+// stages the node.  (Its first key may leave a short node midway: the node is
+// then split, its place taken by new nodes, and needs no mark.)
+__device__ __forceinline__ void descend_key(const NuArgs &a, uint32_t i, DirtyStage &ds) {
   const Pools &P = a.P;
   Stop st;
   st.stop = REF_NULL;
@@ -664,106 +666,133 @@ __global__ __launch_bounds__(256) void k_descend(NuArgs a) {
   st.slot = 0;
   st.less = 0;
   st.pad = 0;
-  KeyRef k;
+  const uint32_t idx = a.u_idx[i];
+  const uint32_t t = a.u_trie[i];
+  const uint32_t mark_from = a.u_first[i] ? 0u : (uint32_t)a.u_lcp[i] + 1u;
+  const KeyRef k = key_of(a, idx);
   ref_t node = REF_NULL, parent = REF_NULL;
   uint32_t pos = 0, pslot = 0;
-  bool done = !active;
-  k.p = nullptr;
-  k.len = 0;
-  if (active) {
-    uint32_t idx = a.u_idx[i];
-    uint32_t t = a.u_trie[i];
-    if (t < a.ntries) {
-      node = P.tries[t].root;
-      if (node != REF_NULL) k = key_of(a, idx);  // an empty trie needs no key bytes
-    } else {
-      done = true;
-      raise_error(P.cnt, ERR_BAD_KEY, idx);
-    }
+  bool done = false;
+  if (t < a.ntries) {
+    node = P.tries[t].root;
+  } else {
+    done = true;
+    raise_error(P.cnt, ERR_BAD_KEY, idx);
   }
+  const uint32_t real = k.len - 1;  // nibbles before the terminator
+  uint64_t kw = 0;                  // nibbles kpos .. kpos + 15 of the key
+  uint32_t kpos = 0;
+  bool kw_ok = false;
   for (int guard = 0; guard < 2 * kMaxKeyNibbles + 4 && !done; guard++) {
-    bool want_mark = false;
-    ref_t mark_ref = REF_NULL;
-    if (!done) {
-      uint32_t ty = ref_type(node);
-      if (node == REF_NULL) {
-        if (parent == REF_NULL) {
-          st.kind = STOP_ROOT_EMPTY;
-          st.base = 0;
-        } else {
-          st.kind = STOP_BRANCH_SLOT;
-          st.attach = parent;
-          st.slot = (uint8_t)pslot;
-          st.base = (uint16_t)pos;
-        }
-        done = true;
-      } else if (ty == T_BRANCH) {
-        const Branch &B = P.branch[ref_idx(node)];
-        want_mark = true;
-        mark_ref = node;
-        if (pos >= k.len || B.depth != pos) {
-          raise_error(P.cnt, ERR_INTERNAL, 12);
-          done = true;
-          break;
-        }
-        uint32_t nib = k.nib(pos);
-        parent = node;
-        pslot = nib;
-        node = B.child[nib];
-        pos += 1;
-      } else if (ty == T_SHORT) {
-        const ref_t cur = node;
-        const Short &S = P.shrt[ref_idx(cur)];
-        uint32_t ml = S.key_len;
-        uint32_t p = 0;
-        while (p < ml && pos + p < k.len && short_nib(P, S, pos + p) == k.nib(pos + p)) p++;
-        if (p == ml) {
-          want_mark = true;
-          mark_ref = cur;
-          if (ref_type(S.child) == T_VALUE) {
-            st.kind = STOP_LEAF_UPDATE;
-            st.stop = cur;
-            st.attach = parent;
-            st.slot = (uint8_t)pslot;
-            st.base = (uint16_t)pos;
-            done = true;
-          } else {
-            parent = cur;
-            pslot = 0;
-            node = S.child;
-            pos += ml;
-          }
-        } else if (pos + p >= k.len) {
-          raise_error(P.cnt, ERR_INTERNAL, 11);
-          done = true;
-        } else {
-          uint32_t d = pos + p;
-          uint32_t kn = k.nib(d), sn = short_nib(P, S, d);
-          st.kind = STOP_SHORT_SPLIT;
-          st.stop = cur;
-          st.attach = parent;
-          st.slot = (uint8_t)pslot;
-          st.base = (uint16_t)pos;
-          st.div = (uint16_t)d;
-          st.less = (kn == kNibbleT) || (sn != kNibbleT && kn < sn);
-          done = true;
-        }
-      } else {  // value in a branch slot: the key ends here
-        st.kind = STOP_VALUE_UPDATE;
-        st.stop = parent;
+    const uint32_t ty = ref_type(node);
+    if (node == REF_NULL) {
+      if (parent == REF_NULL) {
+        st.kind = STOP_ROOT_EMPTY;
+        st.base = 0;
+      } else {
+        st.kind = STOP_BRANCH_SLOT;
         st.attach = parent;
         st.slot = (uint8_t)pslot;
         st.base = (uint16_t)pos;
+      }
+      done = true;
+    } else if (ty == T_BRANCH) {
+      Branch &B = P.branch[ref_idx(node)];
+      if (pos >= k.len) {
+        raise_error(P.cnt, ERR_INTERNAL, 12);
+        done = true;
+        break;
+      }
+      uint32_t nib = kNibbleT;
+      if (pos < real) {
+        if (!kw_ok || pos - kpos >= 16) {
+          kw = nib_word(k.p, pos, real);
+          kpos = pos;
+          kw_ok = true;
+        }
+        nib = (uint32_t)(kw >> (60 - 4 * (pos - kpos))) & 15u;
+      }
+      const uint32_t depth = B.depth, flag = B.dirty;
+      const ref_t child = B.child[nib];
+      if (depth != pos) {
+        raise_error(P.cnt, ERR_INTERNAL, 12);
+        done = true;
+        break;
+      }
+      if (flag == 0 && pos >= mark_from) {
+        B.dirty = 1;
+        ds.push(P, node);
+      }
+      parent = node;
+      pslot = nib;
+      node = child;
+      pos += 1;
+    } else if (ty == T_SHORT) {
+      Short &S = P.shrt[ref_idx(node)];
+      const uint32_t ml = S.key_len, term = S.term, ks = S.key_start, flag = S.dirty;
+      const ref_t child = S.child;
+      const uint32_t sreal = ml - term, kleft = real - min(pos, real);
+      const uint32_t mreal = min(sreal, kleft);
+      uint32_t p = match_nibbles(P.keys + S.key_off, ks, ks + sreal, k.p, pos, real, mreal);
+      if (p == mreal && p == sreal && term && p == kleft) p++;  // both at the terminator
+      if (p == ml) {
+        if (flag == 0 && pos >= mark_from) {
+          S.dirty = 1;
+          ds.push(P, node);
+        }
+        if (ref_type(child) == T_VALUE) {
+          st.kind = STOP_LEAF_UPDATE;
+          st.stop = node;
+          st.attach = parent;
+          st.slot = (uint8_t)pslot;
+          st.base = (uint16_t)pos;
+          done = true;
+        } else {
+          parent = node;
+          pslot = 0;
+          node = child;
+          pos += ml;
+        }
+      } else if (pos + p >= k.len) {
+        raise_error(P.cnt, ERR_INTERNAL, 11);
+        done = true;
+      } else {
+        const uint32_t d = pos + p;
+        const uint32_t kn = k.nib(d), sn = short_nib(P, S, d);
+        st.kind = STOP_SHORT_SPLIT;
+        st.stop = node;
+        st.attach = parent;
+        st.slot = (uint8_t)pslot;
+        st.base = (uint16_t)pos;
+        st.div = (uint16_t)d;
+        st.less = (kn == kNibbleT) || (sn != kNibbleT && kn < sn);
         done = true;
       }
+    } else {  // value in a branch slot: the key ends here
+      st.kind = STOP_VALUE_UPDATE;
+      st.stop = parent;
+      st.attach = parent;
+      st.slot = (uint8_t)pslot;
+      st.base = (uint16_t)pos;
+      done = true;
     }
-    if (want_mark) ds.mark(P, mark_ref);
   }
-  if (active) {
-    if (!done) raise_error(P.cnt, ERR_INTERNAL, 10);
-    a.stop[i] = st;
-  }
-  dirty_flush(P, ds);
+  if (!done) raise_error(P.cnt, ERR_INTERNAL, 10);
+  a.stop[i] = st;
+}
+
+__global__ __launch_bounds__(256) void k_descend(NuArgs a) {
+  // the sort needs a fallback pass: the order (and with it which key marks a
+  // node) is not final, and the host runs the descent again
+  if (a.P.cnt->flag_fallback) return;
+  __shared__ ref_t dbuf[kDirtyStage];
+  __shared__ uint32_t dcnt;
+  if (threadIdx.x == 0) dcnt = 0;
+  __syncthreads();
+  DirtyStage ds{dbuf, &dcnt, kDirtyStage};
+  const uint32_t i = grid_tid();
+  if (i < a.scal[SC_M_UNIQ]) descend_key(a, i, ds);
+  dirty_flush(a.P, ds);
 }
 
 __device__ __forceinline__ bool same_group(const Stop &x, uint32_t tx, const Stop &y, uint32_t ty) {
@@ -778,6 +807,7 @@ __device__ __forceinline__ bool same_group(const Stop &x, uint32_t tx, const Sto
 }
 
 __global__ __launch_bounds__(256) void k_group_flags(NuArgs a) {
+  if (a.P.cnt->flag_fallback) return;  // no stops yet (k_descend)
   uint32_t i = grid_tid();
   uint32_t m = a.scal[SC_M_UNIQ];
   if (i >= a.n) return;
@@ -792,6 +822,7 @@ __global__ __launch_bounds__(256) void k_group_flags(NuArgs a) {
 // grp[] = exclusive scan of the start flags in ecount[]; make it inclusive,
 // i.e. 1-based group ids.
 __global__ __launch_bounds__(256) void k_group_fix(NuArgs a) {
+  if (a.P.cnt->flag_fallback) return;  // no stops yet (k_descend)
   uint32_t i = grid_tid();
   if (i >= a.n) return;
   a.grp[i] += a.ecount[i];
@@ -799,6 +830,7 @@ __global__ __launch_bounds__(256) void k_group_fix(NuArgs a) {
 
 // grp[] now holds the inclusive scan; group id = grp - 1.
 __global__ __launch_bounds__(256) void k_group_info(NuArgs a) {
+  if (a.P.cnt->flag_fallback) return;  // no stops yet (k_descend)
   uint32_t i = grid_tid();
   uint32_t m = a.scal[SC_M_UNIQ];
   if (i >= m) return;
@@ -819,6 +851,7 @@ __global__ __launch_bounds__(256) void k_group_info(NuArgs a) {
 }
 
 __global__ __launch_bounds__(256) void k_group_split(NuArgs a) {
+  if (a.P.cnt->flag_fallback) return;  // no stops yet (k_descend)
   uint32_t i = grid_tid();
   uint32_t m = a.scal[SC_M_UNIQ];
   if (i >= m) return;
@@ -845,6 +878,7 @@ __device__ bool key_before_block(const NuArgs &a, uint32_t j, uint32_t trie, con
 }
 
 __global__ __launch_bounds__(256) void k_group_merge(NuArgs a) {
+  if (a.P.cnt->flag_fallback) return;  // no stops yet (k_descend)
   uint32_t i = grid_tid();
   uint32_t m = a.scal[SC_M_UNIQ];
   if (i >= m) return;

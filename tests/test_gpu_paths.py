@@ -1,0 +1,51 @@
+"""Edges of the kernels' size and shape rules, bit for bit against the CPU oracle."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+PUTS = {"2phase": "puts_2phase_with_valuehp", "latching": "puts_latching_with_valuehp_v2"}
+
+
+def _put(t, b, mode="2phase"):
+    targets, n = getattr(t, PUTS[mode])(b)
+    t.hash_onepass_v2(targets, n)
+    return t.get_root_hash()
+
+
+def _after(oracle, batches):
+    o = oracle.OracleMPT()
+    for b in batches:
+        o.puts(b)
+        o.hash()
+    return o.root()
+
+
+@pytest.mark.parametrize("mode", list(PUTS))
+@pytest.mark.parametrize("first", [0, 1, 5])
+def test_keys_leaving_a_long_leaf_at_every_nibble(gmpt, workloads, oracle, mode, first):
+    # a key matched 16 nibbles per word: one key, then keys that differ from it
+    # at each nibble (word edges 15, 16, 17, 31, 32, ... among them), its own
+    # update, and reads of present, absent and invalid keys
+    rng = np.random.default_rng(40 + first)
+    base = [int(x) for x in rng.integers(0, 16, 64)]
+    hexes = [bytes(base[:first] + base[first:] + [16])]
+    one = workloads.batch_from_hex(hexes, [b"first value of the shared leaf"])
+    others = []
+    for d in range(first, 64):
+        k = list(base)
+        k[d] = (k[d] + 1 + d % 3) % 16
+        others.append(bytes(k + [16]))
+    others.append(hexes[0])
+    more = workloads.batch_from_hex(others, [b"v%d" % i * (1 + i % 40) for i in range(len(others))])
+    t = gmpt.MPT(device=0)
+    _put(t, one, mode)
+    assert _put(t, more, mode) == _after(oracle, [one, more])
+    # a second batch of updates along the same path
+    upd = workloads.batch_from_hex(others[::3], [b"w%d" % i * 9 for i in range(len(others[::3]))])
+    assert _put(t, upd, mode) == _after(oracle, [one, more, upd])
+    assert t.get_values(more)[1] == more.value(1)
+    bad = [bytes(base[:20] + [0x10 | base[20]] + base[21:] + [16]), bytes(base[:40] + [16]), bytes(base + [3]),
+           bytes(base[:63] + [17, 16]), bytes(base[:15] + [0xF0 | base[15]] + base[16:] + [16])]
+    assert t.get_values(workloads.batch_from_hex(bad, [b""] * len(bad))) == [None] * len(bad)
+    assert t.get_values(upd) == [upd.value(i) for i in range(upd.n)]
