@@ -167,6 +167,9 @@ class Forest {
   int carve_nu(NuArgs &a, const BatchDesc &d, uint64_t vbase, bool has_tid, void **temp);
   int sort_unique(NuArgs &a, uint32_t trie_bits, void *temp, int pass, int *cur);
   int next_pass(int pass);
+  void finish_build(const NuArgs &a);
+  int merge_sorted(NuArgs &a, void *temp);
+  bool bulk_fits(const BatchDesc &b) const;
   uint8_t *value_space(uint64_t bytes);
 
   int device_ = 0;

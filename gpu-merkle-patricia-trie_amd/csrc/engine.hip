@@ -560,6 +560,43 @@ int Forest::next_pass(int pass) {
   return 1;
 }
 
+// After a build's closing counter read: the key arena's new end, and the new
+// nodes' hashing records.
+void Forest::finish_build(const NuArgs &a) {
+  // the batch's packed keys stay only if a new node refers to them: a batch
+  // of updates alone (no elements) leaves them unused, so the arena keeps
+  // its place (keys of repeated updates do not accumulate)
+  if (cnt_.scal[SC_NE] != 0) {
+    key_used_ += *(const uint64_t *)(cnt_.scal + SC_KTOT);
+    key_used_ = align_up(key_used_, 8);
+  }
+  // the new leaves' hashing bins, valid until the next change to the trie
+  rec_.pk = a.leaf_pk;
+  rec_.meta = a.leaf_meta;
+  rec_.lo = cnt_.scal[SC_DBASE];
+  rec_.n = cnt_.scal[SC_NE];
+  rec_.bdesc = a.bdesc;
+  rec_.blo = rec_.lo + rec_.n;
+  rec_.bn = cnt_.scal[SC_NREP_TOT];
+}
+
+// After the descent's counter read: the rest of an insert into tries that
+// are not empty.
+int Forest::merge_sorted(NuArgs &a, void *temp) {
+  int r;
+  if (cnt_.scal[SC_MERGE]) {
+    // a split group straddles a subtree: make every group contiguous
+    uint32_t m = cnt_.scal[SC_M_UNIQ];
+    HIP_TRY(nu_regroup(a, m, m, temp, stream_));
+    stats_.regroups++;
+  }
+  HIP_TRY(nu_emit(a, temp, stream_, false));
+  HIP_TRY(nu_build(a, temp, stream_, false));
+  if ((r = sync_counters())) return r;
+  finish_build(a);
+  return 0;
+}
+
 int Forest::puts_2phase(const BatchDesc &b, void **targets, int *n_targets) {
   int r;
   if ((r = set_device())) return r;
@@ -585,11 +622,14 @@ int Forest::puts_2phase(const BatchDesc &b, void **targets, int *n_targets) {
       HIP_TRY(hipStreamWaitEvent(side_.stream, side_.fork, 0));
     }
     const uint32_t n = b.n;
-    // slots: branches <= 2n+2, shorts <= 2(2n+2), values: 2n+2 for elements + n for updates
-    if ((r = ensure_pools(2ull * n + 2, 4ull * n + 4, 3ull * n + 2, d.key_slots))) return r;
     const bool has_tid = d.trie_ids != nullptr && ntries_ > 1;
     // a bulk build into a forest of empty tries skips the descent and grouping
     const bool empty = all_empty_;
+    // Elements are the unique keys, plus one per split short node (none in an
+    // empty trie); per element at most one branch, two shorts and one value.
+    if ((r = empty ? ensure_pools(n, 2ull * n, n, d.key_slots)
+                   : ensure_pools(2ull * n + 2, 4ull * n + 4, 2ull * n + 2, d.key_slots)))
+      return r;
     all_empty_ = false;
     NuArgs a;
     void *temp = nullptr;
@@ -633,32 +673,10 @@ int Forest::puts_2phase(const BatchDesc &b, void **targets, int *n_targets) {
       if (r == 0) break;
       if (run > 0 || !grow_key_arena_after_error()) return r;
     }
-    if (!empty) {
-      if (cnt_.scal[SC_MERGE]) {
-        // a split group straddles a subtree: make every group contiguous
-        uint32_t m = cnt_.scal[SC_M_UNIQ];
-        HIP_TRY(nu_regroup(a, m, m, temp, stream_));
-        stats_.regroups++;
-      }
-      HIP_TRY(nu_emit(a, temp, stream_, false));
-      HIP_TRY(nu_build(a, temp, stream_, false));
-      if ((r = sync_counters())) return r;
-    }
-    // the batch's packed keys stay only if a new node refers to them: a batch
-    // of updates alone (no elements) leaves them unused, so the arena keeps
-    // its place (keys of repeated updates do not accumulate)
-    if (cnt_.scal[SC_NE] != 0) {
-      key_used_ += *(const uint64_t *)(cnt_.scal + SC_KTOT);
-      key_used_ = align_up(key_used_, 8);
-    }
-    // the new leaves' hashing bins, valid until the next change to the trie
-    rec_.pk = a.leaf_pk;
-    rec_.meta = a.leaf_meta;
-    rec_.lo = cnt_.scal[SC_DBASE];
-    rec_.n = cnt_.scal[SC_NE];
-    rec_.bdesc = a.bdesc;
-    rec_.blo = rec_.lo + rec_.n;
-    rec_.bn = cnt_.scal[SC_NREP_TOT];
+    if (empty)
+      finish_build(a);
+    else if ((r = merge_sorted(a, temp)))
+      return r;
   }
   if (targets) *targets = dirty_.p;
   if (n_targets) *n_targets = (int)cnt_.n_dirty;
@@ -1125,10 +1143,50 @@ int Forest::export_nodes(const BatchDesc &keys, uint8_t **hashes, uint8_t **encs
   return export_paths(this, d, hashes, encs, enc_indexs, num);
 }
 
+// Whether a bulk build of the batch and its hash pass are sure to fit what is
+// left of a fixed region: a bound for each array both take, the batch itself
+// included.
+bool Forest::bulk_fits(const BatchDesc &b) const {
+  const uint64_t n = b.n;
+  uint64_t kb = b.keys_bytes, vb = b.values_total, keys;
+  if (b.on_device) {
+    // packed keys: at first from the key buffer's size, then (pairs that overlap) the real total
+    keys = kb / 2 + 8 * n + n * (kMaxKeyNibbles / 2 + 9);
+  } else {
+    keys = 0;
+    for (uint64_t i = 0; i < n; i++) {
+      const int64_t s = b.keys_indexs[2 * i], e = b.keys_indexs[2 * i + 1];
+      kb = std::max<int64_t>(kb, e + 1);
+      vb = std::max<int64_t>(vb, b.values_indexs[2 * i + 1] + 1);
+      keys += s >= 0 && e >= s ? std::min<int64_t>(e - s + 1, kMaxKeyNibbles) / 2 + 8 : 8;
+    }
+  }
+  const uint64_t staged = b.on_device ? (b.adopt_values ? 0 : vb) : kb + 32 * n + vb;
+  const uint64_t pools = n * (sizeof(Branch) + 2 * sizeof(Short) + sizeof(Value) + 16);
+  const uint64_t dirty = 3 * n;  // elements, branches and extension entries
+  const uint64_t hash = dirty * 48 + hc_temp_bytes((uint32_t)dirty) + 64 * kHcBins;
+  // Messages, in 136-byte blocks: branches of k children take at most
+  // 1.2 + k / 4, their children are at most 2n in all; an extension takes at
+  // most 2; a long leaf 2 and its value, which a branch's slot 16 may hold
+  // instead.
+  const uint64_t scratch = 136 * (2 * n + 2 * n + 2 * n) + vb;
+  return arena_->used + staged + keys + pools + nu_ws_bytes(n, b.trie_ids != nullptr) + hash + scratch + (1u << 20) <=
+         arena_->cap;
+}
+
 // LockNU.  Writes of the same key are combined first (the batch is sorted
 // and only each key's last write is kept, which is the final state the
 // sequential order gives), then the surviving writes insert concurrently with
 // optimistic lock coupling.
+// Latches pay while the writes spread over the trie.  Into a trie with fewer
+// keys than the batch, many lanes want the same few latches and restart (a
+// failed try is repeated from the root): insert + hash of 100,000 uniform
+// keys took 18.9 ms into an empty trie, 1,071 us onto 2,000 keys, 821 onto
+// 20,000 and 630 onto 200,000; PhaseNU's sorted build, which needs no
+// latches, takes 0.3 ms, 585, 605 and 647 us.  So a batch of more distinct
+// keys than the trie holds is built by position instead; the tries that
+// result are the same.  The forest's value slots count its keys; of a
+// multi-trie forest the average trie's share is taken.
 int Forest::puts_latching(const BatchDesc &b, void **targets, int *n_targets) {
   int r;
   if ((r = set_device())) return r;
@@ -1140,6 +1198,9 @@ int Forest::puts_latching(const BatchDesc &b, void **targets, int *n_targets) {
     set_error("device batch needs keys_bytes and values_total");
     return -3;
   }
+  stats_.restarts = 0;
+  stats_.lock_fails = 0;
+  if (all_empty_ && (!arena_ || bulk_fits(b))) return puts_2phase(b, targets, n_targets);
   stats_.fallback_sorts = 0;
   stats_.regroups = 0;
   if (b.n > 0) {
@@ -1147,6 +1208,7 @@ int Forest::puts_latching(const BatchDesc &b, void **targets, int *n_targets) {
     uint64_t vbase = 0;
     if ((r = stage_batch(b, &d, &vbase, true))) return r;
     const uint32_t n = b.n;
+    const bool was_empty = all_empty_;
     all_empty_ = false;
     if ((r = ensure_pools(n, 2ull * n, n, d.key_slots))) return r;
     const bool has_tid = d.trie_ids != nullptr && ntries_ > 1;
@@ -1159,7 +1221,6 @@ int Forest::puts_latching(const BatchDesc &b, void **targets, int *n_targets) {
     for (int run = 0;; run++) {
       if ((r = carve_nu(a, d, vbase, has_tid, &temp))) return r;
       a.seq_base = lock_seq_;
-      a.skref = nullptr;  // the latched insert reads keys through kref only
       HIP_TRY(hipMemsetAsync(&d_cnt_->n_restarts, 0, 8, stream_));
       HIP_TRY(nu_prepare_keys(a, temp, stream_));
       int cur = 0;
@@ -1172,6 +1233,18 @@ int Forest::puts_latching(const BatchDesc &b, void **targets, int *n_targets) {
       if (r == 0) break;
       if (run > 0 || !grow_key_arena_after_error()) return r;
     }
+    lock_seq_ += n;
+    const uint32_t m = cnt_.scal[SC_M_UNIQ];
+    if (!was_empty && m > cnt_.n_value / ntries_) {
+      if ((r = ensure_pools(2ull * m + 2, 4ull * m + 4, 2ull * m + 2, d.key_slots))) return r;
+      a.P = pools();
+      HIP_TRY(nu_descend_and_group(a, temp, stream_));
+      if ((r = sync_counters())) return r;
+      if ((r = merge_sorted(a, temp))) return r;
+      if (targets) *targets = dirty_.p;
+      if (n_targets) *n_targets = (int)cnt_.n_dirty;
+      return 0;
+    }
     const uint64_t ktot = *(const uint64_t *)(cnt_.scal + SC_KTOT);
     const uint32_t values_before = cnt_.n_value;
     HIP_TRY(lock_insert(a, key_used_ + ktot, temp, stream_));
@@ -1179,7 +1252,6 @@ int Forest::puts_latching(const BatchDesc &b, void **targets, int *n_targets) {
     // only new keys' nodes refer to the batch's packed keys: a batch that
     // only overwrites leaves the arena where it was
     if (cnt_.n_value != values_before) key_used_ = align_up(key_used_ + ktot, 8);
-    lock_seq_ += n;
     stats_.restarts = cnt_.n_restarts;
     stats_.lock_fails = cnt_.n_lock_fail;
   }

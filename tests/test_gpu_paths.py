@@ -49,3 +49,44 @@ def test_keys_leaving_a_long_leaf_at_every_nibble(gmpt, workloads, oracle, mode,
            bytes(base[:63] + [17, 16]), bytes(base[:15] + [0xF0 | base[15]] + base[16:] + [16])]
     assert t.get_values(workloads.batch_from_hex(bad, [b""] * len(bad))) == [None] * len(bad)
     assert t.get_values(upd) == [upd.value(i) for i in range(upd.n)]
+
+
+@pytest.mark.parametrize("tries", [1, 3])
+@pytest.mark.parametrize("share", [0.5, 0.3, 0.05])
+def test_latched_insert_by_the_tries_size(gmpt, workloads, oracle, tries, share):
+    # the latched insert runs while the batch has no more keys than the trie
+    # (share 0.5: both about equal, the line; below: latched); a batch into
+    # empty tries is built by position.  Clustered keys split fresh nodes.
+    rng = np.random.default_rng(int(100 * share) + tries)
+    keys = []
+    for _ in range(250):
+        base = rng.integers(0, 256, 32, dtype=np.uint8)
+        for _ in range(int(rng.integers(2, 30))):
+            k = base.copy()
+            k[int(rng.integers(1, 32)):] = rng.integers(0, 256, 1, dtype=np.uint8)
+            keys.append(k)
+    keys = np.unique(np.array(keys), axis=0)
+    keys = keys[rng.permutation(len(keys))]
+    cut = int(len(keys) * (1 - share))
+    f = gmpt.MPT(device=0, num_tries=tries)
+    os_ = [oracle.OracleMPT() for _ in range(tries)]
+    for part in (keys[:cut], np.concatenate([keys[cut:], keys[:len(keys) // 20]])):
+        flat, lens = workloads.random_values(rng, len(part), 1, 120)
+        b = workloads.batch_from_fixed(part, flat, lens)
+        b.trie_ids = np.sort(rng.integers(0, tries, len(part))).astype(np.int32)
+        _put(f, b, "latching")
+        for t in range(tries):
+            os_[t].puts(b.subset(np.flatnonzero(b.trie_ids == t)))
+            os_[t].hash()
+        assert f.get_root_hashes() == [o.root() for o in os_]
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("n,vlen", [(1, 40), (3000, 40), (32768, 40), (32768, 1000)])
+def test_root_without_allocation_near_its_region(gmpt, workloads, oracle, mode, n, vlen):
+    # the largest batch and, at 1,000-byte values, one whose bound is past the
+    # region (the latched insert keeps it)
+    rng = np.random.default_rng(n + vlen)
+    b = workloads.batch_from_fixed(rng.integers(0, 256, (n, 8), dtype=np.uint8),
+                                   rng.integers(0, 256, n * vlen, dtype=np.uint8), np.full(n, vlen))
+    assert gmpt.build_root_noalloc(b, mode) == oracle.root_of(b)
