@@ -165,7 +165,7 @@ class Forest {
   // the caller stages them later, before anything reads value bytes.
   int stage_batch(const BatchDesc &b, BatchDesc *dev, uint64_t *vbase, bool copy_values, StageSeg *defer = nullptr);
   int carve_nu(NuArgs &a, const BatchDesc &d, uint64_t vbase, bool has_tid, void **temp);
-  int sort_unique(NuArgs &a, uint32_t trie_bits, void *temp, int pass, int *cur);
+  int sort_unique(NuArgs &a, void *temp, int pass, int *cur);
   int next_pass(int pass);
   void finish_build(const NuArgs &a);
   int merge_sorted(NuArgs &a, void *temp);

@@ -433,6 +433,8 @@ int Forest::carve_nu(NuArgs &a, const BatchDesc &d, uint64_t vbase, bool has_tid
   a.vidx = d.values_indexs;
   a.hps = d.values_hps;
   a.tid = has_tid ? d.trie_ids : nullptr;
+  if (has_tid)
+    while ((1ull << a.tbits) < ntries_) a.tbits++;
   a.n = n;
   a.ntries = ntries_;
   a.kh_bytes = d.keys_bytes;
@@ -515,7 +517,7 @@ int Forest::carve_nu(NuArgs &a, const BatchDesc &d, uint64_t vbase, bool has_tid
 // Passes 0 and 2 need no host synchronisation: the caller reads
 // flag_fallback at its next one and, if a flag is set, runs next_pass() and
 // repeats the work that followed.
-int Forest::sort_unique(NuArgs &a, uint32_t trie_bits, void *temp, int pass, int *cur) {
+int Forest::sort_unique(NuArgs &a, void *temp, int pass, int *cur) {
   uint64_t *sk = nullptr;
   uint32_t *sv = nullptr;
   int nwords = 0;
@@ -536,10 +538,10 @@ int Forest::sort_unique(NuArgs &a, uint32_t trie_bits, void *temp, int pass, int
     const int pop = __builtin_popcountll(m);
     if (pop >= 1 && pop <= 56) vmask = m;  // saves at least one 8-bit digit
   }
-  HIP_TRY(nu_sort(a, nwords, trie_bits, temp, stream_, &sk, &sv, pass == 1, cur, vmask, &sk_mask));
+  HIP_TRY(nu_sort(a, nwords, a.tbits, temp, stream_, &sk, &sv, pass == 1, cur, vmask, &sk_mask));
   // the sorted keys are the plain windows unless the whole keys were sorted
   // or the windows were compressed to their varying bits
-  a.u_win_ok = pass != 2 && sk_mask == 0;
+  a.u_win_nibs = pass != 2 && sk_mask == 0 ? (64 - a.tbits) / 4 : 0u;
   if (pass > 0) HIP_TRY(nu_reset_dup(a, stream_));
   HIP_TRY(nu_adjacent(a, sk, sv, pass == 2 ? 1 : 0, stream_, sk_mask));
   HIP_TRY(nu_unique(a, sk, sv, temp, stream_));
@@ -633,17 +635,13 @@ int Forest::puts_2phase(const BatchDesc &b, void **targets, int *n_targets) {
     all_empty_ = false;
     NuArgs a;
     void *temp = nullptr;
-    uint32_t trie_bits = 0;
-    if (has_tid) {
-      while ((1ull << trie_bits) < ntries_) trie_bits++;
-    }
     for (int run = 0;; run++) {
       if ((r = carve_nu(a, d, vbase, has_tid, &temp))) return r;
       a.e_ident = empty && !has_tid ? 1u : 0u;
       HIP_TRY(nu_prepare_keys(a, temp, stream_));
       int cur = 0;
       for (int pass = 0; pass >= 0;) {
-        if ((r = sort_unique(a, trie_bits, temp, pass, &cur))) break;
+        if ((r = sort_unique(a, temp, pass, &cur))) break;
         HIP_TRY(nu_descend_and_group(a, temp, stream_, empty));
         if (empty) {
           // into empty tries no group needs merging: the build follows at
@@ -1214,10 +1212,6 @@ int Forest::puts_latching(const BatchDesc &b, void **targets, int *n_targets) {
     const bool has_tid = d.trie_ids != nullptr && ntries_ > 1;
     NuArgs a;
     void *temp = nullptr;
-    uint32_t trie_bits = 0;
-    if (has_tid) {
-      while ((1ull << trie_bits) < ntries_) trie_bits++;
-    }
     for (int run = 0;; run++) {
       if ((r = carve_nu(a, d, vbase, has_tid, &temp))) return r;
       a.seq_base = lock_seq_;
@@ -1225,7 +1219,7 @@ int Forest::puts_latching(const BatchDesc &b, void **targets, int *n_targets) {
       HIP_TRY(nu_prepare_keys(a, temp, stream_));
       int cur = 0;
       for (int pass = 0; pass >= 0;) {
-        if ((r = sort_unique(a, trie_bits, temp, pass, &cur))) break;
+        if ((r = sort_unique(a, temp, pass, &cur))) break;
         if ((r = sync_counters())) break;
         pass = next_pass(pass);
         if (pass >= 0) HIP_TRY(hipMemsetAsync(&d_cnt_->flag_fallback, 0, 4, stream_));

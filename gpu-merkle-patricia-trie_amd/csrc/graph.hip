@@ -74,9 +74,6 @@ int Forest::capture_rebuild(const BatchDesc &b) {
   uint64_t vbase = 0;
   if ((r = stage_batch(b, &d, &vbase, true))) return r;
   const bool has_tid = d.trie_ids != nullptr && ntries_ > 1;
-  uint32_t trie_bits = 0;
-  if (has_tid)
-    while ((1ull << trie_bits) < ntries_) trie_bits++;
   GRAPH_TRY(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
   hipGraph_t g = nullptr;
   auto fail = [&](int code) {
@@ -96,9 +93,9 @@ int Forest::capture_rebuild(const BatchDesc &b) {
   uint64_t sk_mask = 0;
   int cur = 0;
   if ((e = nu_prepare_keys(a, temp, stream_)) != hipSuccess ||
-      (e = nu_sort(a, 0, trie_bits, temp, stream_, &sk, &sv, false, &cur, 0, &sk_mask)) != hipSuccess)
+      (e = nu_sort(a, 0, a.tbits, temp, stream_, &sk, &sv, false, &cur, 0, &sk_mask)) != hipSuccess)
     return fail(-1);
-  a.u_win_ok = sk_mask == 0;
+  a.u_win_nibs = sk_mask == 0 ? (64 - a.tbits) / 4 : 0u;
   if ((e = nu_adjacent(a, sk, sv, 0, stream_, sk_mask)) != hipSuccess ||
       (e = nu_unique(a, sk, sv, temp, stream_)) != hipSuccess ||
       (e = nu_descend_and_group(a, temp, stream_, true)) != hipSuccess ||

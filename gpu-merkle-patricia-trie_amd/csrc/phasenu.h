@@ -76,11 +76,11 @@ struct NuArgs {
   uint32_t *merge;       // per run: run whose group it joins (split groups around a subtree)
   uint32_t *u_idx2, *u_trie2, *perm0, *perm1, *gkey0, *gkey1;
   // each unique key's kref and sort window, gathered in unique order so the
-  // build reads them in sequence (u_win holds the 16 nibbles from W only when
-  // u_win_ok: the last sort's keys were the plain windows)
+  // build reads them in sequence (u_win holds u_win_nibs nibbles from W)
   uint64_t *skref;       // per sorted position: kref of that key (null: not gathered)
   uint64_t *u_kref, *u_kref2, *u_win, *u_win2;
-  uint32_t u_win_ok;
+  uint32_t u_win_nibs;   // nibbles from W that u_win holds, from the top (0: u_win is not written)
+  uint32_t tbits;        // multi-trie batches: the sort key is the trie id (tbits bits) above the window's top bits
   uint8_t *u_lcp2;
   Stop *stop2;
   // E elements (M <= 2m)
@@ -137,8 +137,10 @@ enum {
 hipError_t nu_init_scalars(const NuArgs &a, hipStream_t s);
 hipError_t nu_prepare_keys(const NuArgs &a, void *temp, hipStream_t s);
 // Sorts the batch: by the 16-nibble windows (full = 0; first by their top bits
-// with a fix-up of equal runs, or by all 64 bits when win_all_bits) or by the
-// whole keys (full = number of 16-nibble words), then by trie.  *cur_io (if
+// with a fix-up of equal runs, or by all 64 bits when win_all_bits), which for
+// a multi-trie batch hold the trie id above the window's leading bits
+// (a.tbits), or by the whole keys (full = number of 16-nibble words), then by
+// trie.  *cur_io (if
 // given) is the ping-pong buffer holding the current order, in and out.
 // With win_all_bits and a mask of the window bits that vary across the batch
 // (vmask, from nu_window_mask), the windows are first compressed to those

@@ -14,6 +14,9 @@
 //      split joins its group as one more element ("virtual" element)
 // The result is the same trie the sequential insert produces.
 #include <limits.h>
+
+#include <algorithm>
+
 #include "hc_leaf.h"
 #include "phasenu.h"
 #include "prims.h"
@@ -202,6 +205,15 @@ struct KeyChunks {
   }
 };
 
+// The first sort's key: the window, or, in a multi-trie batch, the trie id
+// above the window's leading bits, so that one sort orders by (trie, path).
+// (A sort by window, then a stable one by trie, then a gather of the windows
+// in the new order took 2.3 ms for 8 M keys of 4,096 tries, 1.5 of them the
+// gather's random reads; the one sort takes 0.5.)
+__device__ __forceinline__ uint64_t sort_key(const NuArgs &a, uint32_t i, uint64_t win) {
+  return a.tbits ? (uint64_t)(uint32_t)a.tid[i] << (64 - a.tbits) | win >> a.tbits : win;
+}
+
 // Validates every key, and reduces per block the common prefix with key 0
 // and the longest key (no global atomics: one slot per block).  A key as long
 // as key 0 is also packed at once to slot i of a layout with equal slots: when
@@ -253,7 +265,7 @@ __global__ __launch_bounds__(256) void k_keys_scan(NuArgs a, uint32_t *blk_w, ui
           // the sort window of a batch with no common prefix (W = 0), as
           // k_keys_pack builds it from the slot: that pass skips such a batch
           if (a.sk0) {
-            a.sk0[i] = __builtin_bswap64(first);
+            a.sk0[i] = sort_key(a, i, __builtin_bswap64(first));
             a.sv0[i] = i;
           }
         }
@@ -405,7 +417,7 @@ __global__ __launch_bounds__(256) void k_keys_pack(NuArgs a) {
     const uint32_t q = W / 16, d = W % 16;
     const uint64_t hi = __builtin_bswap64(src[q]);
     const uint64_t lo = (q + 1) * 8 < slot ? __builtin_bswap64(src[q + 1]) : 0ull;
-    a.sk0[i] = d ? (hi << (4 * d)) | (lo >> (64 - 4 * d)) : hi;
+    a.sk0[i] = sort_key(a, i, d ? (hi << (4 * d)) | (lo >> (64 - 4 * d)) : hi);
     a.sv0[i] = i;
     return;
   }
@@ -427,7 +439,7 @@ __global__ __launch_bounds__(256) void k_keys_pack(NuArgs a) {
   if (a.kbase + *(const uint64_t *)(a.scal + SC_KTOT) > a.key_cap) {
     a.kref[i] = 1ull << 48;
     if (a.sk0) {
-      a.sk0[i] = 0;
+      a.sk0[i] = sort_key(a, i, 0);
       a.sv0[i] = i;
     }
     if (i == 0) raise_error(a.P.cnt, ERR_POOL, kErrArgKeyArena);
@@ -442,7 +454,7 @@ __global__ __launch_bounds__(256) void k_keys_pack(NuArgs a) {
   uint32_t W = a.scal[SC_W];
   uint64_t h0 = W < nn ? ldn(k + W, min(8u, nn - W)) : 0ull;
   uint64_t h1 = W + 8 < nn ? ldn(k + W + 8, min(8u, nn - W - 8)) : 0ull;
-  a.sk0[i] = ((uint64_t)__builtin_bswap32(pack8(h0)) << 32) | __builtin_bswap32(pack8(h1));
+  a.sk0[i] = sort_key(a, i, ((uint64_t)__builtin_bswap32(pack8(h0)) << 32) | __builtin_bswap32(pack8(h1)));
   a.sv0[i] = i;
 }
 
@@ -451,22 +463,13 @@ __global__ __launch_bounds__(256) void k_keys_pack(NuArgs a) {
 __global__ __launch_bounds__(256) void k_gather_word(NuArgs a, const uint32_t *sv, uint64_t *sk, int w) {
   uint32_t j = grid_tid();
   if (j >= a.n) return;
-  uint32_t i = sv[j];
-  uint32_t L = a.klen[i];
+  const KeyRef k = key_of(a, sv[j]);
   if (w < 0) {
-    sk[j] = L;
+    sk[j] = k.len;
     return;
   }
-  const uint8_t *k = a.kh + (key_range_ok(a, i) ? a.kidx[2 * i] : 0);
-  uint32_t nn = L - 1;
-  uint32_t W = a.scal[SC_W] + 16u * (uint32_t)w;
-  uint64_t win = 0;
-  for (int q = 0; q < 16; q++) {
-    uint32_t jj = W + q;
-    uint64_t v = jj < nn ? (uint64_t)k[jj] : 0ull;
-    win |= v << (60 - 4 * q);
-  }
-  sk[j] = win;
+  const uint32_t at = a.scal[SC_W] + 16u * (uint32_t)w;
+  sk[j] = at + 1 < k.len ? nib_word(k.p, at, k.len - 1) : 0ull;  // the slot is zero past the key's nibbles
 }
 
 __global__ __launch_bounds__(256) void k_gather_trie(NuArgs a, const uint32_t *sv, uint32_t *tk) {
@@ -569,6 +572,7 @@ __global__ __launch_bounds__(256) void k_adjacent(NuArgs a, const uint64_t *sk, 
       bool ident;
       uint64_t x = full ? 0ull : (sk[j - 1] ^ sk[j]);
       if (x != 0 && cmask != 0) x = scatter_bits(x >> (64 - __popcll(cmask)), cmask);
+      x <<= a.tbits;  // one trie: the keys' trie bits agree
       if (x != 0) {
         p = W + (uint32_t)(__clzll((long long)x) >> 2);
         if (ka.len != kb.len) p = min(p, mn - 1);
@@ -577,7 +581,7 @@ __global__ __launch_bounds__(256) void k_adjacent(NuArgs a, const uint64_t *sk, 
         // windows agree (or full mode): compare nibble by nibble; with
         // different lengths the shorter key's terminator (0 in the window)
         // differs from the longer key's nibble at mn - 1
-        p = full ? 0u : min(W + 16u, mn);
+        p = full ? 0u : min(W + (64u - a.tbits) / 4u, mn);
         if (ka.len != kb.len) p = min(p, mn - 1);
         while (p < mn && ka.nib(p) == kb.nib(p)) p++;
         ident = (p == mn) && ka.len == kb.len;
@@ -597,7 +601,7 @@ __global__ __launch_bounds__(256) void k_adjacent(NuArgs a, const uint64_t *sk, 
   a.u_idx[j] = ib;
   if (a.skref) {
     a.u_kref[j] = rb;
-    if (a.u_win_ok) a.u_win[j] = sk[j];
+    if (a.u_win_nibs) a.u_win[j] = sk[j] << a.tbits;
   }
   if (fl & 1) atomicOr(&a.scal[SC_DUP], 1u);
   }
@@ -637,7 +641,7 @@ __global__ __launch_bounds__(256) void k_unique(NuArgs a, const uint64_t *sk, co
     a.u_idx[r] = sv[j];
     if (a.skref) {
       a.u_kref[r] = a.skref[j];
-      if (a.u_win_ok) a.u_win[r] = sk[j];
+      if (a.u_win_nibs) a.u_win[r] = sk[j] << a.tbits;
     }
   }
   if (j + 1 == a.n) a.scal[SC_M_UNIQ] = r + 1;
@@ -1030,7 +1034,7 @@ __global__ __launch_bounds__(256) void k_permute(NuArgs a, const uint32_t *perm,
   uint32_t p = perm[i];
   a.u_idx2[i] = a.u_idx[p];
   a.u_kref2[i] = a.u_kref[p];
-  if (a.u_win_ok) a.u_win2[i] = a.u_win[p];
+  if (a.u_win_nibs) a.u_win2[i] = a.u_win[p];
   a.u_trie2[i] = a.u_trie[p];
   a.u_lcp2[i] = a.u_lcp[p];
   a.stop2[i] = a.stop[p];
@@ -1420,7 +1424,7 @@ struct ElemKey {
   uint32_t end;       // absolute end of the element's path (exclusive)
   uint8_t term;       // path ends with the terminator
   bool virt;
-  bool has_win;       // win holds nibbles W .. W + 15 of the key
+  uint32_t win_nibs;  // win holds this many nibbles of the key from nibble W
   uint32_t uidx;      // unique index (new key) or short node idx (virtual)
   uint64_t win;
 };
@@ -1436,7 +1440,7 @@ __device__ __forceinline__ ElemKey elem_key(const NuArgs &a, uint32_t e) {
     k.end = S.depth + S.key_len;
     k.term = S.term;
     k.virt = true;
-    k.has_win = false;
+    k.win_nibs = 0;
     k.win = 0;
     k.uidx = src & 0x7fffffffu;
   } else {
@@ -1447,19 +1451,19 @@ __device__ __forceinline__ ElemKey elem_key(const NuArgs &a, uint32_t e) {
     k.end = (uint32_t)(r >> 48);
     k.term = 1;
     k.virt = false;
-    k.has_win = a.u_win_ok != 0;
-    k.win = k.has_win ? a.u_win[src] : 0ull;
+    k.win_nibs = a.u_win_nibs;
+    k.win = k.win_nibs ? a.u_win[src] : 0ull;
     k.uidx = src;
   }
   return k;
 }
 
 // Nibble j of the element's path; W is the batch's common prefix (the sort
-// window's first nibble): nibbles W .. W + 15 of a new key come from its
-// window when the window is at hand.
+// window's first nibble): the nibbles of a new key that its window holds come
+// from there.
 __device__ __forceinline__ uint32_t elem_nib(const Pools &P, const ElemKey &k, uint32_t j, uint32_t W) {
   if (k.term && j + 1 == k.end) return kNibbleT;
-  if (k.has_win && j >= W && j - W < 16) return (uint32_t)(k.win >> (60 - 4 * (j - W))) & 15u;
+  if (j >= W && j - W < k.win_nibs) return (uint32_t)(k.win >> (60 - 4 * (j - W))) & 15u;
   return packed_nibble(P.keys + k.off, k.start + (j - k.origin));
 }
 
@@ -1793,21 +1797,21 @@ hipError_t nu_prepare_keys(const NuArgs &a, void *temp, hipStream_t s) {
 
 namespace {
 
-// After a stable sort by the windows' top kTopBits bits: every run of equal
-// top bits is sorted by the whole window with a stable insertion sort by the
+// After a stable sort by the keys' top bits: every run of equal top bits is
+// sorted by the whole window with a stable insertion sort by the
 // thread at the run's start (runs of uniform keys hold one or two entries).
 // A run longer than kFixMaxRun sets bit 1 of flag_fallback: the host then
 // sorts by all 64 bits.
-constexpr int kTopBits = 24;
+constexpr int kTopBits = 24;  // a single trie's: runs of one or two up to tens of millions of uniform keys
 constexpr uint32_t kFixMaxRun = 64;
 
-__global__ __launch_bounds__(256) void k_fix_runs(NuArgs a, uint64_t *sk, uint32_t *sv) {
+__global__ __launch_bounds__(256) void k_fix_runs(NuArgs a, uint64_t *sk, uint32_t *sv, int top) {
   uint32_t j = grid_tid();
   if (j >= a.n) return;
-  const uint64_t top = sk[j] >> (64 - kTopBits);
-  if (j > 0 && (sk[j - 1] >> (64 - kTopBits)) == top) return;  // not a run start
+  const uint64_t lead = sk[j] >> (64 - top);
+  if (j > 0 && (sk[j - 1] >> (64 - top)) == lead) return;  // not a run start
   uint32_t L = 1;
-  while (j + L < a.n && L <= kFixMaxRun && (sk[j + L] >> (64 - kTopBits)) == top) L++;
+  while (j + L < a.n && L <= kFixMaxRun && (sk[j + L] >> (64 - top)) == lead) L++;
   if (L == 1) return;
   if (L > kFixMaxRun) {
     atomicOr(&a.P.cnt->flag_fallback, 2u);
@@ -1891,18 +1895,32 @@ hipError_t nu_sort(NuArgs &a, int full, uint32_t trie_bits, void *temp, hipStrea
   uint32_t *v[2] = {a.sv0, a.sv1};
   int cur = cur_io ? *cur_io : 0, which = 0;
   hipError_t e;
-  if (!full && !win_all_bits && a.n <= kBucketSortMaxN) {
-    // whole windows (ties by input position) in one pass plus a sort of each
+  // The bucket sort's 8 leading bits split a multi-trie batch by trie first;
+  // above one workgroup's capacity it runs when even a batch for a single
+  // trie would leave buckets that fit (its uniform keys fill 1 / 2^(8 -
+  // trie_bits) of them).
+  const bool buckets = a.n <= kBucketCap || (a.n <= kBucketSortMaxN && trie_bits < 8 &&
+                                             (a.n >> (8 - trie_bits)) <= kBucketSortMaxN / 256);
+  if (!full && !win_all_bits && buckets) {
+    // whole keys (ties by input position) in one pass plus a sort of each
     // top-8-bit bucket in LDS; a bucket too large for LDS asks for pass 1
     e = bucket_sort_u64(k[cur], v[cur], k[cur ^ 1], v[cur ^ 1], a.n, &which, temp, s, &a.P.cnt->flag_fallback);
     if (e != hipSuccess) return e;
     cur ^= which;
   } else if (!full && !win_all_bits) {
-    // top bits, then each run of equal top bits by the whole window
-    e = radix_sort_u64(k[cur], v[cur], k[cur ^ 1], v[cur ^ 1], a.n, 64 - kTopBits, 64, &which, temp, s);
+    // top bits, then each run of equal top bits by the whole key.  Above the
+    // trie id, enough window bits that a run holds 8 entries on average when
+    // one trie has the whole batch.
+    int top = kTopBits;
+    if (trie_bits) {
+      uint32_t lg = 0;
+      while ((1ull << lg) < a.n) lg++;
+      top = std::min(64, std::max(top, (int)((trie_bits + (lg > 3 ? lg - 3 : 0) + 7) & ~7u)));
+    }
+    e = radix_sort_u64(k[cur], v[cur], k[cur ^ 1], v[cur ^ 1], a.n, 64 - top, 64, &which, temp, s);
     if (e != hipSuccess) return e;
     cur ^= which;
-    k_fix_runs<<<nblk(a.n), kB, 0, s>>>(a, k[cur], v[cur]);
+    k_fix_runs<<<nblk(a.n), kB, 0, s>>>(a, k[cur], v[cur], top);
     GMPT_LAUNCH_CHECK();
   } else if (!full) {
     // compressed to the varying bits (all of them: no fix-up needed), or all 64
@@ -1927,26 +1945,19 @@ hipError_t nu_sort(NuArgs &a, int full, uint32_t trie_bits, void *temp, hipStrea
       cur ^= which;
     }
   }
-  if (trie_bits > 0) {
-    // stable sort of the current permutation by trie id, then regather the
-    // windows in the new order
+  if (full && trie_bits > 0) {
+    // stable sort of the current permutation by trie id
     uint32_t *t[2] = {a.tk0, a.tk1};
     k_gather_trie<<<nblk(a.n), kB, 0, s>>>(a, v[cur], t[0]);
     GMPT_LAUNCH_CHECK();
     e = radix_sort_u32(t[0], v[cur], t[1], v[cur ^ 1], a.n, 0, (int)((trie_bits + 7) & ~7u), &which, temp, s);
     if (e != hipSuccess) return e;
     if (which) cur ^= 1;
-    if (!full) {
-      k_gather_word<<<nblk(a.n), kB, 0, s>>>(a, v[cur], k[cur], 0);
-      GMPT_LAUNCH_CHECK();
-    }
   }
   *sk = k[cur];
   *sv = v[cur];
   if (cur_io) *cur_io = cur;
-  // the trie pass regathered raw windows
-  if (sk_mask) *sk_mask = (!full && win_all_bits && vmask && __builtin_popcountll(vmask) < 64 && trie_bits == 0)
-                              ? vmask : 0ull;
+  if (sk_mask) *sk_mask = !full && win_all_bits && vmask && __builtin_popcountll(vmask) < 64 ? vmask : 0ull;
   return hipSuccess;
 }
 

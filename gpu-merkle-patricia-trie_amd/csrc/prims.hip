@@ -318,16 +318,18 @@ hipError_t radix_impl(K *k0, uint32_t *v0, K *k1, uint32_t *v1, size_t n, int be
 // [goff[d * nblocks], goff[(d + 1) * nblocks]) of the pass's output (the
 // exclusive scan of the digit-major per-tile counts), or the whole array
 // without goff.  The bucket is counting-sorted in LDS by the next 12 key bits
-// (4,096 sub-buckets: about one entry each for a bucket of uniform keys),
-// then each sub-bucket's run is insertion-sorted by (key, value), which also
-// fixes the order the LDS atomics placed equal sub-buckets in.  A bucket
-// with a run longer than kSubMaxRun is left as it came and sets bit 1 of
-// *overflow.
+// (4,096 sub-buckets: about one entry each for a bucket of uniform keys);
+// then each entry counts the entries of its sub-bucket's run that are smaller
+// by (key, value), which is its place in the run.  A run's entries count side
+// by side, so a run of hundreds (keys of a few tries, or with a fixed field)
+// costs its length in LDS reads, where an insertion sort by one thread cost
+// its square.  A bucket with a run longer than kSubMaxRun is left as it came
+// and sets bit 1 of *overflow.
 constexpr int kBkThreads = 1024;
 constexpr uint32_t kBkPer = (uint32_t)(kBucketCap / kBkThreads);  // entries per thread
 constexpr uint32_t kSubs = 4096;
 constexpr uint32_t kSubPer = kSubs / kBkThreads;                    // sub-buckets per thread
-constexpr uint32_t kSubMaxRun = 64;
+constexpr uint32_t kSubMaxRun = 1024;
 static_assert(kBucketCap % kBkThreads == 0 && kSubs % kBkThreads == 0, "bucket tiling");
 
 __global__ __launch_bounds__(1024) void k_bucket_sort(uint64_t *__restrict__ keys, uint32_t *__restrict__ vals,
@@ -335,7 +337,7 @@ __global__ __launch_bounds__(1024) void k_bucket_sort(uint64_t *__restrict__ key
                                                       uint32_t nblocks, uint32_t *overflow) {
   __shared__ uint64_t sk[kBucketCap];
   __shared__ uint32_t sv[kBucketCap];
-  __shared__ uint32_t start[kSubs];
+  __shared__ uint32_t start[kSubs + 1];
   __shared__ uint32_t wsum[kBkThreads / 64];
   const uint32_t d = blockIdx.x;
   const uint32_t lo = goff ? goff[(size_t)d * nblocks] : 0u;
@@ -377,20 +379,19 @@ __global__ __launch_bounds__(1024) void k_bucket_sort(uint64_t *__restrict__ key
   __syncthreads();
   uint32_t base = 0;
   for (uint32_t w = 0; w < (t >> 6); w++) base += wsum[w];
-  uint32_t first[kSubPer];
   bool long_run = false;
   {
     uint32_t x = base + incl - sum;
 #pragma unroll
     for (uint32_t j = 0; j < kSubPer; j++) {
-      first[j] = x;
       start[kSubPer * t + j] = x;  // only this thread reads or writes these entries here
       x += cnt[j];
       long_run |= cnt[j] > kSubMaxRun;
     }
+    if (t + 1 == kBkThreads) start[kSubs] = x;
   }
-  // a run too long to insertion-sort: the bucket stays as it came (in the
-  // previous pass's stable order, which the caller's other sort relies on)
+  // a run too long to rank: the bucket stays as it came (in the previous
+  // pass's stable order, which the caller's other sort relies on)
   if (__syncthreads_or(long_run)) {
     if (t == 0) atomicOr(overflow, 2u);
     return;
@@ -406,20 +407,25 @@ __global__ __launch_bounds__(1024) void k_bucket_sort(uint64_t *__restrict__ key
   }
   __syncthreads();
 #pragma unroll
-  for (uint32_t j = 0; j < kSubPer; j++) {
-    if (cnt[j] < 2) continue;
-    const uint32_t f = first[j];
-    for (uint32_t q = 1; q < cnt[j]; q++) {
-      const uint64_t kk = sk[f + q];
-      const uint32_t vv = sv[f + q];
-      uint32_t p = q;
-      while (p > 0 && (sk[f + p - 1] > kk || (sk[f + p - 1] == kk && sv[f + p - 1] > vv))) {
-        sk[f + p] = sk[f + p - 1];
-        sv[f + p] = sv[f + p - 1];
-        p--;
+  for (uint32_t q = 0; q < kBkPer; q++) {
+    const uint32_t e = t + q * kBkThreads;
+    if (e < c) {
+      const uint32_t f = start[sub[q]], g = start[sub[q] + 1];
+      uint32_t less = 0;
+      for (uint32_t p = f; g - f > 1 && p < g; p++) {
+        const uint64_t kk = sk[p];
+        less += kk < k[q] || (kk == k[q] && sv[p] < v[q]) ? 1u : 0u;
       }
-      sk[f + p] = kk;
-      sv[f + p] = vv;
+      pos[q] = f + less;
+    }
+  }
+  __syncthreads();  // every run ranked
+#pragma unroll
+  for (uint32_t q = 0; q < kBkPer; q++) {
+    const uint32_t e = t + q * kBkThreads;
+    if (e < c) {
+      sk[pos[q]] = k[q];
+      sv[pos[q]] = v[q];
     }
   }
   __syncthreads();

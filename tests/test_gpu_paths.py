@@ -90,3 +90,27 @@ def test_root_without_allocation_near_its_region(gmpt, workloads, oracle, mode, 
     b = workloads.batch_from_fixed(rng.integers(0, 256, (n, 8), dtype=np.uint8),
                                    rng.integers(0, 256, n * vlen, dtype=np.uint8), np.full(n, vlen))
     assert gmpt.build_root_noalloc(b, mode) == oracle.root_of(b)
+
+
+@pytest.mark.parametrize("tries,per", [(2, 3000), (3, 4000), (130, 70), (130, 700), (257, 40), (5000, 3)])
+@pytest.mark.parametrize("shape", ["uniform", "tied", "one-trie"])
+def test_batches_ordered_by_trie_and_path(gmpt, workloads, oracle, tries, per, shape):
+    # one sort by the trie id above the window's leading bits: trie counts with
+    # 1 to 13 bits, batches of one workgroup and more, tries in random order,
+    # keys that tie in the window's kept nibbles, all keys in one trie
+    rng = np.random.default_rng(tries + per)
+    n = tries * per
+    keys = rng.integers(0, 256, (n, 12), dtype=np.uint8)
+    if shape == "tied":  # 4 bytes in common after the first, then a long tail in common
+        keys[:, 1:5] = 7
+        keys[:, 6:9] = rng.integers(0, 2, (n, 3), dtype=np.uint8)
+    tid = np.full(n, tries - 1, np.int32) if shape == "one-trie" else rng.integers(0, tries, n).astype(np.int32)
+    flat, lens = workloads.random_values(rng, n, 1, 60)
+    b = workloads.batch_from_fixed(keys, flat, lens)
+    b.trie_ids = tid
+    f = gmpt.MPT(device=0, num_tries=tries)
+    _put(f, b)
+    roots = f.get_root_hashes()
+    for t in sorted(set(tid[:: max(1, n // 12)].tolist())):
+        assert roots[t] == oracle.root_of(b.subset(np.flatnonzero(tid == t))), t
+    assert all(roots[t] == b"" for t in set(range(tries)) - set(tid.tolist()))
