@@ -160,7 +160,8 @@ def bench_phase(pkg, args):
     perms = st["perms"]
     hms = sum(hash_ms) / len(hash_ms)
     leaf_ms = sum(leaf_ms_l) / len(leaf_ms_l)
-    achieved = st["leaf_perms"] / (leaf_ms * 1e-3) / 1e9
+    # a short dirty list's leaves have no launch of their own to time
+    achieved = st["leaf_perms"] / (leaf_ms * 1e-3) / 1e9 if leaf_ms else 0.0
     # whole-path roofline: input bytes + node bytes over HBM, Keccak over VALU
     b_in = b.key_bytes + 8 * b.n + b.value_bytes + 16 * b.n + 8 * b.n
     b_nodes = st["enc_bytes"] + 32 * st["hashed_nodes"]

@@ -37,10 +37,10 @@ struct Branch {
   uint8_t hash_size;     // 32, or the raw encoding length (< 32)
   uint8_t pad0;
   uint16_t depth;        // nibble position this branch dispatches on
-  uint32_t dirty;        // 1 while the node waits for re-hashing
+  uint32_t dirty;        // not 0 while the node waits for re-hashing (a hash pass may keep its parent here)
   uint64_t lock;         // OLC version word: bit1 locked, bit0 obsolete, +4 per write
   ref_t child[17];       // slots 0..15 by nibble, 16 for a key ending here
-  uint32_t pad1;
+  uint32_t pad1;         // within a hash pass: dirty children still to be hashed
   uint8_t pad2[8];
 };
 static_assert(sizeof(Branch) == 128, "Branch layout");
@@ -98,6 +98,7 @@ struct Counters {
   unsigned long long leaf_perms; // PhaseHC: permutations of the leaf level
   unsigned long long leaf_bytes; // PhaseHC: encoding bytes of the leaf level
   uint32_t scal[20];             // the current insert's device scalars (PhaseNU / LockNU)
+  uint32_t hc_nodes, hc_leaves, hc_listed;  // PhaseHC climb: nodes and leaves hashed, nodes of the dirty list
   uint32_t root0_size;           // trie 0's root as the last hash pass left it (k_hc_roots), so that
   uint8_t root0[32];             // the pass's closing counter read also brings the root to the host
 };

@@ -147,6 +147,10 @@ class Forest {
   int grow(DevBuf &b, size_t need, size_t keep);
   int ensure_ws(DevBuf &b, size_t bytes);
   int arena_exhausted();
+  // hash()'s two forms: a short dirty list as one climb (*done: every node
+  // was hashed), any list by levels.
+  int hash_tree(uint32_t n, bool *done);
+  int hash_by_level(uint32_t n);
   int hash_levels(const Pools &P, const uint32_t *hist, bool direct_leaves, bool captured, uint32_t *n_leaf_out);
   // rebuild_graph's parts (graph.hip)
   int rebuild_eager(const BatchDesc &b);
@@ -190,6 +194,12 @@ class Forest {
   DevBuf st_keys_, st_kidx_, st_vidx_, st_hps_, st_tid_;
   DevBuf ws_, ws2_, rw_;
   HostStager *stager_ = nullptr; // pinned chunked staging of large host batches (made on first use)
+  DevBuf hc_tree_;
+  bool tree_zero_ = false;       // hc_tree_ holds zeroes (its state between passes)
+  // since the last hash pass: distinct keys written (about a dirty leaf each)
+  // and null entries the builds left in the dirty list
+  uint64_t dirty_keys_ = 0, dirty_holes_ = 0;
+  bool by_level_ = false;        // the next hash pass is to classify its nodes (rebuild_graph captures their bins)
   DevBuf hc_sorted_, hc_meta_, hc_cursor_, hc_slot_, hc_enc_, hc_scratch_, hc_lmeta_, hc_lmeta_tmp_;
   void *h_meta_ = nullptr;       // pinned HcMeta mirror
   bool root0_ok_ = false;        // cnt_.root0 is trie 0's current root (set by hash, cleared by every other call)

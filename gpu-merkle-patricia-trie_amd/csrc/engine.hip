@@ -119,7 +119,7 @@ Forest::~Forest() {
   delete stager_;
   DevBuf *bufs[] = {&branch_, &shrt_, &value_, &keys_, &tries_, &dirty_, &st_keys_, &st_kidx_, &st_vidx_,
                     &st_hps_, &st_tid_, &ws_, &ws2_, &hc_sorted_, &hc_meta_, &hc_cursor_, &hc_slot_, &hc_enc_, &hc_scratch_,
-                    &hc_lmeta_, &hc_lmeta_tmp_, &rw_};
+                    &hc_lmeta_, &hc_lmeta_tmp_, &hc_tree_, &rw_};
   for (DevBuf *b : bufs) release(*b);
   for (DevBuf &b : vchunks_) release(b);
   if (d_cnt_) (void)hipFree(d_cnt_);
@@ -580,6 +580,8 @@ void Forest::finish_build(const NuArgs &a) {
   rec_.bdesc = a.bdesc;
   rec_.blo = rec_.lo + rec_.n;
   rec_.bn = cnt_.scal[SC_NREP_TOT];
+  dirty_keys_ += cnt_.scal[SC_M_UNIQ];
+  dirty_holes_ += cnt_.scal[SC_NREP_TOT] - cnt_.scal[SC_NEXT];
 }
 
 // After the descent's counter read: the rest of an insert into tries that
@@ -689,7 +691,56 @@ int Forest::hash(void *targets, int n_targets) {
     return -3;
   }
   (void)n_targets;  // the whole dirty list is hashed: a subset would leave stale ancestors
-  uint32_t n = cnt_.n_dirty;
+  const uint32_t n = cnt_.n_dirty;
+  // The climb's waves use the spread layout, which hc_spread_max 0 turns off,
+  // and its counts are atomics on the nodes, which host pools do not get.
+  const uint64_t others = dirty_keys_ + dirty_holes_, inner = n > others ? n - others : 0;
+  dirty_keys_ = dirty_holes_ = 0;
+  if (n > 0 && n <= kTreeMax && inner <= kTreeMaxInner && !by_level_ && hc_fuse_leaves_ && hc_fuse_inner_ && hc_spread_max_ > 0 &&
+      !branch_.host && !shrt_.host) {
+    bool done = false;
+    if ((r = hash_tree(n, &done)) || done) return r;
+  }
+  return hash_by_level(n);
+}
+
+int Forest::hash_tree(uint32_t n, bool *done) {
+  int r;
+  if ((r = ensure_ws(hc_sorted_, sizeof(ref_t) * (size_t)n))) return r;
+  if ((r = ensure_ws(hc_enc_, sizeof(uint32_t) * (size_t)n))) return r;
+  if (!hc_tree_.p) tree_zero_ = false;
+  if ((r = ensure_ws(hc_tree_, sizeof(TreeState)))) return r;
+  TreeState *tree = (TreeState *)hc_tree_.p;
+  if (!tree_zero_) HIP_TRY(hipMemsetAsync(tree, 0, sizeof(TreeState), stream_));
+  tree_zero_ = false;
+  if (ev0_) HIP_TRY(hipEventRecord(ev0_, stream_));
+  HIP_TRY(hc_tree(pools(), (const ref_t *)dirty_.p, n, (ref_t *)hc_sorted_.p, (ref_t *)hc_enc_.p, tree, stream_));
+  HIP_TRY(hc_roots(pools(), ntries_, nullptr, stream_, tree));
+  if ((r = sync_counters(ev0_ ? ev1_ : nullptr))) return r;
+  tree_zero_ = true;
+  if (cnt_.hc_nodes != cnt_.hc_listed) return 0;
+  *done = true;
+  rec_ = LeafRecords();
+  stats_.hash_launches = 1;
+  stats_.hashed_nodes = cnt_.hc_nodes;
+  stats_.leaf_nodes = cnt_.hc_leaves;
+  stats_.ext_direct_nodes = 0;
+  stats_.perms = cnt_.n_perms;
+  stats_.enc_bytes = cnt_.enc_bytes;
+  stats_.leaf_perms = cnt_.leaf_perms;
+  stats_.leaf_bytes = cnt_.leaf_bytes;
+  stats_.leaf_perm_ms = stats_.last_hash_ms = 0;
+  if (ev0_) {
+    float ms = 0;
+    HIP_TRY(hipEventElapsedTime(&ms, ev0_, ev1_));
+    stats_.last_hash_ms = ms;
+  }
+  root0_ok_ = cnt_.root0_size <= 32;
+  return 0;
+}
+
+int Forest::hash_by_level(uint32_t n) {
+  int r;
   stats_.hash_launches = 0;
   stats_.hashed_nodes = 0;
   stats_.leaf_nodes = 0;
@@ -897,6 +948,7 @@ int Forest::clear() {
   rec_ = LeafRecords();
   HIP_TRY(hc_clear(d_cnt_, (TrieHdr *)tries_.p, ntries_, stream_));
   memset(&cnt_, 0, sizeof(cnt_));
+  dirty_keys_ = dirty_holes_ = 0;
   all_empty_ = true;
   key_used_ = 0;
   // keep the first value chunk, release the others
@@ -1248,6 +1300,7 @@ int Forest::puts_latching(const BatchDesc &b, void **targets, int *n_targets) {
     if (cnt_.n_value != values_before) key_used_ = align_up(key_used_ + ktot, 8);
     stats_.restarts = cnt_.n_restarts;
     stats_.lock_fails = cnt_.n_lock_fail;
+    dirty_keys_ += m;
   }
   if (targets) *targets = dirty_.p;
   if (n_targets) *n_targets = (int)cnt_.n_dirty;

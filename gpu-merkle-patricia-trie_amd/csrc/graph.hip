@@ -52,7 +52,10 @@ int Forest::rebuild_eager(const BatchDesc &b) {
   plan_.n_dirty = cnt_.n_dirty;
   plan_.ne = cnt_.scal[SC_NE];
   plan_.key_used = key_used_;
-  if ((r = hash(targets, nt))) return r;
+  by_level_ = true;  // for the bins the capture launches by
+  r = hash(targets, nt);
+  by_level_ = false;
+  if (r) return r;
   if (plan_.n_dirty) memcpy(plan_.hist, ((const HcMeta *)h_meta_)->hist, sizeof(plan_.hist));
   return 0;
 }

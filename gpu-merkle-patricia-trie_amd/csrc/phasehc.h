@@ -103,9 +103,36 @@ hipError_t hc_graph_check(const Pools &P, const HcMeta *meta, const uint32_t *pl
                           const uint32_t *scal, hipStream_t s);
 // Zeroes the forest's counters and every trie header (empty tries).
 hipError_t hc_clear(Counters *cnt, TrieHdr *tries, uint32_t ntries, hipStream_t s);
+// Work counts and list lengths of a climb (hc_tree); all zero between passes.
+constexpr uint32_t kTreeParts = 256;
+struct TreeState {
+  unsigned long long lists;     // ready, leaf and listed nodes (21 bits each)
+  unsigned long long pad[15];
+  unsigned long long parts[kTreeParts][8];  // permutations, bytes, those of the leaves, nodes, leaves
+};
+// Hashes the dirty list list[0 .. n) (n <= kTreeMax) without classifying it:
+// every node is hashed by the wave that hashed its last dirty child.  ready
+// and leaves hold n entries each; hc_roots with the same state folds the
+// counts and clears it.  A pass whose hc_nodes differ from its hc_listed left
+// nodes out (a dirty node that no dirty path reaches) and is to be repeated by
+// levels.
+constexpr uint32_t kTreeMax = 1u << 17;
+// A climb gives an inner node a wave of its own, so it wins while their
+// latency, not their number, sets the time.  Insert + hash by levels / as a
+// climb, by inner nodes: 1,450 303 / 184 us, 6,900 364 / 251, 12,300 369 / 293,
+// 21,500 382 / 364, 26,500 681 / 672, 30,100 397 / 440, 35,600 742 / 779.
+constexpr uint32_t kTreeMaxInner = 24576;
+// Up to here a leaf has a wave of its own too (8,200 entries: 113 us, leaves by
+// lane 132); above, its permutations fill the SIMDs and lanes do more per
+// cycle (17,000 entries: 147 by wave, 121 by lane).
+constexpr uint32_t kTreeSpreadLeaves = 8192;
+hipError_t hc_tree(const Pools &P, const ref_t *list, uint32_t n, ref_t *ready, ref_t *leaves, TreeState *tree,
+                   hipStream_t s);
 // Copies every trie's root hash into its header and empties the dirty list;
-// with parts (from hc_count), adds the pass's work counts to the counters.
-hipError_t hc_roots(const Pools &P, uint32_t ntries, const unsigned long long *parts, hipStream_t s);
+// with parts (from hc_count), adds the pass's work counts to the counters;
+// with tree (from hc_tree), sets them from it.
+hipError_t hc_roots(const Pools &P, uint32_t ntries, const unsigned long long *parts, hipStream_t s,
+                    TreeState *tree = nullptr);
 // Node export: encoding lengths, then encodings at offs and 32-byte hash slots.
 hipError_t hc_enc_len(const Pools &P, const ref_t *refs, uint32_t m, uint64_t *len, hipStream_t s);
 hipError_t hc_enc_write(const Pools &P, const ref_t *refs, uint32_t m, const uint64_t *offs, uint8_t *encs,

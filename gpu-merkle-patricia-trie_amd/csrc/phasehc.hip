@@ -1669,7 +1669,404 @@ __global__ __launch_bounds__(256) void k_hc_small2(Pools P, const ref_t *__restr
   hash_pair_spread2(P, list, slot, n, scratch, enc_len, 4 * blockIdx.x + wave, lds + 2 * wave);
 }
 
-__global__ __launch_bounds__(256) void k_hc_roots(Pools P, uint32_t ntries, const unsigned long long *parts) {
+
+// ------------------------------------------------- small passes: one climb --
+//
+// A pass over a short dirty list is bound by latency: a classification (five
+// launches), a copy of its bins to the host, and one launch per level, each
+// waiting for the one before, hash a few hundred nodes in ten times what
+// their permutations take.  Such a pass runs as one climb instead:
+//   k_tree_link    every dirty node gets its dirty parent (in its own dirty
+//                  word) and a branch the number of its dirty children; the
+//                  nodes without one are ready
+//   k_tree_leaves  (longer lists only) the leaves, one per lane
+//   k_tree_climb   one wave per ready node hashes it in the spread layout and
+//                  counts it off at its parent; the wave that was last goes on
+//                  with the parent.  No wave waits for another, and no level
+//                  for the slowest node of the one below.
+// The host reads nothing back in between.
+//
+// A dirty word: 1 = dirty without a dirty parent, else 1 | (parent is a short
+// node) << 1 | (parent's slot + 1) << 2.
+__device__ __forceinline__ uint32_t tree_parent_word(ref_t parent) {
+  return 1u | (ref_type(parent) == T_SHORT ? 2u : 0u) | (ref_idx(parent) + 1) << 2;
+}
+
+// TreeState::lists: ready entries, leaf entries and listed nodes, 21 bits each
+// (one atomic gives a block its place in both lists).
+constexpr uint32_t kTreeListBits = 21;
+constexpr unsigned long long kTreeListMask = (1ull << kTreeListBits) - 1;
+static_assert(kTreeMax < (1u << kTreeListBits), "the lists' counts are packed");
+
+// Words 4 (hash size, depth, dirty) of a branch and 6 (depth, hash size,
+// terminator flag, dirty) of a short node.
+static_assert(offsetof(Branch, hash_size) == 32 && offsetof(Branch, depth) == 34 && offsetof(Branch, dirty) == 36 &&
+                  offsetof(Branch, pad1) == 116,
+              "branch words");
+static_assert(offsetof(Short, depth) == 48 && offsetof(Short, hash_size) == 50 && offsetof(Short, term) == 51 &&
+                  offsetof(Short, dirty) == 52,
+              "short node words");
+
+__device__ __forceinline__ unsigned long long tree_reserve(TreeState *T, unsigned long long mine, uint32_t lane) {
+  unsigned long long base = 0;
+  if (lane == 0) base = atomicAdd(&T->lists, mine);
+  return (unsigned long long)__shfl((long long)base, 0);
+}
+
+// One thread per dirty-list entry (64 per block: the loads of a few thousand
+// nodes spread over the CUs).  With leaf_lanes the leaves the word builder
+// takes go to the leaf list, otherwise every leaf is ready.
+__global__ __launch_bounds__(64) void k_tree_link(Pools P, const ref_t *__restrict__ list, uint32_t n,
+                                                  ref_t *__restrict__ ready, ref_t *__restrict__ leaves,
+                                                  TreeState *T, int leaf_lanes) {
+  const uint32_t lane = threadIdx.x, i = blockIdx.x * 64 + lane;
+  const ref_t r = i < n ? list[i] : REF_NULL;  // builds leave null holes
+  bool rdy = false, leaf = false, listed = false;
+  if (ref_type(r) == T_BRANCH) {
+    Branch &B = P.branch[ref_idx(r)];
+    ref_t c[16];
+    const uint4 *cw = (const uint4 *)B.child;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const uint4 v = cw[q];
+      c[4 * q] = v.x;
+      c[4 * q + 1] = v.y;
+      c[4 * q + 2] = v.z;
+      c[4 * q + 3] = v.w;
+    }
+    uint32_t f[16];
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+      const uint32_t t = ref_type(c[q]);
+      f[q] = t == T_BRANCH || t == T_SHORT ? *node_dirty_flag(P, c[q]) : 0u;
+    }
+    const uint32_t me = tree_parent_word(r);
+    uint32_t k = 0;
+#pragma unroll
+    for (int q = 0; q < 16; q++)
+      if (f[q]) {
+        *node_dirty_flag(P, c[q]) = me;
+        k++;
+      }
+    B.pad1 = k;  // dirty children still to be hashed
+    rdy = k == 0;
+    listed = true;
+  } else if (ref_type(r) == T_SHORT) {
+    Short &S = P.shrt[ref_idx(r)];
+    const ref_t c = S.child;
+    if (ref_type(c) == T_VALUE) {
+      listed = true;
+      leaf = leaf_lanes && (uint32_t)S.key_len - S.term <= kLeafFastNibbles &&
+             P.value[ref_idx(c)].size <= kLeafDirectMaxValue;
+      rdy = !leaf;
+    } else if (S.lock & 1) {
+      S.dirty = 0;  // replaced by a split since it was listed: no node's child any more, and its child another's
+    } else {
+      listed = true;
+      uint32_t *f = node_dirty_flag(P, c);
+      rdy = *f == 0;
+      if (!rdy) *f = tree_parent_word(r);
+    }
+  }
+  const uint64_t mr = __ballot(rdy), ml = __ballot(leaf), ma = __ballot(listed);
+  if (ma == 0) return;
+  const unsigned long long base = tree_reserve(
+      T, (unsigned long long)__popcll(mr) | (unsigned long long)__popcll(ml) << kTreeListBits |
+             (unsigned long long)__popcll(ma) << (2 * kTreeListBits), lane);
+  const uint64_t below = (1ull << lane) - 1;
+  if (rdy) ready[(uint32_t)(base & kTreeListMask) + (uint32_t)__popcll(mr & below)] = r;
+  if (leaf) leaves[(uint32_t)(base >> kTreeListBits & kTreeListMask) + (uint32_t)__popcll(ml & below)] = r;
+}
+
+// Adds the wave's work counts (v on lanes 0 .. 5 as TreeState::parts' words).
+__device__ __forceinline__ void tree_count(TreeState *T, uint32_t wave, uint32_t lane, unsigned long long v) {
+  if (lane < 6 && v) atomicAdd(&T->parts[wave % kTreeParts][lane], v);
+}
+
+// The leaf list, one leaf per lane (as k_hc_leaf_direct); a branch whose last
+// dirty child was one of them becomes ready.
+__global__ __launch_bounds__(256) void k_tree_leaves(Pools P, const ref_t *__restrict__ leaves, ref_t *ready,
+                                                     TreeState *T) {
+  __shared__ uint64_t head[256][kLeafDirectHead];
+  const uint32_t i = grid_tid(), lane = __lane_id();
+  const uint32_t n = (uint32_t)(T->lists >> kTreeListBits & kTreeListMask);  // only the ready count moves here
+  if (i - lane >= n) return;
+  uint32_t enc = 0;
+  ref_t up = REF_NULL;
+  if (i < n) {
+    const ref_t r = leaves[i];
+    const uint32_t par = P.shrt[ref_idx(r)].dirty;
+    uint64_t m[2];
+    leaf_meta(P, r, m);
+    enc = hash_leaf_shaped(P, r, m[0], m[1], head[threadIdx.x]);
+    // a leaf's parent is a branch
+    if (par >> 2 && __hip_atomic_fetch_add(&P.branch[(par >> 2) - 1].pad1, ~0u, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT) == 1u)
+      up = make_ref(T_BRANCH, (par >> 2) - 1);
+  }
+  const uint64_t mu = __ballot(up != REF_NULL);
+  if (mu) {
+    const uint32_t base = (uint32_t)(tree_reserve(T, (unsigned long long)__popcll(mu), lane) & kTreeListMask);
+    if (up != REF_NULL) ready[base + (uint32_t)__popcll(mu & ((1ull << lane) - 1))] = up;
+  }
+  uint32_t bytes = enc, perms = enc >= 32 ? keccak_blocks(enc) : 0u;
+  for (int off = 32; off > 0; off >>= 1) {
+    bytes += (uint32_t)__shfl_xor((int)bytes, off);
+    perms += (uint32_t)__shfl_xor((int)perms, off);
+  }
+  const uint32_t nodes = min(n - (i - lane), 64u);
+  tree_count(T, i / 64, lane,
+             lane == 0 || lane == 2 ? perms : lane == 1 || lane == 3 ? bytes : nodes);
+}
+
+// Agent-scope accesses for what waves on other dies write in the same launch.
+template <typename T>
+__device__ __forceinline__ T ld_agent(const T *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_agent(uint64_t *p, uint64_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// A wave's LDS operations complete in order: only the compiler must not move
+// them across.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// A child's digest word q and its size, as another wave may just have stored them.
+__device__ __forceinline__ void tree_child(const Pools &P, ref_t c, uint32_t q, uint64_t &h, uint32_t &hs) {
+  if (ref_type(c) == T_BRANCH) {
+    const uint64_t *w = (const uint64_t *)&P.branch[ref_idx(c)];
+    h = ld_agent(w + q);
+    hs = (uint32_t)ld_agent(w + 4) & 255u;
+  } else {
+    const uint64_t *w = (const uint64_t *)&P.shrt[ref_idx(c)];
+    h = ld_agent(w + q);
+    hs = (uint32_t)(ld_agent(w + 6) >> 16) & 255u;
+  }
+}
+
+// A node's message: plen bytes in LDS, then the vsz bytes at va; enc = both.
+struct TreeMsg {
+  uint32_t plen, vsz, enc;
+  uint64_t va;
+};
+
+// The size and place of a value's string item; its first byte for a 1-byte
+// value (raw when <= 0x7f).
+struct TreeStr {
+  uint64_t va = 0;
+  uint32_t vsz = 0, b0 = 0x80;
+  __device__ __forceinline__ void load(const Pools &P, ref_t v) {
+    const Value &V = P.value[ref_idx(v)];
+    va = V.addr;
+    vsz = V.size;
+    if (vsz == 1) b0 = (uint32_t)value_word(va, 1, 0) & 255u;
+  }
+  __device__ __forceinline__ bool raw() const { return vsz == 1 && b0 <= 0x7f; }
+};
+
+// Ends a message at LDS offset p with the string item: its header (or raw
+// byte) in LDS, its bytes left where they are.
+__device__ __forceinline__ void tree_tail(uint8_t *b, uint32_t p, uint32_t lane, const TreeStr &s, TreeMsg &m) {
+  uint32_t n = 1;
+  const uint64_t h = s.raw() ? (uint64_t)s.b0 : rlp_hdr(s.vsz, 0x80, 0xB7, &n);
+  if (lane < n) b[p + lane] = (uint8_t)(h >> (8 * lane));
+  m.plen = p + n;
+  m.va = s.va;
+  m.vsz = s.raw() ? 0u : s.vsz;
+}
+
+// Four lanes per nibble slot: each takes 8 bytes of the child's digest (or raw
+// encoding, written as a string like the digest).
+__device__ __forceinline__ void tree_branch(const Pools &P, const Branch &B, uint32_t lane, uint8_t *b, TreeMsg &m) {
+  const uint32_t s = lane >> 2, q = lane & 3;
+  const ref_t c = B.child[s], c16 = B.child[16];
+  uint64_t h = 0;
+  uint32_t hs = 0;
+  if (c != REF_NULL) tree_child(P, c, q, h, hs);
+  TreeStr v;
+  if (c16 != REF_NULL) v.load(P, c16);
+  const uint32_t len = c == REF_NULL ? 1u : 1u + hs;
+  uint32_t incl = len;  // over the slots (the same in a slot's four lanes)
+#pragma unroll
+  for (uint32_t d = 4; d < 64; d <<= 1) {
+    const uint32_t t = (uint32_t)__shfl_up((int)incl, d);
+    if (lane >= d) incl += t;
+  }
+  const uint32_t total = (uint32_t)__shfl((int)incl, 63);
+  const uint32_t payload = total + (v.raw() || c16 == REF_NULL ? 1u : rlp_hdr_len(v.vsz) + v.vsz);
+  uint32_t hn;
+  const uint64_t hdr = rlp_hdr(payload, 0xC0, 0xF7, &hn);
+  if (lane < hn) b[lane] = (uint8_t)(hdr >> (8 * lane));
+  const uint32_t pos = hn + incl - len;
+  if (q == 0) b[pos] = (uint8_t)(0x80 + hs);  // an empty slot is an empty string
+  if (hs == 32) {
+#pragma unroll
+    for (uint32_t t = 0; t < 8; t++) b[pos + 1 + 8 * q + t] = (uint8_t)(h >> (8 * t));
+  } else {
+    for (uint32_t t = 0; t < 8 && 8 * q + t < hs; t++) b[pos + 1 + 8 * q + t] = (uint8_t)(h >> (8 * t));
+  }
+  m.enc = hn + payload;
+  if (c16 != REF_NULL) {
+    tree_tail(b, hn + total, lane, v, m);
+  } else {
+    if (lane == 0) b[hn + total] = 0x80;
+    m.plen = hn + total + 1;
+    m.va = 0;
+    m.vsz = 0;
+  }
+}
+
+// One lane per byte of the compact key.
+__device__ __forceinline__ void tree_short(const Pools &P, const Short &S, uint32_t lane, uint8_t *b, TreeMsg &m) {
+  const ref_t c = S.child;
+  const uint32_t term = S.term, cnt = (uint32_t)S.key_len - term, kc = cnt / 2 + 1, ks = S.key_start;
+  const uint8_t *key = P.keys + S.key_off;
+  const bool leaf = ref_type(c) == T_VALUE;
+  TreeStr v;
+  uint64_t h = 0;
+  uint32_t hs = 0;
+  if (leaf)
+    v.load(P, c);
+  else
+    tree_child(P, c, lane & 3, h, hs);
+  uint32_t khn = 0, hn;
+  const uint64_t khdr = kc == 1 ? 0ull : rlp_hdr(kc, 0x80, 0xB7, &khn);  // a lone byte is <= 0x3f: raw
+  const uint32_t payload = khn + kc + (!leaf ? 1u + hs : v.raw() ? 1u : rlp_hdr_len(v.vsz) + v.vsz);
+  const uint64_t hdr = rlp_hdr(payload, 0xC0, 0xF7, &hn);
+  if (lane < hn) b[lane] = (uint8_t)(hdr >> (8 * lane));
+  if (lane < khn) b[hn + lane] = (uint8_t)(khdr >> (8 * lane));
+  const uint32_t odd = cnt & 1;
+  for (uint32_t k = lane; k < kc; k += 64) {
+    uint32_t x;
+    if (k == 0) {
+      x = (term << 5) | (odd << 4) | (odd ? packed_nibble(key, ks) : 0u);
+    } else {
+      const uint32_t j = ks + odd + 2 * (k - 1);
+      x = (packed_nibble(key, j) << 4) | packed_nibble(key, j + 1);
+    }
+    b[hn + khn + k] = (uint8_t)x;
+  }
+  m.enc = hn + payload;
+  const uint32_t p = hn + khn + kc;
+  if (leaf) {
+    tree_tail(b, p, lane, v, m);
+  } else {
+    if (lane == 0) b[p] = (uint8_t)(0x80 + hs);
+    for (uint32_t t = 0; lane < 4 && t < 8 && 8 * lane + t < hs; t++) b[p + 1 + 8 * lane + t] = (uint8_t)(h >> (8 * t));
+    m.plen = p + 1 + hs;
+    m.va = 0;
+    m.vsz = 0;
+  }
+}
+
+// Message word w: LDS bytes, value bytes and, with nb, Keccak padding.
+__device__ __forceinline__ uint64_t tree_word(const uint64_t *b, const TreeMsg &m, uint32_t nb, uint32_t w) {
+  const uint32_t x0 = 8 * w;
+  uint64_t v = 0;
+  if (x0 < m.plen) v = low_bytes(b[w], m.plen - x0);
+  if (m.vsz && x0 + 8 > m.plen && x0 < m.enc) v |= value_word(m.va, m.vsz, (int64_t)x0 - (int64_t)m.plen);
+  if (nb) {
+    if (m.enc >= x0 && m.enc < x0 + 8) v |= 0x01ull << (8 * (m.enc - x0));
+    if (w + 1 == 17 * nb) v |= 0x80ull << 56;
+  }
+  return v;
+}
+
+// One wave per ready node; the wave climbs as long as it hashed its node's
+// parent's last dirty child.  Its stores of a node (digest, then the word with
+// the size) are written through and complete before the parent's count goes
+// down; the last wave's loads of its siblings' nodes start after its own count
+// came back.  Every wave ends: a step goes one node up.
+// Bound by latency: a level costs its permutations (3.3 us each in the spread
+// layout) and about 2.5 us of dependent loads, stores and the count.
+constexpr uint32_t kTreeMsgWords = 80;  // a branch's items and value header take at most 536 bytes
+__global__ __launch_bounds__(256) void k_tree_climb(Pools P, const ref_t *__restrict__ ready, TreeState *T) {
+  __shared__ uint64_t lds[256 / 64][kTreeMsgWords];
+  const uint32_t lane = __lane_id(), g = threadIdx.x / 64;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (256 / 64) + g);
+  if (wave >= (uint32_t)(T->lists & kTreeListMask)) return;
+  uint64_t *msg = lds[g];
+  uint8_t *b = (uint8_t *)msg;
+  const SpreadLane sl(lane);
+  const int w = SpreadLane::word_of(lane);
+  uint32_t perms = 0, bytes = 0, lperms = 0, lbytes = 0, nodes = 0, lnodes = 0;
+  ref_t r = __builtin_amdgcn_readfirstlane(ready[wave]);
+  for (;;) {
+    const bool branch = ref_type(r) == T_BRANCH;
+    const uint32_t idx = ref_idx(r);
+    uint64_t *node = branch ? (uint64_t *)&P.branch[idx] : (uint64_t *)&P.shrt[idx];
+    const uint64_t meta = node[branch ? 4 : 6];  // dirty word in the upper half: the parent
+    bool leaf = false;
+    TreeMsg m;
+    if (branch) {
+      tree_branch(P, P.branch[idx], lane, b, m);
+    } else {
+      leaf = ref_type(P.shrt[idx].child) == T_VALUE;
+      tree_short(P, P.shrt[idx], lane, b, m);
+    }
+    wave_lds_order();
+    m.enc = __builtin_amdgcn_readfirstlane(m.enc);
+    const uint32_t nb = m.enc >= 32 ? keccak_blocks(m.enc) : 0u;
+    uint32_t hs = 32;
+    if (nb == 0) {  // shorter than a digest: the raw encoding is the "hash"
+      hs = m.enc;
+      if (lane < 4) st_agent(node + lane, tree_word(msg, m, 0, lane));
+    } else {
+      uint32_t l = 0, h = 0;
+      // the words of two blocks are in flight before the first permutation
+      uint64_t cur = w >= 0 ? tree_word(msg, m, nb, (uint32_t)w) : 0ull;
+      uint64_t nxt = w >= 0 && nb > 1 ? tree_word(msg, m, nb, 17 + (uint32_t)w) : 0ull;
+      for (uint32_t k = 0; k < nb; k++) {
+        l ^= (uint32_t)cur;
+        h ^= (uint32_t)(cur >> 32);
+        cur = nxt;
+        if (k + 2 < nb && w >= 0) nxt = tree_word(msg, m, nb, 17 * (k + 2) + (uint32_t)w);
+        keccak_spread(l, h, sl);
+      }
+      if (spread_digest_lane(lane)) st_agent(node + (lane >> 3), ((uint64_t)h << 32) | l);
+    }
+    if (lane == 0) {
+      const uint32_t lo = (uint32_t)meta;
+      if (branch)
+        st_agent(node + 4, (uint64_t)((lo & 0xffffff00u) | hs));
+      else
+        st_agent(node + 6, (uint64_t)((lo & 0xff00ffffu) | hs << 16));
+    }
+    perms += nb;
+    bytes += m.enc;
+    nodes++;
+    if (leaf) {
+      lperms += nb;
+      lbytes += m.enc;
+      lnodes++;
+    }
+    const uint32_t par = __builtin_amdgcn_readfirstlane((uint32_t)(meta >> 32));
+    if (par >> 2 == 0) break;  // a root
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0);  // the node's stores have completed
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    if (par & 2) {
+      r = make_ref(T_SHORT, (par >> 2) - 1);  // an extension's only child
+    } else {
+      uint32_t left = 0;
+      if (lane == 0)
+        left = __hip_atomic_fetch_add(&P.branch[(par >> 2) - 1].pad1, ~0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      left = __builtin_amdgcn_readfirstlane(left);
+      if (left != 1) break;  // another child's wave goes on
+      r = make_ref(T_BRANCH, (par >> 2) - 1);
+    }
+    wave_lds_order();
+  }
+  tree_count(T, wave, lane,
+             lane == 0 ? perms : lane == 1 ? bytes : lane == 2 ? lperms : lane == 3 ? lbytes : lane == 4 ? nodes : lnodes);
+}
+
+__global__ __launch_bounds__(256) void k_hc_roots(Pools P, uint32_t ntries, const unsigned long long *parts,
+                                                  TreeState *tree) {
   uint32_t t = grid_tid();
   // the root's hash first: its two dependent loads overlap the counts' reduction
   uint32_t hs = 0;
@@ -1703,6 +2100,34 @@ __global__ __launch_bounds__(256) void k_hc_roots(Pools P, uint32_t ntries, cons
                                 : threadIdx.x == 2 ? &P.cnt->leaf_perms
                                                    : &P.cnt->leaf_bytes;
       *dst += sh[0][threadIdx.x] + sh[1][threadIdx.x] + sh[2][threadIdx.x] + sh[3][threadIdx.x];
+    }
+  }
+  if (tree && blockIdx.x == 0) {  // a climb's counts (uniform branch); its state is left zero for the next one
+    static_assert(kTreeParts == 256, "one partial per thread");
+    __shared__ unsigned long long st[4][6];
+    unsigned long long v[6];
+#pragma unroll
+    for (int q = 0; q < 6; q++) {
+      v[q] = tree->parts[threadIdx.x][q];
+      tree->parts[threadIdx.x][q] = 0;
+    }
+#pragma unroll
+    for (int q = 0; q < 6; q++)
+      for (int off = 32; off > 0; off >>= 1) v[q] += (unsigned long long)__shfl_xor((long long)v[q], off);
+    if (__lane_id() == 0)
+#pragma unroll
+      for (int q = 0; q < 6; q++) st[threadIdx.x >> 6][q] = v[q];
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int q = 0; q < 6; q++) v[q] = st[0][q] + st[1][q] + st[2][q] + st[3][q];
+      P.cnt->n_perms = v[0];
+      P.cnt->enc_bytes = v[1];
+      P.cnt->leaf_perms = v[2];
+      P.cnt->leaf_bytes = v[3];
+      P.cnt->hc_nodes = (uint32_t)v[4];
+      P.cnt->hc_leaves = (uint32_t)v[5];
+      P.cnt->hc_listed = (uint32_t)(tree->lists >> (2 * kTreeListBits));
+      tree->lists = 0;
     }
   }
   if (t >= ntries) return;
@@ -1984,8 +2409,22 @@ hipError_t hc_clear(Counters *cnt, TrieHdr *tries, uint32_t ntries, hipStream_t 
   return hipGetLastError();
 }
 
-hipError_t hc_roots(const Pools &P, uint32_t ntries, const unsigned long long *parts, hipStream_t s) {
-  k_hc_roots<<<nblk(ntries), kB, 0, s>>>(P, ntries, parts);
+hipError_t hc_roots(const Pools &P, uint32_t ntries, const unsigned long long *parts, hipStream_t s, TreeState *tree) {
+  k_hc_roots<<<nblk(ntries), kB, 0, s>>>(P, ntries, parts, tree);
+  return hipGetLastError();
+}
+
+hipError_t hc_tree(const Pools &P, const ref_t *list, uint32_t n, ref_t *ready, ref_t *leaves, TreeState *tree,
+                   hipStream_t s) {
+  if (n == 0 || n > kTreeMax) return hipErrorInvalidValue;
+  const bool lanes = n > kTreeSpreadLeaves;
+  k_tree_link<<<(n + 63) / 64, 64, 0, s>>>(P, list, n, ready, leaves, tree, lanes ? 1 : 0);
+  GMPT_LAUNCH_CHECK();
+  if (lanes) {
+    k_tree_leaves<<<nblk(n), kB, 0, s>>>(P, leaves, ready, tree);
+    GMPT_LAUNCH_CHECK();
+  }
+  k_tree_climb<<<(n + 3) / 4, kB, 0, s>>>(P, ready, tree);
   return hipGetLastError();
 }
 

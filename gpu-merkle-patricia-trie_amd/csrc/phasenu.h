@@ -126,7 +126,7 @@ __host__ __device__ inline size_t mt_bytes(size_t stride) {
 // device scalar slots in NuArgs::scal
 enum {
   SC_W = 0, SC_MAXLEN = 1, SC_M_UNIQ = 2, SC_NGROUP = 3, SC_NE = 4, SC_KTOT = 6 /* u64 */, SC_MERGE = 8,
-  SC_NREP = 9, SC_DBASE = 10, SC_NREP_TOT = 11,
+  SC_NEXT = 9 /* extensions a build of at most kCountExtBlocks blocks made */, SC_DBASE = 10, SC_NREP_TOT = 11,
   SC_WOR = 12 /* u64: OR of the windows */, SC_WAND = 14 /* u64: AND of the windows */,
   SC_UNIFORM = 16 /* 1: every key has key 0's length (packed by the validation pass) */,
   SC_NFRESH = 17 /* LockNU: keys the insert creates */,

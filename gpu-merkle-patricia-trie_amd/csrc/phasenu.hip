@@ -1489,13 +1489,14 @@ __device__ __forceinline__ void install(const NuArgs &a, const GroupInfo &gi, re
 }
 
 // Branches: link each to its parent (through an extension when depths skip).
+// Returns whether it made an extension.
 template <class Sink>
-__device__ __forceinline__ void link_branch(const NuArgs &a, uint32_t j, uint32_t rank, const Slots &q,
+__device__ __forceinline__ bool link_branch(const NuArgs &a, uint32_t j, uint32_t rank, const Slots &q,
                                             const Sink &sink) {
   ST s = st_of(a);
-  if (j >= s.nsp) return;
+  if (j >= s.nsp) return false;
   uint32_t L = s.at(0, j);
-  if (L == 0 || a.repof[j] != j) return;
+  if (L == 0 || a.repof[j] != j) return false;
   // the interval's bounding split points, found by k_split_reps
   const uint64_t lh = a.plohi[j];
   const int lo = (int)(uint32_t)lh;
@@ -1534,6 +1535,7 @@ __device__ __forceinline__ void link_branch(const NuArgs &a, uint32_t j, uint32_
     install(a, gi, me);
   else
     sink(a, parent, slot, me);
+  return ext != REF_NULL;
 }
 
 // Elements: new keys become a leaf short node + value node; a split short
@@ -1584,6 +1586,7 @@ __device__ __forceinline__ void link_elem(const NuArgs &a, uint32_t e, const Slo
   uint32_t vsz = 0;
   if (ek.virt) {
     child = a.P.shrt[ek.uidx].child;
+    a.P.shrt[ek.uidx].lock |= 1;  // the split node is no one's child any more (a dirty list may still name it)
   } else {
     uint32_t vid = a.base_value + e;
     if (vid >= a.P.cap_value) {
@@ -1630,6 +1633,7 @@ __device__ __forceinline__ void link_elem(const NuArgs &a, uint32_t e, const Slo
 // to the cross list (xp, xs, xm), which k_link_cross applies afterwards; no
 // other branch line is written piecewise.  Thread j links the branch whose
 // representative is split point j, if any, and element j.
+constexpr uint32_t kCountExtBlocks = 512;         // blocks of a build that counts its extensions (one atomic each)
 constexpr uint32_t kCrossPerBlock = 2 * kSpTile;  // a thread makes at most two links
 struct OwnedLinks {
   ref_t (*kid)[17];
@@ -1708,9 +1712,10 @@ __global__ __launch_bounds__(256) void k_build_links(NuArgs a, int pre) {
   }
   __syncthreads();  // child arrays cleared, local indices set
   const OwnedLinks sink{kid, krec, own, &xn, blockIdx.x * kSpTile};
-  link_branch(a, j, rank, q, sink);
+  const bool ext = link_branch(a, j, rank, q, sink);
   link_elem(a, j, q, sink);
-  __syncthreads();  // every owned link in LDS
+  const uint32_t exts = (uint32_t)__syncthreads_count(ext);  // every owned link in LDS
+  if (exts && gridDim.x <= kCountExtBlocks && threadIdx.x == 0) atomicAdd(&a.scal[SC_NEXT], exts);
   // the owned branches, 16 bytes per thread: hash (zero), hash_size 0 |
   // depth | dirty 1 | lock 0, child[0 .. 15], child[16] and padding
   const uint32_t b0 = a.base_branch + base;

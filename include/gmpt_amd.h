@@ -60,7 +60,8 @@ typedef struct gmpt_stats {
   uint64_t enc_bytes;             /* node encoding bytes produced by the last hash */
   uint64_t pool_bytes_used;       /* HBM held by nodes, keys and values */
   uint64_t pool_bytes_reserved;   /* HBM reserved by the pools */
-  double leaf_perm_ms;            /* device time of the leaf level's permutation kernel (last hash) */
+  double leaf_perm_ms;            /* device time of the leaf level's permutation kernel (last hash; 0 when a short
+                                     dirty list was hashed in one climb) */
   uint64_t leaf_perms;            /* its permutations */
   uint64_t leaf_bytes;            /* encoding bytes of the leaf level */
   uint32_t leaf_nodes;            /* leaf nodes hashed */

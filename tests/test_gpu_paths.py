@@ -114,3 +114,86 @@ def test_batches_ordered_by_trie_and_path(gmpt, workloads, oracle, tries, per, s
     for t in sorted(set(tid[:: max(1, n // 12)].tolist())):
         assert roots[t] == oracle.root_of(b.subset(np.flatnonzero(tid == t))), t
     assert all(roots[t] == b"" for t in set(range(tries)) - set(tid.tolist()))
+
+
+COUNTS = ("perms", "enc_bytes", "leaf_perms", "leaf_bytes", "leaf_nodes", "hashed_nodes")
+
+
+def _mixed_keys(rng, n, kind):
+    if kind == "uniform":
+        return [bytes(k) for k in rng.integers(0, 256, (n, 32), dtype=np.uint8)]
+    if kind == "short":  # keys that are prefixes of others (values in branches), encodings under 32 bytes
+        return [bytes(rng.integers(0, 256, int(rng.integers(1, 5)), dtype=np.uint8)) for _ in range(n)]
+    # long: remainders past 64 nibbles, extensions of every length
+    stems = [bytes(rng.integers(0, 256, int(rng.integers(1, 60)), dtype=np.uint8)) for _ in range(1 + n // 6)]
+    return [stems[int(rng.integers(len(stems)))] + bytes(rng.integers(0, 256, int(rng.integers(1, 60)), dtype=np.uint8))
+            for _ in range(n)]
+
+
+@pytest.mark.parametrize("mode", list(PUTS))
+@pytest.mark.parametrize("kind,n", [("uniform", 1), ("uniform", 2), ("uniform", 36), ("short", 700), ("long", 700),
+                                    ("uniform", 4650), ("uniform", 4850), ("short", 9000), ("long", 6000),
+                                    ("uniform", 66_000), ("uniform", 75_000)])
+def test_short_dirty_lists_hashed_in_one_climb(gmpt, workloads, oracle, mode, kind, n):
+    # list lengths around a block of 64, around the lines to leaves by lane
+    # (8,192 entries) and to levels (24,576 inner nodes); empty, 1-byte and many-block
+    # values, in leaves and in branches; a second batch hashed over a clean trie;
+    # the same root as by levels, and for a build into an empty trie the same
+    # work counts (later batches may split a node after listing it, which only
+    # the levels hash)
+    rng = np.random.default_rng(n + len(kind))
+    keys = list(dict.fromkeys(_mixed_keys(rng, n, kind)))
+    lens = rng.choice([0, 1, 1, 5, 32, 55, 56, 90, 135, 136, 137, 300, 1000], len(keys))
+    lens[:: max(1, n // 3)] = rng.choice([255, 256, 16_382, 16_383, 70_000], len(lens[:: max(1, n // 3)]))
+    vals = [bytes(rng.integers(0, 256, int(k), dtype=np.uint8)) for k in lens]
+    b = workloads.batch_from_bytes(keys, vals)
+    some = rng.permutation(len(keys))[: 1 + n // 8]
+    more = workloads.batch_from_bytes([keys[i] for i in some] + [b"\x31" + keys[i][:20] for i in some],
+                                      [b"u%d" % i for i in range(2 * len(some))])
+    t, by_level = gmpt.MPT(device=0), gmpt.MPT(device=0)
+    by_level.set_option("hc_fuse_leaves", 0)
+    o = oracle.OracleMPT()
+    for part in (b, more):
+        nt = getattr(t, PUTS[mode])(part)[1]
+        t.hash_onepass_v2(None, nt)
+        o.puts(part)
+        o.hash()
+        assert t.get_root_hash() == o.root()
+        st = t.stats()
+        if part is b:
+            assert (st["hash_launches"] == 1) == (st["hashed_nodes"] - st["leaf_nodes"] <= 24576)
+        assert _put(by_level, part, mode) == o.root()
+        if part is b:
+            assert [t.stats()[k] for k in COUNTS] == [by_level.stats()[k] for k in COUNTS]
+    assert _put(t, b, mode) == _after(oracle, [b, more, b])
+
+
+@pytest.mark.parametrize("modes", [("2phase", "2phase"), ("latching", "latching"), ("2phase", "latching"),
+                                   ("latching", "2phase")])
+@pytest.mark.parametrize("tries", [1, 7])
+def test_dirty_nodes_split_before_they_are_hashed(gmpt, workloads, oracle, modes, tries):
+    # two inserts before one hash: the second splits leaves and extensions the
+    # first left in the dirty list, at their first nibble and further in
+    rng = np.random.default_rng(len(modes[0]) + tries)
+    first, second = [], []
+    for _ in range(300):
+        stem = [int(x) for x in rng.integers(0, 16, int(rng.integers(1, 24)))]
+        tail = [int(x) for x in rng.integers(0, 16, 64 - len(stem))]
+        first += [bytes(stem + [q] + tail[1:] + [16]) for q in (1, 9)]  # a branch below the stem
+        cut = int(rng.integers(0, len(stem)))
+        second.append(bytes(stem[:cut] + [(stem[cut] + 1) % 16] + stem[cut + 1:] + tail + [16]))
+        second.append(bytes(stem + [1] + tail[1:30] + [(tail[30] + 1) % 16] + tail[31:] + [16]))
+    f = gmpt.MPT(device=0, num_tries=tries)
+    os_ = [oracle.OracleMPT() for _ in range(tries)]
+    for hexes, mode in ((first, modes[0]), (second, modes[1]), (first[::5] + second[::3], modes[0])):
+        hexes = list(dict.fromkeys(hexes))
+        b = workloads.batch_from_hex(hexes, [b"%d" % i * 9 for i in range(len(hexes))])
+        b.trie_ids = np.array([h[0] % tries for h in hexes], np.int32)
+        n = getattr(f, PUTS[mode])(b)[1]
+        for t in range(tries):
+            os_[t].puts(b.subset(np.flatnonzero(b.trie_ids == t)))
+    f.hash_onepass_v2(None, n)
+    assert f.stats()["hash_launches"] == 1  # no node was left out of the climb
+    for o in os_:
+        o.hash()
+    assert f.get_root_hashes() == [o.root() for o in os_]
