@@ -631,8 +631,11 @@ int Forest::puts_2phase(const BatchDesc &b, void **targets, int *n_targets) {
     const bool empty = all_empty_;
     // Elements are the unique keys, plus one per split short node (none in an
     // empty trie); per element at most one branch, two shorts and one value.
-    if ((r = empty ? ensure_pools(n, 2ull * n, n, d.key_slots)
-                   : ensure_pools(2ull * n + 2, 4ull * n + 4, 2ull * n + 2, d.key_slots)))
+    // A forest that may allocate reserves for as many again when its tries are
+    // empty: the next insert would otherwise grow the pools by copy (200,000
+    // keys, then 100,000 more, in a new forest: 3,970 us, 3,440 with).
+    if ((r = empty && arena_ ? ensure_pools(n, 2ull * n, n, d.key_slots)
+                             : ensure_pools(2ull * n + 2, 4ull * n + 4, 2ull * n + 2, d.key_slots)))
       return r;
     all_empty_ = false;
     NuArgs a;
