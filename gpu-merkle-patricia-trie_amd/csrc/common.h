@@ -97,12 +97,12 @@ struct Counters {
   unsigned long long enc_bytes;  // PhaseHC: bytes of node encodings produced
   unsigned long long leaf_perms; // PhaseHC: permutations of the leaf level
   unsigned long long leaf_bytes; // PhaseHC: encoding bytes of the leaf level
-  uint32_t scal[20];             // the current insert's device scalars (PhaseNU / LockNU)
+  uint32_t scal[22];             // the current insert's device scalars (PhaseNU / LockNU)
   uint32_t hc_nodes, hc_leaves, hc_listed;  // PhaseHC climb: nodes and leaves hashed, nodes of the dirty list
   uint32_t root0_size;           // trie 0's root as the last hash pass left it (k_hc_roots), so that
   uint8_t root0[32];             // the pass's closing counter read also brings the root to the host
 };
-static_assert(offsetof(Counters, root0) % 4 == 0, "Counters layout");
+static_assert(offsetof(Counters, root0) % 4 == 0 && offsetof(Counters, scal) % 8 == 0, "Counters layout");
 
 enum : uint32_t {
   ERR_NONE = 0,

@@ -531,10 +531,13 @@ int Forest::sort_unique(NuArgs &a, void *temp, int pass, int *cur) {
   if (pass == 1 && 4ull * ((a.n + 255) / 256) <= a.n) {
     // keys with long shared stretches inside the window (ASCII digits, fixed
     // fields) sort by fewer radix digits once the constant bits are dropped
-    HIP_TRY(nu_window_mask(a, *cur ? a.sk1 : a.sk0, stream_));
-    if ((r = sync_counters())) return r;
-    const uint64_t wor = *(const uint64_t *)(cnt_.scal + SC_WOR), wand = *(const uint64_t *)(cnt_.scal + SC_WAND);
-    const uint64_t m = wor & ~wand;
+    uint64_t m = *(const uint64_t *)(cnt_.scal + SC_WVAR);  // when the packing pass noted them
+    if (m == 0) {
+      HIP_TRY(nu_window_mask(a, *cur ? a.sk1 : a.sk0, stream_));
+      if ((r = sync_counters())) return r;
+      const uint64_t wor = *(const uint64_t *)(cnt_.scal + SC_WOR), wand = *(const uint64_t *)(cnt_.scal + SC_WAND);
+      m = wor & ~wand;
+    }
     const int pop = __builtin_popcountll(m);
     if (pop >= 1 && pop <= 56) vmask = m;  // saves at least one 8-bit digit
   }

@@ -130,7 +130,8 @@ enum {
   SC_WOR = 12 /* u64: OR of the windows */, SC_WAND = 14 /* u64: AND of the windows */,
   SC_UNIFORM = 16 /* 1: every key has key 0's length (packed by the validation pass) */,
   SC_NFRESH = 17 /* LockNU: keys the insert creates */,
-  SC_DUP = 18 /* nonzero: the sorted batch holds equal keys (set by k_adjacent) */, SC_COUNT = 20
+  SC_DUP = 18 /* nonzero: the sorted batch holds equal keys (set by k_adjacent) */,
+  SC_WVAR = 20 /* u64: sort key bits that vary across the batch, and no others vary (0: not known) */, SC_COUNT = 22
 };
 
 // Zeroes the call's device scalars (SC_W starts at all ones for its minimum).

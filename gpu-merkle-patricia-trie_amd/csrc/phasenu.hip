@@ -214,6 +214,21 @@ __device__ __forceinline__ uint64_t sort_key(const NuArgs &a, uint32_t i, uint64
   return a.tbits ? (uint64_t)(uint32_t)a.tid[i] << (64 - a.tbits) | win >> a.tbits : win;
 }
 
+// The window of a key of nn nibbles (k: its hex bytes) from nibble W on.
+__device__ __forceinline__ uint64_t window_at(const uint8_t *k, uint32_t nn, uint32_t W) {
+  const uint64_t h0 = W < nn ? ldn(k + W, min(8u, nn - W)) : 0ull;
+  const uint64_t h1 = W + 8 < nn ? ldn(k + W + 8, min(8u, nn - W - 8)) : 0ull;
+  return ((uint64_t)__builtin_bswap32(pack8(h0)) << 32) | __builtin_bswap32(pack8(h1));
+}
+// Records the bits in which some lane's sort key differs from key 0's (diff).
+// Every lane of the wave calls it; a wave with nothing new issues no atomic.
+__device__ __forceinline__ void note_varying(const NuArgs &a, uint64_t diff) {
+  for (int off = 32; off > 0; off >>= 1) diff |= (uint64_t)__shfl_xor((unsigned long long)diff, off);
+  unsigned long long *var = (unsigned long long *)(a.scal + SC_WVAR);
+  if (__lane_id() == 0 && (diff & ~__hip_atomic_load(var, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
+    atomicOr(var, (unsigned long long)diff);
+}
+
 // Validates every key, and reduces per block the common prefix with key 0
 // and the longest key (no global atomics: one slot per block).  A key as long
 // as key 0 is also packed at once to slot i of a layout with equal slots: when
@@ -226,6 +241,11 @@ __global__ __launch_bounds__(256) void k_keys_scan(NuArgs a, uint32_t *blk_w, ui
   uint32_t i = grid_tid();
   uint32_t lcp0 = UINT_MAX, len = 0, odd = 0;
   uint64_t sbytes = 0;  // the key's packed slot size
+  // Bits in which the sort key differs from key 0's, noted for a multi-trie
+  // batch that the bucket sort may take (one trie's keys without a common
+  // prefix vary in their leading bits, where it looks without a mask).
+  const bool note = a.tbits && a.sk0 && a.n <= kBucketSortMaxN;
+  uint64_t diff = 0;
   const uint32_t L0 = key_range_ok(a, 0) ? (uint32_t)(a.kidx[1] - a.kidx[0] + 1) : 0u;
   if (i < a.n) {
     bool ok = key_range_ok(a, i);
@@ -265,8 +285,10 @@ __global__ __launch_bounds__(256) void k_keys_scan(NuArgs a, uint32_t *blk_w, ui
           // the sort window of a batch with no common prefix (W = 0), as
           // k_keys_pack builds it from the slot: that pass skips such a batch
           if (a.sk0) {
-            a.sk0[i] = sort_key(a, i, __builtin_bswap64(first));
+            const uint64_t key = sort_key(a, i, __builtin_bswap64(first));
+            a.sk0[i] = key;
             a.sv0[i] = i;
+            if (note) diff = key ^ sort_key(a, 0, window_at(a.kh + a.kidx[0], L0 - 1, 0));
           }
         }
       } else {
@@ -318,6 +340,7 @@ __global__ __launch_bounds__(256) void k_keys_scan(NuArgs a, uint32_t *blk_w, ui
       a.kref[i] = koff | ((uint64_t)len << 48);
     }
   }
+  if (note) note_varying(a, diff);
   for (int off = 32; off > 0; off >>= 1) {
     lcp0 = min(lcp0, (uint32_t)__shfl_xor(lcp0, off));
     len = max(len, (uint32_t)__shfl_xor(len, off));
@@ -390,8 +413,11 @@ __global__ __launch_bounds__(256) void k_keys_reduce(NuArgs a, const uint32_t *b
     }
   }
   if (threadIdx.x == 0) {
-    a.scal[SC_W] = min(min(sw[0], sw[1]), min(sw[2], sw[3]));
-    a.scal[SC_MAXLEN] = max(max(sl[0], sl[1]), max(sl[2], sl[3]));
+    const uint32_t W = min(min(sw[0], sw[1]), min(sw[2], sw[3])), maxlen = max(max(sl[0], sl[1]), max(sl[2], sl[3]));
+    a.scal[SC_W] = W;
+    a.scal[SC_MAXLEN] = maxlen;
+    // other windows than k_keys_scan's follow (k_keys_pack)
+    if (!(uni && W == 0 && maxlen <= kFastKeyBytes)) *(uint64_t *)(a.scal + SC_WVAR) = 0;
     a.scal[SC_UNIFORM] = uni;
     *(uint64_t *)(a.scal + SC_KTOT) = kbytes;
   }
@@ -410,15 +436,23 @@ __global__ __launch_bounds__(256) void k_keys_pack(NuArgs a) {
     // every key took k_keys_scan's register path (equal lengths of at most
     // kFastKeyBytes), which wrote the windows for W = 0
     if (W == 0 && a.scal[SC_MAXLEN] <= kFastKeyBytes) return;
-    if (i >= a.n || !a.sk0) return;
-    const uint32_t L = a.klen[i];
-    const uint32_t slot = slot_bytes(L);
-    const uint64_t *src = (const uint64_t *)(a.P.keys + a.kbase + (uint64_t)i * slot);
-    const uint32_t q = W / 16, d = W % 16;
-    const uint64_t hi = __builtin_bswap64(src[q]);
-    const uint64_t lo = (q + 1) * 8 < slot ? __builtin_bswap64(src[q + 1]) : 0ull;
-    a.sk0[i] = sort_key(a, i, d ? (hi << (4 * d)) | (lo >> (64 - 4 * d)) : hi);
-    a.sv0[i] = i;
+    if (!a.sk0) return;
+    uint64_t diff = 0;
+    if (i < a.n) {
+      const uint32_t slot = slot_bytes(a.klen[i]);
+      const uint32_t q = W / 16, d = W % 16;
+      const auto window = [&](uint32_t k) {
+        const uint64_t *src = (const uint64_t *)(a.P.keys + a.kbase + (uint64_t)k * slot);
+        const uint64_t hi = __builtin_bswap64(src[q]);
+        const uint64_t lo = (q + 1) * 8 < slot ? __builtin_bswap64(src[q + 1]) : 0ull;
+        return sort_key(a, k, d ? (hi << (4 * d)) | (lo >> (64 - 4 * d)) : hi);
+      };
+      const uint64_t key = window(i);
+      a.sk0[i] = key;
+      a.sv0[i] = i;
+      diff = key ^ window(0);
+    }
+    note_varying(a, diff);
     return;
   }
   const KeyStager stg = stage_keys(a, lds);
@@ -429,14 +463,14 @@ __global__ __launch_bounds__(256) void k_keys_pack(NuArgs a) {
   uint64_t btot;
   const uint64_t koff =
       a.kpoff[blockIdx.x] + block_exclusive_scan_256<uint64_t>(i < a.n ? slot_bytes(Li) : 0u, s64, &btot);
-  if (i >= a.n) return;
   // The packed keys must fit the arena.  The host reserves it from the key
   // buffer's size, which index pairs that overlap or repeat a key range can
   // exceed: then no key is packed, every key reads as the empty key (its
   // terminator only, so every later read stays at the batch's first arena
   // bytes) and the call fails with an arena error; the host grows the arena
   // to the total and runs the insert again.
-  if (a.kbase + *(const uint64_t *)(a.scal + SC_KTOT) > a.key_cap) {
+  if (a.kbase + *(const uint64_t *)(a.scal + SC_KTOT) > a.key_cap) {  // uniform over the grid
+    if (i >= a.n) return;
     a.kref[i] = 1ull << 48;
     if (a.sk0) {
       a.sk0[i] = sort_key(a, i, 0);
@@ -445,17 +479,23 @@ __global__ __launch_bounds__(256) void k_keys_pack(NuArgs a) {
     if (i == 0) raise_error(a.P.cnt, ERR_POOL, kErrArgKeyArena);
     return;
   }
-  const uint32_t L = Li;
-  const uint8_t *k = key_range_ok(a, i) ? stg.at(a, a.kidx[2 * i]) : a.kh;
-  a.kref[i] = koff | ((uint64_t)L << 48);
-  pack_key((uint64_t *)(a.P.keys + a.kbase + koff), k, L);
-  const uint32_t nn = L - 1;  // real nibbles (0 for a rejected key)
-  if (!a.sk0) return;  // LockNU packs keys without sorting them
-  uint32_t W = a.scal[SC_W];
-  uint64_t h0 = W < nn ? ldn(k + W, min(8u, nn - W)) : 0ull;
-  uint64_t h1 = W + 8 < nn ? ldn(k + W + 8, min(8u, nn - W - 8)) : 0ull;
-  a.sk0[i] = sort_key(a, i, ((uint64_t)__builtin_bswap32(pack8(h0)) << 32) | __builtin_bswap32(pack8(h1)));
-  a.sv0[i] = i;
+  uint64_t diff = 0;
+  if (i < a.n) {
+    const uint32_t L = Li;
+    const uint8_t *k = key_range_ok(a, i) ? stg.at(a, a.kidx[2 * i]) : a.kh;
+    a.kref[i] = koff | ((uint64_t)L << 48);
+    pack_key((uint64_t *)(a.P.keys + a.kbase + koff), k, L);
+    const uint32_t nn = L - 1;  // real nibbles (0 for a rejected key)
+    if (a.sk0) {  // LockNU packs keys without sorting them
+      const uint32_t W = a.scal[SC_W];
+      const uint64_t key = sort_key(a, i, window_at(k, nn, W));
+      a.sk0[i] = key;
+      a.sv0[i] = i;
+      // klen[0] is 1 for a rejected key 0
+      diff = key ^ sort_key(a, 0, window_at(key_range_ok(a, 0) ? a.kh + a.kidx[0] : a.kh, a.klen[0] - 1, W));
+    }
+  }
+  if (a.sk0) note_varying(a, diff);
 }
 
 // Full-key sort support: word `w` (16 nibbles from W + 16w) of key sv[j], or
@@ -1907,9 +1947,11 @@ hipError_t nu_sort(NuArgs &a, int full, uint32_t trie_bits, void *temp, hipStrea
   const bool buckets = a.n <= kBucketCap || (a.n <= kBucketSortMaxN && trie_bits < 8 &&
                                              (a.n >> (8 - trie_bits)) <= kBucketSortMaxN / 256);
   if (!full && !win_all_bits && buckets) {
-    // whole keys (ties by input position) in one pass plus a sort of each
-    // top-8-bit bucket in LDS; a bucket too large for LDS asks for pass 1
-    e = bucket_sort_u64(k[cur], v[cur], k[cur ^ 1], v[cur ^ 1], a.n, &which, temp, s, &a.P.cnt->flag_fallback);
+    // whole keys (ties by input position) in one pass by the 8 highest varying
+    // bits plus a sort of each bucket in LDS; a bucket too large for LDS asks
+    // for pass 1
+    e = bucket_sort_u64(k[cur], v[cur], k[cur ^ 1], v[cur ^ 1], a.n, &which, temp, s, &a.P.cnt->flag_fallback,
+                        (const uint64_t *)(a.scal + SC_WVAR));
     if (e != hipSuccess) return e;
     cur ^= which;
   } else if (!full && !win_all_bits) {

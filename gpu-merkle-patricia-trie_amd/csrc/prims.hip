@@ -189,17 +189,55 @@ constexpr int kRsItems = 4;
 constexpr int kRsTile = kRsBlock * kRsItems;
 constexpr int kRsWaves = kRsBlock / 64;
 
+// The digit of a pass: eight bits from `shift` on, or, with a mask of the bits
+// that vary among the keys (in device memory; 0: not known), the eight highest
+// of those.  Keys with constant bits between the varying ones (ASCII digits:
+// every other nibble) then fill as many buckets as their values allow.
+struct Digit {
+  uint64_t m = 0;  // scattered bits to gather, or 0: eight in a row from shift
+  int shift;
+  __device__ __forceinline__ Digit(int s, const uint64_t *mask) : shift(s) {
+    if (mask) {
+      uint64_t v = *mask;
+      for (uint32_t k = 0; k < 8 && v; k++) {  // the same on every lane
+        const uint64_t b = 1ull << (63 - __clzll((long long)v));
+        m |= b;
+        v ^= b;
+      }
+      if (m == 0) return;  // not known: the top eight
+      const int lo = __ffsll((unsigned long long)m) - 1;
+      if (m >> lo == 255) {
+        shift = lo;
+        m = 0;
+      }
+    }
+  }
+  template <typename K>
+  __device__ __forceinline__ uint32_t of(K k) const {
+    if (m == 0) return (uint32_t)(k >> shift) & 255u;
+    uint32_t d = 0;
+    for (uint64_t v = m; v;) {
+      const int p = 63 - __clzll((long long)v);
+      d = d << 1 | ((uint32_t)((uint64_t)k >> p) & 1u);
+      v ^= 1ull << p;
+    }
+    return d;
+  }
+};
+
 template <typename K>
 __global__ __launch_bounds__(256) void k_rs_hist(const K *__restrict__ keys, size_t n, int shift,
-                                                 uint32_t *__restrict__ hist, uint32_t nblocks) {
+                                                 uint32_t *__restrict__ hist, uint32_t nblocks,
+                                                 const uint64_t *mask = nullptr) {
   __shared__ uint32_t h[256];
+  const Digit digit(shift, mask);
   h[threadIdx.x] = 0;
   __syncthreads();
   size_t base = (size_t)blockIdx.x * kRsTile;
 #pragma unroll
   for (int r = 0; r < kRsItems; r++) {
     size_t j = base + (size_t)r * kRsBlock + threadIdx.x;
-    if (j < n) atomicAdd(&h[(uint32_t)(keys[j] >> shift) & 255u], 1u);
+    if (j < n) atomicAdd(&h[digit.of(keys[j])], 1u);
   }
   __syncthreads();
   hist[(size_t)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
@@ -209,7 +247,8 @@ template <typename K>
 __global__ __launch_bounds__(256) void k_rs_scatter(const K *__restrict__ kin, const uint32_t *__restrict__ vin,
                                                     K *__restrict__ kout, uint32_t *__restrict__ vout, size_t n,
                                                     int shift, const uint32_t *__restrict__ goff,
-                                                    uint32_t nblocks) {
+                                                    uint32_t nblocks, const uint64_t *mask = nullptr) {
+  const Digit digit(shift, mask);
   __shared__ uint16_t cnt[kRsItems][kRsWaves][256];
   __shared__ K sk[kRsTile];
   __shared__ uint32_t sv[kRsTile];
@@ -234,7 +273,7 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const K *__restrict__ kin, c
     valid[r] = j < n;
     key[r] = valid[r] ? kin[j] : K(0);
     val[r] = valid[r] ? vin[j] : 0u;
-    dig[r] = (uint32_t)(key[r] >> shift) & 255u;
+    dig[r] = digit.of(key[r]);
     uint64_t m = __ballot(valid[r]);
 #pragma unroll
     for (int b = 0; b < 8; b++) {
@@ -278,7 +317,7 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const K *__restrict__ kin, c
     uint32_t i = r * kRsBlock + t;
     if (i < valid_n) {
       K k = sk[i];
-      uint32_t d = (uint32_t)(k >> shift) & 255u;
+      uint32_t d = digit.of(k);
       size_t dst = (size_t)goff[(size_t)d * nblocks + blockIdx.x] + (i - tstart[d]);
       kout[dst] = k;
       vout[dst] = sv[i];
@@ -314,23 +353,102 @@ hipError_t radix_impl(K *k0, uint32_t *v0, K *k1, uint32_t *v1, size_t n, int be
   return hipSuccess;
 }
 
-// One bucket of the top-8-bit pass per workgroup: bucket d spans
+// One bucket of the first pass per workgroup: bucket d spans
 // [goff[d * nblocks], goff[(d + 1) * nblocks]) of the pass's output (the
 // exclusive scan of the digit-major per-tile counts), or the whole array
-// without goff.  The bucket is counting-sorted in LDS by the next 12 key bits
-// (4,096 sub-buckets: about one entry each for a bucket of uniform keys);
-// then each entry counts the entries of its sub-bucket's run that are smaller
-// by (key, value), which is its place in the run.  A run's entries count side
-// by side, so a run of hundreds (keys of a few tries, or with a fixed field)
-// costs its length in LDS reads, where an insertion sort by one thread cost
-// its square.  A bucket with a run longer than kSubMaxRun is left as it came
-// and sets bit 1 of *overflow.
+// without goff.  The bucket is counting-sorted in LDS by the 12 highest bits
+// that vary among its keys (4,096 sub-buckets: about one entry each for keys
+// that spread evenly over those bits' values, constant bits between them or
+// not); then each entry counts the entries of its sub-bucket's run that are
+// smaller by (key, value), which is its place in the run.  With a run longer
+// than kSubMaxRun (a key repeated hundreds of times, keys that share a long
+// stretch) the counting would cost its square: the bucket is sorted instead by
+// all its varying bits, six at a time from the lowest, stably (it came in
+// value order), at about 4 us per six bits.  Only a bucket above kBucketCap
+// entries is left as it came, setting bit 1 of *overflow.
 constexpr int kBkThreads = 1024;
 constexpr uint32_t kBkPer = (uint32_t)(kBucketCap / kBkThreads);  // entries per thread
+constexpr uint32_t kBkWaves = kBkThreads / 64;
 constexpr uint32_t kSubs = 4096;
 constexpr uint32_t kSubPer = kSubs / kBkThreads;                    // sub-buckets per thread
-constexpr uint32_t kSubMaxRun = 1024;
+constexpr uint32_t kSubMaxRun = 64;
+constexpr uint32_t kLsdBits = 6;
+constexpr uint32_t kLsdCnts = (1u << kLsdBits) * kBkPer * kBkWaves;  // a count per digit, round and wave
 static_assert(kBucketCap % kBkThreads == 0 && kSubs % kBkThreads == 0, "bucket tiling");
+static_assert(kLsdCnts * sizeof(uint16_t) <= kSubs * sizeof(uint32_t) && kLsdCnts == 8 * kBkThreads,
+              "the counts fit the sub-bucket starts, eight per thread");
+
+// Exclusive scan of one value per thread over the block.
+__device__ __forceinline__ uint32_t bk_scan(uint32_t sum, uint32_t *wsum) {
+  const uint32_t t = threadIdx.x, incl = wave_inclusive_scan(sum);
+  if (__lane_id() == 63) wsum[t >> 6] = incl;
+  __syncthreads();
+  uint32_t base = 0;
+  for (uint32_t w = 0; w < (t >> 6); w++) base += wsum[w];
+  return base + incl - sum;
+}
+
+// The c entries (k, v in registers, entry t + q * kBkThreads of the bucket in
+// round q) sorted stably by the bits of var, in place.  Every thread of the
+// block calls it; the sorted entries end in sk, sv (after its last barrier).
+__device__ __forceinline__ void bk_lsd(uint64_t *k, uint32_t *v, uint32_t c, uint64_t var, uint64_t *sk, uint32_t *sv,
+                                       uint16_t *cnt, uint32_t *wsum) {
+  const uint32_t t = threadIdx.x, lane = __lane_id(), w = t >> 6;
+  const uint64_t below = (1ull << lane) - 1;
+  do {
+    uint64_t m = 0;  // this pass's bits: the lowest left (the same on every lane)
+    for (uint32_t j = 0; j < kLsdBits && var; j++) {
+      m |= var & (0ull - var);
+      var &= var - 1;
+    }
+    for (uint32_t j = t; j < kLsdCnts / 2; j += kBkThreads) ((uint32_t *)cnt)[j] = 0;
+    __syncthreads();
+    uint32_t dig[kBkPer], rank[kBkPer];
+#pragma unroll
+    for (uint32_t q = 0; q < kBkPer; q++) {
+      const bool in = t + q * kBkThreads < c;
+      uint64_t same = __ballot(in);
+      uint32_t d = 0, j = 0;
+      for (uint64_t x = m; x; x &= x - 1, j++) {
+        const bool bit = in && (k[q] & x & (0ull - x)) != 0;
+        const uint64_t bb = __ballot(bit);
+        same &= bit ? bb : ~bb;
+        d |= (uint32_t)bit << j;
+      }
+      dig[q] = (d * kBkPer + q) * kBkWaves + w;
+      rank[q] = (uint32_t)__popcll(same & below);
+      if (in && rank[q] == 0) cnt[dig[q]] = (uint16_t)__popcll(same);
+    }
+    __syncthreads();
+    uint32_t own[8], sum = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < 8; j++) {
+      own[j] = cnt[8 * t + j];
+      sum += own[j];
+    }
+    uint32_t x = bk_scan(sum, wsum);
+#pragma unroll
+    for (uint32_t j = 0; j < 8; j++) {
+      cnt[8 * t + j] = (uint16_t)x;
+      x += own[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t q = 0; q < kBkPer; q++)
+      if (t + q * kBkThreads < c) {
+        const uint32_t p = cnt[dig[q]] + rank[q];
+        sk[p] = k[q];
+        sv[p] = v[q];
+      }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t q = 0; q < kBkPer; q++)
+      if (t + q * kBkThreads < c) {
+        k[q] = sk[t + q * kBkThreads];
+        v[q] = sv[t + q * kBkThreads];
+      }
+  } while (var);
+}
 
 __global__ __launch_bounds__(1024) void k_bucket_sort(uint64_t *__restrict__ keys, uint32_t *__restrict__ vals,
                                                       uint32_t n, const uint32_t *__restrict__ goff,
@@ -338,7 +456,8 @@ __global__ __launch_bounds__(1024) void k_bucket_sort(uint64_t *__restrict__ key
   __shared__ uint64_t sk[kBucketCap];
   __shared__ uint32_t sv[kBucketCap];
   __shared__ uint32_t start[kSubs + 1];
-  __shared__ uint32_t wsum[kBkThreads / 64];
+  __shared__ uint32_t wsum[kBkWaves];
+  __shared__ uint64_t wvar[kBkWaves];
   const uint32_t d = blockIdx.x;
   const uint32_t lo = goff ? goff[(size_t)d * nblocks] : 0u;
   const uint32_t hi = goff && d + 1 < 256 ? goff[(size_t)(d + 1) * nblocks] : n;
@@ -348,21 +467,50 @@ __global__ __launch_bounds__(1024) void k_bucket_sort(uint64_t *__restrict__ key
     if (threadIdx.x == 0) atomicOr(overflow, 2u);
     return;
   }
-  // the sub-bucket bits: below the bucket's 8, or the top 12 of a single bucket
-  const int sub_shift = goff ? 44 : 52;
   const uint32_t t = threadIdx.x;
 #pragma unroll
   for (uint32_t j = 0; j < kSubPer; j++) start[t + j * kBkThreads] = 0;
-  __syncthreads();
   uint64_t k[kBkPer];
   uint32_t v[kBkPer], sub[kBkPer], pos[kBkPer];
+  // the bits that vary: those in which some key differs from the first
+  const uint64_t k0 = keys[lo];
+  uint64_t var = 0;
 #pragma unroll
   for (uint32_t q = 0; q < kBkPer; q++) {
     const uint32_t e = t + q * kBkThreads;
     if (e < c) {
       k[q] = keys[lo + e];
       v[q] = vals[lo + e];
-      sub[q] = (uint32_t)(k[q] >> sub_shift) & (kSubs - 1);
+      var |= k[q] ^ k0;
+    }
+  }
+  for (int off = 32; off > 0; off >>= 1) var |= (uint64_t)__shfl_xor((unsigned long long)var, off);
+  if (__lane_id() == 0) wvar[t >> 6] = var;
+  __syncthreads();  // and the counts cleared
+  var = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < kBkWaves; w++) var |= wvar[w];
+  // the 12 highest of them (the same on every lane): in a row from sub_shift,
+  // as for uniform keys, or gathered
+  uint64_t top = 0;
+  for (uint32_t j = 0; j < 12 && (var ^ top); j++) top |= 1ull << (63 - __clzll((long long)(var ^ top)));
+  const int sub_shift = top ? __ffsll((unsigned long long)top) - 1 : 0;
+  const bool row = ((top >> sub_shift) & ((top >> sub_shift) + 1)) == 0;
+#pragma unroll
+  for (uint32_t q = 0; q < kBkPer; q++) {
+    const uint32_t e = t + q * kBkThreads;
+    if (e < c) {
+      if (row) {
+        sub[q] = (uint32_t)((k[q] & top) >> sub_shift);
+      } else {
+        uint32_t x = 0;
+        for (uint64_t m = top; m;) {
+          const int p = 63 - __clzll((long long)m);
+          x = x << 1 | ((uint32_t)(k[q] >> p) & 1u);
+          m ^= 1ull << p;
+        }
+        sub[q] = x;
+      }
       pos[q] = atomicAdd(&start[sub[q]], 1u);
     }
   }
@@ -374,14 +522,9 @@ __global__ __launch_bounds__(1024) void k_bucket_sort(uint64_t *__restrict__ key
     cnt[j] = start[kSubPer * t + j];
     sum += cnt[j];
   }
-  const uint32_t incl = wave_inclusive_scan(sum);
-  if (__lane_id() == 63) wsum[t >> 6] = incl;
-  __syncthreads();
-  uint32_t base = 0;
-  for (uint32_t w = 0; w < (t >> 6); w++) base += wsum[w];
   bool long_run = false;
   {
-    uint32_t x = base + incl - sum;
+    uint32_t x = bk_scan(sum, wsum);
 #pragma unroll
     for (uint32_t j = 0; j < kSubPer; j++) {
       start[kSubPer * t + j] = x;  // only this thread reads or writes these entries here
@@ -390,10 +533,16 @@ __global__ __launch_bounds__(1024) void k_bucket_sort(uint64_t *__restrict__ key
     }
     if (t + 1 == kBkThreads) start[kSubs] = x;
   }
-  // a run too long to rank: the bucket stays as it came (in the previous
-  // pass's stable order, which the caller's other sort relies on)
   if (__syncthreads_or(long_run)) {
-    if (t == 0) atomicOr(overflow, 2u);
+    bk_lsd(k, v, c, var, sk, sv, (uint16_t *)start, wsum);
+#pragma unroll
+    for (uint32_t q = 0; q < kBkPer; q++) {
+      const uint32_t e = t + q * kBkThreads;
+      if (e < c) {
+        keys[lo + e] = k[q];
+        vals[lo + e] = v[q];
+      }
+    }
     return;
   }
 #pragma unroll
@@ -438,7 +587,7 @@ __global__ __launch_bounds__(1024) void k_bucket_sort(uint64_t *__restrict__ key
 }  // namespace
 
 hipError_t bucket_sort_u64(uint64_t *k0, uint32_t *v0, uint64_t *k1, uint32_t *v1, size_t n, int *which, void *temp,
-                           hipStream_t s, uint32_t *overflow) {
+                           hipStream_t s, uint32_t *overflow, const uint64_t *varying) {
   *which = 0;
   if (n <= 1) return hipSuccess;
   if (n > kBucketSortMaxN) return hipErrorInvalidValue;
@@ -449,11 +598,11 @@ hipError_t bucket_sort_u64(uint64_t *k0, uint32_t *v0, uint64_t *k1, uint32_t *v
   const uint32_t nb = (uint32_t)((n + kRsTile - 1) / kRsTile);
   uint32_t *hist = (uint32_t *)temp;
   uint32_t *scan_tmp = hist + (size_t)256 * nb + 16;
-  k_rs_hist<uint64_t><<<nb, kRsBlock, 0, s>>>(k0, n, 56, hist, nb);
+  k_rs_hist<uint64_t><<<nb, kRsBlock, 0, s>>>(k0, n, 56, hist, nb, varying);
   GMPT_LAUNCH_CHECK();
   hipError_t e = scan_impl<uint32_t>(hist, hist, (size_t)256 * nb, nullptr, scan_tmp, s);
   if (e != hipSuccess) return e;
-  k_rs_scatter<uint64_t><<<nb, kRsBlock, 0, s>>>(k0, v0, k1, v1, n, 56, hist, nb);
+  k_rs_scatter<uint64_t><<<nb, kRsBlock, 0, s>>>(k0, v0, k1, v1, n, 56, hist, nb, varying);
   GMPT_LAUNCH_CHECK();
   k_bucket_sort<<<256, kBkThreads, 0, s>>>(k1, v1, (uint32_t)n, hist, nb, overflow);
   GMPT_LAUNCH_CHECK();

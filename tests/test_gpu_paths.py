@@ -197,3 +197,37 @@ def test_dirty_nodes_split_before_they_are_hashed(gmpt, workloads, oracle, modes
     for o in os_:
         o.hash()
     assert f.get_root_hashes() == [o.root() for o in os_]
+
+
+@pytest.mark.parametrize("n", [2, 64, 66, 700, 8191, 8192, 8193, 30_000])
+@pytest.mark.parametrize("shape", ["digits", "hot", "hot-digits", "field", "ends", "one-key"])
+@pytest.mark.parametrize("tries", [1, 200])
+def test_sort_by_the_bits_that_vary(gmpt, workloads, oracle, n, shape, tries):
+    # one workgroup's capacity (8,192) and the first pass above it; runs up to
+    # 64 and longer: decimal digits behind a common prefix, a key repeated in a
+    # third of the batch (the last write stands), keys equal but for a few bits
+    # at the window's end, all writes to one key
+    rng = np.random.default_rng(n + len(shape) + tries)
+    if shape in ("digits", "hot-digits"):
+        keys = [b"user%019d" % int(x) for x in rng.integers(0, 10 * n, n)]
+    elif shape == "field":  # every other byte the same
+        k = rng.integers(0, 256, (n, 24), dtype=np.uint8)
+        k[:, ::2] = 0x5A
+        keys = [bytes(r) for r in k]
+    elif shape == "ends":
+        keys = [b"\x11" * 6 + int(x).to_bytes(2, "big") + bytes(4) for x in rng.integers(0, min(n, 60_000), n)]
+    elif shape == "one-key":
+        keys = [b"the only key"] * n
+    else:
+        keys = [bytes(r) for r in rng.integers(0, 256, (n, 32), dtype=np.uint8)]
+    if shape.startswith("hot"):
+        for i in rng.choice(n, n // 3, replace=False):
+            keys[i] = keys[0]
+    b = workloads.batch_from_bytes(keys, [b"%d" % i * (1 + i % 5) for i in range(n)])
+    b.trie_ids = np.full(n, tries // 2, np.int32) if tries > 1 and n % 2 else rng.integers(0, tries, n).astype(np.int32)
+    f = gmpt.MPT(device=0, num_tries=tries)
+    _put(f, b)
+    roots = f.get_root_hashes()
+    for t in sorted(set(b.trie_ids.tolist()))[:: 1 + tries // 12]:
+        assert roots[t] == oracle.root_of(b.subset(np.flatnonzero(b.trie_ids == t))), t
+    assert _put(f, b, "latching") == roots[0]
