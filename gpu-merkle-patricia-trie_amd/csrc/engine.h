@@ -136,7 +136,7 @@ class Forest {
   uint32_t ntries() const { return ntries_; }
   uint64_t pool_bytes_used() const;
   uint64_t pool_bytes_reserved() const;
-  const OpStats &stats() const { return stats_; }
+  const OpStats &stats();  // waits for the last hash pass's timing events
   hipStream_t stream() const { return stream_; }
   int device() const { return device_; }
   Pools pools() const;
@@ -160,9 +160,16 @@ class Forest {
   void drop_graph();
   bool is_pool(const DevBuf &b) const;
   void release(DevBuf &b);
-  // Reads the counters back (raising a kernel's error); with mark, the host
-  // waits for that event, recorded after the read, instead of the stream.
-  int sync_counters(hipEvent_t mark = nullptr);
+  // Reads the counters back (raising a kernel's error), after everything
+  // queued on the stream.
+  int sync_counters();
+  // The same without waiting for the stream: the last kernel queued, or one
+  // launched here, sends the counters to the host, which waits for their
+  // number.  (Copies to pageable host memory need sync_counters.)
+  Publish next_publish();
+  int await_counters(const Publish &pub);
+  int publish_and_await();
+  int take_counters();
   bool grow_key_arena_after_error();
   // With defer, a host batch large enough for the pinned stager leaves its
   // values out and describes them in *defer (bytes 0 when nothing is left):
@@ -172,7 +179,8 @@ class Forest {
   int sort_unique(NuArgs &a, void *temp, int pass, int *cur);
   int next_pass(int pass);
   void finish_build(const NuArgs &a);
-  int merge_sorted(NuArgs &a, void *temp);
+  int build_sorted(NuArgs &a, void *temp, bool empty);
+  int merge_groups(NuArgs &a, void *temp);
   bool bulk_fits(const BatchDesc &b) const;
   uint8_t *value_space(uint64_t bytes);
 
@@ -185,6 +193,9 @@ class Forest {
   DevBuf branch_, shrt_, value_, keys_, tries_, dirty_;
   Counters *d_cnt_ = nullptr;
   Counters *h_cnt_ = nullptr;  // pinned
+  uint32_t *h_seq_ = nullptr;  // pinned, after h_cnt_: number of the counters' last publication
+  uint32_t pub_seq_ = 0;
+  bool scal_zero_ = false;     // the device scalars are zero (left so by a hash pass or a clear)
   uint32_t *h_scal_ = nullptr; // pinned
   Counters cnt_{};             // host mirror after the last sync
   uint64_t key_used_ = 0;
@@ -212,6 +223,7 @@ class Forest {
   bool pool_host_ = false;
   LeafRecords rec_;              // bins the last build recorded for its new leaves (in ws_)
   hipEvent_t ev0_ = nullptr, ev1_ = nullptr;  // around a hash pass (after the bins' copy; after the counters' read)
+  hipEvent_t hash_from_ = nullptr, leaf_from_ = nullptr;  // start events of times stats() has not read yet
   hipEvent_t ev2_ = nullptr, ev3_ = nullptr;  // around the leaf level's permutation kernel
   hipEvent_t ev_meta_ = nullptr;               // the classification bins have reached the host
   hipEvent_t meta_mark_ = nullptr;             // the event hash() recorded after the bins' copy (ev0_ or ev_meta_)

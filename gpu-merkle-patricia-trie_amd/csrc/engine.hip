@@ -71,7 +71,10 @@ Forest::Forest(int device, uint32_t ntries) : device_(device), ntries_(ntries) {
   }
   if (hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking) != hipSuccess) return;
   if (hipMalloc(&d_cnt_, sizeof(Counters)) != hipSuccess) return;
-  if (hipHostMalloc(&h_cnt_, sizeof(Counters)) != hipSuccess) return;
+  constexpr size_t kSeqAt = (sizeof(Counters) + 63) / 64 * 64;
+  if (hipHostMalloc(&h_cnt_, kSeqAt + 64) != hipSuccess) return;
+  memset(h_cnt_, 0, kSeqAt + 64);
+  h_seq_ = (uint32_t *)((uint8_t *)h_cnt_ + kSeqAt);
   if (hipHostMalloc(&h_scal_, 64) != hipSuccess) return;
   if (hipMemset(d_cnt_, 0, sizeof(Counters)) != hipSuccess) return;
   if (hipEventCreate(&ev0_) != hipSuccess || hipEventCreate(&ev1_) != hipSuccess) return;
@@ -270,16 +273,47 @@ int Forest::ensure_pools(uint64_t nb, uint64_t ns, uint64_t nv, uint64_t key_byt
   return 0;
 }
 
-int Forest::sync_counters(hipEvent_t mark) {
+int Forest::sync_counters() {
   HIP_TRY(hipMemcpyAsync(h_cnt_, d_cnt_, sizeof(Counters), hipMemcpyDeviceToHost, stream_));
-  if (mark) {
-    // the host waits for the caller's event, recorded after the copy: one
-    // packet instead of a synchronisation marker beside the event's own
-    HIP_TRY(hipEventRecord(mark, stream_));
-    HIP_TRY(hipEventSynchronize(mark));
-  } else {
-    HIP_TRY(hipStreamSynchronize(stream_));
+  HIP_TRY(hipStreamSynchronize(stream_));
+  return take_counters();
+}
+
+// An empty Publish where the host mirror is no pinned memory (a forest over a
+// fixed region): then the counters are copied.
+Publish Forest::next_publish() {
+  Publish p;
+  if (h_seq_) {
+    p.host = h_cnt_;
+    p.seq = h_seq_;
+    p.val = ++pub_seq_;
   }
+  return p;
+}
+
+int Forest::await_counters(const Publish &pub) {
+  if (!pub.host) return sync_counters();
+  // A small operation ends within microseconds of the host's wait; after a few
+  // milliseconds the runtime waits (and reports a failed launch).
+  for (uint32_t spins = 0; __atomic_load_n(pub.seq, __ATOMIC_ACQUIRE) != pub.val; spins++) {
+    if (spins >= 1u << 20) {
+      HIP_TRY(hipStreamSynchronize(stream_));
+      if (__atomic_load_n(pub.seq, __ATOMIC_ACQUIRE) == pub.val) break;
+      set_error("the counters did not reach the host");
+      return -1;
+    }
+    __builtin_ia32_pause();
+  }
+  return take_counters();
+}
+
+int Forest::publish_and_await() {
+  const Publish pub = next_publish();
+  if (pub.host) HIP_TRY(publish_counters(d_cnt_, pub, stream_));
+  return await_counters(pub);
+}
+
+int Forest::take_counters() {
   cnt_ = *h_cnt_;
   if (cnt_.err != ERR_NONE) {
     uint32_t code = cnt_.err, arg = cnt_.err_arg;
@@ -504,7 +538,8 @@ int Forest::carve_nu(NuArgs &a, const BatchDesc &d, uint64_t vbase, bool has_tid
     set_error("workspace carve overflow");
     return -4;
   }
-  HIP_TRY(nu_init_scalars(a, stream_));
+  if (!scal_zero_) HIP_TRY(nu_init_scalars(a, stream_));
+  scal_zero_ = false;
   return 0;
 }
 
@@ -523,7 +558,7 @@ int Forest::sort_unique(NuArgs &a, void *temp, int pass, int *cur) {
   int nwords = 0;
   int r;
   if (pass == 2) {
-    if ((r = sync_counters())) return r;
+    if ((r = publish_and_await())) return r;
     uint32_t W = cnt_.scal[SC_W], maxlen = cnt_.scal[SC_MAXLEN];
     nwords = (int)((maxlen > W ? maxlen - W : 1) + 15) / 16;
   }
@@ -534,7 +569,7 @@ int Forest::sort_unique(NuArgs &a, void *temp, int pass, int *cur) {
     uint64_t m = *(const uint64_t *)(cnt_.scal + SC_WVAR);  // when the packing pass noted them
     if (m == 0) {
       HIP_TRY(nu_window_mask(a, *cur ? a.sk1 : a.sk0, stream_));
-      if ((r = sync_counters())) return r;
+      if ((r = publish_and_await())) return r;
       const uint64_t wor = *(const uint64_t *)(cnt_.scal + SC_WOR), wand = *(const uint64_t *)(cnt_.scal + SC_WAND);
       m = wor & ~wand;
     }
@@ -587,19 +622,30 @@ void Forest::finish_build(const NuArgs &a) {
   dirty_holes_ += cnt_.scal[SC_NREP_TOT] - cnt_.scal[SC_NEXT];
 }
 
-// After the descent's counter read: the rest of an insert into tries that
-// are not empty.
-int Forest::merge_sorted(NuArgs &a, void *temp) {
+// The sorted, deduplicated keys into the tries: descent (or, into empty tries,
+// the groups alone), element sequence and build, without a wait in between
+// (the build's kernels skip themselves while the sort asks for another pass,
+// groups are to be merged or an error is pending).
+int Forest::build_sorted(NuArgs &a, void *temp, bool empty) {
+  HIP_TRY(nu_descend_and_group(a, temp, stream_, empty));
+  HIP_TRY(nu_emit(a, temp, stream_, empty));
+  HIP_TRY(nu_build(a, temp, stream_, empty));
+  return 0;
+}
+
+// After the build's counter read: a split group that straddles a subtree makes
+// every group contiguous and builds again.
+int Forest::merge_groups(NuArgs &a, void *temp) {
   int r;
   if (cnt_.scal[SC_MERGE]) {
-    // a split group straddles a subtree: make every group contiguous
-    uint32_t m = cnt_.scal[SC_M_UNIQ];
+    const uint32_t m = cnt_.scal[SC_M_UNIQ];
+    HIP_TRY(hipMemsetAsync(a.scal + SC_MERGE, 0, 4, stream_));
     HIP_TRY(nu_regroup(a, m, m, temp, stream_));
     stats_.regroups++;
+    HIP_TRY(nu_emit(a, temp, stream_, false));
+    HIP_TRY(nu_build(a, temp, stream_, false));
+    if ((r = publish_and_await())) return r;
   }
-  HIP_TRY(nu_emit(a, temp, stream_, false));
-  HIP_TRY(nu_build(a, temp, stream_, false));
-  if ((r = sync_counters())) return r;
   finish_build(a);
   return 0;
 }
@@ -650,14 +696,7 @@ int Forest::puts_2phase(const BatchDesc &b, void **targets, int *n_targets) {
       int cur = 0;
       for (int pass = 0; pass >= 0;) {
         if ((r = sort_unique(a, temp, pass, &cur))) break;
-        HIP_TRY(nu_descend_and_group(a, temp, stream_, empty));
-        if (empty) {
-          // into empty tries no group needs merging: the build follows at
-          // once (its kernels skip themselves while the sort asks for another
-          // pass or an error is pending), one synchronisation per pass
-          HIP_TRY(nu_emit(a, temp, stream_, true));
-          HIP_TRY(nu_build(a, temp, stream_, true));
-        }
+        if ((r = build_sorted(a, temp, empty))) return r;
         if (vals.bytes) {
           // no insert kernel reads value bytes (only their index pairs): the
           // values cross PCIe on the second stream while they run, and the
@@ -667,7 +706,7 @@ int Forest::puts_2phase(const BatchDesc &b, void **targets, int *n_targets) {
           HIP_TRY(hipStreamWaitEvent(stream_, side_.join, 0));
           vals.bytes = 0;
         }
-        if ((r = sync_counters())) break;
+        if ((r = publish_and_await())) break;
         pass = next_pass(pass);
         if (pass >= 0) {
           // redo from the sort; marks the discarded descent made are on the
@@ -679,10 +718,7 @@ int Forest::puts_2phase(const BatchDesc &b, void **targets, int *n_targets) {
       if (r == 0) break;
       if (run > 0 || !grow_key_arena_after_error()) return r;
     }
-    if (empty)
-      finish_build(a);
-    else if ((r = merge_sorted(a, temp)))
-      return r;
+    if ((r = merge_groups(a, temp))) return r;
   }
   if (targets) *targets = dirty_.p;
   if (n_targets) *n_targets = (int)cnt_.n_dirty;
@@ -697,6 +733,7 @@ int Forest::hash(void *targets, int n_targets) {
     return -3;
   }
   (void)n_targets;  // the whole dirty list is hashed: a subset would leave stale ancestors
+  hash_from_ = leaf_from_ = nullptr;
   const uint32_t n = cnt_.n_dirty;
   // The climb's waves use the spread layout, which hc_spread_max 0 turns off,
   // and its counts are atomics on the nodes, which host pools do not get.
@@ -721,9 +758,11 @@ int Forest::hash_tree(uint32_t n, bool *done) {
   tree_zero_ = false;
   if (ev0_) HIP_TRY(hipEventRecord(ev0_, stream_));
   HIP_TRY(hc_tree(pools(), (const ref_t *)dirty_.p, n, (ref_t *)hc_sorted_.p, (ref_t *)hc_enc_.p, tree, stream_));
-  HIP_TRY(hc_roots(pools(), ntries_, nullptr, stream_, tree));
-  if ((r = sync_counters(ev0_ ? ev1_ : nullptr))) return r;
-  tree_zero_ = true;
+  const Publish pub = next_publish();
+  HIP_TRY(hc_roots(pools(), ntries_, nullptr, stream_, tree, pub));
+  if (ev0_) HIP_TRY(hipEventRecord(ev1_, stream_));
+  if ((r = await_counters(pub))) return r;
+  tree_zero_ = scal_zero_ = true;
   if (cnt_.hc_nodes != cnt_.hc_listed) return 0;
   *done = true;
   rec_ = LeafRecords();
@@ -736,11 +775,7 @@ int Forest::hash_tree(uint32_t n, bool *done) {
   stats_.leaf_perms = cnt_.leaf_perms;
   stats_.leaf_bytes = cnt_.leaf_bytes;
   stats_.leaf_perm_ms = stats_.last_hash_ms = 0;
-  if (ev0_) {
-    float ms = 0;
-    HIP_TRY(hipEventElapsedTime(&ms, ev0_, ev1_));
-    stats_.last_hash_ms = ms;
-  }
+  hash_from_ = ev0_;
   root0_ok_ = cnt_.root0_size <= 32;
   return 0;
 }
@@ -802,10 +837,13 @@ int Forest::hash_by_level(uint32_t n) {
     HIP_TRY(hc_count(encl, (const HcMeta *)hc_meta_.p, n, n_leaf, parts, stream_));
     stats_.leaf_nodes = n_leaf;
   }
-  HIP_TRY(hc_roots(pools(), ntries_, parts, stream_));  // also empties the dirty list
+  const Publish pub = next_publish();
+  HIP_TRY(hc_roots(pools(), ntries_, parts, stream_, nullptr, pub));  // also empties the dirty list
   rec_ = LeafRecords();
-  // ev1_ closes the hash timing after the roots and the counters' read
-  if ((r = sync_counters(n > 0 && ev0_ ? ev1_ : nullptr))) return r;
+  // ev1_ closes the hash timing after the roots and the counters' way out
+  if (n > 0 && ev0_) HIP_TRY(hipEventRecord(ev1_, stream_));
+  if ((r = await_counters(pub))) return r;
+  scal_zero_ = true;
   // the counters are zeroed by the classification, so only a pass that ran sets them
   stats_.perms = n ? cnt_.n_perms : 0;
   stats_.enc_bytes = n ? cnt_.enc_bytes : 0;
@@ -813,13 +851,8 @@ int Forest::hash_by_level(uint32_t n) {
   stats_.leaf_bytes = n ? cnt_.leaf_bytes : 0;
   stats_.leaf_perm_ms = 0;
   if (n > 0 && ev0_) {
-    float ms = 0;
-    HIP_TRY(hipEventElapsedTime(&ms, ev0_, ev1_));
-    stats_.last_hash_ms = ms;
-    if (stats_.leaf_nodes) {
-      HIP_TRY(hipEventElapsedTime(&ms, leaf_from_ev0 ? ev0_ : ev2_, ev3_));
-      stats_.leaf_perm_ms = ms;
-    }
+    hash_from_ = ev0_;
+    if (stats_.leaf_nodes) leaf_from_ = leaf_from_ev0 ? ev0_ : ev2_;
   }
   root0_ok_ = cnt_.root0_size <= 32;
   return 0;
@@ -896,6 +929,16 @@ int Forest::hash_levels(const Pools &P, const uint32_t *hist, bool direct_leaves
   return 0;
 }
 
+const OpStats &Forest::stats() {
+  float ms = 0;
+  if (hash_from_ && hipEventSynchronize(ev1_) == hipSuccess) {
+    if (hipEventElapsedTime(&ms, hash_from_, ev1_) == hipSuccess) stats_.last_hash_ms = ms;
+    if (leaf_from_ && hipEventElapsedTime(&ms, leaf_from_, ev3_) == hipSuccess) stats_.leaf_perm_ms = ms;
+  }
+  hash_from_ = leaf_from_ = nullptr;
+  return stats_;
+}
+
 int Forest::root_hash(uint32_t trie, uint8_t *out, int *size) {
   if (trie == 0 && ntries_ > 0 && root0_ok_) {  // no call since the last hash pass, whose counter read brought it
     *size = (int)cnt_.root0_size;
@@ -955,6 +998,7 @@ int Forest::clear() {
   HIP_TRY(hc_clear(d_cnt_, (TrieHdr *)tries_.p, ntries_, stream_));
   memset(&cnt_, 0, sizeof(cnt_));
   dirty_keys_ = dirty_holes_ = 0;
+  scal_zero_ = true;
   all_empty_ = true;
   key_used_ = 0;
   // keep the first value chunk, release the others
@@ -1278,7 +1322,7 @@ int Forest::puts_latching(const BatchDesc &b, void **targets, int *n_targets) {
       int cur = 0;
       for (int pass = 0; pass >= 0;) {
         if ((r = sort_unique(a, temp, pass, &cur))) break;
-        if ((r = sync_counters())) break;
+        if ((r = publish_and_await())) break;
         pass = next_pass(pass);
         if (pass >= 0) HIP_TRY(hipMemsetAsync(&d_cnt_->flag_fallback, 0, 4, stream_));
       }
@@ -1290,9 +1334,9 @@ int Forest::puts_latching(const BatchDesc &b, void **targets, int *n_targets) {
     if (!was_empty && m > cnt_.n_value / ntries_) {
       if ((r = ensure_pools(2ull * m + 2, 4ull * m + 4, 2ull * m + 2, d.key_slots))) return r;
       a.P = pools();
-      HIP_TRY(nu_descend_and_group(a, temp, stream_));
-      if ((r = sync_counters())) return r;
-      if ((r = merge_sorted(a, temp))) return r;
+      if ((r = build_sorted(a, temp, false))) return r;
+      if ((r = publish_and_await())) return r;
+      if ((r = merge_groups(a, temp))) return r;
       if (targets) *targets = dirty_.p;
       if (n_targets) *n_targets = (int)cnt_.n_dirty;
       return 0;
@@ -1300,7 +1344,7 @@ int Forest::puts_latching(const BatchDesc &b, void **targets, int *n_targets) {
     const uint64_t ktot = *(const uint64_t *)(cnt_.scal + SC_KTOT);
     const uint32_t values_before = cnt_.n_value;
     HIP_TRY(lock_insert(a, key_used_ + ktot, temp, stream_));
-    if ((r = sync_counters())) return r;
+    if ((r = publish_and_await())) return r;
     // only new keys' nodes refer to the batch's packed keys: a batch that
     // only overwrites leaves the arena where it was
     if (cnt_.n_value != values_before) key_used_ = align_up(key_used_ + ktot, 8);

@@ -89,6 +89,7 @@ int Forest::capture_rebuild(const BatchDesc &b) {
   if ((e = hc_clear(d_cnt_, (TrieHdr *)tries_.p, ntries_, stream_)) != hipSuccess) return fail(-1);
   NuArgs a;
   void *temp = nullptr;
+  scal_zero_ = false;  // the captured pass zeroes them itself
   if ((r = carve_nu(a, d, vbase, has_tid, &temp))) return fail(r);
   a.e_ident = has_tid ? 0u : 1u;  // the pass builds into emptied tries
   uint64_t *sk = nullptr;

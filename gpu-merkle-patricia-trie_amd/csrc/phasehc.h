@@ -131,8 +131,19 @@ hipError_t hc_tree(const Pools &P, const ref_t *list, uint32_t n, ref_t *ready, 
 // Copies every trie's root hash into its header and empties the dirty list;
 // with parts (from hc_count), adds the pass's work counts to the counters;
 // with tree (from hc_tree), sets them from it.
+// Then zeroes the insert's scalars for the next insert and, with pub, sends
+// the counters to the host as publish_counters does.
+struct Publish {
+  Counters *host = nullptr;  // pinned host memory
+  uint32_t *seq = nullptr;   // set to val once the counters are there
+  uint32_t val = 0;
+};
 hipError_t hc_roots(const Pools &P, uint32_t ntries, const unsigned long long *parts, hipStream_t s,
-                    TreeState *tree = nullptr);
+                    TreeState *tree = nullptr, Publish pub = Publish());
+// Copies the counters to pinned host memory and then stores val at seq, which
+// the host waits for: a launch of ours in place of a copy's blit kernel, and
+// no wait for the stream's completion signal.
+hipError_t publish_counters(const Counters *cnt, Publish pub, hipStream_t s);
 // Node export: encoding lengths, then encodings at offs and 32-byte hash slots.
 hipError_t hc_enc_len(const Pools &P, const ref_t *refs, uint32_t m, uint64_t *len, hipStream_t s);
 hipError_t hc_enc_write(const Pools &P, const ref_t *refs, uint32_t m, const uint64_t *offs, uint8_t *encs,

@@ -2065,8 +2065,30 @@ __global__ __launch_bounds__(256) void k_tree_climb(Pools P, const ref_t *__rest
              lane == 0 ? perms : lane == 1 ? bytes : lane == 2 ? lperms : lane == 3 ? lbytes : lane == 4 ? nodes : lnodes);
 }
 
+// One wave: the counters, then (once those stores have completed) the number.
+__device__ __forceinline__ void publish_wave(const Counters *cnt, const Publish &pub, uint32_t lane) {
+  constexpr uint32_t kWords = sizeof(Counters) / 4;
+  for (uint32_t q = lane; q < kWords; q += 64)
+    __hip_atomic_store((uint32_t *)pub.host + q, ((const uint32_t *)cnt)[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");  // system scope; the wave's lanes store and wait as one
+  if (lane == 0) __hip_atomic_store(pub.seq, pub.val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__global__ __launch_bounds__(64) void k_publish(const Counters *cnt, Publish pub) {
+  publish_wave(cnt, pub, threadIdx.x);
+}
+
+__device__ __forceinline__ void roots_body(const Pools &P, uint32_t ntries, const unsigned long long *parts,
+                                           TreeState *tree);
 __global__ __launch_bounds__(256) void k_hc_roots(Pools P, uint32_t ntries, const unsigned long long *parts,
-                                                  TreeState *tree) {
+                                                  TreeState *tree, Publish pub) {
+  roots_body(P, ntries, parts, tree);
+  if (grid_tid() < sizeof(P.cnt->scal) / 4) P.cnt->scal[grid_tid()] = 0;
+  if (!pub.host) return;
+  __syncthreads();  // one block: its counters are complete
+  if (threadIdx.x < 64) publish_wave(P.cnt, pub, threadIdx.x);
+}
+__device__ __forceinline__ void roots_body(const Pools &P, uint32_t ntries, const unsigned long long *parts,
+                                           TreeState *tree) {
   uint32_t t = grid_tid();
   // the root's hash first: its two dependent loads overlap the counts' reduction
   uint32_t hs = 0;
@@ -2409,8 +2431,16 @@ hipError_t hc_clear(Counters *cnt, TrieHdr *tries, uint32_t ntries, hipStream_t 
   return hipGetLastError();
 }
 
-hipError_t hc_roots(const Pools &P, uint32_t ntries, const unsigned long long *parts, hipStream_t s, TreeState *tree) {
-  k_hc_roots<<<nblk(ntries), kB, 0, s>>>(P, ntries, parts, tree);
+hipError_t hc_roots(const Pools &P, uint32_t ntries, const unsigned long long *parts, hipStream_t s, TreeState *tree,
+                    Publish pub) {
+  const bool one = nblk(ntries) == 1;
+  k_hc_roots<<<nblk(ntries), kB, 0, s>>>(P, ntries, parts, tree, one ? pub : Publish());
+  GMPT_LAUNCH_CHECK();
+  return one || !pub.host ? hipSuccess : publish_counters(P.cnt, pub, s);
+}
+
+hipError_t publish_counters(const Counters *cnt, Publish pub, hipStream_t s) {
+  k_publish<<<1, 64, 0, s>>>(cnt, pub);
   return hipGetLastError();
 }
 

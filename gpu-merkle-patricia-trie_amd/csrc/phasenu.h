@@ -134,7 +134,7 @@ enum {
   SC_WVAR = 20 /* u64: sort key bits that vary across the batch, and no others vary (0: not known) */, SC_COUNT = 22
 };
 
-// Zeroes the call's device scalars (SC_W starts at all ones for its minimum).
+// Zeroes the call's device scalars.
 hipError_t nu_init_scalars(const NuArgs &a, hipStream_t s);
 hipError_t nu_prepare_keys(const NuArgs &a, void *temp, hipStream_t s);
 // Sorts the batch: by the 16-nibble windows (full = 0; first by their top bits

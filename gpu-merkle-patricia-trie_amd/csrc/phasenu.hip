@@ -1117,7 +1117,16 @@ __device__ __forceinline__ Emit emit_of(const NuArgs &a, uint32_t i, uint32_t m)
   return e;
 }
 
+// An insert's kernels from here on run before the host has seen how the sort
+// and the grouping went: they skip while the sort asks for another pass, the
+// groups are to be merged (nu_regroup) or an error is pending, and the host
+// runs them again.
+__device__ __forceinline__ bool build_waits(const NuArgs &a) {
+  return a.P.cnt->flag_fallback || a.P.cnt->err || a.scal[SC_MERGE];
+}
+
 __global__ __launch_bounds__(256) void k_emit_count(NuArgs a) {
+  if (build_waits(a)) return;
   uint32_t i = grid_tid();
   uint32_t m = a.scal[SC_M_UNIQ];
   if (i >= a.n) return;
@@ -1133,6 +1142,7 @@ __global__ __launch_bounds__(256) void k_emit_count(NuArgs a) {
 // split point q (between E[q] and E[q+1]), lcp(E[q], E[q+1]) + 1, or 0 across
 // a group boundary.
 __global__ __launch_bounds__(256) void k_emit_write(NuArgs a) {
+  if (build_waits(a)) return;
   uint32_t i = grid_tid();
   uint32_t m = a.scal[SC_M_UNIQ];
   if (i >= m) return;
@@ -1199,6 +1209,7 @@ constexpr int kMtMaxLevels = 8;  // 16^8 split points
 // Level k from level k - 1, one entry per thread (entries past the level's
 // valid count are never read by a query).
 __global__ __launch_bounds__(256) void k_mt_level(NuArgs a, int k) {
+  if (build_waits(a)) return;
   const uint32_t b = grid_tid();
   const uint32_t ne = a.scal[SC_NE];
   uint32_t cnt = ne > 0 ? ne - 1 : 0;  // valid entries of level k - 1
@@ -1390,9 +1401,7 @@ __device__ __forceinline__ ST st_window(const ST &g, uint32_t t0, uint8_t *w, ui
 // points (plohi).  The queries run on the workgroup's window of split points
 // in LDS.
 __global__ __launch_bounds__(256) void k_split_reps(NuArgs a, uint32_t ne_max) {
-  // the sort needs a fallback pass, or an error is pending: the build waits
-  // for the host (which may run it before reading either)
-  if (a.P.cnt->flag_fallback || a.P.cnt->err) return;
+  if (build_waits(a)) return;
   static_assert(kSpTile == 256, "one split point per thread");
   __shared__ __align__(16) uint8_t win[kSpWinBytes];
   const uint32_t j = blockIdx.x * kSpTile + threadIdx.x;
@@ -1699,9 +1708,7 @@ struct OwnedLinks {
 };
 
 __global__ __launch_bounds__(256) void k_build_links(NuArgs a, int pre) {
-  // the sort needs a fallback pass, or an error is pending: the build waits
-  // for the host (which may run it before reading either)
-  if (a.P.cnt->flag_fallback || a.P.cnt->err) return;
+  if (build_waits(a)) return;
   static_assert(kSpTile == 256, "one split point per thread");
   static_assert(offsetof(Branch, hash_size) == 32 && offsetof(Branch, depth) == 34 && offsetof(Branch, dirty) == 36 &&
                     offsetof(Branch, lock) == 40 && offsetof(Branch, child) == 48 && sizeof(Branch) == 128,
@@ -1783,7 +1790,7 @@ __global__ __launch_bounds__(256) void k_build_links(NuArgs a, int pre) {
 // The cross links of k_build_links (block b's in its segment of the list):
 // each into its parent's child slot, and counted in the parent's record.
 __global__ __launch_bounds__(256) void k_link_cross(NuArgs a) {
-  if (a.P.cnt->flag_fallback || a.P.cnt->err) return;
+  if (build_waits(a)) return;
   const uint32_t n = a.xcnt[blockIdx.x];
   for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) {
     const uint32_t x = blockIdx.x * kCrossPerBlock + k;
@@ -1799,6 +1806,7 @@ __global__ __launch_bounds__(256) void k_link_cross(NuArgs a) {
 // The key's value node is rewritten in place (no node is allocated per
 // update; only this key refers to it).
 __global__ __launch_bounds__(256) void k_updates(NuArgs a) {
+  if (build_waits(a)) return;
   uint32_t i = grid_tid();
   uint32_t m = a.scal[SC_M_UNIQ];
   if (i >= m) return;
@@ -1821,7 +1829,7 @@ __global__ __launch_bounds__(256) void k_updates(NuArgs a) {
 namespace {
 __global__ void k_init_scalars(uint32_t *scal) {
   uint32_t t = threadIdx.x;
-  if (t < SC_COUNT) scal[t] = t == SC_W ? 0xffffffffu : 0u;
+  if (t < SC_COUNT) scal[t] = 0;
 }
 }  // namespace
 
