@@ -31,6 +31,7 @@ struct BatchDesc {
   uint64_t values_total = 0;
   uint64_t key_slots = 0;                  // key arena bytes of the packed keys (set by stage_batch)
   bool on_device = false;                  // all pointers above are device pointers
+  bool pinned = false;                     // host batch in pinned memory (copied to the device as it is)
   bool adopt_values = false;               // device batch: nodes point into values_bytes (caller keeps it alive)
 };
 
@@ -86,7 +87,9 @@ class Forest {
   // A forest that allocates nothing: its device memory comes from `arena`,
   // its host mirrors from `host`, and it runs on `stream` (not owned).  It
   // keeps no timing events, so its stats carry no kernel times.
-  Forest(int device, uint32_t ntries, Arena *arena, HostMirror *host, hipStream_t stream);
+  // Batches of up to stage_cap bytes are packed in `stage` (host memory).
+  Forest(int device, uint32_t ntries, Arena *arena, HostMirror *host, hipStream_t stream, uint8_t *stage = nullptr,
+         size_t stage_cap = 0);
   ~Forest();
   bool ok() const { return init_ok_; }
 
@@ -144,7 +147,8 @@ class Forest {
  private:
   int set_device();
   int ensure_pools(uint64_t nb, uint64_t ns, uint64_t nv, uint64_t key_bytes);
-  int grow(DevBuf &b, size_t need, size_t keep);
+  int grow(DevBuf &b, size_t need, size_t keep, bool fill = true);
+  int ready_pin();
   int ensure_ws(DevBuf &b, size_t bytes);
   int arena_exhausted();
   // hash()'s two forms: a short dirty list as one climb (*done: every node
@@ -202,8 +206,16 @@ class Forest {
   uint64_t lock_seq_ = 1;    // LockNU order stamps (PhaseNU values carry 0)
   std::vector<DevBuf> vchunks_;
   size_t vchunk_used_ = 0;
-  DevBuf st_keys_, st_kidx_, st_vidx_, st_hps_, st_tid_;
+  DevBuf st_;                    // a host batch's arrays on the device (values apart)
   DevBuf ws_, ws2_, rw_;
+  // Pinned memory small host batches go through on their way to the device,
+  // and small results on theirs back.  An operation waits for its last kernel
+  // before it returns; stage_busy_ marks one that failed before it did.
+  void *pin_ = nullptr;
+  size_t pin_used_ = 0;
+  uint8_t *host_stage_ = nullptr;  // a forest over a fixed region: its caller's host memory for packing a batch
+  size_t host_stage_cap_ = 0;
+  bool stage_busy_ = false;
   HostStager *stager_ = nullptr; // pinned chunked staging of large host batches (made on first use)
   DevBuf hc_tree_;
   bool tree_zero_ = false;       // hc_tree_ holds zeroes (its state between passes)

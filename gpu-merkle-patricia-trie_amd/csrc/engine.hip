@@ -20,6 +20,11 @@ namespace gmpt {
 namespace {
 thread_local std::string g_err;
 
+// Pinned memory a forest packs host batches in.  Up to 1 MiB its allocation
+// costs a new forest 50 us at most (4 MiB: 300), and an array that does not
+// fit is large enough that the runtime's own copy is as fast.
+constexpr size_t kPinBytes = 1u << 20;
+
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // Carves aligned sub-buffers out of one workspace allocation.
@@ -93,22 +98,27 @@ Forest::Forest(int device, uint32_t ntries) : device_(device), ntries_(ntries) {
   init_ok_ = true;
 }
 
-Forest::Forest(int device, uint32_t ntries, Arena *arena, HostMirror *host, hipStream_t stream)
-    : device_(device), ntries_(ntries), arena_(arena), stream_(stream) {
+Forest::Forest(int device, uint32_t ntries, Arena *arena, HostMirror *host, hipStream_t stream, uint8_t *stage,
+               size_t stage_cap)
+    : device_(device), ntries_(ntries), arena_(arena), stream_(stream), host_stage_(stage), host_stage_cap_(stage_cap) {
   if (hipSetDevice(device) != hipSuccess) {
     set_error("hipSetDevice failed");
     return;
   }
+  // the counters, trie headers and climb state, cleared in one go
+  const size_t from = arena->used;
   d_cnt_ = (Counters *)arena->take(sizeof(Counters));
-  if (!d_cnt_) {
+  hc_tree_.p = arena->take(hc_tree_.cap = align_up(sizeof(TreeState), 256));
+  if (!d_cnt_ || !hc_tree_.p) {
     set_error("device scratch region too small for the counters");
     return;
   }
   h_cnt_ = &host->cnt;
   h_scal_ = host->scal;
   h_meta_ = &host->meta;
-  if (hipMemsetAsync(d_cnt_, 0, sizeof(Counters), stream_) != hipSuccess) return;
-  if (grow(tries_, sizeof(TrieHdr) * std::max<uint32_t>(ntries, 1), 0) != 0) return;
+  if (grow(tries_, sizeof(TrieHdr) * std::max<uint32_t>(ntries, 1), 0, false) != 0) return;
+  if (hipMemsetAsync(arena->base + from, 0, arena->used - from, stream_) != hipSuccess) return;
+  tree_zero_ = scal_zero_ = true;
   hc_spread_max_ = kHcSpreadMaxDefault;
   init_ok_ = true;
 }
@@ -120,14 +130,14 @@ Forest::~Forest() {
   drop_graph();
   release(plan_hist_);
   delete stager_;
-  DevBuf *bufs[] = {&branch_, &shrt_, &value_, &keys_, &tries_, &dirty_, &st_keys_, &st_kidx_, &st_vidx_,
-                    &st_hps_, &st_tid_, &ws_, &ws2_, &hc_sorted_, &hc_meta_, &hc_cursor_, &hc_slot_, &hc_enc_, &hc_scratch_,
+  DevBuf *bufs[] = {&branch_, &shrt_, &value_, &keys_, &tries_, &dirty_, &st_, &ws_, &ws2_, &hc_sorted_, &hc_meta_, &hc_cursor_, &hc_slot_, &hc_enc_, &hc_scratch_,
                     &hc_lmeta_, &hc_lmeta_tmp_, &hc_tree_, &rw_};
   for (DevBuf *b : bufs) release(*b);
   for (DevBuf &b : vchunks_) release(b);
   if (d_cnt_) (void)hipFree(d_cnt_);
   if (h_cnt_) (void)hipHostFree(h_cnt_);
   if (h_scal_) (void)hipHostFree(h_scal_);
+  if (pin_) (void)hipHostFree(pin_);
   if (h_meta_) (void)hipHostFree(h_meta_);
   if (ev0_) (void)hipEventDestroy(ev0_);
   if (ev1_) (void)hipEventDestroy(ev1_);
@@ -192,7 +202,8 @@ void Forest::release(DevBuf &b) {
 
 // Regrow a device buffer to at least `need` bytes, keeping the first `keep`.
 // With pool_memory = host, the trie's pools grow in pinned host memory.
-int Forest::grow(DevBuf &b, size_t need, size_t keep) {
+// fill = false leaves the rest of the buffer to the caller.
+int Forest::grow(DevBuf &b, size_t need, size_t keep, bool fill) {
   if (b.cap >= need) return 0;
   void *p = nullptr;
   size_t cap;
@@ -216,10 +227,10 @@ int Forest::grow(DevBuf &b, size_t need, size_t keep) {
   if (host) {
     HIP_TRY(hipStreamSynchronize(stream_));
     memset((uint8_t *)p + keep, 0, cap - keep);
-  } else {
+  } else if (fill) {
     HIP_TRY(hipMemsetAsync((uint8_t *)p + keep, 0, cap - keep, stream_));
   }
-  HIP_TRY(hipStreamSynchronize(stream_));
+  if (!arena_) HIP_TRY(hipStreamSynchronize(stream_));  // a region's memory is not given back: nothing to wait for
   release(b);
   b.p = p;
   b.cap = cap;
@@ -255,16 +266,31 @@ int Forest::ensure_ws(DevBuf &b, size_t bytes) {
   return 0;
 }
 
+// Makes the pinned memory free to write.
+int Forest::ready_pin() {
+  if (stage_busy_) {
+    HIP_TRY(hipStreamSynchronize(stream_));
+    stage_busy_ = false;
+  }
+  pin_used_ = 0;
+  if (!pin_) HIP_TRY(hipHostMalloc(&pin_, kPinBytes, hipHostMallocDefault));
+  return 0;
+}
+
 int Forest::ensure_pools(uint64_t nb, uint64_t ns, uint64_t nv, uint64_t key_bytes) {
   int r;
-  if ((r = grow(branch_, (cnt_.n_branch + nb) * sizeof(Branch), cnt_.n_branch * sizeof(Branch)))) return r;
-  if ((r = grow(shrt_, (cnt_.n_short + ns) * sizeof(Short), cnt_.n_short * sizeof(Short)))) return r;
-  if ((r = grow(value_, (cnt_.n_value + nv) * sizeof(Value), cnt_.n_value * sizeof(Value)))) return r;
-  if ((r = grow(keys_, key_used_ + key_bytes + 64, key_used_))) return r;
+  // a region's first pools lie side by side: one fill for all
+  const bool fresh = arena_ && !branch_.p && !shrt_.p && !value_.p && !keys_.p && !dirty_.p;
+  const size_t from = fresh ? arena_->used : 0;
+  if ((r = grow(branch_, (cnt_.n_branch + nb) * sizeof(Branch), cnt_.n_branch * sizeof(Branch), !fresh))) return r;
+  if ((r = grow(shrt_, (cnt_.n_short + ns) * sizeof(Short), cnt_.n_short * sizeof(Short), !fresh))) return r;
+  if ((r = grow(value_, (cnt_.n_value + nv) * sizeof(Value), cnt_.n_value * sizeof(Value), !fresh))) return r;
+  if ((r = grow(keys_, key_used_ + key_bytes + 64, key_used_, !fresh))) return r;
   // every existing node is listed at most once, a build adds at most
   // 3 entries (holes included) per slot it reserved
   size_t dcap = ((size_t)cnt_.n_dirty + cnt_.n_branch + cnt_.n_short + 2 * nb + ns + 64) * sizeof(ref_t);
-  if ((r = grow(dirty_, dcap, cnt_.n_dirty * sizeof(ref_t)))) return r;
+  if ((r = grow(dirty_, dcap, cnt_.n_dirty * sizeof(ref_t), !fresh))) return r;
+  if (fresh) HIP_TRY(hipMemsetAsync(arena_->base + from, 0, arena_->used - from, stream_));
   if ((uint64_t)(cnt_.n_branch + nb) > 0x3fffffffull || (uint64_t)(cnt_.n_short + ns) > 0x3fffffffull ||
       (uint64_t)(cnt_.n_value + nv) > 0x3fffffffull) {
     set_error("node pool exceeds 2^30 nodes of one kind");
@@ -315,6 +341,7 @@ int Forest::publish_and_await() {
 
 int Forest::take_counters() {
   cnt_ = *h_cnt_;
+  stage_busy_ = false;
   if (cnt_.err != ERR_NONE) {
     uint32_t code = cnt_.err, arg = cnt_.err_arg;
     HIP_TRY(hipMemsetAsync(&d_cnt_->err, 0, 2 * sizeof(uint32_t), stream_));
@@ -372,61 +399,95 @@ int Forest::stage_batch(const BatchDesc &b, BatchDesc *d, uint64_t *vbase, bool 
       return -2;
     }
     if (staged) {
-      stager_->extents(b.keys_indexs, b.values_indexs, n, &kb, &vb, &ks, kMaxKeyNibbles);
+      stager_->extents(b.keys_indexs, copy_values ? b.values_indexs : nullptr, n, &kb, &vb, &ks, kMaxKeyNibbles);
     } else {
+      int64_t kmax = -1, vmax = -1;
       for (uint32_t i = 0; i < n; i++) {
         const int64_t s = b.keys_indexs[2 * (size_t)i], e = b.keys_indexs[2 * (size_t)i + 1];
-        if (e >= 0 && (uint64_t)e + 1 > kb) kb = (uint64_t)e + 1;
+        kmax = std::max(kmax, e);
         const int64_t L = (s >= 0 && e >= s && e - s < kMaxKeyNibbles) ? e - s + 1 : 1;
         ks += (uint64_t)((L / 2 + 8) & ~7ll);
-        if (b.values_indexs) {
-          int64_t ve = b.values_indexs[2 * (size_t)i + 1];
-          if (ve >= 0 && (uint64_t)ve + 1 > vb) vb = (uint64_t)ve + 1;
-        }
       }
+      for (uint32_t i = 0; copy_values && b.values_indexs && i < n; i++)
+        vmax = std::max(vmax, b.values_indexs[2 * (size_t)i + 1]);
+      kb = (uint64_t)(kmax + 1);
+      vb = (uint64_t)(vmax + 1);
     }
     d->keys_bytes = kb;
     d->values_total = vb;
     d->key_slots = ks;
     int r;
-    if ((r = ensure_ws(st_keys_, kb + 64))) return r;
-    if ((r = ensure_ws(st_kidx_, 8ull * n + 64))) return r;
-    if ((r = ensure_ws(st_vidx_, 16ull * n + 64))) return r;
+    // every array but the values side by side in one device buffer (256-byte
+    // aligned; the keys, often the largest, last), the values in the value
+    // arena
     StageSeg seg[6];
     int ns = 0;
-    seg[ns++] = {st_keys_.p, b.keys_hexs, kb};
-    seg[ns++] = {st_kidx_.p, b.keys_indexs, 8ull * n};
-    d->keys_hexs = (const uint8_t *)st_keys_.p;
-    d->keys_indexs = (const int32_t *)st_kidx_.p;
-    if (b.values_indexs) {
-      seg[ns++] = {st_vidx_.p, b.values_indexs, 16ull * n};
-      d->values_indexs = (const int64_t *)st_vidx_.p;
-    }
-    if (b.values_hps) {
-      if ((r = ensure_ws(st_hps_, 8ull * n + 64))) return r;
-      seg[ns++] = {st_hps_.p, b.values_hps, 8ull * n};
-      d->values_hps = (const uint64_t *)st_hps_.p;
-    }
-    if (b.trie_ids) {
-      if ((r = ensure_ws(st_tid_, 4ull * n + 64))) return r;
-      seg[ns++] = {st_tid_.p, b.trie_ids, 4ull * n};
-      d->trie_ids = (const int32_t *)st_tid_.p;
-    }
+    size_t at[6], off = 0;
+    const auto add = [&](const void *src, size_t bytes) {
+      at[ns] = off;
+      seg[ns++] = {nullptr, src, bytes};
+      off += align_up(bytes, 256);
+    };
+    add(b.keys_indexs, 8ull * n);
+    // reads have no use for value pairs
+    const int vi = copy_values && b.values_indexs ? ns : -1;
+    if (vi >= 0) add(b.values_indexs, 16ull * n);
+    const int hi = b.values_hps ? ns : -1;
+    if (hi >= 0) add(b.values_hps, 8ull * n);
+    const int ti = b.trie_ids ? ns : -1;
+    if (ti >= 0) add(b.trie_ids, 4ull * n);
+    const int ki = ns;
+    add(b.keys_hexs, kb);
+    if ((r = ensure_ws(st_, off + 64))) return r;
+    for (int q = 0; q < ns; q++) seg[q].dst = (uint8_t *)st_.p + at[q];
+    d->keys_indexs = (const int32_t *)seg[0].dst;
+    d->values_indexs = vi >= 0 ? (const int64_t *)seg[vi].dst : nullptr;
+    if (hi >= 0) d->values_hps = (const uint64_t *)seg[hi].dst;
+    if (ti >= 0) d->trie_ids = (const int32_t *)seg[ti].dst;
+    d->keys_hexs = (const uint8_t *)seg[ki].dst;
     d->on_device = true;
+    uint8_t *vs = nullptr;
     if (copy_values) {
-      uint8_t *vs = value_space(vb);
+      vs = value_space(vb);
       if (!vs) return -2;
-      if (staged && defer)
-        *defer = StageSeg{vs, b.values_bytes, vb};
-      else
-        seg[ns++] = {vs, b.values_bytes, vb};
       d->values_bytes = vs;
+      if (staged && defer) {
+        *defer = StageSeg{vs, b.values_bytes, vb};
+      } else {
+        at[ns] = off;
+        seg[ns++] = {vs, b.values_bytes, vb};
+      }
     }
+    // What fits is packed into pinned memory first (leaving room for a read's
+    // results): one copy from there costs the runtime about 10 us, one from
+    // pageable memory 15 to 60 per array (its bounce buffer, or pinning the
+    // pages), and the packing 1 us per 60 KB.
+    uint8_t *pin = host_stage_;
+    size_t cap = host_stage_cap_;
+    if (!staged && !b.pinned && !arena_) {
+      if ((r = ready_pin())) return r;
+      pin = (uint8_t *)pin_;
+      cap = copy_values ? kPinBytes : kPinBytes - std::min<size_t>(kPinBytes, 12ull * n + 256);
+    }
+    int packed = 0;  // the arrays packed, from the first on
+    while (!staged && !b.pinned && packed < ns && at[packed] + seg[packed].bytes <= cap) packed++;
     if (staged) {
       HIP_TRY(stager_->copy(stream_, seg, ns));
     } else {
-      for (int q = 0; q < ns; q++)
-        if (seg[q].bytes) HIP_TRY(hipMemcpyAsync(seg[q].dst, seg[q].src, seg[q].bytes, hipMemcpyDefault, stream_));
+      size_t end = 0;  // of the packed part of st_
+      for (int q = 0; q < packed; q++) {
+        if (seg[q].bytes) memcpy(pin + at[q], seg[q].src, seg[q].bytes);
+        pin_used_ = at[q] + seg[q].bytes;
+        if (!(copy_values && q + 1 == ns)) end = pin_used_;
+      }
+      stage_busy_ = packed > 0;
+      if (end) HIP_TRY(hipMemcpyAsync(st_.p, pin, end, hipMemcpyHostToDevice, stream_));
+      for (int q = 0; q < ns; q++) {
+        const bool value = copy_values && q + 1 == ns;
+        if (!seg[q].bytes || (q < packed && !value)) continue;
+        HIP_TRY(hipMemcpyAsync(seg[q].dst, q < packed ? (const void *)(pin + at[q]) : seg[q].src, seg[q].bytes,
+                               hipMemcpyDefault, stream_));
+      }
     }
   } else if (copy_values && !b.adopt_values) {
     uint8_t *vs = value_space(b.values_total);
@@ -967,6 +1028,17 @@ int Forest::root_hashes(uint32_t first, uint32_t count, uint8_t *out, int32_t *s
     return -3;
   }
   if (count == 0) return 0;
+  const size_t bytes = 36ull * count;
+  if (!arena_ && bytes <= kPinBytes) {  // gathered into pinned memory
+    if ((r = ready_pin())) return r;
+    uint8_t *h = (uint8_t *)pin_;
+    int32_t *s = (int32_t *)(h + 32ull * count);
+    HIP_TRY(gather_roots((const TrieHdr *)tries_.p + first, count, h, s, stream_));
+    if ((r = publish_and_await())) return r;
+    memcpy(out, h, 32ull * count);
+    memcpy(sizes, s, 4ull * count);
+    return 0;
+  }
   std::vector<TrieHdr> h(count);
   HIP_TRY(hipMemcpyAsync(h.data(), (TrieHdr *)tries_.p + first, sizeof(TrieHdr) * count, hipMemcpyDefault,
                          stream_));
@@ -1105,17 +1177,33 @@ int Forest::gets(const BatchDesc &keys, uint64_t *hps, int32_t *sizes) {
   BatchDesc d;
   uint64_t vb;
   if ((r = stage_batch(keys, &d, &vb, false))) return r;
-  if ((r = ensure_ws(ws2_, 16ull * n + 1024))) return r;
+  if ((r = ensure_ws(ws2_, 20ull * n + 1024))) return r;
   Carver c(ws2_.p);
-  uint64_t *d_hp = c.take<uint64_t>(n);
   uint64_t *d_addr = c.take<uint64_t>(n);
+  uint64_t *d_hp = c.take<uint64_t>(n);
   int32_t *d_size = c.take<int32_t>(n);
   if (c.off > ws2_.cap && (r = ensure_ws(ws2_, c.off))) return r;
+  // the kernel writes a small batch's results to pinned memory itself, past
+  // what is packed there of the batch
+  const size_t bytes = 12ull * n;
+  if (!arena_ && !stage_busy_ && (r = ready_pin())) return r;
+  const size_t from = align_up(pin_used_, 256);
+  const bool pin = !arena_ && from + bytes <= kPinBytes;
+  if (pin) {
+    d_hp = (uint64_t *)((uint8_t *)pin_ + from);
+    d_size = (int32_t *)(d_hp + n);
+  }
   GetArgs g{pools(), d.keys_hexs, d.keys_indexs, ntries_ > 1 ? d.trie_ids : nullptr, n, d.keys_bytes, ntries_, d_hp, d_addr, d_size};
   HIP_TRY(launch_gets(g, stream_));
-  if (hps) HIP_TRY(hipMemcpyAsync(hps, d_hp, 8ull * n, hipMemcpyDeviceToHost, stream_));
-  if (sizes) HIP_TRY(hipMemcpyAsync(sizes, d_size, 4ull * n, hipMemcpyDeviceToHost, stream_));
-  return sync_counters();
+  if (!pin) {
+    if (hps) HIP_TRY(hipMemcpyAsync(hps, d_hp, 8ull * n, hipMemcpyDeviceToHost, stream_));
+    if (sizes) HIP_TRY(hipMemcpyAsync(sizes, d_size, 4ull * n, hipMemcpyDeviceToHost, stream_));
+    return sync_counters();
+  }
+  if ((r = publish_and_await())) return r;
+  if (hps) memcpy(hps, d_hp, 8ull * n);
+  if (sizes) memcpy(sizes, d_size, 4ull * n);
+  return 0;
 }
 
 int Forest::puts_with_read(const BatchDesc &b, const uint8_t *rw_flags, int mode, uint32_t *read_num,

@@ -23,6 +23,11 @@ constexpr int kMaxDevices = 64;
 
 static __device__ __align__(256) uint8_t scratch[kScratchBytes];
 
+// Host memory a small batch is packed in, so that one copy takes it to the
+// device (a copy from pageable memory costs 15 us and more per array).
+constexpr size_t kStageBytes = 512u << 10;
+uint8_t g_stage[kMaxDevices][kStageBytes];
+
 std::mutex g_mu[kMaxDevices];        // one call at a time per device: they share its region
 uint8_t *g_ptr[kMaxDevices] = {};    // scratch's device address on each device (set under g_mu)
 
@@ -80,7 +85,7 @@ extern "C" int gmpt_build_root_noalloc(const gmpt_batch *b, int mode, uint8_t ou
   arena.cap = kScratchBytes;
   gmpt::HostMirror host;
   memset(&host, 0, sizeof(host));
-  gmpt::Forest f(dev, 1, &arena, &host, nullptr);
+  gmpt::Forest f(dev, 1, &arena, &host, nullptr, g_stage[dev], kStageBytes);
   if (!f.ok()) return -1;
   void *targets = nullptr;
   int nt = 0;

@@ -140,9 +140,11 @@ struct Publish {
 };
 hipError_t hc_roots(const Pools &P, uint32_t ntries, const unsigned long long *parts, hipStream_t s,
                     TreeState *tree = nullptr, Publish pub = Publish());
-// Copies the counters to pinned host memory and then stores val at seq, which
+// (publish_counters) Copies the counters to pinned host memory and then stores val at seq, which
 // the host waits for: a launch of ours in place of a copy's blit kernel, and
 // no wait for the stream's completion signal.
+// Root hashes (32-byte slots) and sizes of count tries, to pinned host memory.
+hipError_t gather_roots(const TrieHdr *tries, uint32_t count, uint8_t *hash, int32_t *size, hipStream_t s);
 hipError_t publish_counters(const Counters *cnt, Publish pub, hipStream_t s);
 // Node export: encoding lengths, then encodings at offs and 32-byte hash slots.
 hipError_t hc_enc_len(const Pools &P, const ref_t *refs, uint32_t m, uint64_t *len, hipStream_t s);

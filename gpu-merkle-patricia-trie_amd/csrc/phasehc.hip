@@ -2439,6 +2439,20 @@ hipError_t hc_roots(const Pools &P, uint32_t ntries, const unsigned long long *p
   return one || !pub.host ? hipSuccess : publish_counters(P.cnt, pub, s);
 }
 
+namespace {
+__global__ __launch_bounds__(256) void k_roots_out(const TrieHdr *tries, uint32_t count, uint64_t *hash, int32_t *size) {
+  const uint32_t i = grid_tid(), t = i / 4, q = i % 4;  // 8 bytes per thread: the slots are written in a row
+  if (t >= count) return;
+  hash[i] = ((const uint64_t *)tries[t].root_hash)[q];
+  if (q == 0) size[t] = (int32_t)tries[t].root_hash_size;
+}
+}  // namespace
+
+hipError_t gather_roots(const TrieHdr *tries, uint32_t count, uint8_t *hash, int32_t *size, hipStream_t s) {
+  k_roots_out<<<nblk(4 * (size_t)count), kB, 0, s>>>(tries, count, (uint64_t *)hash, size);
+  return hipGetLastError();
+}
+
 hipError_t publish_counters(const Counters *cnt, Publish pub, hipStream_t s) {
   k_publish<<<1, 64, 0, s>>>(cnt, pub);
   return hipGetLastError();

@@ -286,6 +286,7 @@ int Server::run_batch(Lane &L, const std::vector<Req *> &batch) {
   d.values_indexs = vidx;
   d.trie_ids = L.local_tries > 1 ? tid : nullptr;
   d.n = (uint32_t)n;
+  d.pinned = true;
   void *targets = nullptr;
   int nt = 0;
   rc = mode_ == 0 ? L.f->puts_2phase(d, &targets, &nt) : L.f->puts_latching(d, &targets, &nt);

@@ -352,7 +352,10 @@ class MPT:
         out = np.zeros(32 * max(count, 1), np.uint8)
         sz = np.zeros(max(count, 1), np.int32)
         _check(lib().gmpt_get_root_hashes(self._f, first, count, _p(out), _p(sz)))
-        return [out[32 * i:32 * i + sz[i]].tobytes() for i in range(count)]
+        roots = out.view("V32").tolist()[:count]  # bytes objects
+        if (sz[:count] == 32).all():
+            return roots
+        return [r[:k] for r, k in zip(roots, sz.tolist())]
 
     # --- gets (gpu_mpt.cuh:139-140) -------------------------------------------
     def gets_parallel(self, batch):

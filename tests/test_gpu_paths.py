@@ -231,3 +231,28 @@ def test_sort_by_the_bits_that_vary(gmpt, workloads, oracle, n, shape, tries):
     for t in sorted(set(b.trie_ids.tolist()))[:: 1 + tries // 12]:
         assert roots[t] == oracle.root_of(b.subset(np.flatnonzero(b.trie_ids == t))), t
     assert _put(f, b, "latching") == roots[0]
+
+
+@pytest.mark.parametrize("mode", list(PUTS))
+@pytest.mark.parametrize("n", [1, 3900, 4200, 11_000, 22_000, 45_000, 60_000, 90_000])
+def test_host_batches_around_the_pinned_packing(gmpt, workloads, oracle, mode, n):
+    # host batches whose arrays (8 to 65 bytes a key) pass the 1 MiB packed in
+    # pinned memory one after the other, with host pointers and trie ids, and
+    # reads whose results (12 bytes a key) fit behind them or do not
+    rng = np.random.default_rng(n)
+    keys = workloads.unique_random_keys(rng, n, 32)
+    flat, lens = workloads.random_values(rng, n, 0, 90)
+    b = workloads.batch_from_fixed(keys, flat, lens)
+    b.trie_ids = rng.integers(0, 2, n).astype(np.int32)
+    hps = rng.integers(1, 1 << 60, n).astype(np.uint64)
+    f = gmpt.MPT(device=0, num_tries=2)
+    targets, m = getattr(f, PUTS[mode])(b, hps)
+    f.hash_onepass_v2(targets, m)
+    assert f.get_root_hashes() == [oracle.root_of(b.subset(np.flatnonzero(b.trie_ids == t))) for t in range(2)]
+    got, sizes = f.gets_parallel(b)
+    assert (got == hps).all() and (sizes == lens).all()
+    absent = b.subset(range(n))
+    absent.trie_ids = 1 - b.trie_ids
+    got, sizes = f.gets_parallel(absent)
+    assert (got == 0).all() and (sizes == f.gets_parallel(absent.subset([0]))[1][0]).all()
+    assert f.get_values(b.subset(range(0, n, 1 + n // 9)))[0] == b.value(0)
