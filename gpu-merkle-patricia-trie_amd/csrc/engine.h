@@ -149,6 +149,12 @@ class Forest {
   int ensure_pools(uint64_t nb, uint64_t ns, uint64_t nv, uint64_t key_bytes);
   int grow(DevBuf &b, size_t need, size_t keep, bool fill = true);
   int ready_pin();
+  struct FetchSeg {
+    size_t at;   // bytes [at, at + bytes) of the device block
+    void *dst;   // host
+    size_t bytes;
+  };
+  int fetch(const void *src, size_t total, const FetchSeg *seg, int ns);
   int ensure_ws(DevBuf &b, size_t bytes);
   int arena_exhausted();
   // hash()'s two forms: a short dirty list as one climb (*done: every node
@@ -216,6 +222,8 @@ class Forest {
   uint8_t *host_stage_ = nullptr;  // a forest over a fixed region: its caller's host memory for packing a batch
   size_t host_stage_cap_ = 0;
   bool stage_busy_ = false;
+  DevBuf exp_map_, exp_ws_, exp_out_;  // node export: bitmap (zero between calls), references and offsets, results
+  bool exp_zero_ = false;
   HostStager *stager_ = nullptr; // pinned chunked staging of large host batches (made on first use)
   DevBuf hc_tree_;
   bool tree_zero_ = false;       // hc_tree_ holds zeroes (its state between passes)

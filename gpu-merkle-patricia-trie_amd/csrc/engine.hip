@@ -131,7 +131,7 @@ Forest::~Forest() {
   release(plan_hist_);
   delete stager_;
   DevBuf *bufs[] = {&branch_, &shrt_, &value_, &keys_, &tries_, &dirty_, &st_, &ws_, &ws2_, &hc_sorted_, &hc_meta_, &hc_cursor_, &hc_slot_, &hc_enc_, &hc_scratch_,
-                    &hc_lmeta_, &hc_lmeta_tmp_, &hc_tree_, &rw_};
+                    &hc_lmeta_, &hc_lmeta_tmp_, &hc_tree_, &rw_, &exp_map_, &exp_ws_, &exp_out_};
   for (DevBuf *b : bufs) release(*b);
   for (DevBuf &b : vchunks_) release(b);
   if (d_cnt_) (void)hipFree(d_cnt_);
@@ -277,6 +277,38 @@ int Forest::ready_pin() {
   return 0;
 }
 
+// Copies total bytes at src (device) through the two halves of the pinned
+// memory into the segments: the host empties one half while the other fills.
+int Forest::fetch(const void *src, size_t total, const FetchSeg *seg, int ns) {
+  int r;
+  if ((r = ready_pin())) return r;
+  constexpr size_t kHalf = kPinBytes / 2;
+  Publish pub[2];
+  const auto empty_half = [&](size_t p) -> int {
+    const size_t lo = p * kHalf, hi = std::min(total, lo + kHalf);
+    const uint8_t *h = (const uint8_t *)pin_ + (p & 1) * kHalf;
+    int e = await_counters(pub[p & 1]);
+    if (e) return e;
+    for (int q = 0; q < ns; q++) {
+      const size_t a = std::max(lo, seg[q].at), b = std::min(hi, seg[q].at + seg[q].bytes);
+      if (a < b) memcpy((uint8_t *)seg[q].dst + (a - seg[q].at), h + (a - lo), b - a);
+    }
+    return 0;
+  };
+  const size_t parts = (total + kHalf - 1) / kHalf;
+  for (size_t p = 0; p < parts + 1; p++) {
+    if (p < parts) {
+      const size_t lo = p * kHalf;
+      HIP_TRY(hipMemcpyAsync((uint8_t *)pin_ + (p & 1) * kHalf, (const uint8_t *)src + lo, std::min(total - lo, kHalf),
+                             hipMemcpyDeviceToHost, stream_));
+      pub[p & 1] = next_publish();
+      HIP_TRY(publish_counters(d_cnt_, pub[p & 1], stream_));
+    }
+    if (p > 0 && (r = empty_half(p - 1))) return r;
+  }
+  return 0;
+}
+
 int Forest::ensure_pools(uint64_t nb, uint64_t ns, uint64_t nv, uint64_t key_bytes) {
   int r;
   // a region's first pools lie side by side: one fill for all
@@ -321,10 +353,12 @@ int Forest::await_counters(const Publish &pub) {
   if (!pub.host) return sync_counters();
   // A small operation ends within microseconds of the host's wait; after a few
   // milliseconds the runtime waits (and reports a failed launch).
-  for (uint32_t spins = 0; __atomic_load_n(pub.seq, __ATOMIC_ACQUIRE) != pub.val; spins++) {
+  // (Later publications may have passed it.)
+  const auto there = [&] { return (int32_t)(__atomic_load_n(pub.seq, __ATOMIC_ACQUIRE) - pub.val) >= 0; };
+  for (uint32_t spins = 0; !there(); spins++) {
     if (spins >= 1u << 20) {
       HIP_TRY(hipStreamSynchronize(stream_));
-      if (__atomic_load_n(pub.seq, __ATOMIC_ACQUIRE) == pub.val) break;
+      if (there()) break;
       set_error("the counters did not reach the host");
       return -1;
     }
@@ -1328,7 +1362,49 @@ int Forest::export_nodes(const BatchDesc &keys, uint8_t **hashes, uint8_t **encs
   BatchDesc d;
   uint64_t vb;
   if ((r = stage_batch(keys, &d, &vb, false))) return r;
-  return export_paths(this, d, hashes, encs, enc_indexs, num);
+  // the paths' nodes, marked in a bitmap of the pools' slots
+  const uint32_t bw = (cnt_.n_branch + 63) / 64, words = bw + (cnt_.n_short + 63) / 64;
+  if (words == 0) return 0;  // no node was ever made
+  if (exp_map_.cap < 8ull * words) exp_zero_ = false;
+  if ((r = ensure_ws(exp_map_, 8ull * words))) return r;
+  if (!exp_zero_) HIP_TRY(hipMemsetAsync(exp_map_.p, 0, exp_map_.cap, stream_));
+  exp_zero_ = false;
+  const size_t nb = (words + 255) / 256;
+  if ((r = ensure_ws(ws2_, 4 * nb + scan_temp_bytes(nb) + 1024))) return r;
+  Carver c(ws2_.p);
+  uint32_t *bcnt = c.take<uint32_t>(nb);
+  GetArgs g{pools(), d.keys_hexs, d.keys_indexs, ntries_ > 1 ? d.trie_ids : nullptr, n, d.keys_bytes, ntries_,
+            nullptr, nullptr, nullptr};
+  HIP_TRY(path_mark(g, (uint64_t *)exp_map_.p, words, bw, bcnt, &d_cnt_->exp_nodes, c.take<uint8_t>(scan_temp_bytes(nb)),
+                    stream_));
+  if ((r = publish_and_await())) return r;
+  const uint32_t m = cnt_.exp_nodes;
+  if (m == 0) {
+    exp_zero_ = true;
+    return 0;
+  }
+  // their references and encoding lengths
+  if ((r = ensure_ws(exp_ws_, 20ull * m + scan_temp_bytes(m) + 2048))) return r;
+  Carver w(exp_ws_.p);
+  uint64_t *len = w.take<uint64_t>(m), *off = w.take<uint64_t>(m);
+  ref_t *refs = w.take<ref_t>(m);
+  HIP_TRY(mark_emit((uint64_t *)exp_map_.p, words, bw, bcnt, refs, stream_));
+  HIP_TRY(hc_enc_len(pools(), refs, m, len, stream_));
+  HIP_TRY(scan_exclusive_u64(len, off, m, &d_cnt_->exp_bytes, w.take<uint8_t>(scan_temp_bytes(m)), stream_));
+  if ((r = publish_and_await())) return r;
+  exp_zero_ = true;
+  // the results side by side: hash slots, index pairs, encodings
+  const size_t ebytes = cnt_.exp_bytes, pairs_at = 32ull * m, encs_at = 48ull * m, total = encs_at + ebytes;
+  if ((r = ensure_ws(exp_out_, total))) return r;
+  uint8_t *out = (uint8_t *)exp_out_.p;
+  HIP_TRY(hc_enc_write(pools(), refs, m, off, out + encs_at, (uint64_t *)out, (uint64_t *)(out + pairs_at), stream_));
+  *hashes = new uint8_t[32ull * m];
+  *encs = new uint8_t[ebytes ? ebytes : 1];
+  *enc_indexs = new uint64_t[2ull * m];
+  const FetchSeg seg[3] = {{0, *hashes, 32ull * m}, {pairs_at, *enc_indexs, 16ull * m}, {encs_at, *encs, ebytes}};
+  if ((r = fetch(out, total, seg, 3))) return r;
+  *num = m;
+  return 0;
 }
 
 // Whether a bulk build of the batch and its hash pass are sure to fit what is

@@ -30,10 +30,14 @@ hipError_t rw_split(const uint8_t *flags, uint32_t n, const int32_t *kidx, const
                     int32_t *wk, int64_t *wv, uint64_t *whp, int32_t *wtid, uint32_t *err, void *temp,
                     hipStream_t s);
 
-// Exports every node on the paths of the (device-staged) keys once, as the
-// reference's nodeset (libgmpt.h:13-18): 32-byte hash slots, RLP encodings,
-// inclusive [start, end] u64 pairs.  Host arrays are new[]-allocated.
-int export_paths(Forest *f, const BatchDesc &keys, uint8_t **hashes, uint8_t **encs, uint64_t **enc_indexs,
-                 uint64_t *num);
+// Node export.  Marks the nodes on the keys' paths in a bitmap (words 64-bit
+// words, all zero before: the branch slots, then from branch_words on the short
+// node slots); *total (device) receives their number and bcnt, an entry per 256
+// words, the numbers before each.  temp: scan workspace for bcnt's entries.
+hipError_t path_mark(const GetArgs &g, uint64_t *map, uint32_t words, uint32_t branch_words, uint32_t *bcnt,
+                     uint32_t *total, void *temp, hipStream_t s);
+// The marked nodes' references in ascending order; clears the bitmap.
+hipError_t mark_emit(uint64_t *map, uint32_t words, uint32_t branch_words, const uint32_t *bcnt, ref_t *out,
+                     hipStream_t s);
 
 }  // namespace gmpt

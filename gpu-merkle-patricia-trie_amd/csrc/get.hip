@@ -5,9 +5,6 @@
 // insert and the value size; flush_dirty_nodes (gpu_mpt.cuh:1039-1122,
 // kernels :2342-2588) exports (hash, encoding) of every node on the given
 // keys' paths.
-#include <string.h>
-
-#include <vector>
 
 #include "get.h"
 #include "phasehc.h"
@@ -130,40 +127,48 @@ __global__ __launch_bounds__(256) void k_gather_values(const uint64_t *addr, con
   for (int32_t q = threadIdx.x; q < size[i]; q += blockDim.x) out[off[i] + q] = src[q];
 }
 
-__global__ __launch_bounds__(256) void k_path_count(GetArgs g, uint32_t *cnt) {
+// The nodes on the keys' paths as a bitmap over the pools' slots (branches,
+// then short nodes from word branch_words on): their references come out of it
+// in order and once each, with no list per key and no sort.  (Counting and
+// writing every key's path, a radix sort and a compaction took 17 launches,
+// 250 us for 2,000 keys; marking takes one descent, 21 us, and the pass over
+// the bitmap of 340,000 slots 8 us.)  The upper levels' bits are set by the
+// first keys to arrive: the others see them and issue no atomic.
+__global__ __launch_bounds__(256) void k_path_mark(GetArgs g, unsigned long long *map, uint32_t branch_words,
+                                                   uint32_t words) {
   uint32_t i = grid_tid();
   if (i >= g.n) return;
   HexKey k = hex_key(g, i);
   uint32_t t = g.tid ? (uint32_t)g.tid[i] : 0u;
-  uint32_t c = 0;
-  if (t < g.ntries && k.len > 0) walk(g.P, g.P.tries[t].root, k, [&](ref_t) { c++; });
-  cnt[i] = c;
-}
-
-__global__ __launch_bounds__(256) void k_path_write(GetArgs g, const uint32_t *off, ref_t *out, uint32_t *idx) {
-  uint32_t i = grid_tid();
-  if (i >= g.n) return;
-  HexKey k = hex_key(g, i);
-  uint32_t t = g.tid ? (uint32_t)g.tid[i] : 0u;
-  uint32_t o = off[i];
   if (t < g.ntries && k.len > 0)
     walk(g.P, g.P.tries[t].root, k, [&](ref_t r) {
-      idx[o] = o;
-      out[o++] = r;
+      const uint32_t s = ref_idx(r), w = (ref_type(r) == T_SHORT ? branch_words : 0u) + s / 64;
+      const unsigned long long bit = 1ull << (s % 64);
+      if (w < words && !(__hip_atomic_load(map + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & bit))
+        atomicOr(map + w, bit);
     });
 }
 
-__global__ __launch_bounds__(256) void k_unique_refs(const ref_t *sorted, uint32_t m, uint32_t *flag) {
-  uint32_t i = grid_tid();
-  if (i >= m) return;
-  flag[i] = (i == 0 || sorted[i] != sorted[i - 1]) ? 1u : 0u;
+__global__ __launch_bounds__(256) void k_mark_count(const uint64_t *map, uint32_t words, uint32_t *bcnt) {
+  __shared__ uint32_t sh[4];
+  const uint32_t i = grid_tid();
+  uint32_t tot;
+  (void)block_exclusive_scan_256<uint32_t>(i < words ? (uint32_t)__popcll(map[i]) : 0u, sh, &tot);
+  if (threadIdx.x == 0) bcnt[blockIdx.x] = tot;
 }
 
-__global__ __launch_bounds__(256) void k_compact_refs(const ref_t *sorted, const uint32_t *flag,
-                                                      const uint32_t *pos, uint32_t m, ref_t *out) {
-  uint32_t i = grid_tid();
-  if (i >= m) return;
-  if (flag[i]) out[pos[i]] = sorted[i];
+// bcnt holds the exclusive scan of the blocks' counts.  The map is left clear.
+__global__ __launch_bounds__(256) void k_mark_emit(uint64_t *map, uint32_t words, uint32_t branch_words,
+                                                   const uint32_t *bcnt, ref_t *out) {
+  __shared__ uint32_t sh[4];
+  const uint32_t i = grid_tid();
+  uint64_t m = i < words ? map[i] : 0ull;
+  if (m) map[i] = 0;
+  uint32_t tot;
+  uint32_t o = bcnt[blockIdx.x] + block_exclusive_scan_256<uint32_t>((uint32_t)__popcll(m), sh, &tot);
+  const bool branch = i < branch_words;
+  const uint32_t type = branch ? T_BRANCH : T_SHORT, s0 = 64 * (branch ? i : i - branch_words);
+  for (; m; m &= m - 1) out[o++] = make_ref(type, s0 + (uint32_t)__ffsll((unsigned long long)m) - 1);
 }
 
 }  // namespace
@@ -181,93 +186,20 @@ hipError_t launch_gather_values(const uint64_t *addr, const int32_t *size, const
   return hipGetLastError();
 }
 
-#define EXP_TRY(expr)                                                                   \
-  do {                                                                                  \
-    hipError_t e__ = (expr);                                                            \
-    if (e__ != hipSuccess) {                                                            \
-      set_error(std::string("node export: ") + #expr + ": " + hipGetErrorString(e__));  \
-      rc = -1;                                                                          \
-      goto done;                                                                        \
-    }                                                                                   \
-  } while (0)
+hipError_t path_mark(const GetArgs &g, uint64_t *map, uint32_t words, uint32_t branch_words, uint32_t *bcnt,
+                     uint32_t *total, void *temp, hipStream_t s) {
+  if (g.n == 0 || words == 0) return hipErrorInvalidValue;
+  k_path_mark<<<nblk(g.n), kB, 0, s>>>(g, (unsigned long long *)map, branch_words, words);
+  GMPT_LAUNCH_CHECK();
+  k_mark_count<<<nblk(words), kB, 0, s>>>(map, words, bcnt);
+  GMPT_LAUNCH_CHECK();
+  return scan_exclusive_u32(bcnt, bcnt, nblk(words), total, temp, s);
+}
 
-int export_paths(Forest *f, const BatchDesc &keys, uint8_t **hashes, uint8_t **encs, uint64_t **enc_indexs,
-                 uint64_t *num) {
-  int rc = 0;
-  hipStream_t s = f->stream();
-  uint32_t n = keys.n;
-  GetArgs g{f->pools(), keys.keys_hexs, keys.keys_indexs, f->ntries() > 1 ? keys.trie_ids : nullptr, n,
-            keys.keys_bytes, f->ntries(), nullptr, nullptr, nullptr};
-  uint32_t *cnt = nullptr, *off = nullptr, *idx0 = nullptr, *idx1 = nullptr, *flag = nullptr, *pos = nullptr;
-  ref_t *r0 = nullptr, *r1 = nullptr, *uniq = nullptr;
-  uint64_t *len = nullptr, *eoff = nullptr;
-  uint8_t *d_enc = nullptr, *d_hash = nullptr;
-  void *temp = nullptr;
-  uint32_t total = 0, m = 0;
-  uint64_t ebytes = 0;
-  int which = 0;
-  std::vector<uint64_t> hlen, hoff;
-  EXP_TRY(hipMalloc(&cnt, 4ull * n + 4));
-  EXP_TRY(hipMalloc(&off, 4ull * n + 4));
-  EXP_TRY(hipMalloc(&temp, scan_temp_bytes(n + 1) + 64));
-  k_path_count<<<nblk(n), kB, 0, s>>>(g, cnt);
-  EXP_TRY(hipGetLastError());
-  EXP_TRY(scan_exclusive_u32(cnt, off, n, off + n, temp, s));
-  EXP_TRY(hipMemcpyAsync(&total, off + n, 4, hipMemcpyDeviceToHost, s));
-  EXP_TRY(hipStreamSynchronize(s));
-  if (total == 0) goto done;
-  EXP_TRY(hipMalloc(&r0, 4ull * total));
-  EXP_TRY(hipMalloc(&r1, 4ull * total));
-  EXP_TRY(hipMalloc(&idx0, 4ull * total));
-  EXP_TRY(hipMalloc(&idx1, 4ull * total));
-  EXP_TRY(hipMalloc(&flag, 4ull * total + 4));
-  EXP_TRY(hipMalloc(&pos, 4ull * total + 4));
-  EXP_TRY(hipFree(temp));
-  temp = nullptr;
-  EXP_TRY(hipMalloc(&temp, radix_temp_bytes(total) + scan_temp_bytes(total + 1) + 64));
-  k_path_write<<<nblk(n), kB, 0, s>>>(g, off, r0, idx0);
-  EXP_TRY(hipGetLastError());
-  EXP_TRY(radix_sort_u32(r0, idx0, r1, idx1, total, 0, 32, &which, temp, s));
-  {
-    ref_t *sorted = which ? r1 : r0;
-    k_unique_refs<<<nblk(total), kB, 0, s>>>(sorted, total, flag);
-    EXP_TRY(hipGetLastError());
-    EXP_TRY(scan_exclusive_u32(flag, pos, total, pos + total, temp, s));
-    EXP_TRY(hipMemcpyAsync(&m, pos + total, 4, hipMemcpyDeviceToHost, s));
-    EXP_TRY(hipStreamSynchronize(s));
-    EXP_TRY(hipMalloc(&uniq, 4ull * m));
-    k_compact_refs<<<nblk(total), kB, 0, s>>>(sorted, flag, pos, total, uniq);
-    EXP_TRY(hipGetLastError());
-  }
-  EXP_TRY(hipMalloc(&len, 8ull * m + 8));
-  EXP_TRY(hipMalloc(&eoff, 8ull * m + 8));
-  EXP_TRY(hc_enc_len(f->pools(), uniq, m, len, s));
-  EXP_TRY(scan_exclusive_u64(len, eoff, m, eoff + m, temp, s));
-  EXP_TRY(hipMemcpyAsync(&ebytes, eoff + m, 8, hipMemcpyDeviceToHost, s));
-  EXP_TRY(hipStreamSynchronize(s));
-  EXP_TRY(hipMalloc(&d_enc, ebytes + 8));
-  EXP_TRY(hipMalloc(&d_hash, 32ull * m + 8));
-  EXP_TRY(hc_enc_write(f->pools(), uniq, m, eoff, d_enc, d_hash, s));
-  hlen.resize(m);
-  hoff.resize(m);
-  *hashes = new uint8_t[32ull * m];
-  *encs = new uint8_t[ebytes ? ebytes : 1];
-  *enc_indexs = new uint64_t[2ull * m];
-  EXP_TRY(hipMemcpyAsync(*hashes, d_hash, 32ull * m, hipMemcpyDeviceToHost, s));
-  EXP_TRY(hipMemcpyAsync(*encs, d_enc, ebytes, hipMemcpyDeviceToHost, s));
-  EXP_TRY(hipMemcpyAsync(hlen.data(), len, 8ull * m, hipMemcpyDeviceToHost, s));
-  EXP_TRY(hipMemcpyAsync(hoff.data(), eoff, 8ull * m, hipMemcpyDeviceToHost, s));
-  EXP_TRY(hipStreamSynchronize(s));
-  for (uint32_t i = 0; i < m; i++) {
-    (*enc_indexs)[2 * i] = hoff[i];
-    (*enc_indexs)[2 * i + 1] = hoff[i] + hlen[i] - 1;
-  }
-  *num = m;
-done:
-  void *bufs[] = {cnt, off, idx0, idx1, flag, pos, r0, r1, uniq, len, eoff, d_enc, d_hash, temp};
-  for (void *b : bufs)
-    if (b) (void)hipFree(b);
-  return rc;
+hipError_t mark_emit(uint64_t *map, uint32_t words, uint32_t branch_words, const uint32_t *bcnt, ref_t *out,
+                     hipStream_t s) {
+  k_mark_emit<<<nblk(words), kB, 0, s>>>(map, words, branch_words, bcnt, out);
+  return hipGetLastError();
 }
 
 namespace {

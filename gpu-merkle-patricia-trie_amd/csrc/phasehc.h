@@ -146,10 +146,11 @@ hipError_t hc_roots(const Pools &P, uint32_t ntries, const unsigned long long *p
 // Root hashes (32-byte slots) and sizes of count tries, to pinned host memory.
 hipError_t gather_roots(const TrieHdr *tries, uint32_t count, uint8_t *hash, int32_t *size, hipStream_t s);
 hipError_t publish_counters(const Counters *cnt, Publish pub, hipStream_t s);
-// Node export: encoding lengths, then encodings at offs and 32-byte hash slots.
+// Node export: encoding lengths; then, with their exclusive sums offs, the
+// encodings, 32-byte hash slots and inclusive [start, end] pairs.
 hipError_t hc_enc_len(const Pools &P, const ref_t *refs, uint32_t m, uint64_t *len, hipStream_t s);
 hipError_t hc_enc_write(const Pools &P, const ref_t *refs, uint32_t m, const uint64_t *offs, uint8_t *encs,
-                        uint8_t *hashes, hipStream_t s);
+                        uint64_t *hashes, uint64_t *pairs, hipStream_t s);
 // Keccak-256 of n messages (test hook for the sponge): scratch holds
 // keccak_scratch_bytes(len, n) bytes, slot n entries, temp scan workspace.
 // spread = 1 runs the 25-lane layout, 0 one state per lane.

@@ -256,3 +256,43 @@ def test_host_batches_around_the_pinned_packing(gmpt, workloads, oracle, mode, n
     got, sizes = f.gets_parallel(absent)
     assert (got == 0).all() and (sizes == f.gets_parallel(absent.subset([0]))[1][0]).all()
     assert f.get_values(b.subset(range(0, n, 1 + n // 9)))[0] == b.value(0)
+
+
+@pytest.mark.parametrize("kind,n", [("uniform", 1), ("uniform", 90), ("short", 800), ("long", 800),
+                                    ("uniform", 20_000)])
+@pytest.mark.parametrize("tries", [1, 3])
+def test_export_of_marked_paths(gmpt, workloads, oracle, kind, n, tries):
+    # results of less than one and of several halves of the pinned memory, one
+    # value above a half; every key, one, and some with repeats and absent ones;
+    # again after the pools (and with them the bitmap) have grown
+    rng = np.random.default_rng(n + tries)
+    keys = list(dict.fromkeys(_mixed_keys(rng, n, kind)))
+    vals = [bytes(rng.integers(0, 256, int(k), dtype=np.uint8)) for k in rng.choice([0, 1, 1, 3, 40, 56, 300], len(keys))]
+    vals[0] = bytes(rng.integers(0, 256, 700_000, dtype=np.uint8))
+    f = gmpt.MPT(device=0, num_tries=tries)
+    os_, kept = [oracle.OracleMPT() for _ in range(tries)], []
+    for cut in (slice(0, max(1, n // 3)), slice(0, None)):
+        # (new values each time: the oracle exports a leaf that was written again
+        # with the value it had as if the value were empty)
+        part, pv = keys[cut], [v + b"!" * (1 + len(kept)) for v in vals[cut]]
+        b = workloads.batch_from_bytes(part, pv)
+        b.trie_ids = np.array([k[0] % tries for k in part], np.int32)
+        _put(f, b)
+        want = set()
+        for t in range(tries):
+            kept.append(b.subset(np.flatnonzero(b.trie_ids == t)))  # the oracle refers to the values
+            os_[t].puts(kept[-1])
+            os_[t].hash()
+            want |= {(h + bytes(32 - len(h)), e) for h, e in os_[t].export()}
+        every = f.flush_dirty_nodes(b)
+        assert set(every) == want
+        one = f.flush_dirty_nodes(b.subset([0]))
+        order = {x: i for i, x in enumerate(every)}  # references ascend
+        assert set(one) <= want and [order[x] for x in one] == sorted(order[x] for x in one)
+        some = b.subset([0, len(part) // 2, 0, len(part) - 1])
+        some.trie_ids = np.array(some.trie_ids)
+        got = f.flush_dirty_nodes(some)
+        assert set(one) <= set(got) <= want and len(got) <= len(every)
+        gone = workloads.batch_from_bytes([b"\xee" * 40], [b""])
+        gone.trie_ids = np.zeros(1, np.int32)
+        assert set(f.flush_dirty_nodes(gone)) <= want
