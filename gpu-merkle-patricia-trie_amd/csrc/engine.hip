@@ -723,7 +723,6 @@ void Forest::finish_build(const NuArgs &a) {
 // groups are to be merged or an error is pending).
 int Forest::build_sorted(NuArgs &a, void *temp, bool empty) {
   HIP_TRY(nu_descend_and_group(a, temp, stream_, empty));
-  HIP_TRY(nu_emit(a, temp, stream_, empty));
   HIP_TRY(nu_build(a, temp, stream_, empty));
   return 0;
 }
@@ -737,7 +736,6 @@ int Forest::merge_groups(NuArgs &a, void *temp) {
     HIP_TRY(hipMemsetAsync(a.scal + SC_MERGE, 0, 4, stream_));
     HIP_TRY(nu_regroup(a, m, m, temp, stream_));
     stats_.regroups++;
-    HIP_TRY(nu_emit(a, temp, stream_, false));
     HIP_TRY(nu_build(a, temp, stream_, false));
     if ((r = publish_and_await())) return r;
   }

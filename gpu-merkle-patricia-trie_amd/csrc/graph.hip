@@ -103,7 +103,7 @@ int Forest::capture_rebuild(const BatchDesc &b) {
   if ((e = nu_adjacent(a, sk, sv, 0, stream_, sk_mask)) != hipSuccess ||
       (e = nu_unique(a, sk, sv, temp, stream_)) != hipSuccess ||
       (e = nu_descend_and_group(a, temp, stream_, true)) != hipSuccess ||
-      (e = nu_emit(a, temp, stream_, true)) != hipSuccess || (e = nu_build(a, temp, stream_, true)) != hipSuccess)
+      (e = nu_build(a, temp, stream_, true)) != hipSuccess)
     return fail(-1);
   // the hash, with the captured pass's sizes
   const uint32_t n = plan_.n_dirty;

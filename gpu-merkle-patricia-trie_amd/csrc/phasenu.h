@@ -26,11 +26,10 @@ struct Stop {
 
 struct GroupInfo {
   ref_t attach;
-  ref_t split;       // short node being split (REF_NULL if none)
   uint32_t trie;
   uint16_t base;
   uint8_t slot;
-  uint8_t has_split;
+  uint8_t pad;
 };
 
 // Device pointers of one PhaseNU call.  All arrays are sized by the host from
@@ -51,7 +50,8 @@ struct NuArgs {
   uint64_t vbase;        // device address of this batch's value bytes
   // per input key
   uint32_t *klen;
-  uint64_t *kpoff;       // per block of 256 keys: its slot bytes, then (k_keys_reduce) its first slot's offset
+  uint64_t *kpoff;       // per block of 256 keys: its slot bytes, then (k_keys_reduce) its first slot's offset;
+                         // after the descent, its group starts | elements << 32
   uint64_t *kref;        // kpoff | nibbles << 48: one load gives a key's place and length
   uint64_t key_cap;      // key arena bytes allocated (bounds the speculative packing)
   uint32_t *leaf_pk;     // per element: the new leaf's hashing bin (hc_leaf.h), or kLeafPackedNone
@@ -72,8 +72,8 @@ struct NuArgs {
   Stop *stop;
   uint32_t *grp;         // group id of each unique key
   GroupInfo *ginfo;
-  uint32_t *ecount;      // E entries emitted per unique key, scanned to positions
-  uint32_t *merge;       // per run: run whose group it joins (split groups around a subtree)
+  uint32_t *ecount;      // multi-trie builds: the flags of the tries' first keys
+  uint32_t *merge;       // per run: first key of the run whose group it joins (split groups around a subtree)
   uint32_t *u_idx2, *u_trie2, *perm0, *perm1, *gkey0, *gkey1;
   // each unique key's kref and sort window, gathered in unique order so the
   // build reads them in sequence (u_win holds u_win_nibs nibbles from W)
@@ -160,17 +160,15 @@ hipError_t nu_unique(const NuArgs &a, const uint64_t *sk, const uint32_t *sv, vo
 // Before a repeated sort pass (an eager fallback): clears SC_DUP, which the
 // pass's k_adjacent sets again.
 hipError_t nu_reset_dup(const NuArgs &a, hipStream_t s);
-// Descends every unique key and groups them by stop point; sets SC_MERGE when
-// a split group is interrupted by keys below the split node (nu_regroup).
+// Descends every unique key, groups them by stop point, writes updated values
+// and emits every group's elements E; sets SC_MERGE when a split group is
+// interrupted by keys below the split node (nu_regroup).
 // empty: every trie of the forest is empty (the host knows it), so the keys
-// need no descent, the groups are the tries and the elements are emitted
-// here too (nu_emit then does nothing, nu_build skips the update kernel).
+// need no descent and the groups are the tries.
 hipError_t nu_descend_and_group(const NuArgs &a, void *temp, hipStream_t s, bool empty = false);
 // Makes every group contiguous (stable sort of the unique keys by group),
-// swapping the unique-key arrays of `a`, and regroups.
+// swapping the unique-key arrays of `a`, then regroups and emits again.
 hipError_t nu_regroup(NuArgs &a, uint32_t m, uint32_t nruns, void *temp, hipStream_t s);
-// Emits the element sequence E of every group.
-hipError_t nu_emit(const NuArgs &a, void *temp, hipStream_t s, bool empty = false);
 // Builds every group's subtree; node and dirty-list slots are fixed by
 // position from base_branch / base_short / base_value (see phasenu.hip).
 hipError_t nu_build(const NuArgs &a, void *temp, hipStream_t s, bool empty = false);

@@ -552,16 +552,17 @@ __device__ __forceinline__ uint64_t scatter_bits(uint64_t x, uint64_t m) {
 // before it (few blocks: kSelfSumBlocks at most).  Every thread of the block
 // calls it (it synchronises the block unless pre).
 constexpr uint32_t kSelfSumBlocks = 4096;
-__device__ __forceinline__ uint32_t block_offset(const uint32_t *cnt, bool pre, uint32_t *sh) {
+template <typename T>
+__device__ __forceinline__ T block_offset(const T *cnt, bool pre, T *sh) {
   if (pre) return cnt[blockIdx.x];
-  uint32_t part = 0;  // all of the thread's loads in flight at once
+  T part = 0;  // all of the thread's loads in flight at once
 #pragma unroll
   for (uint32_t q = 0; q < kSelfSumBlocks / 256; q++) {
     const uint32_t t = threadIdx.x + 256 * q;
-    part += t < blockIdx.x ? cnt[t] : 0u;
+    part += t < blockIdx.x ? cnt[t] : T(0);
   }
-  uint32_t tot;
-  block_exclusive_scan_256<uint32_t>(part, sh, &tot);
+  T tot;
+  block_exclusive_scan_256<T>(part, sh, &tot);
   return tot;
 }
 
@@ -850,59 +851,6 @@ __device__ __forceinline__ bool same_group(const Stop &x, uint32_t tx, const Sto
   return x.attach == y.attach && x.slot == y.slot;  // branch slot
 }
 
-__global__ __launch_bounds__(256) void k_group_flags(NuArgs a) {
-  if (a.P.cnt->flag_fallback) return;  // no stops yet (k_descend)
-  uint32_t i = grid_tid();
-  uint32_t m = a.scal[SC_M_UNIQ];
-  if (i >= a.n) return;
-  if (i >= m) {
-    a.ecount[i] = 0;
-    return;
-  }
-  bool start = i == 0 || !same_group(a.stop[i - 1], a.u_trie[i - 1], a.stop[i], a.u_trie[i]);
-  a.ecount[i] = start ? 1u : 0u;
-}
-
-// grp[] = exclusive scan of the start flags in ecount[]; make it inclusive,
-// i.e. 1-based group ids.
-__global__ __launch_bounds__(256) void k_group_fix(NuArgs a) {
-  if (a.P.cnt->flag_fallback) return;  // no stops yet (k_descend)
-  uint32_t i = grid_tid();
-  if (i >= a.n) return;
-  a.grp[i] += a.ecount[i];
-}
-
-// grp[] now holds the inclusive scan; group id = grp - 1.
-__global__ __launch_bounds__(256) void k_group_info(NuArgs a) {
-  if (a.P.cnt->flag_fallback) return;  // no stops yet (k_descend)
-  uint32_t i = grid_tid();
-  uint32_t m = a.scal[SC_M_UNIQ];
-  if (i >= m) return;
-  uint32_t g = a.grp[i] - 1;
-  const Stop st = a.stop[i];
-  bool start = i == 0 || a.grp[i - 1] != a.grp[i];
-  if (start) {
-    GroupInfo gi;
-    gi.attach = st.attach;
-    gi.split = (st.kind == STOP_SHORT_SPLIT || st.kind == STOP_LEAF_UPDATE) ? st.stop : REF_NULL;
-    gi.trie = a.u_trie[i];
-    gi.base = st.base;
-    gi.slot = st.slot;
-    gi.has_split = 0;
-    a.ginfo[g] = gi;
-  }
-  if (i + 1 == m) a.scal[SC_NGROUP] = g + 1;
-}
-
-__global__ __launch_bounds__(256) void k_group_split(NuArgs a) {
-  if (a.P.cnt->flag_fallback) return;  // no stops yet (k_descend)
-  uint32_t i = grid_tid();
-  uint32_t m = a.scal[SC_M_UNIQ];
-  if (i >= m) return;
-  if (a.stop[i].kind == STOP_SHORT_SPLIT) a.ginfo[a.grp[i] - 1].has_split = 1;
-}
-
-
 // A split group whose short node S is an extension can be interrupted in the
 // sorted key order by keys that pass through S (they sort between the keys
 // ordered before S's subtree and those after it).  The run after the
@@ -921,19 +869,11 @@ __device__ bool key_before_block(const NuArgs &a, uint32_t j, uint32_t trie, con
   return false;  // kj has the whole prefix: inside the block
 }
 
-__global__ __launch_bounds__(256) void k_group_merge(NuArgs a) {
-  if (a.P.cnt->flag_fallback) return;  // no stops yet (k_descend)
-  uint32_t i = grid_tid();
-  uint32_t m = a.scal[SC_M_UNIQ];
-  if (i >= m) return;
-  uint32_t run = a.grp[i] - 1;
-  bool start = i == 0 || a.grp[i - 1] != a.grp[i];
-  if (!start) return;
-  a.merge[run] = run;
-  const Stop st = a.stop[i];
-  if (st.kind != STOP_SHORT_SPLIT || st.less) return;
+// The start key of the earlier run that the run starting at key i joins, or i.
+__device__ uint32_t merge_target(const NuArgs &a, uint32_t i, const Stop &st) {
+  if (st.kind != STOP_SHORT_SPLIT || st.less) return i;
   const Short &S = a.P.shrt[ref_idx(st.stop)];
-  if (S.term) return;  // a leaf's subtree is one key, already grouped with it
+  if (S.term) return i;  // a leaf's subtree is one key, already grouped with it
   uint32_t trie = a.u_trie[i];
   KeyRef kr = key_of(a, a.u_idx[i]);
   uint32_t blen = S.depth + S.key_len;
@@ -945,13 +885,9 @@ __global__ __launch_bounds__(256) void k_group_merge(NuArgs a) {
     else
       hi = mid;
   }
-  if (lo == 0) return;
-  uint32_t j = lo - 1;
-  const Stop sj = a.stop[j];
-  if (a.u_trie[j] == trie && sj.kind == STOP_SHORT_SPLIT && sj.stop == st.stop && sj.less) {
-    a.merge[run] = a.grp[j] - 1;
-    a.scal[SC_MERGE] = 1;
-  }
+  if (lo == 0) return i;
+  const Stop sj = a.stop[lo - 1];
+  return a.u_trie[lo - 1] == trie && sj.kind == STOP_SHORT_SPLIT && sj.stop == st.stop && sj.less ? lo - 1 : i;
 }
 
 // Every trie of the forest empty (a bulk build): each unique key stops at its
@@ -1002,11 +938,10 @@ __device__ __forceinline__ uint32_t empty_element(const NuArgs &a, uint32_t i, u
   if (start) {
     GroupInfo gi;
     gi.attach = REF_NULL;
-    gi.split = REF_NULL;
     gi.trie = t;
     gi.base = 0;
     gi.slot = 0;
-    gi.has_split = 0;
+    gi.pad = 0;
     a.ginfo[g - 1] = gi;
   }
   if (!a.e_ident) {
@@ -1029,42 +964,11 @@ __global__ __launch_bounds__(256) void k_empty_groups(NuArgs a, int multi) {
   mt_block_levels(a, i < m ? empty_element(a, i, m, multi) : 255u);
 }
 
-// Levels k0 .. of the minimum tree in one workgroup, each from the one below.
-__global__ __launch_bounds__(256) void k_mt_top(NuArgs a, int k0) {
-  const uint32_t ne = a.scal[SC_NE];
-  uint32_t cnt = ne > 0 ? ne - 1 : 0;  // valid entries of level k - 1
-  size_t off = 0;                      // and its offset
-  for (int q = 0; q < k0 - 1; q++) {
-    off += mt_level_len(a.st_stride, q);
-    cnt = (cnt + 15) / 16;
-  }
-  for (int k = k0; k < a.st_levels; k++) {
-    const size_t len = mt_level_len(a.st_stride, k - 1);
-    const uint32_t nout = (cnt + 15) / 16;
-    for (uint32_t b = threadIdx.x; b < nout; b += blockDim.x) {
-      // the entry's 16 children in one load (levels are 16-byte multiples
-      // at 16-byte aligned offsets); children past cnt do not count
-      const uint4 v = *(const uint4 *)(a.st + off + 16 * (size_t)b);
-      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-      uint32_t mn = 255;
-#pragma unroll
-      for (uint32_t i = 0; i < 16; i++)
-        if (16 * b + i < cnt) mn = min(mn, (w[i >> 2] >> (8 * (i & 3))) & 255u);
-      a.st[off + len + b] = (uint8_t)mn;
-    }
-    __syncthreads();  // the level is complete for the next one
-    off += len;
-    cnt = nout;
-  }
-}
-
 __global__ __launch_bounds__(256) void k_gkey(NuArgs a, uint32_t m) {
   uint32_t i = grid_tid();
   if (i >= m) return;
-  uint32_t run = a.grp[i] - 1;
-  uint32_t tgt = a.merge[run];
-  // the target of a target is itself (a run joins at most one earlier run)
-  a.gkey0[i] = tgt;
+  // a run joins at most one earlier run, named by its first key
+  a.gkey0[i] = a.grp[a.merge[a.grp[i] - 1]] - 1;
   a.perm0[i] = i;
 }
 
@@ -1084,37 +988,167 @@ __device__ __forceinline__ bool is_update(uint8_t kind) {
   return kind == STOP_LEAF_UPDATE || kind == STOP_VALUE_UPDATE;
 }
 
-// E layout per group: [keys ordered before the split node's subtree]
-// [the split node as one virtual element] [keys after it]; updates emit nothing.
-struct Emit {
-  bool self, vbefore, vafter;
+__device__ __forceinline__ void init_value(const NuArgs &a, uint32_t vid, uint32_t idx, uint64_t *addr = nullptr,
+                                           uint32_t *size = nullptr) {
+  Value &V = a.P.value[vid];
+  int64_t vs = a.vidx[2 * idx], ve = a.vidx[2 * idx + 1];
+  V.addr = a.vbase + (uint64_t)vs;
+  V.hp = a.hps ? a.hps[idx] : 0ull;
+  V.size = (uint32_t)(ve - vs + 1);
+  V.pad = 0;
+  V.seq = 0;
+  if (addr) *addr = V.addr;
+  if (size) *size = V.size;
+}
+
+// Existing key i's new value: its value node is rewritten in place (no node is
+// allocated per update; only this key refers to it).  Every update precedes the
+// links, so a leaf that is also split carries the new value into its remainder.
+__device__ __forceinline__ void update_value(const NuArgs &a, uint32_t i, const Stop &st) {
+  const ref_t vr = st.kind == STOP_LEAF_UPDATE ? a.P.shrt[ref_idx(st.stop)].child
+                                               : a.P.branch[ref_idx(st.stop)].child[16];
+  if (ref_type(vr) != T_VALUE) {
+    raise_error(a.P.cnt, ERR_INTERNAL, 13);
+    return;
+  }
+  init_value(a, ref_idx(vr), a.u_idx[i]);
+}
+
+// Unique key i among its neighbours: whether it starts a group, and what it
+// emits.  E layout per group: [keys ordered before the split node's subtree]
+// [the split node as one virtual element] [keys after it]; updates emit
+// nothing.  A key that is not an update but shares its group's split node has
+// left that node midway, so it alone says that the group is split.
+struct GroupPos {
+  Stop st;
+  bool start, self, vbefore, vafter;
+  int prev;  // the group's previous element, or -1
+  uint32_t prev_div;
+  __device__ __forceinline__ GroupPos(const NuArgs &a, uint32_t i, uint32_t m) {
+    st = a.stop[i];
+    const uint32_t t = a.u_trie[i];
+    const Stop p = a.stop[i > 0 ? i - 1 : i];
+    const uint32_t tp = a.u_trie[i > 0 ? i - 1 : i];
+    start = i == 0 || !same_group(p, tp, st, t);
+    self = !is_update(st.kind);
+    vbefore = vafter = false;
+    prev = -1;
+    prev_div = 0;
+    if (!self) return;
+    if (!start) {
+      if (!is_update(p.kind)) {
+        prev = (int)i - 1;
+        prev_div = p.div;
+      } else if (i > 1) {
+        const Stop pp = a.stop[i - 2];
+        if (same_group(pp, a.u_trie[i - 2], p, tp)) {
+          prev = (int)i - 2;
+          prev_div = pp.div;
+        }
+      }
+    }
+    if (st.kind != STOP_SHORT_SPLIT) return;
+    if (!st.less) {
+      // first key ordered after the split subtree?
+      vbefore = start || is_update(p.kind) || p.less;
+    } else {
+      // last key ordered before the subtree, with no key after it in the group?
+      vafter = true;
+      if (i + 1 < m) {
+        const Stop n = a.stop[i + 1];
+        const uint32_t tn = a.u_trie[i + 1];
+        if (same_group(st, t, n, tn))
+          vafter = is_update(n.kind) && !(i + 2 < m && same_group(n, tn, a.stop[i + 2], a.u_trie[i + 2]));
+      }
+    }
+  }
+  // group starts in the lower half, elements in the upper
+  __device__ __forceinline__ uint64_t counts() const {
+    return (uint64_t)start | (uint64_t)((uint32_t)self + vbefore + vafter) << 32;
+  }
 };
 
-__device__ __forceinline__ Emit emit_of(const NuArgs &a, uint32_t i, uint32_t m) {
-  Emit e{false, false, false};
-  const Stop st = a.stop[i];
-  if (is_update(st.kind)) return e;
-  e.self = true;
-  uint32_t g = a.grp[i];
-  const GroupInfo &gi = a.ginfo[g - 1];
-  if (!gi.has_split) return e;
-  if (!st.less) {
-    // first key ordered after the split subtree?
-    bool first = true;
-    if (i > 0 && a.grp[i - 1] == g) {
-      const Stop p = a.stop[i - 1];
-      first = is_update(p.kind) || p.less;
-    }
-    e.vbefore = first;
-  } else {
-    // last key ordered before the subtree, with no key after it in the group?
-    bool last = true;
-    uint32_t j = i + 1;
-    if (j < m && a.grp[j] == g && is_update(a.stop[j].kind)) j++;
-    if (j < m && a.grp[j] == g) last = false;
-    e.vafter = last;
+// Groups and elements take two launches (with the updates in the second; a
+// launch of a few thousand keys costs about 5 us whatever it does, and flags,
+// scans, descriptors, merge targets, counts and elements took eleven of them):
+// k_group_count leaves each block's group starts and elements in kpoff, and
+// k_group_write finds every key's group and place from the counts before it
+// (pre: they are scanned already) and its neighbours' stops, without other
+// blocks' results.  The descent's stops are final here, unless the sort needs
+// another pass or an error is pending.
+__global__ __launch_bounds__(256) void k_group_count(NuArgs a) {
+  if (a.P.cnt->flag_fallback || a.P.cnt->err) return;
+  __shared__ uint64_t sh[4];
+  const uint32_t i = grid_tid(), m = a.scal[SC_M_UNIQ];
+  uint64_t v = i < m ? GroupPos(a, i, m).counts() : 0ull;
+  for (int off = 32; off > 0; off >>= 1) v += (uint64_t)__shfl_xor((unsigned long long)v, off);
+  if (__lane_id() == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) a.kpoff[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
+}
+
+// Level 0 of the minimum tree gets, at split point q (between E[q] and
+// E[q+1]), lcp(E[q], E[q+1]) + 1, or 0 across a group boundary.  With merge,
+// a group whose keys are interrupted sets SC_MERGE: the host then makes groups
+// contiguous (nu_regroup) and discards these elements.
+__global__ __launch_bounds__(256) void k_group_write(NuArgs a, int pre, int merge) {
+  if (a.P.cnt->flag_fallback || a.P.cnt->err) return;
+  __shared__ uint64_t sh[4];
+  const uint32_t i = grid_tid(), m = a.scal[SC_M_UNIQ];
+  if (blockIdx.x * kB >= m) return;  // uniform over the block
+  const GroupPos e(a, min(i, m - 1), m);
+  const uint64_t c = i < m ? e.counts() : 0ull;
+  uint64_t btot;
+  const uint64_t at =
+      block_offset<uint64_t>(a.kpoff, pre != 0, sh) + block_exclusive_scan_256<uint64_t>(c, sh, &btot);
+  if (i >= m) return;
+  const Stop &st = e.st;
+  const uint32_t g = (uint32_t)at + e.start;  // 1-based
+  uint32_t pos = (uint32_t)(at >> 32);
+  a.grp[i] = g;
+  if (i + 1 == m) {
+    a.scal[SC_NGROUP] = g;
+    a.scal[SC_NE] = pos + (uint32_t)(c >> 32);
   }
-  return e;
+  if (e.start) {
+    GroupInfo gi;
+    gi.attach = st.attach;
+    gi.trie = a.u_trie[i];
+    gi.base = st.base;
+    gi.slot = st.slot;
+    gi.pad = 0;
+    a.ginfo[g - 1] = gi;
+    if (merge) {
+      const uint32_t to = merge_target(a, i, st);
+      a.merge[g - 1] = to;
+      if (to != i) a.scal[SC_MERGE] = 1;
+    }
+  }
+  if (!e.self) {
+    update_value(a, i, st);
+    return;
+  }
+  uint8_t *sp = a.st;  // level 0
+  if (e.vbefore) {
+    a.e_src[pos] = 0x80000000u | ref_idx(st.stop);
+    a.e_grp[pos] = g - 1;
+    if (pos > 0) sp[pos - 1] = e.prev >= 0 ? (uint8_t)(e.prev_div + 1) : 0;
+    pos++;
+    a.e_src[pos] = i;
+    a.e_grp[pos] = g - 1;
+    sp[pos - 1] = (uint8_t)(st.div + 1);
+    pos++;
+  } else {
+    a.e_src[pos] = i;
+    a.e_grp[pos] = g - 1;
+    if (pos > 0) sp[pos - 1] = e.prev >= 0 ? (uint8_t)(a.u_lcp[i] + 1) : 0;
+    pos++;
+  }
+  if (e.vafter) {
+    a.e_src[pos] = 0x80000000u | ref_idx(st.stop);
+    a.e_grp[pos] = g - 1;
+    sp[pos - 1] = (uint8_t)(st.div + 1);
+  }
 }
 
 // An insert's kernels from here on run before the host has seen how the sort
@@ -1123,76 +1157,6 @@ __device__ __forceinline__ Emit emit_of(const NuArgs &a, uint32_t i, uint32_t m)
 // runs them again.
 __device__ __forceinline__ bool build_waits(const NuArgs &a) {
   return a.P.cnt->flag_fallback || a.P.cnt->err || a.scal[SC_MERGE];
-}
-
-__global__ __launch_bounds__(256) void k_emit_count(NuArgs a) {
-  if (build_waits(a)) return;
-  uint32_t i = grid_tid();
-  uint32_t m = a.scal[SC_M_UNIQ];
-  if (i >= a.n) return;
-  uint32_t c = 0;
-  if (i < m) {
-    Emit e = emit_of(a, i, m);
-    c = (uint32_t)e.self + (uint32_t)e.vbefore + (uint32_t)e.vafter;
-  }
-  a.ecount[i] = c;
-}
-
-// ecount[] holds the exclusive scan.  Level 0 of the minimum tree gets, at
-// split point q (between E[q] and E[q+1]), lcp(E[q], E[q+1]) + 1, or 0 across
-// a group boundary.
-__global__ __launch_bounds__(256) void k_emit_write(NuArgs a) {
-  if (build_waits(a)) return;
-  uint32_t i = grid_tid();
-  uint32_t m = a.scal[SC_M_UNIQ];
-  if (i >= m) return;
-  Emit e = emit_of(a, i, m);
-  if (!e.self) {
-    if (i + 1 == m) a.scal[SC_NE] = a.ecount[i];
-    return;
-  }
-  const Stop st = a.stop[i];
-  uint32_t g = a.grp[i];
-  uint32_t pos = a.ecount[i];
-  uint8_t *sp = a.st;  // level 0
-  const GroupInfo &gi = a.ginfo[g - 1];
-  // does an earlier E element of this group exist, and what is its lcp to us?
-  auto prev_in_group = [&](uint32_t ii) -> int {
-    // index of the previous non-update unique key in the group, or -1
-    if (ii == 0) return -1;
-    uint32_t j = ii - 1;
-    if (a.grp[j] != g) return -1;
-    if (is_update(a.stop[j].kind)) {
-      if (j == 0) return -1;
-      j--;
-      if (a.grp[j] != g) return -1;
-    }
-    return (int)j;
-  };
-  if (e.vbefore) {
-    int pj = prev_in_group(i);
-    a.e_src[pos] = 0x80000000u | ref_idx(gi.split);
-    a.e_grp[pos] = g - 1;
-    if (pos > 0) sp[pos - 1] = pj >= 0 ? (uint8_t)(a.stop[pj].div + 1) : 0;
-    pos++;
-    a.e_src[pos] = i;
-    a.e_grp[pos] = g - 1;
-    sp[pos - 1] = (uint8_t)(st.div + 1);
-    pos++;
-  } else {
-    a.e_src[pos] = i;
-    a.e_grp[pos] = g - 1;
-    int pj = prev_in_group(i);
-    if (pos > 0) sp[pos - 1] = pj >= 0 ? (uint8_t)(a.u_lcp[i] + 1) : 0;
-    pos++;
-  }
-  if (e.vafter) {
-    a.e_src[pos] = 0x80000000u | ref_idx(gi.split);
-    a.e_grp[pos] = g - 1;
-    sp[pos - 1] = (uint8_t)(st.div + 1);
-    pos++;
-  }
-  if (i + 1 == m) a.scal[SC_NE] = pos;
 }
 
 // ------------------------------------------------------------- 4. build --
@@ -1227,6 +1191,39 @@ __global__ __launch_bounds__(256) void k_mt_level(NuArgs a, int k) {
   for (uint32_t i = 0; i < 16; i++)
     if (16 * b + i < cnt) mn = min(mn, (w[i >> 2] >> (8 * (i & 3))) & 255u);
   a.st[off + mt_level_len(a.st_stride, k - 1) + b] = (uint8_t)mn;
+}
+
+// Levels k0 .. in one workgroup, each from the one below: four entries per
+// thread at the first of them, about what another launch would cost.
+constexpr uint32_t kMtTopThreads = 1024;
+constexpr size_t kMtTopMax = 4 * kMtTopThreads;
+__global__ __launch_bounds__(1024) void k_mt_top(NuArgs a, int k0) {
+  if (build_waits(a)) return;
+  const uint32_t ne = a.scal[SC_NE];
+  uint32_t cnt = ne > 0 ? ne - 1 : 0;  // valid entries of level k - 1
+  size_t off = 0;                      // and its offset
+  for (int q = 0; q < k0 - 1; q++) {
+    off += mt_level_len(a.st_stride, q);
+    cnt = (cnt + 15) / 16;
+  }
+  for (int k = k0; k < a.st_levels; k++) {
+    const size_t len = mt_level_len(a.st_stride, k - 1);
+    const uint32_t nout = (cnt + 15) / 16;
+    for (uint32_t b = threadIdx.x; b < nout; b += blockDim.x) {
+      // the entry's 16 children in one load (levels are 16-byte multiples
+      // at 16-byte aligned offsets); children past cnt do not count
+      const uint4 v = *(const uint4 *)(a.st + off + 16 * (size_t)b);
+      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+      uint32_t mn = 255;
+#pragma unroll
+      for (uint32_t i = 0; i < 16; i++)
+        if (16 * b + i < cnt) mn = min(mn, (w[i >> 2] >> (8 * (i & 3))) & 255u);
+      a.st[off + len + b] = (uint8_t)mn;
+    }
+    __syncthreads();  // the level is complete for the next one
+    off += len;
+    cnt = nout;
+  }
 }
 
 // The tree's levels are located from its level-0 length (stride) alone,
@@ -1589,19 +1586,6 @@ __device__ __forceinline__ bool link_branch(const NuArgs &a, uint32_t j, uint32_
 
 // Elements: new keys become a leaf short node + value node; a split short
 // node's remainder is re-attached below the new branch.
-__device__ __forceinline__ void init_value(const NuArgs &a, uint32_t vid, uint32_t idx, uint64_t *addr = nullptr,
-                                           uint32_t *size = nullptr) {
-  Value &V = a.P.value[vid];
-  int64_t vs = a.vidx[2 * idx], ve = a.vidx[2 * idx + 1];
-  V.addr = a.vbase + (uint64_t)vs;
-  V.hp = a.hps ? a.hps[idx] : 0ull;
-  V.size = (uint32_t)(ve - vs + 1);
-  V.pad = 0;
-  V.seq = 0;
-  if (addr) *addr = V.addr;
-  if (size) *size = V.size;
-}
-
 template <class Sink>
 __device__ __forceinline__ void link_elem(const NuArgs &a, uint32_t e, const Slots &q, const Sink &sink) {
   ST s = st_of(a);
@@ -1800,27 +1784,6 @@ __global__ __launch_bounds__(256) void k_link_cross(NuArgs a) {
     count_child(a, rank, slot);
   }
 }
-
-// Existing keys: swap in a new value node (runs before the links, so a leaf
-// that is also split carries the new value into its remainder).
-// The key's value node is rewritten in place (no node is allocated per
-// update; only this key refers to it).
-__global__ __launch_bounds__(256) void k_updates(NuArgs a) {
-  if (build_waits(a)) return;
-  uint32_t i = grid_tid();
-  uint32_t m = a.scal[SC_M_UNIQ];
-  if (i >= m) return;
-  Stop st = a.stop[i];
-  if (!is_update(st.kind)) return;
-  const ref_t vr = st.kind == STOP_LEAF_UPDATE ? a.P.shrt[ref_idx(st.stop)].child
-                                               : a.P.branch[ref_idx(st.stop)].child[16];
-  if (ref_type(vr) != T_VALUE) {
-    raise_error(a.P.cnt, ERR_INTERNAL, 13);
-    return;
-  }
-  init_value(a, ref_idx(vr), a.u_idx[i]);
-}
-
 
 }  // namespace
 
@@ -2044,16 +2007,17 @@ hipError_t nu_unique(const NuArgs &a, const uint64_t *sk, const uint32_t *sv, vo
   return hipGetLastError();
 }
 
-static hipError_t nu_groups(const NuArgs &a, void *temp, hipStream_t s) {
-  k_group_flags<<<nblk(a.n), kB, 0, s>>>(a);
+// Groups and elements from the stops; merge: look for interrupted groups.
+static hipError_t nu_groups(const NuArgs &a, void *temp, hipStream_t s, bool merge) {
+  const uint32_t nb = nblk(a.n);
+  k_group_count<<<nb, kB, 0, s>>>(a);
   GMPT_LAUNCH_CHECK();
-  hipError_t e = scan_exclusive_u32(a.ecount, a.grp, a.n, nullptr, temp, s);
-  if (e != hipSuccess) return e;
-  k_group_fix<<<nblk(a.n), kB, 0, s>>>(a);
-  GMPT_LAUNCH_CHECK();
-  k_group_info<<<nblk(a.n), kB, 0, s>>>(a);
-  GMPT_LAUNCH_CHECK();
-  k_group_split<<<nblk(a.n), kB, 0, s>>>(a);
+  const bool pre = nb > kSelfSumBlocks;
+  if (pre) {
+    hipError_t e = scan_exclusive_u64(a.kpoff, a.kpoff, nb, nullptr, temp, s);
+    if (e != hipSuccess) return e;
+  }
+  k_group_write<<<nb, kB, 0, s>>>(a, pre ? 1 : 0, merge ? 1 : 0);
   return hipGetLastError();
 }
 
@@ -2071,10 +2035,7 @@ hipError_t nu_descend_and_group(const NuArgs &a, void *temp, hipStream_t s, bool
   }
   k_descend<<<nblk(a.n), kB, 0, s>>>(a);
   GMPT_LAUNCH_CHECK();
-  hipError_t e = nu_groups(a, temp, s);
-  if (e != hipSuccess) return e;
-  k_group_merge<<<nblk(a.n), kB, 0, s>>>(a);
-  return hipGetLastError();
+  return nu_groups(a, temp, s, true);
 }
 
 hipError_t nu_regroup(NuArgs &a, uint32_t m, uint32_t nruns, void *temp, hipStream_t s) {
@@ -2094,38 +2055,23 @@ hipError_t nu_regroup(NuArgs &a, uint32_t m, uint32_t nruns, void *temp, hipStre
   t = a.u_trie; a.u_trie = a.u_trie2; a.u_trie2 = t;
   uint8_t *l = a.u_lcp; a.u_lcp = a.u_lcp2; a.u_lcp2 = l;
   Stop *st = a.stop; a.stop = a.stop2; a.stop2 = st;
-  return nu_groups(a, temp, s);
-}
-
-hipError_t nu_emit(const NuArgs &a, void *temp, hipStream_t s, bool empty) {
-  if (empty) return hipSuccess;  // k_empty_groups emitted the elements
-  k_emit_count<<<nblk(a.n), kB, 0, s>>>(a);
-  GMPT_LAUNCH_CHECK();
-  hipError_t e = scan_exclusive_u32(a.ecount, a.ecount, a.n, nullptr, temp, s);
-  if (e != hipSuccess) return e;
-  k_emit_write<<<nblk(a.n), kB, 0, s>>>(a);
-  return hipGetLastError();
+  return nu_groups(a, temp, s, false);
 }
 
 hipError_t nu_build(const NuArgs &a, void *temp, hipStream_t s, bool empty) {
   // elements: the unique keys, plus one virtual element per split short node
   // (none when the tries were empty)
   uint32_t ne_max = empty ? a.n + 1 : 2 * a.n + 2;
-  if (empty) {  // k_empty_groups wrote levels 0 .. 2
-    if (a.st_levels > 3) {
-      k_mt_top<<<1, kB, 0, s>>>(a, 3);
-      GMPT_LAUNCH_CHECK();
-    }
-  } else {
-    size_t cnt = ne_max;  // bound on the entries of each level
-    for (int k = 1; k < a.st_levels; k++) {
-      cnt = (cnt + 15) / 16;
-      k_mt_level<<<nblk(cnt), kB, 0, s>>>(a, k);
-      GMPT_LAUNCH_CHECK();
-    }
+  // the minimum tree's levels above 0, or above 2 where k_empty_groups wrote
+  // them: one launch each while a level fills more than one workgroup
+  int k = empty ? 3 : 1;
+  for (size_t cnt = (ne_max + (k == 1 ? 15 : 4095)) / (k == 1 ? 16 : 4096); k < a.st_levels && cnt > kMtTopMax;
+       k++, cnt = (cnt + 15) / 16) {
+    k_mt_level<<<nblk(cnt), kB, 0, s>>>(a, k);
+    GMPT_LAUNCH_CHECK();
   }
-  if (!empty) {  // empty tries hold no key to update
-    k_updates<<<nblk(a.n), kB, 0, s>>>(a);
+  if (k < a.st_levels) {
+    k_mt_top<<<1, kMtTopThreads, 0, s>>>(a, k);
     GMPT_LAUNCH_CHECK();
   }
   k_split_reps<<<nblk(ne_max), kB, 0, s>>>(a, ne_max);

@@ -296,3 +296,36 @@ def test_export_of_marked_paths(gmpt, workloads, oracle, kind, n, tries):
         gone = workloads.batch_from_bytes([b"\xee" * 40], [b""])
         gone.trie_ids = np.zeros(1, np.int32)
         assert set(f.flush_dirty_nodes(gone)) <= want
+
+
+@pytest.mark.parametrize("inside", [0, 1, 300, 5000, 32_767 - 54, 32_768 - 54, 40_000])
+@pytest.mark.parametrize("tries", [1, 3])
+def test_split_extension_around_keys_below_it(gmpt, workloads, oracle, inside, tries):
+    # keys that leave an extension midway, ordered before and after its subtree,
+    # with new keys and updates below it between them (one group in two runs,
+    # far apart), at sizes around those of a block and of the minimum tree's
+    # one-workgroup levels
+    rng = np.random.default_rng(inside + 7 * tries)
+    pre = [int(x) for x in rng.integers(1, 15, 24)]
+
+    def below(n):
+        return [bytes(pre + [int(x) for x in k] + [16]) for k in rng.integers(0, 16, (n, 40))]
+
+    old = below(9)
+    away = []
+    for d in range(24):
+        for x in (0, 15):
+            away.append(bytes(pre[:d] + [x] + [int(y) for y in rng.integers(0, 16, 63 - d)] + [16]))
+    first = workloads.batch_from_hex(old, [b"old%d" % i for i in range(len(old))])
+    keys = away + below(inside) + old[:6]
+    keys = [keys[i] for i in rng.permutation(len(keys))]
+    more = workloads.batch_from_hex(keys, [b"new%d" % i for i in range(len(keys))])
+    want = _after(oracle, [first, more])
+    t = gmpt.MPT(device=0, num_tries=tries)
+    for b in (first, more):
+        n = b.n
+        b.trie_ids = np.full(n, tries - 1, np.int32) if tries > 1 else None
+        _put(t, b)
+    assert t.stats()["regroups"] == 1
+    assert t.get_root_hash(tries - 1) == want
+    assert t.get_values(more)[:50] == [more.value(i) for i in range(50)]
