@@ -1382,41 +1382,48 @@ __global__ __launch_bounds__(256) void k_hc_ext_direct(Pools P, const ref_t *__r
   node_done(P, r, 32);
 }
 
-// Keccak-f[1600] with one state spread over a wave: lane 8x + y holds word
-// A[x, y] (x, y < 5) as (l, h) halves; lanes 8x + 5 .. 8x + 7 and 40..63 hold
-// zero.  A column sits in one 8-lane half-row, so theta's column parity is a
-// three-step DPP xor butterfly (quad_perm, quad_perm, row_half_mirror) with
-// no LDS traffic; the parities of columns x - 1 and x + 1, and pi with chi's
-// two row neighbours, are gathered with ds_bpermute: 10 permutes per round.
-// A padding lane takes its column parities from lane 40 (a lane of the
-// all-padding group 5, whose parity is zero), does not rotate, and gathers
-// pi and chi's three sources from itself: it stays zero with no masking.
+// Keccak-f[1600] with one state spread over a wave: lane 8y + p (y < 5) holds
+// word A[x, y], x = (p + 4) mod 5, as (l, h) halves; lanes 40 .. 63 hold zero.
+// A plane sits in one 8-lane half-row with its ends repeated (p = 0 and 5 hold
+// x = 4, p = 1 and 6 x = 0, p = 2 and 7 x = 1), so that a round takes one trip
+// through LDS:
+//   theta  the column parities by a DPP xor of the half-rows and lane swaps of
+//          rows, C[x - 1] and C[x + 1] by DPP from the lanes beside (at
+//          p = 1 .. 5, the lanes that are a later source)
+//   pi     one gather (ds_bpermute) per half for B[x, y] at every p, one for
+//          B[x + 2, y]
+//   chi    B[x + 1, y] by DPP from the next lane (at p = 0 .. 6; p = 7 holds
+//          anything, and only p = 6 takes anything from it)
+// Bound by latency: 2.4 us a permutation on an idle CU, 5.2 with four waves on
+// every SIMD.  (A column per half-row, parities and their neighbours gathered
+// and all three of chi's operands too, took 3.05 and 10.9: ten gathers a
+// round in two trips.)
 struct SpreadLane {
-  uint32_t iota, flip, t, cm, cp, s0, s1, s2;  // cm .. s2: source byte addresses for ds_bpermute
-  // pi moves A[x', y'] to B[y', 2x' + 3y']: B[x, y] comes from A[3 (y - 3x) mod 5, x]
-  static __device__ __forceinline__ uint32_t pi_src(uint32_t x, uint32_t y) {
-    return 8 * ((3 * (y + 5 - (3 * x) % 5)) % 5) + x;
+  uint32_t ok, iota, flip, t, s0, s2;  // s0, s2: source byte addresses for ds_bpermute
+  // pi moves A[x', y'] to B[y', 2x' + 3y']: B[x, y] comes from A[3y + x, x].
+  // Lanes 40 .. 63 read themselves, which are zero.
+  static __device__ __forceinline__ uint32_t pi_src(uint32_t x, uint32_t y, uint32_t lane) {
+    return 4 * (y < 5 ? 8 * x + 1 + (3 * y + x) % 5 : lane);
   }
   __device__ __forceinline__ explicit SpreadLane(uint32_t lane) {
-    const uint32_t x = lane >> 3, y = lane & 7;
-    const bool ok = x < 5 && y < 5;
-    iota = lane == 0 ? ~0u : 0u;
+    const uint32_t x = ((lane & 7) + 4) % 5, y = lane >> 3;
+    ok = y < 5 ? ~0u : 0u;
+    iota = x == 0 && y == 0 ? ~0u : 0u;
     // rho as two funnel shifts by t = (32 - r) mod 32 of the halves, swapped
     // first when flip: rotations by 0 and 32 need no other case
     const uint32_t rho = ok ? (uint32_t)kKeccak.rho[x + 5 * y] : 0u, rr = rho & 31;
     flip = (rho >= 32) != (rr == 0) ? ~0u : 0u;
     t = (32 - rr) & 31;
-    cm = ok ? 4 * (8 * ((x + 4) % 5) + y) : 4 * 40;
-    cp = ok ? 4 * (8 * ((x + 1) % 5) + y) : 4 * 40;
-    s0 = ok ? 4 * pi_src(x, y) : 4 * lane;
-    s1 = ok ? 4 * pi_src((x + 1) % 5, y) : 4 * lane;
-    s2 = ok ? 4 * pi_src((x + 2) % 5, y) : 4 * lane;
+    s0 = pi_src(x, y, lane);
+    s2 = pi_src((x + 2) % 5, y, lane);
   }
   // message word this lane absorbs (x + 5y < 17), or -1
   __device__ __forceinline__ static int word_of(uint32_t lane) {
-    const uint32_t x = lane >> 3, y = lane & 7;
-    return x < 5 && y < 5 && x + 5 * y < 17 ? (int)(x + 5 * y) : -1;
+    const uint32_t w = ((lane & 7) + 4) % 5 + 5 * (lane >> 3);
+    return lane < 40 && w < 17 ? (int)w : -1;
   }
+  // digest word q is A[q, 0]
+  __device__ __forceinline__ static bool digest(uint32_t lane) { return lane - 1 < 4; }
 };
 
 __device__ __forceinline__ uint32_t bperm(uint32_t addr, uint32_t v) {
@@ -1432,30 +1439,49 @@ __device__ __forceinline__ uint32_t xor8(uint32_t v) {
   return v;
 }
 
+template <int C>
+__device__ __forceinline__ uint32_t dpp(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, C, 0xF, 0xF, true);
+}
+constexpr int kDppNext = 0x101;  // row_shl 1: the value of lane + 1
+constexpr int kDppPrev = 0x111;  // row_shr 1
+constexpr int kDppHalf = 0x128;  // row_ror 8: of the row's other half
+// a ^ (b & c)
+__device__ __forceinline__ uint32_t xor_and(uint32_t a, uint32_t b, uint32_t c) {
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0x78);
+}
+
 __device__ __forceinline__ void keccak_spread(uint32_t &l, uint32_t &h, const SpreadLane &c) {
 #pragma unroll
   for (int ir = 0; ir < 24; ir++) {
-    // theta: A ^= C[x - 1] ^ rotl(C[x + 1], 1)
-    const uint32_t cl = xor8(l), ch = xor8(h);
-    const uint32_t cml = bperm(c.cm, cl), cmh = bperm(c.cm, ch);
-    const uint32_t cpl = bperm(c.cp, cl), cph = bperm(c.cp, ch);
-    l = xor3(l, cml, __builtin_amdgcn_alignbit(cpl, cph, 31));
-    h = xor3(h, cmh, __builtin_amdgcn_alignbit(cph, cpl, 31));
+    // theta: A ^= C[x - 1] ^ rotl(C[x + 1], 1).  Both halves' parities in one
+    // reduction: after the first swap of 32 lanes the lower lanes hold l's and
+    // the upper ones h's, and the last one gives every lane both.
+    const auto u = __builtin_amdgcn_permlane32_swap(l ^ dpp<kDppHalf>(l), h ^ dpp<kDppHalf>(h), false, false);
+    const uint32_t r = u[0] ^ u[1];
+    const auto v = __builtin_amdgcn_permlane16_swap(r, r, false, false);
+    const uint32_t q = v[0] ^ v[1];
+    const auto p = __builtin_amdgcn_permlane32_swap(q, q, false, false);
+    const uint32_t nxl = dpp<kDppNext>(p[0]), nxh = dpp<kDppNext>(p[1]);
+    l = xor_and(l, dpp<kDppPrev>(p[0]) ^ __builtin_amdgcn_alignbit(nxl, nxh, 31), c.ok);
+    h = xor_and(h, dpp<kDppPrev>(p[1]) ^ __builtin_amdgcn_alignbit(nxh, nxl, 31), c.ok);
     // rho: rotate this lane's word by its own offset
     const uint32_t a = c.flip ? h : l, b = c.flip ? l : h;
     const uint32_t nl = __builtin_amdgcn_alignbit(a, b, c.t);
     const uint32_t nh = __builtin_amdgcn_alignbit(b, a, c.t);
     // pi + chi: B[x, y] ^ (~B[x + 1, y] & B[x + 2, y])
-    l = chi3(bperm(c.s0, nl), bperm(c.s1, nl), bperm(c.s2, nl));
-    h = chi3(bperm(c.s0, nh), bperm(c.s1, nh), bperm(c.s2, nh));
+    const uint32_t b0l = bperm(c.s0, nl), b0h = bperm(c.s0, nh);
+    const uint32_t b2l = bperm(c.s2, nl), b2h = bperm(c.s2, nh);
+    l = chi3(b0l, dpp<kDppNext>(b0l), b2l);
+    h = chi3(b0h, dpp<kDppNext>(b0h), b2h);
     // iota (unrolled: the constants are immediates)
-    l ^= (uint32_t)kKeccak.rc[ir] & c.iota;
-    h ^= (uint32_t)(kKeccak.rc[ir] >> 32) & c.iota;
+    if ((uint32_t)kKeccak.rc[ir]) l = xor_and(l, (uint32_t)kKeccak.rc[ir], c.iota);
+    if ((uint32_t)(kKeccak.rc[ir] >> 32)) h = xor_and(h, (uint32_t)(kKeccak.rc[ir] >> 32), c.iota);
   }
 }
 
 // Sponge over nb padded blocks, state spread over the wave; every lane must
-// call it with the same m and nb.  Digest word q ends on lane 8q (q < 4).
+// call it with the same m and nb.  Digest word q ends on lane q + 1 (q < 4).
 __device__ __forceinline__ void sponge_spread(const uint64_t *m, uint32_t nb, uint32_t lane, const SpreadLane &c,
                                               uint32_t &l, uint32_t &h) {
   l = 0;
@@ -1470,8 +1496,6 @@ __device__ __forceinline__ void sponge_spread(const uint64_t *m, uint32_t nb, ui
     keccak_spread(l, h, c);
   }
 }
-__device__ __forceinline__ bool spread_digest_lane(uint32_t lane) { return (lane & 7) == 0 && lane < 32; }
-
 __global__ __launch_bounds__(256) void k_hc_perm_spread(Pools P, const ref_t *list, const uint64_t *slot,
                                                         const uint32_t *enc_len, uint32_t n,
                                                         const uint64_t *scratch) {
@@ -1485,7 +1509,7 @@ __global__ __launch_bounds__(256) void k_hc_perm_spread(Pools P, const ref_t *li
   sponge_spread(nb ? scratch + slot[i] / 8 : scratch, nb, lane, c, l, h);
   if (nb == 0) return;
   ref_t r = list[i];
-  if (spread_digest_lane(lane)) ((uint64_t *)node_hash(P, r))[lane >> 3] = ((uint64_t)h << 32) | l;
+  if (SpreadLane::digest(lane)) ((uint64_t *)node_hash(P, r))[lane - 1] = ((uint64_t)h << 32) | l;
   if (lane == 0) node_done(P, r, 32);
 }
 
@@ -1518,7 +1542,7 @@ __global__ __launch_bounds__(256) void k_hc_small(Pools P, const ref_t *__restri
   // a fast node's message stays in LDS (at most 4 blocks: 68 of the 80 words)
   sponge_spread(in_lds ? lds[g] : out, nb, lane, c, l, h);
   if (nb == 0) return;
-  if (spread_digest_lane(lane)) ((uint64_t *)node_hash(P, r))[lane >> 3] = ((uint64_t)h << 32) | l;
+  if (SpreadLane::digest(lane)) ((uint64_t *)node_hash(P, r))[lane - 1] = ((uint64_t)h << 32) | l;
   if (lane == 0) node_done(P, r, 32);
 }
 
@@ -1981,7 +2005,7 @@ __device__ __forceinline__ uint64_t tree_word(const uint64_t *b, const TreeMsg &
 // the size) are written through and complete before the parent's count goes
 // down; the last wave's loads of its siblings' nodes start after its own count
 // came back.  Every wave ends: a step goes one node up.
-// Bound by latency: a level costs its permutations (3.3 us each in the spread
+// Bound by latency: a level costs its permutations (2.5 us each in the spread
 // layout) and about 2.5 us of dependent loads, stores and the count.
 constexpr uint32_t kTreeMsgWords = 80;  // a branch's items and value header take at most 536 bytes
 __global__ __launch_bounds__(256) void k_tree_climb(Pools P, const ref_t *__restrict__ ready, TreeState *T) {
@@ -2027,7 +2051,7 @@ __global__ __launch_bounds__(256) void k_tree_climb(Pools P, const ref_t *__rest
         if (k + 2 < nb && w >= 0) nxt = tree_word(msg, m, nb, 17 * (k + 2) + (uint32_t)w);
         keccak_spread(l, h, sl);
       }
-      if (spread_digest_lane(lane)) st_agent(node + (lane >> 3), ((uint64_t)h << 32) | l);
+      if (SpreadLane::digest(lane)) st_agent(node + (lane - 1), ((uint64_t)h << 32) | l);
     }
     if (lane == 0) {
       const uint32_t lo = (uint32_t)meta;
@@ -2207,7 +2231,7 @@ __global__ __launch_bounds__(256) void k_kb_spread(const uint64_t *slot, const u
   SpreadLane c(lane);
   uint32_t l, h;
   sponge_spread(nb ? scratch + slot[i] / 8 : scratch, nb, lane, c, l, h);
-  if (nb && spread_digest_lane(lane)) ((uint64_t *)(out + 32 * (size_t)i))[lane >> 3] = ((uint64_t)h << 32) | l;
+  if (nb && SpreadLane::digest(lane)) ((uint64_t *)(out + 32 * (size_t)i))[lane - 1] = ((uint64_t)h << 32) | l;
 }
 
 // ------------------------------------------------------------- node export --
