@@ -8,12 +8,14 @@ constexpr uint32_t kHcClasses = 8;     // Keccak block-count classes per level
 constexpr uint32_t kHcMaxDepth = 255;  // levels: 0 = leaves, 1 + (255 - depth) otherwise
 constexpr uint32_t kHcLevels = kHcMaxDepth + 2;
 constexpr uint32_t kHcBins = kHcLevels * kHcClasses;
-// Levels with at most this many nodes spread each Keccak state over 25 lanes.
-constexpr uint32_t kHcSpreadMaxDefault = 1024;
+// Levels with at most this many nodes spread each Keccak state over 25 lanes:
+// four waves on every SIMD take 4,096 nodes' permutation in 5.2 us, one state
+// per lane takes 7.2 however few there are, and its messages take longer to
+// lay out.  Builds of 100,000 / 250,000 / 400,000 / 1,000,000 keys with the
+// line at 1,024: 399 / 459 / 506 / 788 us, 8,192: 374 / 438 / 487 / 780.
+constexpr uint32_t kHcSpreadMaxDefault = 8192;
 // Extensions per inner level that get their own (leaf word builder) kernel.
 constexpr uint32_t kExtDirectMin = 16384;
-// Spread-layout levels of at least this many nodes put two states in a wave.
-constexpr uint32_t kSpread2Min = 2048;
 
 // Classification results, read back by the host in one copy.
 struct HcMeta {
@@ -122,10 +124,10 @@ constexpr uint32_t kTreeMax = 1u << 17;
 // climb, by inner nodes: 1,450 303 / 184 us, 6,900 364 / 251, 12,300 369 / 293,
 // 21,500 382 / 364, 26,500 681 / 672, 30,100 397 / 440, 35,600 742 / 779.
 constexpr uint32_t kTreeMaxInner = 24576;
-// Up to here a leaf has a wave of its own too (8,200 entries: 113 us, leaves by
-// lane 132); above, its permutations fill the SIMDs and lanes do more per
-// cycle (17,000 entries: 147 by wave, 121 by lane).
-constexpr uint32_t kTreeSpreadLeaves = 8192;
+// Up to here a leaf has a wave of its own too; above, its permutations fill the
+// SIMDs and lanes do more per cycle (whole builds, leaves by wave / by lane, of
+// 8,200 entries: 181 / 197 us, 13,600: 206 / 209, 19,000: 229 / 217).
+constexpr uint32_t kTreeSpreadLeaves = 16384;
 hipError_t hc_tree(const Pools &P, const ref_t *list, uint32_t n, ref_t *ready, ref_t *leaves, TreeState *tree,
                    hipStream_t s);
 // Copies every trie's root hash into its header and empties the dirty list;
