@@ -101,6 +101,7 @@ struct Counters {
   uint64_t exp_bytes;            // node export: bytes of the encodings
   uint32_t exp_nodes;            // and its nodes
   uint32_t hc_nodes, hc_leaves, hc_listed;  // PhaseHC climb: nodes and leaves hashed, nodes of the dirty list
+  uint32_t hc_exts;                         // and extensions hashed
   uint32_t root0_size;           // trie 0's root as the last hash pass left it (k_hc_roots), so that
   uint8_t root0[32];             // the pass's closing counter read also brings the root to the host
 };

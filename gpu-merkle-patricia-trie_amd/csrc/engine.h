@@ -159,7 +159,7 @@ class Forest {
   int arena_exhausted();
   // hash()'s two forms: a short dirty list as one climb (*done: every node
   // was hashed), any list by levels.
-  int hash_tree(uint32_t n, bool *done);
+  int hash_tree(uint32_t n, int passes, bool *done);
   int hash_by_level(uint32_t n);
   int hash_levels(const Pools &P, const uint32_t *hist, bool direct_leaves, bool captured, uint32_t *n_leaf_out);
   // rebuild_graph's parts (graph.hip)

@@ -832,25 +832,28 @@ int Forest::hash(void *targets, int n_targets) {
   // and its counts are atomics on the nodes, which host pools do not get.
   const uint64_t others = dirty_keys_ + dirty_holes_, inner = n > others ? n - others : 0;
   dirty_keys_ = dirty_holes_ = 0;
-  if (n > 0 && n <= kTreeMax && inner <= kTreeMaxInner && !by_level_ && hc_fuse_leaves_ && hc_fuse_inner_ && hc_spread_max_ > 0 &&
-      !branch_.host && !shrt_.host) {
+  if (n > 0 && n <= kTreeMax && inner <= kTreeRowsMaxInner && !by_level_ && hc_fuse_leaves_ && hc_fuse_inner_ &&
+      hc_spread_max_ > 0 && !branch_.host && !shrt_.host) {
+    const int passes = inner <= kTreeMaxInner ? 0 : kTreeRowPasses;
     bool done = false;
-    if ((r = hash_tree(n, &done)) || done) return r;
+    if ((r = hash_tree(n, passes, &done)) || done) return r;
   }
   return hash_by_level(n);
 }
 
-int Forest::hash_tree(uint32_t n, bool *done) {
+int Forest::hash_tree(uint32_t n, int passes, bool *done) {
   int r;
   if ((r = ensure_ws(hc_sorted_, sizeof(ref_t) * (size_t)n))) return r;
   if ((r = ensure_ws(hc_enc_, sizeof(uint32_t) * (size_t)n))) return r;
+  if (passes && (r = ensure_ws(hc_slot_, sizeof(ref_t) * (size_t)n))) return r;
   if (!hc_tree_.p) tree_zero_ = false;
   if ((r = ensure_ws(hc_tree_, sizeof(TreeState)))) return r;
   TreeState *tree = (TreeState *)hc_tree_.p;
   if (!tree_zero_) HIP_TRY(hipMemsetAsync(tree, 0, sizeof(TreeState), stream_));
   tree_zero_ = false;
   if (ev0_) HIP_TRY(hipEventRecord(ev0_, stream_));
-  HIP_TRY(hc_tree(pools(), (const ref_t *)dirty_.p, n, (ref_t *)hc_sorted_.p, (ref_t *)hc_enc_.p, tree, stream_));
+  HIP_TRY(hc_tree(pools(), (const ref_t *)dirty_.p, n, (ref_t *)hc_sorted_.p, (ref_t *)hc_slot_.p, (ref_t *)hc_enc_.p,
+                  tree, passes, stream_));
   const Publish pub = next_publish();
   HIP_TRY(hc_roots(pools(), ntries_, nullptr, stream_, tree, pub));
   if (ev0_) HIP_TRY(hipEventRecord(ev1_, stream_));
@@ -859,10 +862,10 @@ int Forest::hash_tree(uint32_t n, bool *done) {
   if (cnt_.hc_nodes != cnt_.hc_listed) return 0;
   *done = true;
   rec_ = LeafRecords();
-  stats_.hash_launches = 1;
+  stats_.hash_launches = 1 + (uint32_t)passes;
   stats_.hashed_nodes = cnt_.hc_nodes;
   stats_.leaf_nodes = cnt_.hc_leaves;
-  stats_.ext_direct_nodes = 0;
+  stats_.ext_direct_nodes = cnt_.hc_exts;
   stats_.perms = cnt_.n_perms;
   stats_.enc_bytes = cnt_.enc_bytes;
   stats_.leaf_perms = cnt_.leaf_perms;

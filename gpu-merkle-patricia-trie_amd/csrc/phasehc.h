@@ -107,29 +107,42 @@ hipError_t hc_graph_check(const Pools &P, const HcMeta *meta, const uint32_t *pl
 hipError_t hc_clear(Counters *cnt, TrieHdr *tries, uint32_t ntries, hipStream_t s);
 // Work counts and list lengths of a climb (hc_tree); all zero between passes.
 constexpr uint32_t kTreeParts = 256;
+constexpr int kTreeRowPasses = 2;
 struct TreeState {
   unsigned long long lists;     // ready, leaf and listed nodes (21 bits each)
-  unsigned long long pad[15];
-  unsigned long long parts[kTreeParts][8];  // permutations, bytes, those of the leaves, nodes, leaves
+  unsigned long long tall;      // leaves of more than one block
+  unsigned long long rows[kTreeRowPasses];  // nodes ready after each row launch
+  unsigned long long pad[12];
+  unsigned long long parts[kTreeParts][8];  // permutations, bytes, those of the leaves, nodes, leaves, extensions
 };
 // Hashes the dirty list list[0 .. n) (n <= kTreeMax) without classifying it:
-// every node is hashed by the wave that hashed its last dirty child.  ready
-// and leaves hold n entries each; hc_roots with the same state folds the
-// counts and clears it.  A pass whose hc_nodes differ from its hc_listed left
-// nodes out (a dirty node that no dirty path reaches) and is to be repeated by
-// levels.
-constexpr uint32_t kTreeMax = 1u << 17;
+// every node is hashed by the wave that hashed its last dirty child, after up
+// to `passes` launches that hash ready nodes a lane each while they are many.
+// ready, ready1 (with passes) and leaves hold n entries each; hc_roots with the
+// same state folds the counts and clears it.  A pass whose hc_nodes differ from
+// its hc_listed left nodes out (a dirty node that no dirty path reaches) and is
+// to be repeated by levels.
+constexpr uint32_t kTreeMax = 1u << 20;
+// A row launch takes a ready list of at least this many nodes (the size up to
+// which a wave per node is as fast, kHcSpreadMaxDefault).
+constexpr uint32_t kTreeRowsMin = 8192;
 // A climb gives an inner node a wave of its own, so it wins while their
 // latency, not their number, sets the time.  Insert + hash by levels / as a
 // climb, by inner nodes: 1,450 303 / 184 us, 6,900 364 / 251, 12,300 369 / 293,
 // 21,500 382 / 364, 26,500 681 / 672, 30,100 397 / 440, 35,600 742 / 779.
 constexpr uint32_t kTreeMaxInner = 24576;
+// Up to here the many nodes just above the leaves go by lanes (row launches)
+// and the climb takes the rest; above, levels sorted by block count make better
+// waves.  Insert + hash by levels / so, uniform keys, by inner nodes: 30,000
+// 365 / 314 us, 38,000 370 / 324, 49,000 381 / 355, 64,000 403 / 432, 94,000
+// 434 / 475.
+constexpr uint32_t kTreeRowsMaxInner = 57344;
 // Up to here a leaf has a wave of its own too; above, its permutations fill the
 // SIMDs and lanes do more per cycle (whole builds, leaves by wave / by lane, of
 // 8,200 entries: 181 / 197 us, 13,600: 206 / 209, 19,000: 229 / 217).
 constexpr uint32_t kTreeSpreadLeaves = 16384;
-hipError_t hc_tree(const Pools &P, const ref_t *list, uint32_t n, ref_t *ready, ref_t *leaves, TreeState *tree,
-                   hipStream_t s);
+hipError_t hc_tree(const Pools &P, const ref_t *list, uint32_t n, ref_t *ready, ref_t *ready1, ref_t *leaves,
+                   TreeState *tree, int passes, hipStream_t s);
 // Copies every trie's root hash into its header and empties the dirty list;
 // with parts (from hc_count), adds the pass's work counts to the counters;
 // with tree (from hc_tree), sets them from it.

@@ -900,32 +900,52 @@ __device__ __forceinline__ void hash_spread(const Pools &P, const ref_t *__restr
                                             uint64_t *__restrict__ scratch, uint32_t *__restrict__ enc_len, uint32_t i,
                                             uint64_t *lds);
 template <int NB>
-__global__ __launch_bounds__(64) void k_hc_inner_wave(Pools P, const ref_t *__restrict__ list,
-                                                      const uint64_t *__restrict__ slot, uint32_t n,
-                                                      uint64_t *__restrict__ scratch, uint32_t *__restrict__ enc_len,
-                                                      uint32_t skip_lo, uint32_t skip_hi, uint32_t nx) {
-  if (P.cnt->graph_bad) return;  // a replayed pass whose batch is unlike the captured one
-  constexpr uint32_t RS = 17 * NB + 1;  // row stride in words (odd: lane-strided reads spread over the banks)
-  __shared__ uint64_t rows[64 * RS];
-  static_assert(64 * RS >= kInnerWords, "a node's message fits the rows");
-  if (blockIdx.x < nx) {  // uniform over the block
-    __builtin_amdgcn_s_setprio(2);  // latency-bound waves beside the bulk's permutations
-    hash_spread(P, list + skip_lo, slot + skip_lo, skip_hi - skip_lo, scratch, enc_len + skip_lo, blockIdx.x, rows);
-    return;
-  }
-  constexpr bool kDense = NB >= 4;      // many children per node: (node, slot) pairs dealt out directly
-  __shared__ ref_t cref[kDense ? 64 * 16 : 1];  // the lanes' branches' child references (dense dealing)
-  __shared__ ref_t nref[64];            // the lanes' nodes
-  __shared__ uint32_t nbase[64];        // first child number of each node (compact dealing)
-  __shared__ uint32_t ninfo[64];        // child mask (0 unless the row path encodes the node) | header length << 16
-  __shared__ uint32_t bad[64];          // 1: the node takes the generic encoder
+struct RowsLds {
+  static constexpr uint32_t kStride = 17 * NB + 1;  // words (odd: lane-strided reads spread over the banks)
+  static constexpr bool kDense = NB >= 4;           // many children per node: (node, slot) pairs dealt out directly
+  uint64_t rows[64 * kStride];
+  ref_t cref[kDense ? 64 * 16 : 1];  // the lanes' branches' child references (dense dealing)
+  ref_t nref[64];                    // the lanes' nodes
+  uint32_t nbase[64];                // first child number of each node (compact dealing)
+  uint32_t ninfo[64];                // child mask (0 unless the row path encodes the node) | header length << 16
+  uint32_t bad[64];                  // 1: the node takes the generic encoder
+};
+
+// An extension's message, [compact key, string of the child's digest d], whole
+// into its lane's row, if it takes at most NB blocks.
+template <int NB>
+__device__ __forceinline__ bool ext_row(const Pools &P, const Short &X, const uint64_t *d, uint64_t *row, uint32_t &enc,
+                                        uint32_t &nb) {
+  const uint32_t cnt = (uint32_t)X.key_len - X.term;
+  const uint32_t payload = rlp_item_len(cnt / 2 + 1, 0) + 33;
+  uint32_t hn;
+  const uint64_t hdr = rlp_hdr(payload, 0xC0, 0xF7, &hn);
+  if (keccak_blocks(hn + payload) > (uint32_t)NB) return false;
+  enc = hn + payload;
+  nb = keccak_blocks(enc);
+  WordWriter w(row);
+  w.inline_bytes(hdr, hn);
+  w.rlp_compact(P.keys + X.key_off, X.key_start, cnt, X.term);
+  w.inline_bytes(0xa0, 1);
+#pragma unroll
+  for (int q = 0; q < 4; q++) w.push(d[q], 8);
+  w.finish_keccak(17 * nb);
+  return true;
+}
+
+// Steps 1 and 2 for the wave's nodes, one per lane (r on active lanes): true
+// where the lane's row holds its node's message of nb blocks, enc bytes.
+// Every lane of the one-wave block calls it (it synchronises the block).
+template <int NB>
+__device__ __forceinline__ bool rows_encode(const Pools &P, ref_t r, bool active, RowsLds<NB> &S, uint32_t &enc,
+                                            uint32_t &nb) {
+  constexpr uint32_t RS = RowsLds<NB>::kStride;
+  constexpr bool kDense = RowsLds<NB>::kDense;
   const uint32_t lane = threadIdx.x;
-  const uint32_t i = (gridDim.x - 1 - blockIdx.x) * 64 + lane;
-  const bool active = i < n && (i < skip_lo || i >= skip_hi);
-  const ref_t r = active ? list[i] : REF_NULL;
   const bool branch = active && ref_type(r) == T_BRANCH;
   bool fast = branch, ext = false;
-  uint32_t mask = 0, enc = 0, nb = 0, hn = 0;
+  uint32_t mask = 0, hn = 0;
+  enc = nb = 0;
   uint64_t hdr = 0;
   if (branch) {
     const Branch &B = P.branch[ref_idx(r)];
@@ -933,7 +953,7 @@ __global__ __launch_bounds__(64) void k_hc_inner_wave(Pools P, const ref_t *__re
 #pragma unroll
     for (int q = 0; q < 4; q++) {
       const uint4 v = cw[q];
-      if (kDense) ((uint4 *)(cref + 16 * lane))[q] = v;
+      if (kDense) ((uint4 *)(S.cref + 16 * lane))[q] = v;
       mask |= (v.x != REF_NULL ? 1u : 0u) << (4 * q);
       mask |= (v.y != REF_NULL ? 2u : 0u) << (4 * q);
       mask |= (v.z != REF_NULL ? 4u : 0u) << (4 * q);
@@ -951,11 +971,11 @@ __global__ __launch_bounds__(64) void k_hc_inner_wave(Pools P, const ref_t *__re
   const uint32_t kc = fast ? (uint32_t)__popc(mask) : 0u;
   const uint32_t incl = wave_inclusive_scan(kc);
   const uint32_t total = (uint32_t)__shfl((int)incl, 63, 64);  // the wave's row-path children
-  nref[lane] = r;
-  nbase[lane] = incl - kc;
-  ninfo[lane] = (fast ? mask : 0u) | (hn << 16);
-  bad[lane] = fast ? 0u : 1u;
-  uint64_t *row = rows + lane * RS;
+  S.nref[lane] = r;
+  S.nbase[lane] = incl - kc;
+  S.ninfo[lane] = (fast ? mask : 0u) | (hn << 16);
+  S.bad[lane] = fast ? 0u : 1u;
+  uint64_t *row = S.rows + lane * RS;
   if (fast)
     for (uint32_t w = 0; w < 17 * nb; w++) row[w] = 0;
   __syncthreads();  // rows zeroed; child references, masks visible to the wave
@@ -973,58 +993,44 @@ __global__ __launch_bounds__(64) void k_hc_inner_wave(Pools P, const ref_t *__re
     rb[enc] = 0x01;      // Keccak padding; enc < 136 * nb, so this byte is the message's own
     rb[136 * nb - 1] |= 0x80;
   } else if (ext) {
-    // [compact key, string of the child's digest]: the whole row from this lane
-    const Short &S = P.shrt[ref_idx(r)];
-    const Branch &C = P.branch[ref_idx(S.child)];
+    const Short &X = P.shrt[ref_idx(r)];
+    const Branch &C = P.branch[ref_idx(X.child)];
+    uint64_t d[4];
     const uint4 d0 = ((const uint4 *)C.hash)[0], d1 = ((const uint4 *)C.hash)[1];
-    const uint32_t cnt = (uint32_t)S.key_len - S.term;
-    const uint32_t payload = rlp_item_len(cnt / 2 + 1, 0) + 33;
-    uint32_t ehn;
-    const uint64_t ehdr = rlp_hdr(payload, 0xC0, 0xF7, &ehn);
-    const uint32_t eenc = ehn + payload;
-    if (C.hash_size == 32 && keccak_blocks(eenc) <= (uint32_t)NB) {
-      WordWriter w(row);
-      w.inline_bytes(ehdr, ehn);
-      w.rlp_compact(P.keys + S.key_off, S.key_start, cnt, S.term);
-      w.inline_bytes(0xa0, 1);
-      w.push(((uint64_t)d0.y << 32) | d0.x, 8);
-      w.push(((uint64_t)d0.w << 32) | d0.z, 8);
-      w.push(((uint64_t)d1.y << 32) | d1.x, 8);
-      w.push(((uint64_t)d1.w << 32) | d1.z, 8);
-      nb = keccak_blocks(eenc);
-      w.finish_keccak(17 * nb);
-      enc = eenc;
-      bad[lane] = 0;
-      fast = true;
-    }
+    d[0] = ((uint64_t)d0.y << 32) | d0.x;
+    d[1] = ((uint64_t)d0.w << 32) | d0.z;
+    d[2] = ((uint64_t)d1.y << 32) | d1.x;
+    d[3] = ((uint64_t)d1.w << 32) | d1.z;
+    fast = C.hash_size == 32 && ext_row<NB>(P, X, d, row, enc, nb);
+    if (fast) S.bad[lane] = 0;
   }
   if (!kDense) {
     // the wave's present children, numbered node by node, dealt out round
     // robin (a few per lane)
     for (uint32_t t = lane; t < total; t += 64) {
-      uint32_t lo = 0, hi = 63;  // the node: the last with nbase <= t (it has children)
+      uint32_t lo = 0, hi = 63;  // the node: the last with S.nbase <= t (it has children)
       while (lo < hi) {
         const uint32_t mid = (lo + hi + 1) / 2;
-        if (nbase[mid] <= t)
+        if (S.nbase[mid] <= t)
           lo = mid;
         else
           hi = mid - 1;
       }
-      const uint32_t j = lo, info = ninfo[j];
-      const uint32_t o = t - nbase[j];  // the child's rank among the node's present children
+      const uint32_t j = lo, info = S.ninfo[j];
+      const uint32_t o = t - S.nbase[j];  // the child's rank among the node's present children
       uint32_t mm = info & 0xffffu;     // its slot: the o-th set bit of the mask
       for (uint32_t q = 0; q < o; q++) mm &= mm - 1;
       const uint32_t sl = __ffs(mm) - 1;
-      const ref_t c = P.branch[ref_idx(nref[j])].child[sl];
+      const ref_t c = P.branch[ref_idx(S.nref[j])].child[sl];
       const bool sh = ref_type(c) == T_SHORT;
       const uint8_t *h = sh ? P.shrt[ref_idx(c)].hash : P.branch[ref_idx(c)].hash;
       const uint4 d0 = ((const uint4 *)h)[0], d1 = ((const uint4 *)h)[1];
       const uint32_t hs = sh ? P.shrt[ref_idx(c)].hash_size : P.branch[ref_idx(c)].hash_size;
       if (hs != 32) {
-        bad[j] = 1;  // an embedded child: the node's own lane encodes it generically
+        S.bad[j] = 1;  // an embedded child: the node's own lane encodes it generically
         continue;
       }
-      or_child_item((uint32_t *)(rows + j * RS), (info >> 16) + 33 * o + (sl - o), d0, d1);
+      or_child_item((uint32_t *)(S.rows + j * RS), (info >> 16) + 33 * o + (sl - o), d0, d1);
     }
   }
   // (dense) the wave's (node, slot) pairs: pair p = node p / 16, slot p % 16;
@@ -1038,7 +1044,7 @@ __global__ __launch_bounds__(64) void k_hc_inner_wave(Pools P, const ref_t *__re
     for (int u = 0; u < 4; u++) {
       const uint32_t p = lane + 64 * (q0 + u);
       const uint32_t j = p >> 4, s = p & 15u;
-      const uint32_t info = ninfo[j];
+      const uint32_t info = S.ninfo[j];
       const uint32_t m = info & 0xffffu;
       const uint32_t o = __popc(m & ((1u << s) - 1u));  // the child's rank among the node's present children
       has[u] = (m >> s) & 1u;
@@ -1047,7 +1053,7 @@ __global__ __launch_bounds__(64) void k_hc_inner_wave(Pools P, const ref_t *__re
       hs[u] = 0;
       d0[u] = d1[u] = make_uint4(0, 0, 0, 0);
       if (has[u]) {
-        const ref_t c = cref[16 * j + s];
+        const ref_t c = S.cref[16 * j + s];
         const bool sh = ref_type(c) == T_SHORT;
         const uint8_t *h = sh ? P.shrt[ref_idx(c)].hash : P.branch[ref_idx(c)].hash;
         d0[u] = ((const uint4 *)h)[0];
@@ -1059,15 +1065,47 @@ __global__ __launch_bounds__(64) void k_hc_inner_wave(Pools P, const ref_t *__re
     for (int u = 0; u < 4; u++) {
       if (!has[u]) continue;
       if (hs[u] != 32) {
-        bad[jj[u]] = 1;  // an embedded child: the node's own lane encodes it generically
+        S.bad[jj[u]] = 1;  // an embedded child: the node's own lane encodes it generically
         continue;
       }
-      or_child_item((uint32_t *)(rows + jj[u] * RS), off[u], d0[u], d1[u]);
+      or_child_item((uint32_t *)(S.rows + jj[u] * RS), off[u], d0[u], d1[u]);
     }
   }
   __syncthreads();  // every row complete
+  return fast && S.bad[lane] == 0;
+}
+
+// A digest into its node, and the node clean.
+__device__ __forceinline__ void store_digest(const Pools &P, ref_t r, const uint64_t *st) {
+  uint64_t *hp = (uint64_t *)node_hash(P, r);
+  hp[0] = st[0];
+  hp[1] = st[1];
+  hp[2] = st[2];
+  hp[3] = st[3];
+  node_done(P, r, 32);
+}
+
+template <int NB>
+__global__ __launch_bounds__(64) void k_hc_inner_wave(Pools P, const ref_t *__restrict__ list,
+                                                      const uint64_t *__restrict__ slot, uint32_t n,
+                                                      uint64_t *__restrict__ scratch, uint32_t *__restrict__ enc_len,
+                                                      uint32_t skip_lo, uint32_t skip_hi, uint32_t nx) {
+  if (P.cnt->graph_bad) return;  // a replayed pass whose batch is unlike the captured one
+  __shared__ RowsLds<NB> S;
+  static_assert(64 * RowsLds<NB>::kStride >= kInnerWords, "a node's message fits the rows");
+  if (blockIdx.x < nx) {  // uniform over the block
+    __builtin_amdgcn_s_setprio(2);  // latency-bound waves beside the bulk's permutations
+    hash_spread(P, list + skip_lo, slot + skip_lo, skip_hi - skip_lo, scratch, enc_len + skip_lo, blockIdx.x, S.rows);
+    return;
+  }
+  const uint32_t lane = threadIdx.x;
+  const uint32_t i = (gridDim.x - 1 - blockIdx.x) * 64 + lane;
+  const bool active = i < n && (i < skip_lo || i >= skip_hi);
+  const ref_t r = active ? list[i] : REF_NULL;
+  uint32_t enc, nb;
+  const bool use_row = rows_encode<NB>(P, r, active, S, enc, nb);
   if (!active) return;
-  const bool use_row = fast && bad[lane] == 0;
+  const uint64_t *row = S.rows + lane * RowsLds<NB>::kStride;
   uint64_t *out = scratch + slot[i] / 8;
   if (!use_row) {
     encode_generic(P, r, out, &enc);
@@ -1088,12 +1126,7 @@ __global__ __launch_bounds__(64) void k_hc_inner_wave(Pools P, const ref_t *__re
     }
     keccak_f1600(st);
   }
-  uint64_t *hp = (uint64_t *)node_hash(P, r);
-  hp[0] = st[0];
-  hp[1] = st[1];
-  hp[2] = st[2];
-  hp[3] = st[3];
-  node_done(P, r, 32);
+  store_digest(P, r, st);
 }
 
 __global__ __launch_bounds__(256) void k_hc_perm_lane(Pools P, const ref_t *list, const uint64_t *slot,
@@ -1564,6 +1597,9 @@ __global__ __launch_bounds__(256) void k_hc_small(Pools P, const ref_t *__restri
 //                  word) and a branch the number of its dirty children; the
 //                  nodes without one are ready
 //   k_tree_leaves  (longer lists only) the leaves, one per lane
+//   k_tree_rows    (lists of many inner nodes only, a few launches) while many
+//                  nodes are ready, one per lane; those without a row of a few
+//                  blocks, and parents that became ready, make the next list
 //   k_tree_climb   one wave per ready node hashes it in the spread layout and
 //                  counts it off at its parent; the wave that was last goes on
 //                  with the parent.  No wave waits for another, and no level
@@ -1591,21 +1627,33 @@ static_assert(offsetof(Short, depth) == 48 && offsetof(Short, hash_size) == 50 &
                   offsetof(Short, dirty) == 52,
               "short node words");
 
-__device__ __forceinline__ unsigned long long tree_reserve(TreeState *T, unsigned long long mine, uint32_t lane) {
+__device__ __forceinline__ unsigned long long tree_reserve(unsigned long long *at, unsigned long long mine,
+                                                           uint32_t lane) {
   unsigned long long base = 0;
-  if (lane == 0) base = atomicAdd(&T->lists, mine);
+  if (lane == 0) base = atomicAdd(at, mine);
   return (unsigned long long)__shfl((long long)base, 0);
 }
 
-// One thread per dirty-list entry (64 per block: the loads of a few thousand
-// nodes spread over the CUs).  With leaf_lanes the leaves the word builder
-// takes go to the leaf list, otherwise every leaf is ready.
-__global__ __launch_bounds__(64) void k_tree_link(Pools P, const ref_t *__restrict__ list, uint32_t n,
+// Entries of ready list k: the links' and leaves' (0), or the ones row launch
+// k left.  Row launch k takes list k when it is long enough for lanes (and
+// then makes list k + 1); the climb takes the first list that is not.
+__device__ __forceinline__ uint32_t tree_ready(const TreeState *T, int k) {
+  return (uint32_t)(k == 0 ? T->lists & kTreeListMask : T->rows[k - 1]);
+}
+
+// One thread per dirty-list entry (W waves per block: one, to spread the loads
+// of a few thousand nodes over the CUs, or four, since blocks take their places
+// in the lists by an atomic on one address each).  With leaf_lanes the leaves
+// the word builder takes go to the leaf list, those of one block from its front
+// and the others from its back (a wave of both would take the longer's time),
+// otherwise every leaf is ready.
+template <int W>
+__global__ __launch_bounds__(64 * W) void k_tree_link(Pools P, const ref_t *__restrict__ list, uint32_t n,
                                                   ref_t *__restrict__ ready, ref_t *__restrict__ leaves,
                                                   TreeState *T, int leaf_lanes) {
-  const uint32_t lane = threadIdx.x, i = blockIdx.x * 64 + lane;
+  const uint32_t lane = __lane_id(), i = grid_tid();
   const ref_t r = i < n ? list[i] : REF_NULL;  // builds leave null holes
-  bool rdy = false, leaf = false, listed = false;
+  bool rdy = false, leaf = false, tall = false, listed = false;
   if (ref_type(r) == T_BRANCH) {
     Branch &B = P.branch[ref_idx(r)];
     ref_t c[16];
@@ -1643,6 +1691,8 @@ __global__ __launch_bounds__(64) void k_tree_link(Pools P, const ref_t *__restri
       leaf = leaf_lanes && (uint32_t)S.key_len - S.term <= kLeafFastNibbles &&
              P.value[ref_idx(c)].size <= kLeafDirectMaxValue;
       rdy = !leaf;
+      tall = leaf && leaf_blocks((uint32_t)S.key_len - S.term, P.value[ref_idx(c)].size) > 1;
+      leaf = leaf && !tall;
     } else if (S.lock & 1) {
       S.dirty = 0;  // replaced by a split since it was listed: no node's child any more, and its child another's
     } else {
@@ -1652,55 +1702,159 @@ __global__ __launch_bounds__(64) void k_tree_link(Pools P, const ref_t *__restri
       if (!rdy) *f = tree_parent_word(r);
     }
   }
-  const uint64_t mr = __ballot(rdy), ml = __ballot(leaf), ma = __ballot(listed);
-  if (ma == 0) return;
-  const unsigned long long base = tree_reserve(
-      T, (unsigned long long)__popcll(mr) | (unsigned long long)__popcll(ml) << kTreeListBits |
-             (unsigned long long)__popcll(ma) << (2 * kTreeListBits), lane);
+  const uint64_t mr = __ballot(rdy), ml = __ballot(leaf), mt = __ballot(tall), ma = __ballot(listed);
+  const unsigned long long mine = (unsigned long long)__popcll(mr) | (unsigned long long)__popcll(ml) << kTreeListBits |
+                                  (unsigned long long)__popcll(ma) << (2 * kTreeListBits);
+  unsigned long long base, tbase = 0;
+  if (W == 1) {
+    if (ma == 0) return;
+    base = tree_reserve(&T->lists, mine, lane);
+    if (mt) tbase = tree_reserve(&T->tall, (unsigned long long)__popcll(mt), lane);
+  } else {
+    __shared__ unsigned long long sums[W][2], place[2];
+    const uint32_t g = threadIdx.x / 64;
+    if (lane == 0) {
+      sums[g][0] = mine;
+      sums[g][1] = (unsigned long long)__popcll(mt);
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+      unsigned long long all = 0;
+      for (int q = 0; q < W; q++) all += sums[q][threadIdx.x];
+      place[threadIdx.x] = all ? atomicAdd(threadIdx.x ? &T->tall : &T->lists, all) : 0ull;
+    }
+    __syncthreads();
+    base = place[0];
+    tbase = place[1];
+    for (uint32_t q = 0; q < g; q++) {
+      base += sums[q][0];
+      tbase += sums[q][1];
+    }
+  }
   const uint64_t below = (1ull << lane) - 1;
   if (rdy) ready[(uint32_t)(base & kTreeListMask) + (uint32_t)__popcll(mr & below)] = r;
   if (leaf) leaves[(uint32_t)(base >> kTreeListBits & kTreeListMask) + (uint32_t)__popcll(ml & below)] = r;
+  if (tall) leaves[n - 1 - ((uint32_t)tbase + (uint32_t)__popcll(mt & below))] = r;
 }
 
-// Adds the wave's work counts (v on lanes 0 .. 5 as TreeState::parts' words).
+// Adds the wave's work counts (v on lanes 0 .. 6 as TreeState::parts' words).
 __device__ __forceinline__ void tree_count(TreeState *T, uint32_t wave, uint32_t lane, unsigned long long v) {
-  if (lane < 6 && v) atomicAdd(&T->parts[wave % kTreeParts][lane], v);
+  if (lane < 7 && v) atomicAdd(&T->parts[wave % kTreeParts][lane], v);
 }
 
-// The leaf list, one leaf per lane (as k_hc_leaf_direct); a branch whose last
-// dirty child was one of them becomes ready.
-__global__ __launch_bounds__(256) void k_tree_leaves(Pools P, const ref_t *__restrict__ leaves, ref_t *ready,
-                                                     TreeState *T) {
+// A hashed node counts off at its parent word par: the parent if that was its
+// last dirty child, or null.
+__device__ __forceinline__ ref_t tree_up(const Pools &P, uint32_t par) {
+  if (par >> 2 == 0) return REF_NULL;  // a root
+  if (par & 2) return make_ref(T_SHORT, (par >> 2) - 1);  // an extension's only child
+  return __hip_atomic_fetch_add(&P.branch[(par >> 2) - 1].pad1, ~0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 1u
+             ? make_ref(T_BRANCH, (par >> 2) - 1)
+             : REF_NULL;
+}
+// Appends the lanes' nodes (null: none) to a list with its length at `at`.
+__device__ __forceinline__ void tree_append(unsigned long long *at, ref_t *list, ref_t r, uint32_t lane) {
+  const uint64_t m = __ballot(r != REF_NULL);
+  if (m == 0) return;
+  const uint32_t base = (uint32_t)(tree_reserve(at, (unsigned long long)__popcll(m), lane) & kTreeListMask);
+  if (r != REF_NULL) list[base + (uint32_t)__popcll(m & ((1ull << lane) - 1))] = r;
+}
+__device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
+  for (int off = 32; off > 0; off >>= 1) v += (uint32_t)__shfl_xor((int)v, off);
+  return v;
+}
+
+// The leaf list, one leaf per lane (as k_hc_leaf_direct), the waves of longer
+// leaves first; a node whose last dirty child was one of them becomes ready.
+__global__ __launch_bounds__(256) void k_tree_leaves(Pools P, const ref_t *__restrict__ leaves, uint32_t n_list,
+                                                     ref_t *ready, TreeState *T) {
   __shared__ uint64_t head[256][kLeafDirectHead];
   const uint32_t i = grid_tid(), lane = __lane_id();
-  const uint32_t n = (uint32_t)(T->lists >> kTreeListBits & kTreeListMask);  // only the ready count moves here
-  if (i - lane >= n) return;
+  const uint32_t nt = (uint32_t)T->tall, wt = (nt + 63) / 64 * 64;                 // the longer ones' lanes
+  const uint32_t n1 = (uint32_t)(T->lists >> kTreeListBits & kTreeListMask);  // only the ready count moves here
+  const bool tall = i < wt;                                                        // uniform over the wave
+  const uint32_t k = tall ? i : i - wt, n = tall ? nt : n1;
+  if (k - lane >= n) return;
+  const bool act = k < n;
+  const ref_t r = act ? leaves[tall ? n_list - 1 - k : k] : REF_NULL;
+  uint64_t m[2] = {0, 0};
+  uint32_t wlo = 0xffffu, whi = 0;  // the wave's window of string words (hash_leaf_shaped)
+  if (act) {
+    leaf_meta(P, r, m);
+    leaf_value_words(m[0], wlo, whi);
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    wlo = min(wlo, (uint32_t)__shfl_xor((int)wlo, off));
+    whi = max(whi, (uint32_t)__shfl_xor((int)whi, off));
+  }
+  wlo = __builtin_amdgcn_readfirstlane(wlo);
+  whi = __builtin_amdgcn_readfirstlane(whi);
   uint32_t enc = 0;
   ref_t up = REF_NULL;
-  if (i < n) {
-    const ref_t r = leaves[i];
+  if (act) {
     const uint32_t par = P.shrt[ref_idx(r)].dirty;
-    uint64_t m[2];
-    leaf_meta(P, r, m);
-    enc = hash_leaf_shaped(P, r, m[0], m[1], head[threadIdx.x]);
-    // a leaf's parent is a branch
-    if (par >> 2 && __hip_atomic_fetch_add(&P.branch[(par >> 2) - 1].pad1, ~0u, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT) == 1u)
-      up = make_ref(T_BRANCH, (par >> 2) - 1);
+    enc = hash_leaf_shaped(P, r, m[0], m[1], head[threadIdx.x], wlo, whi);
+    up = tree_up(P, par);
   }
-  const uint64_t mu = __ballot(up != REF_NULL);
-  if (mu) {
-    const uint32_t base = (uint32_t)(tree_reserve(T, (unsigned long long)__popcll(mu), lane) & kTreeListMask);
-    if (up != REF_NULL) ready[base + (uint32_t)__popcll(mu & ((1ull << lane) - 1))] = up;
-  }
-  uint32_t bytes = enc, perms = enc >= 32 ? keccak_blocks(enc) : 0u;
-  for (int off = 32; off > 0; off >>= 1) {
-    bytes += (uint32_t)__shfl_xor((int)bytes, off);
-    perms += (uint32_t)__shfl_xor((int)perms, off);
-  }
-  const uint32_t nodes = min(n - (i - lane), 64u);
+  tree_append(&T->lists, ready, up, lane);
+  const uint32_t bytes = wave_sum(enc), perms = wave_sum(enc >= 32 ? keccak_blocks(enc) : 0u);
+  const uint32_t nodes = min(n - (k - lane), 64u);
   tree_count(T, i / 64, lane,
-             lane == 0 || lane == 2 ? perms : lane == 1 || lane == 3 ? bytes : nodes);
+             lane == 0 || lane == 2 ? perms : lane == 1 || lane == 3 ? bytes : lane < 6 ? nodes : 0u);
+}
+
+// Ready list k (in) one node per lane, with the messages in LDS rows of NB
+// blocks (rows_encode), if it is long enough; an extension whose child a lane
+// has just hashed follows in the same lane.  What the rows do not take (taller
+// nodes, values in branches, embedded children, leaves) and the parents that
+// became ready make list k + 1 (out).
+template <int NB>
+__global__ __launch_bounds__(64) void k_tree_rows(Pools P, const ref_t *__restrict__ in, ref_t *__restrict__ out,
+                                                  TreeState *T, int k) {
+  const uint32_t n = tree_ready(T, k), lane = threadIdx.x;
+  if (n < kTreeRowsMin) return;
+  __shared__ RowsLds<NB> S;
+  uint64_t *row = S.rows + lane * RowsLds<NB>::kStride;
+  uint32_t perms = 0, bytes = 0, nodes = 0, exts = 0;
+  for (uint32_t b = blockIdx.x * 64; b < n; b += gridDim.x * 64) {
+    const bool active = b + lane < n;
+    const ref_t r = active ? in[b + lane] : REF_NULL;
+    uint32_t par = active ? *node_dirty_flag(P, r) : 0u;
+    uint32_t enc, nb;
+    const bool use = rows_encode<NB>(P, r, active, S, enc, nb) && active;
+    ref_t up = r;  // not taken
+    if (use) {
+      ref_t me = r;
+      uint64_t st[25];
+      for (;;) {
+#pragma unroll
+        for (int q = 0; q < 25; q++) st[q] = 0;
+        for (uint32_t j = 0; j < nb; j++) {
+#pragma unroll
+          for (int q = 0; q < 17; q++) st[q] ^= row[17 * j + q];
+          keccak_f1600(st);
+        }
+        store_digest(P, me, st);
+        perms += nb;
+        bytes += enc;
+        nodes++;
+        exts += ref_type(me) == T_SHORT ? 1u : 0u;
+        up = tree_up(P, par);
+        if (up == REF_NULL || ref_type(up) == T_BRANCH) break;
+        const Short &X = P.shrt[ref_idx(up)];
+        if (!is_direct_ext(X) || !ext_row<NB>(P, X, st, row, enc, nb)) break;
+        par = X.dirty;
+        me = up;
+      }
+    }
+    tree_append(&T->rows[k], out, up, lane);
+    __syncthreads();  // the rows are reused
+  }
+  perms = wave_sum(perms);
+  bytes = wave_sum(bytes);
+  nodes = wave_sum(nodes);
+  exts = wave_sum(exts);
+  tree_count(T, blockIdx.x, lane,
+             lane == 0 ? perms : lane == 1 ? bytes : lane == 4 ? nodes : lane == 6 ? exts : 0u);
 }
 
 // Agent-scope accesses for what waves on other dies write in the same launch.
@@ -1868,85 +2022,96 @@ __device__ __forceinline__ uint64_t tree_word(const uint64_t *b, const TreeMsg &
 // Bound by latency: a level costs its permutations (2.5 us each in the spread
 // layout) and about 2.5 us of dependent loads, stores and the count.
 constexpr uint32_t kTreeMsgWords = 80;  // a branch's items and value header take at most 536 bytes
-__global__ __launch_bounds__(256) void k_tree_climb(Pools P, const ref_t *__restrict__ ready, TreeState *T) {
+__global__ __launch_bounds__(256) void k_tree_climb(Pools P, const ref_t *__restrict__ ready,
+                                                    const ref_t *__restrict__ ready1, TreeState *T, int passes) {
   __shared__ uint64_t lds[256 / 64][kTreeMsgWords];
   const uint32_t lane = __lane_id(), g = threadIdx.x / 64;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (256 / 64) + g);
-  if (wave >= (uint32_t)(T->lists & kTreeListMask)) return;
+  int pass = 0;  // the list left by the row launches
+  while (pass < passes && tree_ready(T, pass) >= kTreeRowsMin) pass++;
+  const uint32_t n = tree_ready(T, pass);
+  if (pass & 1) ready = ready1;
+  if (wave >= n) return;
   uint64_t *msg = lds[g];
   uint8_t *b = (uint8_t *)msg;
   const SpreadLane sl(lane);
   const int w = SpreadLane::word_of(lane);
   uint32_t perms = 0, bytes = 0, lperms = 0, lbytes = 0, nodes = 0, lnodes = 0;
-  ref_t r = __builtin_amdgcn_readfirstlane(ready[wave]);
-  for (;;) {
-    const bool branch = ref_type(r) == T_BRANCH;
-    const uint32_t idx = ref_idx(r);
-    uint64_t *node = branch ? (uint64_t *)&P.branch[idx] : (uint64_t *)&P.shrt[idx];
-    const uint64_t meta = node[branch ? 4 : 6];  // dirty word in the upper half: the parent
-    bool leaf = false;
-    TreeMsg m;
-    if (branch) {
-      tree_branch(P, P.branch[idx], lane, b, m);
-    } else {
-      leaf = ref_type(P.shrt[idx].child) == T_VALUE;
-      tree_short(P, P.shrt[idx], lane, b, m);
-    }
-    wave_lds_order();
-    m.enc = __builtin_amdgcn_readfirstlane(m.enc);
-    const uint32_t nb = m.enc >= 32 ? keccak_blocks(m.enc) : 0u;
-    uint32_t hs = 32;
-    if (nb == 0) {  // shorter than a digest: the raw encoding is the "hash"
-      hs = m.enc;
-      if (lane < 4) st_agent(node + lane, tree_word(msg, m, 0, lane));
-    } else {
-      uint32_t l = 0, h = 0;
-      // the words of two blocks are in flight before the first permutation
-      uint64_t cur = w >= 0 ? tree_word(msg, m, nb, (uint32_t)w) : 0ull;
-      uint64_t nxt = w >= 0 && nb > 1 ? tree_word(msg, m, nb, 17 + (uint32_t)w) : 0ull;
-      for (uint32_t k = 0; k < nb; k++) {
-        l ^= (uint32_t)cur;
-        h ^= (uint32_t)(cur >> 32);
-        cur = nxt;
-        if (k + 2 < nb && w >= 0) nxt = tree_word(msg, m, nb, 17 * (k + 2) + (uint32_t)w);
-        keccak_spread(l, h, sl);
+  uint32_t exts = 0;
+  for (uint32_t i = wave; i < n; i += gridDim.x * (256 / 64)) {
+    ref_t r = __builtin_amdgcn_readfirstlane(ready[i]);
+    for (;;) {
+      const bool branch = ref_type(r) == T_BRANCH;
+      const uint32_t idx = ref_idx(r);
+      uint64_t *node = branch ? (uint64_t *)&P.branch[idx] : (uint64_t *)&P.shrt[idx];
+      const uint64_t meta = node[branch ? 4 : 6];  // dirty word in the upper half: the parent
+      bool leaf = false;
+      TreeMsg m;
+      if (branch) {
+        tree_branch(P, P.branch[idx], lane, b, m);
+      } else {
+        leaf = ref_type(P.shrt[idx].child) == T_VALUE;
+        tree_short(P, P.shrt[idx], lane, b, m);
       }
-      if (SpreadLane::digest(lane)) st_agent(node + (lane - 1), ((uint64_t)h << 32) | l);
-    }
-    if (lane == 0) {
-      const uint32_t lo = (uint32_t)meta;
-      if (branch)
-        st_agent(node + 4, (uint64_t)((lo & 0xffffff00u) | hs));
-      else
-        st_agent(node + 6, (uint64_t)((lo & 0xff00ffffu) | hs << 16));
-    }
-    perms += nb;
-    bytes += m.enc;
-    nodes++;
-    if (leaf) {
-      lperms += nb;
-      lbytes += m.enc;
-      lnodes++;
-    }
-    const uint32_t par = __builtin_amdgcn_readfirstlane((uint32_t)(meta >> 32));
-    if (par >> 2 == 0) break;  // a root
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    __builtin_amdgcn_s_waitcnt(0);  // the node's stores have completed
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    if (par & 2) {
-      r = make_ref(T_SHORT, (par >> 2) - 1);  // an extension's only child
-    } else {
-      uint32_t left = 0;
-      if (lane == 0)
-        left = __hip_atomic_fetch_add(&P.branch[(par >> 2) - 1].pad1, ~0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      left = __builtin_amdgcn_readfirstlane(left);
-      if (left != 1) break;  // another child's wave goes on
-      r = make_ref(T_BRANCH, (par >> 2) - 1);
+      wave_lds_order();
+      m.enc = __builtin_amdgcn_readfirstlane(m.enc);
+      const uint32_t nb = m.enc >= 32 ? keccak_blocks(m.enc) : 0u;
+      uint32_t hs = 32;
+      if (nb == 0) {  // shorter than a digest: the raw encoding is the "hash"
+        hs = m.enc;
+        if (lane < 4) st_agent(node + lane, tree_word(msg, m, 0, lane));
+      } else {
+        uint32_t l = 0, h = 0;
+        // the words of two blocks are in flight before the first permutation
+        uint64_t cur = w >= 0 ? tree_word(msg, m, nb, (uint32_t)w) : 0ull;
+        uint64_t nxt = w >= 0 && nb > 1 ? tree_word(msg, m, nb, 17 + (uint32_t)w) : 0ull;
+        for (uint32_t k = 0; k < nb; k++) {
+          l ^= (uint32_t)cur;
+          h ^= (uint32_t)(cur >> 32);
+          cur = nxt;
+          if (k + 2 < nb && w >= 0) nxt = tree_word(msg, m, nb, 17 * (k + 2) + (uint32_t)w);
+          keccak_spread(l, h, sl);
+        }
+        if (SpreadLane::digest(lane)) st_agent(node + (lane - 1), ((uint64_t)h << 32) | l);
+      }
+      if (lane == 0) {
+        const uint32_t lo = (uint32_t)meta;
+        if (branch)
+          st_agent(node + 4, (uint64_t)((lo & 0xffffff00u) | hs));
+        else
+          st_agent(node + 6, (uint64_t)((lo & 0xff00ffffu) | hs << 16));
+      }
+      perms += nb;
+      bytes += m.enc;
+      nodes++;
+      if (leaf) {
+        lperms += nb;
+        lbytes += m.enc;
+        lnodes++;
+      } else if (!branch) {
+        exts++;
+      }
+      const uint32_t par = __builtin_amdgcn_readfirstlane((uint32_t)(meta >> 32));
+      if (par >> 2 == 0) break;  // a root
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      __builtin_amdgcn_s_waitcnt(0);  // the node's stores have completed
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      if (par & 2) {
+        r = make_ref(T_SHORT, (par >> 2) - 1);  // an extension's only child
+      } else {
+        uint32_t left = 0;
+        if (lane == 0)
+          left = __hip_atomic_fetch_add(&P.branch[(par >> 2) - 1].pad1, ~0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        left = __builtin_amdgcn_readfirstlane(left);
+        if (left != 1) break;  // another child's wave goes on
+        r = make_ref(T_BRANCH, (par >> 2) - 1);
+      }
+      wave_lds_order();
     }
     wave_lds_order();
   }
   tree_count(T, wave, lane,
-             lane == 0 ? perms : lane == 1 ? bytes : lane == 2 ? lperms : lane == 3 ? lbytes : lane == 4 ? nodes : lnodes);
+             lane == 0 ? perms : lane == 1 ? bytes : lane == 2 ? lperms : lane == 3 ? lbytes : lane == 4 ? nodes : lane == 5 ? lnodes : exts);
 }
 
 // One wave: the counters, then (once those stores have completed) the number.
@@ -2010,30 +2175,32 @@ __device__ __forceinline__ void roots_body(const Pools &P, uint32_t ntries, cons
   }
   if (tree && blockIdx.x == 0) {  // a climb's counts (uniform branch); its state is left zero for the next one
     static_assert(kTreeParts == 256, "one partial per thread");
-    __shared__ unsigned long long st[4][6];
-    unsigned long long v[6];
+    __shared__ unsigned long long st[4][7];
+    unsigned long long v[7];
 #pragma unroll
-    for (int q = 0; q < 6; q++) {
+    for (int q = 0; q < 7; q++) {
       v[q] = tree->parts[threadIdx.x][q];
       tree->parts[threadIdx.x][q] = 0;
     }
 #pragma unroll
-    for (int q = 0; q < 6; q++)
+    for (int q = 0; q < 7; q++)
       for (int off = 32; off > 0; off >>= 1) v[q] += (unsigned long long)__shfl_xor((long long)v[q], off);
     if (__lane_id() == 0)
 #pragma unroll
-      for (int q = 0; q < 6; q++) st[threadIdx.x >> 6][q] = v[q];
+      for (int q = 0; q < 7; q++) st[threadIdx.x >> 6][q] = v[q];
     __syncthreads();
     if (threadIdx.x == 0) {
-      for (int q = 0; q < 6; q++) v[q] = st[0][q] + st[1][q] + st[2][q] + st[3][q];
+      for (int q = 0; q < 7; q++) v[q] = st[0][q] + st[1][q] + st[2][q] + st[3][q];
       P.cnt->n_perms = v[0];
       P.cnt->enc_bytes = v[1];
       P.cnt->leaf_perms = v[2];
       P.cnt->leaf_bytes = v[3];
       P.cnt->hc_nodes = (uint32_t)v[4];
       P.cnt->hc_leaves = (uint32_t)v[5];
+      P.cnt->hc_exts = (uint32_t)v[6];
       P.cnt->hc_listed = (uint32_t)(tree->lists >> (2 * kTreeListBits));
-      tree->lists = 0;
+      tree->lists = tree->tall = 0;
+      for (uint32_t q = 0; q < kTreeRowPasses; q++) tree->rows[q] = 0;
     }
   }
   if (t >= ntries) return;
@@ -2323,17 +2490,31 @@ hipError_t publish_counters(const Counters *cnt, Publish pub, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t hc_tree(const Pools &P, const ref_t *list, uint32_t n, ref_t *ready, ref_t *leaves, TreeState *tree,
-                   hipStream_t s) {
+hipError_t hc_tree(const Pools &P, const ref_t *list, uint32_t n, ref_t *ready, ref_t *ready1, ref_t *leaves,
+                   TreeState *tree, int passes, hipStream_t s) {
   if (n == 0 || n > kTreeMax) return hipErrorInvalidValue;
   const bool lanes = n > kTreeSpreadLeaves;
-  k_tree_link<<<(n + 63) / 64, 64, 0, s>>>(P, list, n, ready, leaves, tree, lanes ? 1 : 0);
+  if (passes)
+    k_tree_link<4><<<nblk(n), kB, 0, s>>>(P, list, n, ready, leaves, tree, lanes ? 1 : 0);
+  else
+    k_tree_link<1><<<(n + 63) / 64, 64, 0, s>>>(P, list, n, ready, leaves, tree, lanes ? 1 : 0);
   GMPT_LAUNCH_CHECK();
   if (lanes) {
-    k_tree_leaves<<<nblk(n), kB, 0, s>>>(P, leaves, ready, tree);
+    k_tree_leaves<<<nblk(n + 63), kB, 0, s>>>(P, leaves, n, ready, tree);
     GMPT_LAUNCH_CHECK();
   }
-  k_tree_climb<<<(n + 3) / 4, kB, 0, s>>>(P, ready, tree);
+  // (one more block than the CUs hold at a time gains nothing: blocks loop)
+  const unsigned grid = std::min<uint32_t>((n + 63) / 64, 4096);
+  for (int k = 0; k < passes; k++) {
+    const ref_t *in = k & 1 ? ready1 : ready;
+    ref_t *out = k & 1 ? ready : ready1;
+    if (k == 0)
+      k_tree_rows<2><<<grid, 64, 0, s>>>(P, in, out, tree, k);
+    else
+      k_tree_rows<4><<<grid, 64, 0, s>>>(P, in, out, tree, k);
+    GMPT_LAUNCH_CHECK();
+  }
+  k_tree_climb<<<std::min<uint32_t>((n + 3) / 4, passes ? 2048 : ~0u), kB, 0, s>>>(P, ready, ready1, tree, passes);
   return hipGetLastError();
 }
 

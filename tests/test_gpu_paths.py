@@ -329,3 +329,37 @@ def test_split_extension_around_keys_below_it(gmpt, workloads, oracle, inside, t
     assert t.stats()["regroups"] == 1
     assert t.get_root_hash(tries - 1) == want
     assert t.get_values(more)[:50] == [more.value(i) for i in range(50)]
+
+
+@pytest.mark.parametrize("kind,n,launches", [("uniform", 100_000, 3), ("uniform", 150_000, 3), ("uniform", 154_000, 0),
+                                             ("short", 150_000, 3), ("long", 60_000, 3), ("digits", 200_000, 3)])
+def test_dirty_lists_hashed_by_rows_then_climb(gmpt, workloads, oracle, kind, n, launches):
+    # lists whose many lower inner nodes are hashed a lane each before the
+    # climb: leaves of one and of more blocks, embedded children, values in
+    # branches, extension chains (decimal keys) and long extensions; around the
+    # line to levels (57,344 inner nodes); the same root and work counts as by
+    # levels, then a batch over the clean trie
+    rng = np.random.default_rng(n)
+    if kind == "digits":
+        keys = [b"user%019d" % i for i in rng.permutation(2 * n)[:n]]
+    else:
+        keys = list(dict.fromkeys(_mixed_keys(rng, n, kind)))
+    lens = rng.choice([0, 1, 5, 32, 56, 90, 95, 110, 135, 136, 137], len(keys))
+    lens[:: n // 5] = 16_383
+    vals = [bytes(rng.integers(0, 256, int(k), dtype=np.uint8)) for k in lens]
+    b = workloads.batch_from_bytes(keys, vals)
+    some = rng.permutation(len(keys))[: n // 3]
+    more = workloads.batch_from_bytes([keys[i] for i in some] + [b"\x31" + keys[i][:20] for i in some],
+                                      [b"u%d" % i for i in range(2 * len(some))])
+    t, by_level = gmpt.MPT(device=0), gmpt.MPT(device=0)
+    by_level.set_option("hc_fuse_leaves", 0)
+    o = oracle.OracleMPT()
+    for part in (b, more):
+        o.puts(part)
+        o.hash()
+        assert _put(t, part) == o.root()
+        assert _put(by_level, part) == o.root()
+        if part is b:
+            st = t.stats()
+            assert launches in (0, st["hash_launches"]) and (launches or st["hash_launches"] > 3)
+            assert [st[k] for k in COUNTS] == [by_level.stats()[k] for k in COUNTS]
