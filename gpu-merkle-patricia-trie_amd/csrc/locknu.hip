@@ -331,7 +331,13 @@ __device__ __forceinline__ int attempt(const NuArgs &a, const Ctx &c, DirtyStage
         continue;
       }
       if (pos + p >= c.len) return ATT_RESTART;
-      if (!c.fresh) return misclassified(a, c);
+      if (!c.fresh) {
+        // S may have been read halfway through another lane's split (its
+        // terminator flag already cleared, its key length not yet cut)
+        const uint64_t sv = ld(&S->lock);
+        load_order();
+        return sv != v ? ATT_RESTART : misclassified(a, c);
+      }
       // split S at p: a new branch at depth pos + p (the latch upgrades
       // validate everything read above)
       const uint32_t d = pos + p;
