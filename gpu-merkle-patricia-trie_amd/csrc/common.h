@@ -168,6 +168,33 @@ __device__ __forceinline__ uint32_t match_nibbles(const uint8_t *pa, uint32_t sa
   return m;
 }
 
+// The same with the first 64 nibbles' words in flight at once (their places
+// clamped to the keys' own words): a leaf's remainder of ~60 nibbles takes one
+// memory round trip.
+__device__ __forceinline__ uint32_t match_nibbles_wide(const uint8_t *pa, uint32_t sa, uint32_t la, const uint8_t *pb,
+                                                       uint32_t sb, uint32_t lb, uint32_t m) {
+  if (m == 0) return 0;
+  const uint64_t *wa = (const uint64_t *)pa, *wb = (const uint64_t *)pb;
+  const uint32_t ia = sa >> 4, ea = (la - 1) >> 4, ib = sb >> 4, eb = (lb - 1) >> 4;
+  uint64_t a[5], b[5];
+#pragma unroll
+  for (uint32_t q = 0; q < 5; q++) {
+    a[q] = wa[min(ia + q, ea)];
+    b[q] = wb[min(ib + q, eb)];
+  }
+  const uint32_t ha = 4 * (sa & 15), hb = 4 * (sb & 15);
+  uint32_t p = 64;  // the first nibble that differs (those past m do not count)
+#pragma unroll
+  for (int q = 3; q >= 0; q--) {
+    uint64_t x = __builtin_bswap64(a[q]) << ha, y = __builtin_bswap64(b[q]) << hb;
+    if (ha) x |= __builtin_bswap64(a[q + 1]) >> (64 - ha);
+    if (hb) y |= __builtin_bswap64(b[q + 1]) >> (64 - hb);
+    if (x != y) p = 16 * q + ((uint32_t)__clzll((long long)(x ^ y)) >> 2);
+  }
+  if (p < 64 || m <= 64) return min(p, m);
+  return 64 + match_nibbles(pa, sa + 64, la, pb, sb + 64, lb, m - 64);
+}
+
 __device__ __forceinline__ uint32_t *node_dirty_flag(const Pools &P, ref_t r) {
   uint32_t t = ref_type(r), i = ref_idx(r);
   return t == T_BRANCH ? &P.branch[i].dirty : &P.shrt[i].dirty;

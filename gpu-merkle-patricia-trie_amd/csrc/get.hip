@@ -44,28 +44,54 @@ __device__ __forceinline__ uint64_t hex_bytes(const uint8_t *p, uint32_t c) {
   return c >= 8 ? v : v & ((1ull << (8 * c)) - 1);
 }
 
+// 16 hex bytes (h0 first) against the first c nibbles of w: 0 if they agree.
+__device__ __forceinline__ uint64_t nibbles_differ(uint64_t w, uint64_t h0, uint64_t h1, uint32_t c) {
+  if ((h0 | h1) & 0xF0F0F0F0F0F0F0F0ull) return 1;  // a hex byte above 15 matches nothing
+  // bytes 0x0a 0x0b -> one byte 0xab, big-endian nibble order
+  uint64_t b0 = __builtin_bswap64(h0), b1 = __builtin_bswap64(h1);
+  b0 = (b0 | (b0 >> 4)) & 0x00FF00FF00FF00FFull;
+  b1 = (b1 | (b1 >> 4)) & 0x00FF00FF00FF00FFull;
+  b0 = (b0 | (b0 >> 8)) & 0x0000FFFF0000FFFFull;
+  b1 = (b1 | (b1 >> 8)) & 0x0000FFFF0000FFFFull;
+  b0 = (b0 | (b0 >> 16)) & 0xFFFFFFFFull;
+  b1 = (b1 | (b1 >> 16)) & 0xFFFFFFFFull;
+  const uint64_t x = w ^ (b0 << 32 | b1);
+  return c < 16 ? x & ~0ull << (64u - 4u * c) : x;
+}
+
 // Nibbles [s, s + m) of the packed key at kp (8-byte aligned) against the m
-// hex bytes at h, eight per step (byte by byte, a leaf remainder of ~60
-// nibbles made 60 dependent loads: 95 us for 20,000 reads of a 200,000-key
-// trie, 24 now).  A hex byte above 15 matches nothing.
+// hex bytes at h.  The first 64 nibbles' words are all in flight at once, so a
+// leaf remainder of ~60 takes one memory round trip (byte by byte it took 60:
+// 95 us for 20,000 reads of a 200,000-key trie; a word after the other 24).
 __device__ __forceinline__ bool nibbles_equal(const uint8_t *kp, uint32_t s, uint32_t m, const uint8_t *h) {
-  for (uint32_t q = 0; q < m; q += 16) {
-    // a packed word and its 16 hex bytes
-    const uint64_t w = nib_word(kp, s + q, s + m);
+  if (m == 0) return true;
+  // words past the keys' last nibbles are read as the last one instead
+  const uint64_t *wk = (const uint64_t *)kp, *wh = (const uint64_t *)((uintptr_t)h & ~(uintptr_t)7);
+  const uint32_t ik = s >> 4, ek = (s + m - 1) >> 4, hh = (uint32_t)((uintptr_t)h & 7), eh = (hh + m - 1) >> 3;
+  uint64_t a[5], b[9];
+#pragma unroll
+  for (uint32_t q = 0; q < 5; q++) a[q] = wk[min(ik + q, ek)];
+#pragma unroll
+  for (uint32_t q = 0; q < 9; q++) b[q] = wh[min(q, eh)];
+  const auto hex8 = [&](uint32_t q, uint32_t left) {  // hex bytes 8q .. 8q + 7, the first `left` of them
+    uint64_t v = b[q] >> (8 * hh);
+    if (hh) v |= b[q + 1] << (64 - 8 * hh);
+    return left >= 8 ? v : left ? v & ((1ull << (8 * left)) - 1) : 0ull;
+  };
+  const uint32_t sh = 4 * (s & 15);
+  uint64_t x = 0;
+#pragma unroll
+  for (uint32_t q = 0; q < 4; q++) {
+    uint64_t w = __builtin_bswap64(a[q]) << sh;
+    if (sh) w |= __builtin_bswap64(a[q + 1]) >> (64 - sh);
+    const uint32_t c = m > 16 * q ? m - 16 * q : 0u;
+    if (c) x |= nibbles_differ(w, hex8(2 * q, c), hex8(2 * q + 1, c > 8 ? c - 8 : 0u), c);
+  }
+  if (x) return false;
+  for (uint32_t q = 64; q < m; q += 16) {
     const uint32_t c = min(16u, m - q);
-    const uint64_t h0 = hex_bytes(h + q, min(8u, c)), h1 = c > 8 ? hex_bytes(h + q + 8, c - 8) : 0ull;
-    if ((h0 | h1) & 0xF0F0F0F0F0F0F0F0ull) return false;
-    // bytes 0x0a 0x0b -> one byte 0xab, big-endian nibble order
-    uint64_t b0 = __builtin_bswap64(h0), b1 = __builtin_bswap64(h1);
-    b0 = (b0 | (b0 >> 4)) & 0x00FF00FF00FF00FFull;
-    b1 = (b1 | (b1 >> 4)) & 0x00FF00FF00FF00FFull;
-    b0 = (b0 | (b0 >> 8)) & 0x0000FFFF0000FFFFull;
-    b1 = (b1 | (b1 >> 8)) & 0x0000FFFF0000FFFFull;
-    b0 = (b0 | (b0 >> 16)) & 0xFFFFFFFFull;
-    b1 = (b1 | (b1 >> 16)) & 0xFFFFFFFFull;
-    uint64_t x = w ^ (b0 << 32 | b1);
-    if (c < 16) x &= ~0ull << (64u - 4u * c);
-    if (x) return false;
+    if (nibbles_differ(nib_word(kp, s + q, s + m), hex_bytes(h + q, min(8u, c)), c > 8 ? hex_bytes(h + q + 8, c - 8) : 0ull, c))
+      return false;
   }
   return true;
 }
@@ -75,6 +101,10 @@ __device__ __forceinline__ bool nibbles_equal(const uint8_t *kp, uint32_t s, uin
 template <typename F>
 __device__ ref_t walk(const Pools &P, ref_t node, HexKey k, F visit) {
   uint32_t pos = 0;
+  // the key's hex bytes from a multiple of 16 on, loaded 16 at a time: a branch
+  // costs one round trip (its child), not two
+  uint64_t b0 = 0, b1 = 0;
+  uint32_t at = ~0u;
   for (int guard = 0; guard < 2 * kMaxKeyNibbles + 4; guard++) {
     uint32_t t = ref_type(node);
     if (node == REF_NULL) return REF_NULL;
@@ -82,7 +112,13 @@ __device__ ref_t walk(const Pools &P, ref_t node, HexKey k, F visit) {
     visit(node);
     if (t == T_BRANCH) {
       if (pos >= k.len) return REF_NULL;
-      uint32_t nib = k.k[pos];
+      if (pos / 16 != at) {
+        at = pos / 16;
+        const uint32_t left = k.len - 16 * at;
+        b0 = hex_bytes(k.k + 16 * at, min(8u, left));
+        b1 = left > 8 ? hex_bytes(k.k + 16 * at + 8, min(8u, left - 8)) : 0ull;
+      }
+      const uint32_t nib = (uint32_t)((pos & 8 ? b1 : b0) >> (8 * (pos & 7))) & 255u;
       if (nib > 16) return REF_NULL;
       node = P.branch[ref_idx(node)].child[nib];
       pos++;
@@ -99,6 +135,10 @@ __device__ ref_t walk(const Pools &P, ref_t node, HexKey k, F visit) {
   }
   return REF_NULL;
 }
+
+// Threads per block of a walk: some ten thousand keys go a wave per block, so
+// that more CUs share their loads.
+inline unsigned walk_threads(uint32_t n) { return n <= 65536 ? 64 : kB; }
 
 __global__ __launch_bounds__(256) void k_gets(GetArgs g) {
   uint32_t i = grid_tid();
@@ -175,7 +215,8 @@ __global__ __launch_bounds__(256) void k_mark_emit(uint64_t *map, uint32_t words
 
 hipError_t launch_gets(const GetArgs &g, hipStream_t s) {
   if (g.n == 0) return hipSuccess;
-  k_gets<<<nblk(g.n), kB, 0, s>>>(g);
+  const unsigned th = walk_threads(g.n);
+  k_gets<<<(g.n + th - 1) / th, th, 0, s>>>(g);
   return hipGetLastError();
 }
 
@@ -189,7 +230,8 @@ hipError_t launch_gather_values(const uint64_t *addr, const int32_t *size, const
 hipError_t path_mark(const GetArgs &g, uint64_t *map, uint32_t words, uint32_t branch_words, uint32_t *bcnt,
                      uint32_t *total, void *temp, hipStream_t s) {
   if (g.n == 0 || words == 0) return hipErrorInvalidValue;
-  k_path_mark<<<nblk(g.n), kB, 0, s>>>(g, (unsigned long long *)map, branch_words, words);
+  const unsigned th = walk_threads(g.n);
+  k_path_mark<<<(g.n + th - 1) / th, th, 0, s>>>(g, (unsigned long long *)map, branch_words, words);
   GMPT_LAUNCH_CHECK();
   k_mark_count<<<nblk(words), kB, 0, s>>>(map, words, bcnt);
   GMPT_LAUNCH_CHECK();

@@ -714,7 +714,8 @@ __device__ __forceinline__ void descend_key(const NuArgs &a, uint32_t i, DirtySt
   const uint32_t idx = a.u_idx[i];
   const uint32_t t = a.u_trie[i];
   const uint32_t mark_from = a.u_first[i] ? 0u : (uint32_t)a.u_lcp[i] + 1u;
-  const KeyRef k = key_of(a, idx);
+  const uint64_t kr = a.u_kref[i];
+  const KeyRef k{a.P.keys + a.kbase + (kr & kKrefOff), (uint32_t)(kr >> 48)};
   ref_t node = REF_NULL, parent = REF_NULL;
   uint32_t pos = 0, pslot = 0;
   bool done = false;
@@ -778,7 +779,7 @@ __device__ __forceinline__ void descend_key(const NuArgs &a, uint32_t i, DirtySt
       const ref_t child = S.child;
       const uint32_t sreal = ml - term, kleft = real - min(pos, real);
       const uint32_t mreal = min(sreal, kleft);
-      uint32_t p = match_nibbles(P.keys + S.key_off, ks, ks + sreal, k.p, pos, real, mreal);
+      uint32_t p = match_nibbles_wide(P.keys + S.key_off, ks, ks + sreal, k.p, pos, real, mreal);
       if (p == mreal && p == sreal && term && p == kleft) p++;  // both at the terminator
       if (p == ml) {
         if (flag == 0 && pos >= mark_from) {
@@ -826,6 +827,7 @@ __device__ __forceinline__ void descend_key(const NuArgs &a, uint32_t i, DirtySt
   a.stop[i] = st;
 }
 
+constexpr uint32_t kDescendSmall = 32768;
 __global__ __launch_bounds__(256) void k_descend(NuArgs a) {
   // the sort needs a fallback pass: the order (and with it which key marks a
   // node) is not final, and the host runs the descent again
@@ -2033,7 +2035,9 @@ hipError_t nu_descend_and_group(const NuArgs &a, void *temp, hipStream_t s, bool
     k_empty_groups<<<nblk(a.n), kB, 0, s>>>(a, multi);
     return hipGetLastError();
   }
-  k_descend<<<nblk(a.n), kB, 0, s>>>(a);
+  // a few thousand keys: a wave per block, so that more CUs share their loads
+  const unsigned th = a.n <= kDescendSmall ? 64 : kB;
+  k_descend<<<(a.n + th - 1) / th, th, 0, s>>>(a);
   GMPT_LAUNCH_CHECK();
   return nu_groups(a, temp, s, true);
 }
