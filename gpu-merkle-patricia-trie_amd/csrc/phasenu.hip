@@ -1237,6 +1237,7 @@ struct ST {
   uint32_t stride;  // bytes of level 0 (mt_level_len geometry)
   int levels;
   uint32_t nsp;
+  bool small;  // values below 128 only (and 255: none); the same on every lane
   __device__ __forceinline__ uint32_t off(int k) const {  // byte offset of level k
     uint32_t o = 0, len = stride;
     for (int q = 0; q < k; q++) {
@@ -1250,13 +1251,26 @@ struct ST {
   }
   __device__ __forceinline__ uint8_t at(int k, uint32_t q) const { return t[off(k) + q]; }
   // 16-bit mask of the valid entries of the block of level k at base
-  // (a multiple of 16) whose value is below lim (lim <= 256)
+  // (a multiple of 16) whose value is below lim (lim <= 256; 127 when small).
+  // Small values are compared four at a time: bit 7 of (value | 128) - lim is
+  // clear where value < lim, and a byte dot product with powers of two gathers
+  // the bits (19 operations for the 16 entries instead of 64).
   __device__ __forceinline__ uint32_t below(int k, uint32_t base, uint32_t lim) const {
     const uint4 v = *(const uint4 *)(t + off(k) + base);
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
     uint32_t m = 0;
+    if (small) {
+      const uint32_t l4 = lim * 0x01010101u;
+      uint32_t b[4];
 #pragma unroll
-    for (uint32_t i = 0; i < 16; i++) m |= (uint32_t)(((w[i >> 2] >> (8 * (i & 3))) & 255u) < lim) << i;
+      for (uint32_t i = 0; i < 4; i++) b[i] = ~((w[i] | 0x80808080u) - l4) & 0x80808080u;
+      const uint32_t lo = __builtin_amdgcn_udot4(b[1], 0x80402010u, __builtin_amdgcn_udot4(b[0], 0x08040201u, 0, false), false);
+      const uint32_t hi = __builtin_amdgcn_udot4(b[3], 0x80402010u, __builtin_amdgcn_udot4(b[2], 0x08040201u, 0, false), false);
+      m = lo >> 7 | hi << 1;
+    } else {
+#pragma unroll
+      for (uint32_t i = 0; i < 16; i++) m |= (uint32_t)(((w[i >> 2] >> (8 * (i & 3))) & 255u) < lim) << i;
+    }
     const uint32_t valid = cnt(k) - base;  // > 0 for every block a query reads
     return valid >= 16 ? m : m & ((1u << valid) - 1);
   }
@@ -1317,6 +1331,7 @@ __device__ __forceinline__ ST st_of(const NuArgs &a) {
   s.nsp = ne > 0 ? ne - 1 : 0;
   s.levels = min(a.st_levels, kMtMaxLevels);
   s.stride = (uint32_t)a.st_stride;
+  s.small = a.scal[SC_MAXLEN] <= 126;  // LCP + 1 is at most a new key's length, and a limit one more
   return s;
 }
 
@@ -1388,6 +1403,7 @@ __device__ __forceinline__ ST st_window(const ST &g, uint32_t t0, uint8_t *w, ui
   ST s;  // the window's levels follow the tree's geometry with a level 0 of kSpWin bytes
   s.t = w;
   s.levels = 4;
+  s.small = g.small;
   s.nsp = n0;
   s.stride = kSpWin;
   return s;

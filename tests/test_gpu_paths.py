@@ -363,3 +363,29 @@ def test_dirty_lists_hashed_by_rows_then_climb(gmpt, workloads, oracle, kind, n,
             st = t.stats()
             assert launches in (0, st["hash_launches"]) and (launches or st["hash_launches"] > 3)
             assert [st[k] for k in COUNTS] == [by_level.stats()[k] for k in COUNTS]
+
+
+@pytest.mark.parametrize("nibbles", [123, 125, 126, 127, 128, 253])
+def test_split_points_near_the_byte_compare_limit(gmpt, workloads, oracle, nibbles):
+    # split points are compared four bytes at a time while keys (terminator
+    # included) have at most 126 nibbles: branches at every depth up to the last
+    # nibble, of an empty trie and then below its leaves, with fan-outs that
+    # reach past a block of 16 split points
+    rng = np.random.default_rng(nibbles)
+    base = [int(x) for x in rng.integers(0, 16, nibbles)]
+
+    def leaving(d, x):
+        return bytes(base[:d] + [x] + [int(y) for y in rng.integers(0, 16, nibbles - 1 - d)] + [16])
+
+    def batch(keys, tag):
+        keys = [keys[i] for i in rng.permutation(len(keys))]
+        return workloads.batch_from_hex(keys, [b"%s%d" % (tag, i) for i in range(len(keys))])
+
+    last = [bytes(base[:-1] + [x, 16]) for x in range(16)]
+    every = [leaving(d, (base[d] + 1 + d % 5) % 16) for d in range(nibbles - 1)]
+    wide = [leaving(d, x) for d in (0, nibbles // 2, nibbles - 2) for x in range(16) for _ in range(3)]
+    first = batch(list(dict.fromkeys(last[:9] + every[::2] + wide[::2])), b"a")
+    more = batch(list(dict.fromkeys(last + every + wide)), b"b")
+    t = gmpt.MPT(device=0)
+    assert _put(t, first) == _after(oracle, [first])
+    assert _put(t, more) == _after(oracle, [first, more])
