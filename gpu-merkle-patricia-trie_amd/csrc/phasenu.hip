@@ -990,8 +990,7 @@ __device__ __forceinline__ bool is_update(uint8_t kind) {
   return kind == STOP_LEAF_UPDATE || kind == STOP_VALUE_UPDATE;
 }
 
-__device__ __forceinline__ void init_value(const NuArgs &a, uint32_t vid, uint32_t idx, uint64_t *addr = nullptr,
-                                           uint32_t *size = nullptr) {
+__device__ __forceinline__ void init_value(const NuArgs &a, uint32_t vid, uint32_t idx) {
   Value &V = a.P.value[vid];
   int64_t vs = a.vidx[2 * idx], ve = a.vidx[2 * idx + 1];
   V.addr = a.vbase + (uint64_t)vs;
@@ -999,8 +998,6 @@ __device__ __forceinline__ void init_value(const NuArgs &a, uint32_t vid, uint32
   V.size = (uint32_t)(ve - vs + 1);
   V.pad = 0;
   V.seq = 0;
-  if (addr) *addr = V.addr;
-  if (size) *size = V.size;
 }
 
 // Existing key i's new value: its value node is rewritten in place (no node is
@@ -1172,6 +1169,27 @@ __device__ __forceinline__ bool build_waits(const NuArgs &a) {
 // for 2M split points).
 constexpr int kMtMaxLevels = 8;  // 16^8 split points
 
+// The minimum of the first n of 16 byte entries (255 for none): whole blocks as
+// pairs of 16-bit lanes, 20 operations for the 16 entries instead of 48.
+__device__ __forceinline__ uint32_t min16(const uint4 &v, uint32_t n) {
+  typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  uint32_t mn = 255;
+  if (n >= 16) {
+    us2 m[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      m[i] = __builtin_elementwise_min(__builtin_bit_cast(us2, w[i] & 0x00ff00ffu),
+                                       __builtin_bit_cast(us2, (w[i] >> 8) & 0x00ff00ffu));
+    const us2 x = __builtin_elementwise_min(__builtin_elementwise_min(m[0], m[1]), __builtin_elementwise_min(m[2], m[3]));
+    return min((uint32_t)x.x, (uint32_t)x.y);
+  }
+#pragma unroll
+  for (uint32_t i = 0; i < 16; i++)
+    if (i < n) mn = min(mn, (w[i >> 2] >> (8 * (i & 3))) & 255u);
+  return mn;
+}
+
 // Level k from level k - 1, one entry per thread (entries past the level's
 // valid count are never read by a query).
 __global__ __launch_bounds__(256) void k_mt_level(NuArgs a, int k) {
@@ -1186,13 +1204,7 @@ __global__ __launch_bounds__(256) void k_mt_level(NuArgs a, int k) {
   }
   if ((size_t)16 * b >= cnt) return;
   const uint8_t *lo = a.st + off + (size_t)16 * b;
-  const uint4 v = *(const uint4 *)lo;
-  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-  uint32_t mn = 255;
-#pragma unroll
-  for (uint32_t i = 0; i < 16; i++)
-    if (16 * b + i < cnt) mn = min(mn, (w[i >> 2] >> (8 * (i & 3))) & 255u);
-  a.st[off + mt_level_len(a.st_stride, k - 1) + b] = (uint8_t)mn;
+  a.st[off + mt_level_len(a.st_stride, k - 1) + b] = (uint8_t)min16(*(const uint4 *)lo, cnt - 16 * b);
 }
 
 // Levels k0 .. in one workgroup, each from the one below: four entries per
@@ -1214,13 +1226,7 @@ __global__ __launch_bounds__(1024) void k_mt_top(NuArgs a, int k0) {
     for (uint32_t b = threadIdx.x; b < nout; b += blockDim.x) {
       // the entry's 16 children in one load (levels are 16-byte multiples
       // at 16-byte aligned offsets); children past cnt do not count
-      const uint4 v = *(const uint4 *)(a.st + off + 16 * (size_t)b);
-      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-      uint32_t mn = 255;
-#pragma unroll
-      for (uint32_t i = 0; i < 16; i++)
-        if (16 * b + i < cnt) mn = min(mn, (w[i >> 2] >> (8 * (i & 3))) & 255u);
-      a.st[off + len + b] = (uint8_t)mn;
+      a.st[off + len + b] = (uint8_t)min16(*(const uint4 *)(a.st + off + 16 * (size_t)b), cnt - 16 * b);
     }
     __syncthreads();  // the level is complete for the next one
     off += len;
@@ -1377,27 +1383,16 @@ __device__ __forceinline__ ST st_window(const ST &g, uint32_t t0, uint8_t *w, ui
   for (uint32_t q = 0; q < kPer; q++) {
     const uint32_t c = threadIdx.x + kSpTile * q;
     if (c >= kSpL1) break;
-    uint32_t mn = 255;
-    const uint32_t wd[4] = {v[q].x, v[q].y, v[q].z, v[q].w};
-#pragma unroll
-    for (uint32_t i = 0; i < 16; i++)
-      if (16 * c + i < n0) mn = min(mn, (wd[i >> 2] >> (8 * (i & 3))) & 255u);
     ((uint4 *)w)[c] = v[q];
-    w1[c] = (uint8_t)mn;
+    w1[c] = (uint8_t)min16(v[q], 16 * c < n0 ? n0 - 16 * c : 0u);
   }
   __syncthreads();
   for (uint32_t c = threadIdx.x; c < kSpL2Pad; c += blockDim.x) {
-    uint32_t mn = 255;
-    if (c < kSpL2)
-      for (uint32_t i = 0; i < 16; i++) mn = min(mn, (uint32_t)w1[16 * c + i]);
-    w2[c] = (uint8_t)mn;
+    w2[c] = (uint8_t)(c < kSpL2 ? min16(((const uint4 *)w1)[c], 16) : 255u);
   }
   __syncthreads();
   if (threadIdx.x < 16) {
-    uint32_t mn = 255;
-    if (threadIdx.x < kSpL3)
-      for (uint32_t i = 0; i < 16; i++) mn = min(mn, (uint32_t)w2[16 * threadIdx.x + i]);
-    w3[threadIdx.x] = (uint8_t)mn;
+    w3[threadIdx.x] = (uint8_t)(threadIdx.x < kSpL3 ? min16(((const uint4 *)w2)[threadIdx.x], 16) : 255u);
   }
   __syncthreads();
   ST s;  // the window's levels follow the tree's geometry with a level 0 of kSpWin bytes
@@ -1604,8 +1599,19 @@ __device__ __forceinline__ bool link_branch(const NuArgs &a, uint32_t j, uint32_
 
 // Elements: new keys become a leaf short node + value node; a split short
 // node's remainder is re-attached below the new branch.
+// What an element's short node and value hold beyond zeros (write_elems).
+struct ElemNodes {
+  uint64_t addr, hp;   // Value
+  uint64_t key_off;    // Short
+  uint32_t size;
+  uint32_t child, key;  // key_start | key_len << 16
+  uint32_t meta;        // depth | term << 24
+  uint32_t has = 0;     // 1: a short node, 2: a value
+};
+
 template <class Sink>
-__device__ __forceinline__ void link_elem(const NuArgs &a, uint32_t e, const Slots &q, const Sink &sink) {
+__device__ __forceinline__ void link_elem(const NuArgs &a, uint32_t e, const Slots &q, const Sink &sink,
+                                          ElemNodes &o) {
   ST s = st_of(a);
   if (e == 0) {
     // the build's node and dirty-list slots are all assigned by position:
@@ -1645,7 +1651,14 @@ __device__ __forceinline__ void link_elem(const NuArgs &a, uint32_t e, const Slo
       a.leaf_pk[e] = kLeafPackedNone;
       return;
     }
-    init_value(a, vid, a.u_idx[ek.uidx], &va, &vsz);
+    const uint32_t idx = a.u_idx[ek.uidx];
+    const int64_t vs = a.vidx[2 * idx], ve = a.vidx[2 * idx + 1];
+    va = a.vbase + (uint64_t)vs;
+    vsz = (uint32_t)(ve - vs + 1);
+    o.addr = va;
+    o.hp = a.hps ? a.hps[idx] : 0ull;
+    o.size = vsz;
+    o.has = 2;
     child = make_ref(T_VALUE, vid);
   }
   ref_t me = child, sh = REF_NULL;
@@ -1656,7 +1669,11 @@ __device__ __forceinline__ void link_elem(const NuArgs &a, uint32_t e, const Slo
       raise_error(a.P.cnt, ERR_POOL, 2);
     } else {
       const uint32_t ks = ek.start + (start - ek.origin), kl = ek.end - start;
-      init_short(a.P.shrt[sid], ek.off, ks, kl, start, ek.term, child);
+      o.key_off = ek.off;
+      o.child = child;
+      o.key = ks | kl << 16;
+      o.meta = start | (uint32_t)ek.term << 24;
+      o.has |= 1;
       sh = make_ref(T_SHORT, sid);
       me = sh;
       if (!ek.virt) {  // a new leaf: record its hashing bin and metadata
@@ -1671,6 +1688,47 @@ __device__ __forceinline__ void link_elem(const NuArgs &a, uint32_t e, const Slo
     install(a, gi, me);
   else
     sink(a, parent, slot, me);
+}
+
+// The block's element nodes, staged in LDS (lds, 10 KB) and written 16 bytes per
+// lane in sequence: an element's 64 + 32 bytes straight from its own lane made
+// every store instruction touch 64 lines.  Every thread of the block calls it
+// (it synchronises the block).
+constexpr uint32_t kElemLds = kSpTile * 10;  // words
+__device__ __forceinline__ void write_elems(const NuArgs &a, const ElemNodes &o, uint32_t *lds) {
+  static_assert(offsetof(Short, key_off) == 32 && offsetof(Short, child) == 40 && offsetof(Short, key_start) == 44 &&
+                    offsetof(Short, key_len) == 46 && offsetof(Short, depth) == 48 && offsetof(Short, term) == 51 &&
+                    offsetof(Short, dirty) == 52 && offsetof(Short, lock) == 56 && sizeof(Short) == 64,
+                "short nodes are written as four 16-byte words");
+  static_assert(offsetof(Value, addr) == 0 && offsetof(Value, hp) == 8 && offsetof(Value, size) == 16 &&
+                    offsetof(Value, seq) == 24 && sizeof(Value) == 32,
+                "values are written as two 16-byte words");
+  const uint32_t t = threadIdx.x, e0 = blockIdx.x * kSpTile;
+  uint4 *const kw = (uint4 *)lds, *const vw = kw + kSpTile;
+  uint32_t *const meta = (uint32_t *)(vw + kSpTile), *const size = meta + kSpTile;
+  kw[t] = make_uint4((uint32_t)o.key_off, (uint32_t)(o.key_off >> 32), o.child, o.key);
+  vw[t] = make_uint4((uint32_t)o.addr, (uint32_t)(o.addr >> 32), (uint32_t)o.hp, (uint32_t)(o.hp >> 32));
+  meta[t] = o.has & 1 ? o.meta : ~0u;  // no depth is 65,535
+  size[t] = o.has & 2 ? o.size : ~0u;  // a value is below 2 GiB
+  __syncthreads();
+#pragma unroll
+  for (uint32_t q = 0; q < 4; q++) {
+    const uint32_t k = t + kSpTile * q, e = k / 4, w = k % 4, m = meta[e];
+    if (m == ~0u) continue;
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if (w == 2) v = kw[e];
+    if (w == 3) {
+      v.x = m;
+      v.y = 1;  // dirty
+    }
+    ((uint4 *)&a.P.shrt[a.base_short + e0 + e])[w] = v;
+  }
+#pragma unroll
+  for (uint32_t q = 0; q < 2; q++) {
+    const uint32_t k = t + kSpTile * q, e = k / 2, n = size[e];
+    if (n == ~0u) continue;
+    ((uint4 *)&a.P.value[a.base_value + e0 + e])[k % 2] = k % 2 ? make_uint4(n, 0, 0, 0) : vw[e];
+  }
 }
 
 // The build's branches and links in one launch.  Block b ranks the
@@ -1717,7 +1775,8 @@ __global__ __launch_bounds__(256) void k_build_links(NuArgs a, int pre) {
                 "owned branches are written as eight 16-byte words");
   __shared__ uint32_t sh[4];
   __shared__ uint64_t sh2[4];
-  __shared__ ref_t kid[kSpTile][17];
+  __shared__ __align__(16) ref_t kid[kSpTile][17];
+  static_assert(sizeof(kid) >= 4 * kElemLds, "the elements are staged in the child arrays' place");
   __shared__ uint32_t krec[kSpTile];   // the owned branches' records (bdesc): depth, children, slot-16 flag
   __shared__ uint16_t own[kSpTile];    // per split point of the block: its branch's local index
   __shared__ uint32_t xn;
@@ -1762,7 +1821,8 @@ __global__ __launch_bounds__(256) void k_build_links(NuArgs a, int pre) {
   __syncthreads();  // child arrays cleared, local indices set
   const OwnedLinks sink{kid, krec, own, &xn, blockIdx.x * kSpTile};
   const bool ext = link_branch(a, j, rank, q, sink);
-  link_elem(a, j, q, sink);
+  ElemNodes elem;
+  link_elem(a, j, q, sink, elem);
   const uint32_t exts = (uint32_t)__syncthreads_count(ext);  // every owned link in LDS
   if (exts && gridDim.x <= kCountExtBlocks && threadIdx.x == 0) atomicAdd(&a.scal[SC_NEXT], exts);
   // the owned branches, 16 bytes per thread: hash (zero), hash_size 0 |
@@ -1787,6 +1847,8 @@ __global__ __launch_bounds__(256) void k_build_links(NuArgs a, int pre) {
   }
   for (uint32_t k = threadIdx.x; k < btot; k += kSpTile) a.bdesc[base + k] = krec[k];
   if (threadIdx.x == 0) a.xcnt[blockIdx.x] = xn;
+  __syncthreads();  // the child arrays are written
+  write_elems(a, elem, &kid[0][0]);
 }
 
 // The cross links of k_build_links (block b's in its segment of the list):
