@@ -14,6 +14,8 @@ constexpr uint32_t kHcBins = kHcLevels * kHcClasses;
 // lay out.  Builds of 100,000 / 250,000 / 400,000 / 1,000,000 keys with the
 // line at 1,024: 399 / 459 / 506 / 788 us, 8,192: 374 / 438 / 487 / 780.
 constexpr uint32_t kHcSpreadMaxDefault = 8192;
+// Nodes of an inner level's lower classes that get a launch of their own.
+constexpr uint32_t kRowsSplitMin = 16384;
 // Extensions per inner level that get their own (leaf word builder) kernel.
 constexpr uint32_t kExtDirectMin = 16384;
 

@@ -2347,6 +2347,19 @@ hipError_t hc_hash_range(const Pools &P, const ref_t *list, const uint64_t *slot
                       : 16ull * ((uint64_t)c01 + cext) >= 15ull * n       ? (cls[1] ? 2 : 1)
                       : 16ull * ((uint64_t)c01 + c23 + cext) >= 15ull * n ? 4
                                                                             : 0;
+  // Rows of 4 blocks leave a SIMD one wave, which issues at little more than
+  // half its rate: where most of a level fits rows of 2, those nodes get a
+  // launch of their own first (the nodes are sorted by class).  1,194,800 nodes,
+  // 88 in 100 of them such: 451 -> 376 us; 432,200 nodes, 68 in 100: 246 -> 241.
+  if (rows_nb == 4 && c01 >= kRowsSplitMin && 2ull * c01 >= n) {
+    const uint32_t low[kHcClasses] = {cls[0], cls[1]};
+    hipError_t e = hc_hash_range(P, list, slot, c01, scratch, enc_len, false, spread_max, s, perm_begin, nullptr, 0, low);
+    if (e != hipSuccess) return e;
+    uint32_t rest[kHcClasses] = {};
+    std::copy(cls + 2, cls + kHcClasses, rest + 2);
+    return hc_hash_range(P, list + c01, slot + c01, n - c01, scratch, enc_len + c01, false, spread_max, s, nullptr,
+                         perm_end, n_ext, rest);
+  }
   if (rows_nb) {
     // the few nodes taller than the rows (classes rows_nb .. 6, between the
     // row classes and the extensions) would take the generic encoder and hold
