@@ -157,8 +157,8 @@ class Forest {
   int fetch(const void *src, size_t total, const FetchSeg *seg, int ns);
   int ensure_ws(DevBuf &b, size_t bytes);
   int arena_exhausted();
-  // hash()'s two forms: a short dirty list as one climb (*done: every node
-  // was hashed), any list by levels.
+  // hash()'s two forms: a short dirty list as one climb after `passes` row
+  // launches (*done: every node was hashed), any list by levels.
   int hash_tree(uint32_t n, int passes, bool *done);
   int hash_by_level(uint32_t n);
   int hash_levels(const Pools &P, const uint32_t *hist, bool direct_leaves, bool captured, uint32_t *n_leaf_out);

@@ -129,9 +129,9 @@ constexpr uint32_t kTreeMax = 1u << 20;
 // which a wave per node is as fast, kHcSpreadMaxDefault).
 constexpr uint32_t kTreeRowsMin = 8192;
 // A climb gives an inner node a wave of its own, so it wins while their
-// latency, not their number, sets the time.  Insert + hash by levels / as a
-// climb, by inner nodes: 1,450 303 / 184 us, 6,900 364 / 251, 12,300 369 / 293,
-// 21,500 382 / 364, 26,500 681 / 672, 30,100 397 / 440, 35,600 742 / 779.
+// latency, not their number, sets the time.  Insert + hash of uniform keys by
+// levels / as a climb alone, by inner nodes: 11,000 356 / 250 us, 17,000
+// 364 / 276, 22,500 362 / 307, 30,000 365 / 355, 38,000 370 / 401.
 constexpr uint32_t kTreeMaxInner = 24576;
 // Up to here the many nodes just above the leaves go by lanes (row launches)
 // and the climb takes the rest; above, levels sorted by block count make better

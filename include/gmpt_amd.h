@@ -50,7 +50,8 @@ typedef struct gmpt_batch {
 
 typedef struct gmpt_stats {
   double last_hash_ms;            /* device time of the last hash pass, from its bins to its counters read */
-  uint32_t hash_launches;         /* hash kernel launches (levels) of the last hash */
+  uint32_t hash_launches;         /* hash kernel launches (levels) of the last hash; a climb over a short dirty list
+                                     is one, with two more where lanes hash its lower nodes first */
   uint32_t hashed_nodes;          /* nodes re-hashed by the last hash */
   uint32_t restarts;              /* LockNU optimistic restarts in the last insert */
   uint32_t lock_fails;            /* LockNU keys that restarted at least once */
@@ -65,7 +66,7 @@ typedef struct gmpt_stats {
   uint64_t leaf_perms;            /* its permutations */
   uint64_t leaf_bytes;            /* encoding bytes of the leaf level */
   uint32_t leaf_nodes;            /* leaf nodes hashed */
-  uint32_t ext_direct_nodes;      /* extension nodes hashed by the leaf word builder (last hash) */
+  uint32_t ext_direct_nodes;      /* extension nodes hashed by the leaf word builder or in a climb (last hash) */
 } gmpt_stats;
 
 /* Creates a forest of num_tries empty tries on device `device`.
