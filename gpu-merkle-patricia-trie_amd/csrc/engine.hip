@@ -830,7 +830,10 @@ int Forest::hash(void *targets, int n_targets) {
   const uint32_t n = cnt_.n_dirty;
   // The climb's waves use the spread layout, which hc_spread_max 0 turns off,
   // and its counts are atomics on the nodes, which host pools do not get.
-  const uint64_t others = dirty_keys_ + dirty_holes_, inner = n > others ? n - others : 0;
+  // Inner nodes: what the inserts' keys and holes leave of the list.  Batches
+  // that write the same keys before one pass count them each time, so a long
+  // list is taken to hold a sixth of them at least (uniform keys: a quarter).
+  const uint64_t others = dirty_keys_ + dirty_holes_, inner = std::max<uint64_t>(n > others ? n - others : 0, n / 6);
   dirty_keys_ = dirty_holes_ = 0;
   if (n > 0 && n <= kTreeMax && inner <= kTreeRowsMaxInner && !by_level_ && hc_fuse_leaves_ && hc_fuse_inner_ &&
       hc_spread_max_ > 0 && !branch_.host && !shrt_.host) {
