@@ -134,7 +134,9 @@ class Forest {
   // first call for a batch (its buffers and sizes) runs eagerly and captures
   // the pass; later calls replay it, and a replay whose batch turns out unlike
   // the captured one (sort fallback, other hash levels) is redone eagerly and
-  // captured again.  *replayed tells which ran.
+  // captured again.  A call in between that replaces a device buffer drops the
+  // capture, which holds the buffers' addresses; the next rebuild captures
+  // anew.  *replayed tells which ran.
   int rebuild_graph(const BatchDesc &b, bool *replayed);
   uint32_t ntries() const { return ntries_; }
   uint64_t pool_bytes_used() const;

@@ -231,6 +231,7 @@ int Forest::grow(DevBuf &b, size_t need, size_t keep, bool fill) {
     HIP_TRY(hipMemsetAsync((uint8_t *)p + keep, 0, cap - keep, stream_));
   }
   if (!arena_) HIP_TRY(hipStreamSynchronize(stream_));  // a region's memory is not given back: nothing to wait for
+  if (b.p) drop_graph();  // its kernels hold the old address
   release(b);
   b.p = p;
   b.cap = cap;
@@ -254,6 +255,7 @@ int Forest::ensure_ws(DevBuf &b, size_t bytes) {
   }
   if (b.p) {
     HIP_TRY(hipStreamSynchronize(stream_));
+    drop_graph();  // its kernels hold the old address
     release(b);
   }
   size_t cap = align_up(bytes + bytes / 4, 1 << 20);
