@@ -836,13 +836,18 @@ __device__ __forceinline__ void descend_key(const NuArgs &a, uint32_t i, DirtySt
 
 constexpr uint32_t kDescendSmall = 32768;
 __global__ __launch_bounds__(256) void k_descend(NuArgs a) {
-  // the sort needs a fallback pass: the order (and with it which key marks a
-  // node) is not final, and the host runs the descent again
-  if (a.P.cnt->flag_fallback) return;
   __shared__ ref_t dbuf[kDirtyStage];
-  __shared__ uint32_t dcnt;
-  if (threadIdx.x == 0) dcnt = 0;
+  __shared__ uint32_t dcnt, skip;
+  if (threadIdx.x == 0) {
+    dcnt = 0;
+    // Which key marks a node rests on the keys' order.  It is not final while
+    // the sort needs a fallback pass (the host runs the descent again), and a
+    // refused key (its trie id may have another trie's low bits) can stand
+    // between two keys of a trie: both would list the nodes they share.
+    skip = a.P.cnt->flag_fallback | a.P.cnt->err;
+  }
   __syncthreads();
+  if (skip) return;
   DirtyStage ds{dbuf, &dcnt, kDirtyStage};
   const uint32_t i = grid_tid();
   if (i < a.scal[SC_M_UNIQ]) descend_key(a, i, ds);

@@ -13,6 +13,14 @@ def _put(t, b, mode="2phase"):
     return t.get_root_hash()
 
 
+def _after(oracle, batches):
+    o = oracle.OracleMPT()
+    for b in batches:
+        o.puts(b)
+        o.hash()
+    return o.root()
+
+
 def _random_batch(workloads, rng, n):
     flat, lens = workloads.random_values(rng, n, 1, 60)
     return workloads.batch_from_fixed(workloads.unique_random_keys(rng, n, 32), flat, lens)
@@ -45,3 +53,33 @@ def test_graph_is_captured_again_after_a_buffer_moved(gmpt, workloads, oracle, b
     assert (sizes == np.diff(small.values_indexs.reshape(-1, 2), axis=1).ravel() + 1).all()
     t.close()
     db.free()
+
+
+def test_refused_batch_leaves_the_dirty_list_as_it_was(gmpt, workloads, oracle):
+    # trie 1 holds a branch below slot 0 and a chain of branches below slot 5;
+    # the chain waits for its hash.  A batch with a trie id past the last one is
+    # refused: two of its keys end in the branch, either side of the key with
+    # the bad id in sorted order (id 9 has trie 1's low three bits).
+    rng = np.random.default_rng(9)
+
+    def key(*head):
+        return bytes(list(head) + [int(x) for x in rng.integers(1, 15, 64 - len(head))] + [16])
+
+    chain = [key(*[5] * d, 6) for d in range(1, 40)] + [key(*[5] * 41)]
+    base = workloads.batch_from_hex([key(0, 1), key(0, 2), key(9)] + chain, [b"%d" % i * 30 for i in range(43)])
+    deep = workloads.batch_from_hex([chain[-1]], [b"another value of the chain's last key"])
+    bad = workloads.batch_from_hex([key(*[0] * 18), key(3), key(0, 3)], [b"x" * 40, b"y" * 40, b"z" * 40])
+    f = gmpt.MPT(device=0, num_tries=5)
+    for b in (base, deep, bad):
+        b.trie_ids = np.full(b.n, 1, np.int32)
+    bad.trie_ids[1] = 9
+    _put(f, base)
+    f.puts_2phase_with_valuehp(deep)
+    with pytest.raises(gmpt.GmptError, match="trie id out of range"):
+        f.puts_2phase_with_valuehp(bad)
+    f.hash_onepass_v2(None, 0)
+    assert f.get_root_hash(1) == _after(oracle, [base, deep])
+    assert f.stats()["hashed_nodes"] == 41  # the last key's leaf and the branches at depths 0 .. 39 above it
+    bad.trie_ids[1] = 2
+    _put(f, bad)
+    assert f.get_root_hash(1) == _after(oracle, [base, deep, bad.subset([0, 2])])
