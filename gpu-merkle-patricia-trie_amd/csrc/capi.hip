@@ -257,6 +257,7 @@ int gmpt_get_stats(gmpt_forest *f, gmpt_stats *out) {
   do {                                                                 \
     hipError_t e__ = (expr);                                           \
     if (e__ != hipSuccess) {                                           \
+      (void)hipGetLastError();                                         \
       gmpt::set_error(std::string(#expr) + ": " + hipGetErrorString(e__)); \
       return -1;                                                       \
     }                                                                  \
@@ -331,6 +332,7 @@ int gmpt_keccak256_batch_mode(const uint8_t *data, const uint64_t *offsets, cons
       (e = gmpt::keccak_batch(d_data, d_off, d_len, n, d_out, d_slot, d_scratch, d_temp, mode, nullptr)) !=
           hipSuccess ||
       (e = hipMemcpy(out, d_out, 32ull * n, hipMemcpyDeviceToHost)) != hipSuccess) {
+    (void)hipGetLastError();
     gmpt::set_error(std::string("keccak batch: ") + hipGetErrorString(e));
     rc = -1;
   }

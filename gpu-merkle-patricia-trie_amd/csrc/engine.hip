@@ -60,10 +60,13 @@ size_t nu_ws_bytes(size_t n, bool tries) {
 void set_error(const std::string &e) { g_err = e; }
 const char *last_error() { return g_err.c_str(); }
 
+// A failed call's error is taken off the runtime's record here: left there, it
+// would be reported again by the next kernel launch's check, of another call.
 #define HIP_TRY(expr)                                                              \
   do {                                                                             \
     hipError_t e__ = (expr);                                                       \
     if (e__ != hipSuccess) {                                                       \
+      (void)hipGetLastError();                                                     \
       set_error(std::string(#expr) + ": " + hipGetErrorString(e__));              \
       return -1;                                                                   \
     }                                                                              \
@@ -216,6 +219,7 @@ int Forest::grow(DevBuf &b, size_t need, size_t keep, bool fill) {
     cap = align_up(std::max(need, b.cap + b.cap / 2), 4096);
     hipError_t e = host ? hipHostMalloc(&p, cap, hipHostMallocDefault) : hipMalloc(&p, cap);
     if (e != hipSuccess) {
+      (void)hipGetLastError();
       set_error(std::string(host ? "host pool allocation failed: " : "device pool allocation failed: ") +
                 hipGetErrorString(e));
       return -2;
@@ -261,6 +265,7 @@ int Forest::ensure_ws(DevBuf &b, size_t bytes) {
   size_t cap = align_up(bytes + bytes / 4, 1 << 20);
   hipError_t e = hipMalloc(&b.p, cap);
   if (e != hipSuccess) {
+    (void)hipGetLastError();
     set_error(std::string("workspace allocation failed: ") + hipGetErrorString(e));
     return -2;
   }
@@ -404,6 +409,7 @@ uint8_t *Forest::value_space(uint64_t bytes) {
     c.cap = align_up(std::max<uint64_t>(bytes, 64ull << 20), 1 << 20);
     c.host = pool_host_;
     if ((c.host ? hipHostMalloc(&c.p, c.cap, hipHostMallocDefault) : hipMalloc(&c.p, c.cap)) != hipSuccess) {
+      (void)hipGetLastError();
       set_error("value arena allocation failed");
       return nullptr;
     }

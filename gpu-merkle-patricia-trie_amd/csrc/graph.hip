@@ -22,6 +22,7 @@ namespace gmpt {
   do {                                                                             \
     hipError_t e__ = (expr);                                                       \
     if (e__ != hipSuccess) {                                                       \
+      (void)hipGetLastError();                                                     \
       set_error(std::string(#expr) + ": " + hipGetErrorString(e__));              \
       return -1;                                                                   \
     }                                                                              \
@@ -82,6 +83,7 @@ int Forest::capture_rebuild(const BatchDesc &b) {
   auto fail = [&](int code) {
     (void)hipStreamEndCapture(stream_, &g);
     if (g) (void)hipGraphDestroy(g);
+    (void)hipGetLastError();
     return code;
   };
   hipError_t e = hipSuccess;
@@ -143,6 +145,7 @@ int Forest::capture_rebuild(const BatchDesc &b) {
   GRAPH_TRY(hipStreamEndCapture(stream_, &g));
   hipGraphExec_t x = nullptr;
   if (hipGraphInstantiate(&x, g, nullptr, nullptr, 0) != hipSuccess) {
+    (void)hipGetLastError();
     (void)hipGraphDestroy(g);
     set_error("hipGraphInstantiate failed");
     return -1;

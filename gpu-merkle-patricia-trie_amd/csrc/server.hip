@@ -59,6 +59,7 @@ int Server::Pinned::reserve(size_t bytes) {
   cap = 0;
   size_t c = std::max<size_t>(bytes + bytes / 2, 1 << 16);
   if (hipHostMalloc(&p, c) != hipSuccess) {
+    (void)hipGetLastError();
     p = nullptr;
     set_error("pinned staging allocation failed");
     return -2;

@@ -83,3 +83,30 @@ def test_refused_batch_leaves_the_dirty_list_as_it_was(gmpt, workloads, oracle):
     bad.trie_ids[1] = 2
     _put(f, bad)
     assert f.get_root_hash(1) == _after(oracle, [base, deep, bad.subset([0, 2])])
+
+
+def _huge_values_in_branches(workloads, rng):
+    # stems that end at a branch with a value of 512 MiB (one buffer for all),
+    # above a branch of two leaves: the levels' messages exceed any device
+    stems = list({bytes(s) for s in rng.integers(0, 16, (640, 8), dtype=np.uint8)})
+    keys = [s + bytes([1, c, 7, 16]) for s in stems for c in (2, 3)] + [s + b"\x10" for s in stems]
+    b = workloads.batch_from_hex(keys, [b""] * len(keys))
+    big = 512 << 20
+    b.values_bytes = np.zeros(big, np.uint8)
+    b.values_indexs = np.array([(0, 39)] * (2 * len(stems)) + [(0, big - 1)] * len(stems), np.int64).ravel()
+    return b
+
+
+def test_failed_allocation_is_reported_once(gmpt, workloads, oracle):
+    rng = np.random.default_rng(511)
+    db = gmpt.DeviceBatch(_huge_values_in_branches(workloads, rng), adopt_values=True)
+    f = gmpt.MPT(device=0)
+    f.set_option("hc_fuse_inner", 0)  # by levels
+    targets, m = f.puts_2phase_with_valuehp(db)
+    with pytest.raises(gmpt.GmptError, match="workspace allocation failed"):
+        f.hash_onepass_v2(targets, m)
+    f.clear()
+    few = _random_batch(workloads, rng, 500)
+    assert _put(f, few) == oracle.root_of(few)
+    f.close()
+    db.free()
