@@ -147,7 +147,8 @@ hipError_t hc_tree(const Pools &P, const ref_t *list, uint32_t n, ref_t *ready, 
                    TreeState *tree, int passes, hipStream_t s);
 // Copies every trie's root hash into its header and empties the dirty list;
 // with parts (from hc_count), adds the pass's work counts to the counters;
-// with tree (from hc_tree), sets them from it.
+// with tree (from hc_tree), sets them from it, and keeps the dirty list, and
+// the headers of roots not hashed yet, if the climb left nodes out.
 // Then zeroes the insert's scalars for the next insert and, with pub, sends
 // the counters to the host as publish_counters does.
 struct Publish {

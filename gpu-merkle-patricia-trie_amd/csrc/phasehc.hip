@@ -2131,17 +2131,19 @@ __device__ __forceinline__ void roots_body(const Pools &P, uint32_t ntries, cons
   uint32_t t = grid_tid();
   // the root's hash first: its two dependent loads overlap the counts' reduction
   uint32_t hs = 0;
+  bool left = false;  // a climb left the root out (see hc_tree): its trie keeps the root hash it had
   uint4 h[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
   if (t < ntries) {
     const ref_t r = P.tries[t].root;
     if (ref_type(r) == T_SHORT || ref_type(r) == T_BRANCH) {
+      left = tree && *node_dirty_flag(P, r) != 0;
       hs = node_hash_size(P, r);
       const uint4 *src = (const uint4 *)node_hash(P, r);  // offset 0 of a 64- or 128-byte node
       h[0] = src[0];
       h[1] = src[1];
     }
   }
-  if (t == 0) P.cnt->n_dirty = 0;  // every listed node has been hashed
+  if (t == 0 && !tree) P.cnt->n_dirty = 0;  // every listed node has been hashed
   if (parts && blockIdx.x == 0) {  // the pass's work counts (uniform branch)
     static_assert(kHcCountParts == 256, "one partial per thread");
     __shared__ unsigned long long sh[4][4];
@@ -2189,11 +2191,12 @@ __device__ __forceinline__ void roots_body(const Pools &P, uint32_t ntries, cons
       P.cnt->hc_leaves = (uint32_t)v[5];
       P.cnt->hc_exts = (uint32_t)v[6];
       P.cnt->hc_listed = (uint32_t)(tree->lists >> (2 * kTreeListBits));
+      if (P.cnt->hc_nodes == P.cnt->hc_listed) P.cnt->n_dirty = 0;  // otherwise the list stands for the levels
       tree->lists = tree->tall = 0;
       for (uint32_t q = 0; q < kTreeRowPasses; q++) tree->rows[q] = 0;
     }
   }
-  if (t >= ntries) return;
+  if (t >= ntries || left) return;
   // bytes past the hash size (a root encoding under 32 bytes) read as zero
   uint32_t w[8] = {h[0].x, h[0].y, h[0].z, h[0].w, h[1].x, h[1].y, h[1].z, h[1].w};
 #pragma unroll

@@ -85,6 +85,33 @@ def test_refused_batch_leaves_the_dirty_list_as_it_was(gmpt, workloads, oracle):
     assert f.get_root_hash(1) == _after(oracle, [base, deep, bad.subset([0, 2])])
 
 
+@pytest.mark.parametrize("n,tries", [(3000, 1), (3000, 300), (80_000, 1)])
+def test_nodes_a_climb_leaves_out_are_hashed_by_levels(gmpt, workloads, oracle, n, tries):
+    # every key gets the value it has, and one branch is taken out of the dirty
+    # list: its parent then waits for it in vain, the climb (alone, and after
+    # row launches) ends without the branches above, and the levels take over
+    rng = np.random.default_rng(n + tries)
+    b = _random_batch(workloads, rng, n)
+    b.trie_ids = np.zeros(n, np.int32)
+    b.trie_ids[::3] = tries - 1
+    want = [oracle.root_of(b.subset(np.flatnonzero(b.trie_ids == t))) for t in sorted({0, tries - 1})]
+    f = gmpt.MPT(device=0, num_tries=tries)
+    _put(f, b)
+    assert f.stats()["hash_launches"] in (1, 3)
+    targets, m = f.puts_2phase_with_valuehp(b)
+    listed = np.zeros(m, np.uint32)
+    L = gmpt.gmpt.lib()
+    assert L.gmpt_memcpy_dtoh(listed.ctypes.data, targets, listed.nbytes) == 0
+    branches = np.flatnonzero(listed >> 30 == 1)
+    at = int(branches[np.argmax(listed[branches])])  # (the roots come first)
+    assert L.gmpt_memcpy_htod(targets + 4 * at, np.zeros(1, np.uint32).ctypes.data, 4) == 0
+    f.hash_onepass_v2(targets, m)
+    st = f.stats()
+    assert st["hash_launches"] > 3 and st["hashed_nodes"] == np.count_nonzero(listed) - 1
+    assert [f.get_root_hash(t) for t in sorted({0, tries - 1})] == want
+    assert f.puts_2phase_with_valuehp(b.subset([]))[1] == 0  # the dirty list is empty
+
+
 def _huge_values_in_branches(workloads, rng):
     # stems that end at a branch with a value of 512 MiB (one buffer for all),
     # above a branch of two leaves: the levels' messages exceed any device
@@ -108,5 +135,29 @@ def test_failed_allocation_is_reported_once(gmpt, workloads, oracle):
     f.clear()
     few = _random_batch(workloads, rng, 500)
     assert _put(f, few) == oracle.root_of(few)
+    f.close()
+    db.free()
+
+
+def test_a_hash_pass_that_fails_keeps_its_dirty_list(gmpt, workloads):
+    # the leaves are taken out of the dirty list: the climb reaches no branch,
+    # and the levels ask for more message memory than the device has
+    rng = np.random.default_rng(512)
+    b = _huge_values_in_branches(workloads, rng)
+    one = workloads.batch_from_hex([b.key(0)], [b"another value of one key, after which no new leaf is recorded"])
+    db = gmpt.DeviceBatch(b, adopt_values=True)
+    f = gmpt.MPT(device=0)
+    f.puts_2phase_with_valuehp(db)
+    targets, m = f.puts_2phase_with_valuehp(one)
+    listed = np.zeros(m, np.uint32)
+    L = gmpt.gmpt.lib()
+    assert L.gmpt_memcpy_dtoh(listed.ctypes.data, targets, listed.nbytes) == 0
+    listed[listed >> 30 != 1] = 0
+    assert L.gmpt_memcpy_htod(targets, listed.ctypes.data, listed.nbytes) == 0
+    for _ in range(2):
+        with pytest.raises(gmpt.GmptError, match="workspace allocation failed"):
+            f.hash_onepass_v2(targets, m)
+        assert f.puts_2phase_with_valuehp(one.subset([]))[1] == m  # nothing was hashed, all is still listed
+        assert f.get_root_hash() == b""
     f.close()
     db.free()
