@@ -258,6 +258,7 @@ class Forest {
     uint32_t n_dirty = 0, ne = 0;  // dirty nodes and elements of the captured pass
     uint64_t key_used = 0;         // key arena bytes after it
     uint32_t hist[kHcBins];        // its hash bins
+    uint32_t launches = 0, nodes = 0, leaves = 0, exts = 0;  // and its hash pass's statistics
   };
   GraphPlan plan_;
   DevBuf plan_hist_;                 // plan_.hist on the device, for the replay check

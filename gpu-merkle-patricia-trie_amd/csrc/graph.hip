@@ -153,6 +153,10 @@ int Forest::capture_rebuild(const BatchDesc &b) {
   graph_ = g;
   gexec_ = x;
   plan_.batch = b;
+  plan_.launches = stats_.hash_launches;
+  plan_.nodes = stats_.hashed_nodes;
+  plan_.leaves = stats_.leaf_nodes;
+  plan_.exts = stats_.ext_direct_nodes;
   plan_.valid = true;
   return 0;
 }
@@ -203,11 +207,17 @@ bool Forest::graph_ok() {
   all_empty_ = false;
   rec_ = LeafRecords();
   stats_.fallback_sorts = stats_.regroups = 0;
+  stats_.hash_launches = plan_.launches;
+  stats_.hashed_nodes = plan_.nodes;
+  stats_.leaf_nodes = plan_.leaves;
+  stats_.ext_direct_nodes = plan_.exts;
   stats_.perms = cnt_.n_perms;
   stats_.enc_bytes = cnt_.enc_bytes;
   stats_.leaf_perms = cnt_.leaf_perms;
   stats_.leaf_bytes = cnt_.leaf_bytes;
   stats_.last_hash_ms = stats_.leaf_perm_ms = 0;
+  hash_from_ = leaf_from_ = nullptr;  // the events of an earlier, eager pass
+  dirty_keys_ = dirty_holes_ = 0;     // inserts the replay's clear undid
   return true;
 }
 

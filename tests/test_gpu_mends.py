@@ -161,3 +161,25 @@ def test_a_hash_pass_that_fails_keeps_its_dirty_list(gmpt, workloads):
         assert f.get_root_hash() == b""
     f.close()
     db.free()
+
+
+def test_stats_of_a_replay_hold_no_other_pass(gmpt, workloads):
+    # a replay records no times; those of the eager pass before it were not read.
+    # Its node counts are the captured pass's
+    rng = np.random.default_rng(77)
+    db = gmpt.DeviceBatch(_random_batch(workloads, rng, 3000), adopt_values=True)
+    t = gmpt.MPT(device=0)
+    for replayed in (False, True):
+        assert t.rebuild_graph(db) is replayed
+        st = t.stats()
+        assert st["last_hash_ms"] == st["leaf_perm_ms"] == 0 and st["leaf_nodes"] == 3000
+    _put(t, _random_batch(workloads, rng, 5000))
+    assert t.rebuild_graph(db) is False  # the insert moved buffers
+    assert t.stats()["last_hash_ms"] == 0
+    _put(t, _random_batch(workloads, rng, 50))
+    assert t.rebuild_graph(db) is True
+    again = t.stats()
+    keys = ("last_hash_ms", "leaf_perm_ms", "hash_launches", "hashed_nodes", "leaf_nodes", "ext_direct_nodes", "perms")
+    assert [again[k] for k in keys] == [st[k] for k in keys]
+    t.close()
+    db.free()
