@@ -127,7 +127,8 @@ class Forest {
   int set_option(const std::string &name, int64_t value);
   int get_option(const std::string &name, int64_t *value) const;
   // Times PhaseHC on `sample` (inserted into a scratch forest on the same
-  // device) for each candidate spread threshold and keeps the fastest.
+  // device) by levels for each spread threshold that changes its launches, and
+  // keeps the fastest.
   int autotune(const BatchDesc &sample, int mode, int64_t *chosen, double *best_ms);
   // Bulk rebuild of a device batch (values adopted) into the emptied forest
   // -- clear, PhaseNU, PhaseHC -- as one replay of a captured HIP graph.  The

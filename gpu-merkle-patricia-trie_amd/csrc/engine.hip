@@ -1176,30 +1176,61 @@ int Forest::get_option(const std::string &name, int64_t *value) const {
   return -3;
 }
 
+// The sample's passes go by levels: the option says which level launches use the
+// spread layout, and nothing of a climb but whether there is one.  Candidates
+// that part the sample's launches alike are the same work, so one of them is
+// timed, the option's present value where it is among them: a sample that
+// cannot tell them apart leaves it as it is.
 int Forest::autotune(const BatchDesc &sample, int mode, int64_t *chosen, double *best_ms) {
-  static const uint32_t kCand[] = {0, 256, 1024, 4096, 16384, 65536};
+  const uint32_t cand[] = {hc_spread_max_, 0, 256, 1024, 4096, kHcSpreadMaxDefault, 16384, 65536};
   Forest t(device_, ntries_);
   if (!t.ok()) return -1;
+  t.hc_fuse_leaves_ = hc_fuse_leaves_;
+  t.hc_fuse_inner_ = hc_fuse_inner_;
+  t.by_level_ = true;
+  const auto pass = [&]() -> int {
+    int r;
+    void *tg = nullptr;
+    int nt = 0;
+    if ((r = t.clear())) return r;
+    if ((r = mode == 0 ? t.puts_2phase(sample, &tg, &nt) : t.puts_latching(sample, &tg, &nt))) return r;
+    return t.hash(tg, nt);
+  };
+  int r;
+  if ((r = pass())) return r;  // warms the pools, and brings the levels' sizes
+  std::vector<uint32_t> sizes;  // of the launches the option decides on
+  if (t.stats_.hashed_nodes) {
+    const uint32_t *hist = ((const HcMeta *)t.h_meta_)->hist;
+    for (uint32_t lv = hc_fuse_leaves_ ? 1 : 0; lv < kHcLevels; lv++) {
+      const uint32_t *c = hist + lv * kHcClasses;
+      uint32_t n = 0;
+      for (uint32_t q = 0; q < kHcClasses; q++) n += c[q];
+      sizes.push_back(n);
+      if (hc_fuse_inner_ && c[0] + c[1] >= kRowsSplitMin) {  // hc_hash_range may take them apart
+        sizes.push_back(c[0] + c[1]);
+        sizes.push_back(n - c[0] - c[1]);
+      }
+    }
+  }
+  const auto largest = [&](uint32_t max) {
+    uint32_t m = 0;
+    for (uint32_t n : sizes)
+      if (n <= max) m = std::max(m, n);
+    return m;
+  };
   double best = 1e30;
   uint32_t arg = hc_spread_max_;
-  for (uint32_t c : kCand) {
-    t.hc_spread_max_ = c;
-    t.hc_fuse_leaves_ = hc_fuse_leaves_;
-    t.hc_fuse_inner_ = hc_fuse_inner_;
+  for (const uint32_t *c = std::begin(cand); c != std::end(cand); c++) {
+    if (std::any_of(std::begin(cand), c, [&](uint32_t o) { return largest(o) == largest(*c); })) continue;
+    t.hc_spread_max_ = *c;
     double ms = 1e30;
-    for (int rep = 0; rep < 4; rep++) {  // the first run warms the pools; the best of the other three counts
-      int r;
-      void *tg = nullptr;
-      int nt = 0;
-      if ((r = t.clear())) return r;
-      r = mode == 0 ? t.puts_2phase(sample, &tg, &nt) : t.puts_latching(sample, &tg, &nt);
-      if (r) return r;
-      if ((r = t.hash(tg, nt))) return r;
+    for (int rep = 0; rep < 4; rep++) {  // the best of the last three counts
+      if ((r = pass())) return r;
       if (rep > 0) ms = std::min(ms, (double)t.stats().last_hash_ms);
     }
     if (ms < best) {
       best = ms;
-      arg = c;
+      arg = *c;
     }
   }
   hc_spread_max_ = arg;

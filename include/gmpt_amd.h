@@ -145,8 +145,10 @@ int gmpt_synchronize(gmpt_forest *f);
 int gmpt_set_option(gmpt_forest *f, const char *name, int64_t value);
 int gmpt_get_option(gmpt_forest *f, const char *name, int64_t *value);
 /* Autotuner: inserts `sample` (mode 0 PhaseNU, 1 LockNU) into a scratch forest
- * on the same device, times PhaseHC for each candidate hc_spread_max, and sets
- * the fastest on f.  No reference counterpart. */
+ * on the same device, times PhaseHC by levels for each candidate hc_spread_max
+ * (the present value among them), and sets the fastest on f.  Candidates that
+ * launch the sample's levels alike count as one, so a sample too small to tell
+ * any apart leaves the option as it is.  No reference counterpart. */
 int gmpt_autotune(gmpt_forest *f, const gmpt_batch *sample, int mode, int64_t *chosen, double *best_ms);
 int gmpt_get_stats(gmpt_forest *f, gmpt_stats *out);
 /* Bulk rebuild of device batch b (on_device and adopt_values set; trie_ids

@@ -183,3 +183,18 @@ def test_stats_of_a_replay_hold_no_other_pass(gmpt, workloads):
     assert [again[k] for k in keys] == [st[k] for k in keys]
     t.close()
     db.free()
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_autotune_keeps_what_its_sample_cannot_tell_apart(gmpt, workloads, mode):
+    # no inner level of 200 uniform keys passes 256 nodes: every threshold from
+    # there on launches the same kernels, and 0 (a state per lane) is the slower
+    sample = _random_batch(workloads, np.random.default_rng(200), 200)
+    t = gmpt.MPT(device=0)
+    for value in (None, 256, 5000, 1 << 30):
+        if value is None:
+            value = t.get_option("hc_spread_max")
+        else:
+            t.set_option("hc_spread_max", value)
+        assert t.autotune(sample, mode)[0] == value == t.get_option("hc_spread_max")
+    t.close()
