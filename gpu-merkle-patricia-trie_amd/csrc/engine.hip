@@ -5,6 +5,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <chrono>
 #include <mutex>
 #include <new>
 
@@ -24,6 +25,8 @@ thread_local std::string g_err;
 // costs a new forest 50 us at most (4 MiB: 300), and an array that does not
 // fit is large enough that the runtime's own copy is as fast.
 constexpr size_t kPinBytes = 1u << 20;
+
+constexpr std::chrono::milliseconds kPollFor(3);
 
 size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
@@ -358,12 +361,14 @@ Publish Forest::next_publish() {
 
 int Forest::await_counters(const Publish &pub) {
   if (!pub.host) return sync_counters();
-  // A small operation ends within microseconds of the host's wait; after a few
-  // milliseconds the runtime waits (and reports a failed launch).
-  // (Later publications may have passed it.)
+  // A small operation ends within microseconds of the host's wait, which polls
+  // for at most kPollFor (a core of the caller's, and one per lane of a server);
+  // from then on the runtime waits, and reports a failed launch.
+  // (Later publications may have passed this one.)
   const auto there = [&] { return (int32_t)(__atomic_load_n(pub.seq, __ATOMIC_ACQUIRE) - pub.val) >= 0; };
-  for (uint32_t spins = 0; !there(); spins++) {
-    if (spins >= 1u << 20) {
+  const auto until = std::chrono::steady_clock::now() + kPollFor;
+  for (uint32_t spins = 1; !there(); spins++) {
+    if (spins % 64 == 0 && std::chrono::steady_clock::now() >= until) {
       HIP_TRY(hipStreamSynchronize(stream_));
       if (there()) break;
       set_error("the counters did not reach the host");
