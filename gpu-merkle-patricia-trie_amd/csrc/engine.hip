@@ -653,10 +653,11 @@ int Forest::carve_nu(NuArgs &a, const BatchDesc &d, uint64_t vbase, bool has_tid
 
 // Sorts the packed keys (by trie, then nibble path) and keeps the last
 // occurrence of each key: u_idx[0 .. scal[SC_M_UNIQ]) in sorted order.  pass 0
-// sorts by the whole windows (top-8-bit buckets sorted in LDS; above
-// kBucketSortMaxN keys, by the windows' leading bits with a fix-up of equal
-// runs), pass 1 by every window bit that varies across the batch, pass 2 by
-// the whole keys.
+// sorts by the sort keys (top-8-bit buckets sorted in LDS; above
+// kBucketSortMaxN keys, by their leading bits with a fix-up of equal runs),
+// pass 1 by every bit of them that varies across the batch, pass 2 by the
+// whole keys and then by trie, pass 3 by the whole windows and then by trie (a
+// multi-trie batch's sort keys hold part of the window only).
 // Passes 0 and 2 need no host synchronisation: the caller reads
 // flag_fallback at its next one and, if a flag is set, runs next_pass() and
 // repeats the work that followed.
@@ -665,16 +666,22 @@ int Forest::sort_unique(NuArgs &a, void *temp, int pass, int *cur) {
   uint32_t *sv = nullptr;
   int nwords = 0;
   int r;
+  uint32_t trie_bits = 0;
+  if (a.tid)
+    while ((1ull << trie_bits) < ntries_) trie_bits++;
   if (pass == 2) {
     if ((r = publish_and_await())) return r;
     uint32_t W = cnt_.scal[SC_W], maxlen = cnt_.scal[SC_MAXLEN];
     nwords = (int)((maxlen > W ? maxlen - W : 1) + 15) / 16;
   }
+  if (pass == 3) HIP_TRY(nu_windows(a, *cur, stream_));
+  if (pass >= 2) a.tbits = 0;
+  const bool bits = pass == 1 || pass == 3;
   uint64_t vmask = 0, sk_mask = 0;
-  if (pass == 1 && 4ull * ((a.n + 255) / 256) <= a.n) {
+  if (bits && 4ull * ((a.n + 255) / 256) <= a.n) {
     // keys with long shared stretches inside the window (ASCII digits, fixed
     // fields) sort by fewer radix digits once the constant bits are dropped
-    uint64_t m = *(const uint64_t *)(cnt_.scal + SC_WVAR);  // when the packing pass noted them
+    uint64_t m = pass == 1 ? *(const uint64_t *)(cnt_.scal + SC_WVAR) : 0ull;  // when the packing pass noted them
     if (m == 0) {
       HIP_TRY(nu_window_mask(a, *cur ? a.sk1 : a.sk0, stream_));
       if ((r = publish_and_await())) return r;
@@ -684,7 +691,7 @@ int Forest::sort_unique(NuArgs &a, void *temp, int pass, int *cur) {
     const int pop = __builtin_popcountll(m);
     if (pop >= 1 && pop <= 56) vmask = m;  // saves at least one 8-bit digit
   }
-  HIP_TRY(nu_sort(a, nwords, a.tbits, temp, stream_, &sk, &sv, pass == 1, cur, vmask, &sk_mask));
+  HIP_TRY(nu_sort(a, nwords, trie_bits, temp, stream_, &sk, &sv, bits, cur, vmask, &sk_mask));
   // the sorted keys are the plain windows unless the whole keys were sorted
   // or the windows were compressed to their varying bits
   a.u_win_nibs = pass != 2 && sk_mask == 0 ? (64 - a.tbits) / 4 : 0u;
@@ -695,17 +702,15 @@ int Forest::sort_unique(NuArgs &a, void *temp, int pass, int *cur) {
 }
 
 // After a synchronisation: the sort pass to redo with, or -1 when the last
-// sort stands.  A run of equal leading window bits too long to fix up asks
-// for a sort by every varying window bit; two distinct keys with equal
-// windows ask for a sort by whole keys.
+// sort stands.
 int Forest::next_pass(int pass) {
   uint32_t f = cnt_.flag_fallback;
   if (f == 0 || pass == 2) return -1;
-  if (f & 1u) {
+  if (f & kFallbackWhole) {
     stats_.fallback_sorts++;
     return 2;
   }
-  return 1;
+  return f & kFallbackWindow ? 3 : 1;
 }
 
 // After a build's closing counter read: the key arena's new end, and the new

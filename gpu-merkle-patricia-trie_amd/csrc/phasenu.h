@@ -137,12 +137,18 @@ enum {
 // Zeroes the call's device scalars.
 hipError_t nu_init_scalars(const NuArgs &a, hipStream_t s);
 hipError_t nu_prepare_keys(const NuArgs &a, void *temp, hipStream_t s);
+// Bits of Counters::flag_fallback: what a sort asks the host to do again.
+constexpr uint32_t kFallbackWhole = 1;   // distinct keys agree in their windows: by whole keys
+constexpr uint32_t kFallbackBits = 2;    // a bucket or run too long for its kernel: by all bits
+constexpr uint32_t kFallbackWindow = 4;  // many keys of a trie agree in the window's part beside the trie id:
+                                         // by window, then by trie
 // Sorts the batch: by the 16-nibble windows (full = 0; first by their top bits
-// with a fix-up of equal runs, or by all 64 bits when win_all_bits), which for
-// a multi-trie batch hold the trie id above the window's leading bits
-// (a.tbits), or by the whole keys (full = number of 16-nibble words), then by
-// trie.  *cur_io (if
-// given) is the ping-pong buffer holding the current order, in and out.
+// with a fix-up of equal runs, or by all 64 bits when win_all_bits), or by the
+// whole keys (full = number of 16-nibble words).  For a multi-trie batch the
+// windows hold the trie id above their leading bits (a.tbits); with a.tbits
+// set to 0 a sort by trie (trie_bits) follows the one by window or whole key.
+// *cur_io (if given) is the ping-pong buffer holding the current order, in and
+// out.
 // With win_all_bits and a mask of the window bits that vary across the batch
 // (vmask, from nu_window_mask), the windows are first compressed to those
 // bits (an order-preserving bit gather to the top) and sorted by them only;
@@ -154,6 +160,8 @@ hipError_t nu_sort(NuArgs &a, int full, uint32_t trie_bits, void *temp, hipStrea
 // OR and AND of the n windows sk[0 .. n) into scal[SC_WOR], scal[SC_WAND]
 // (per-block partials in a.ecount, which needs 4 words per 256 keys).
 hipError_t nu_window_mask(const NuArgs &a, const uint64_t *sk, hipStream_t s);
+// The plain windows of the order in buffer cur.
+hipError_t nu_windows(const NuArgs &a, int cur, hipStream_t s);
 hipError_t nu_adjacent(const NuArgs &a, const uint64_t *sk, const uint32_t *sv, int full, hipStream_t s,
                        uint64_t sk_mask = 0);
 hipError_t nu_unique(const NuArgs &a, const uint64_t *sk, const uint32_t *sv, void *temp, hipStream_t s);

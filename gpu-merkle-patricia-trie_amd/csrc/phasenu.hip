@@ -209,7 +209,12 @@ struct KeyChunks {
 // above the window's leading bits, so that one sort orders by (trie, path).
 // (A sort by window, then a stable one by trie, then a gather of the windows
 // in the new order took 2.3 ms for 8 M keys of 4,096 tries, 1.5 of them the
-// gather's random reads; the one sort takes 0.5.)
+// gather's random reads; the one sort takes 0.5.)  The trie id takes the place
+// of the window's last tbits bits: keys of one trie that agree in the rest tie,
+// and are ordered by their nibbles afterwards (k_fix_runs).  Insert and hash of
+// 1,000,000 decimal keys of 4,096 tries, tied keys in most: 2,125 us when ties
+// sent the batch to the sort by whole keys, 984 with their runs ordered; 8,000
+// of 200 tries: 430 and 205.
 __device__ __forceinline__ uint64_t sort_key(const NuArgs &a, uint32_t i, uint64_t win) {
   return a.tbits ? (uint64_t)(uint32_t)a.tid[i] << (64 - a.tbits) | win >> a.tbits : win;
 }
@@ -567,6 +572,19 @@ __device__ __forceinline__ T block_offset(const T *cnt, bool pre, T *sh) {
 }
 
 // Adjacent keys of the sorted order: LCP, duplicate and new-trie flags.
+// Whether key ia of a trie comes after key ib of it in path order, given that
+// they agree up to the batch's common prefix: the order k_gather_word's words
+// (then lengths) sort in.
+__device__ bool key_after(const NuArgs &a, uint32_t ia, uint32_t ib) {
+  const KeyRef x = key_of(a, ia), y = key_of(a, ib);
+  for (uint32_t at = a.scal[SC_W]; at + 1 < x.len || at + 1 < y.len; at += 16) {
+    const uint64_t u = at + 1 < x.len ? nib_word(x.p, at, x.len - 1) : 0ull;
+    const uint64_t v = at + 1 < y.len ? nib_word(y.p, at, y.len - 1) : 0ull;
+    if (u != v) return u > v;
+  }
+  return x.len > y.len;
+}
+
 // With cmask != 0 the keys are windows compressed to the bits of cmask
 // (k_compress_windows): the XOR of two is scattered back to window bits
 // before its leading zeros give the first differing nibble.
@@ -626,7 +644,16 @@ __global__ __launch_bounds__(256) void k_adjacent(NuArgs a, const uint64_t *sk, 
         if (ka.len != kb.len) p = min(p, mn - 1);
         while (p < mn && ka.nib(p) == kb.nib(p)) p++;
         ident = (p == mn) && ka.len == kb.len;
-        if (!ident && !full) atomicOr(&a.P.cnt->flag_fallback, 1u);
+        // Distinct keys with equal sort keys: a single trie's need the sort by
+        // whole keys.  A multi-trie batch's are in order already, but for runs
+        // too long for k_fix_runs: those need it if they agree in whole
+        // windows, else the sort by window and trie.
+        if (!ident && !full) {
+          if (a.tbits == 0)
+            atomicOr(&a.P.cnt->flag_fallback, kFallbackWhole);
+          else if (key_after(a, sv[j - 1], ib))
+            atomicOr(&a.P.cnt->flag_fallback, p >= W + 16 ? kFallbackWhole : kFallbackWindow);
+        }
       }
       fl = ident ? 1 : 0;
       l = (uint8_t)min(p, 255u);
@@ -1906,10 +1933,11 @@ hipError_t nu_prepare_keys(const NuArgs &a, void *temp, hipStream_t s) {
 namespace {
 
 // After a stable sort by the keys' top bits: every run of equal top bits is
-// sorted by the whole window with a stable insertion sort by the
-// thread at the run's start (runs of uniform keys hold one or two entries).
-// A run longer than kFixMaxRun sets bit 1 of flag_fallback: the host then
-// sorts by all 64 bits.
+// sorted by the whole sort key, and in a multi-trie batch equal sort keys by
+// the keys' nibbles, with a stable insertion sort by the thread at the run's
+// start (runs of uniform keys hold one or two entries).  A run longer than
+// kFixMaxRun asks the host for a sort by all 64 bits; if those are all equal
+// (top = 64) it is left as it is, for k_adjacent to look at.
 constexpr int kTopBits = 24;  // a single trie's: runs of one or two up to tens of millions of uniform keys
 constexpr uint32_t kFixMaxRun = 64;
 
@@ -1922,14 +1950,14 @@ __global__ __launch_bounds__(256) void k_fix_runs(NuArgs a, uint64_t *sk, uint32
   while (j + L < a.n && L <= kFixMaxRun && (sk[j + L] >> (64 - top)) == lead) L++;
   if (L == 1) return;
   if (L > kFixMaxRun) {
-    atomicOr(&a.P.cnt->flag_fallback, 2u);
+    if (top < 64) atomicOr(&a.P.cnt->flag_fallback, kFallbackBits);
     return;
   }
   for (uint32_t q = 1; q < L; q++) {
     const uint64_t k = sk[j + q];
     const uint32_t v = sv[j + q];
     uint32_t p = q;
-    while (p > 0 && sk[j + p - 1] > k) {
+    while (p > 0 && (sk[j + p - 1] > k || (a.tbits && sk[j + p - 1] == k && key_after(a, sv[j + p - 1], v)))) {
       sk[j + p] = sk[j + p - 1];
       sv[j + p] = sv[j + p - 1];
       p--;
@@ -1997,6 +2025,11 @@ hipError_t nu_window_mask(const NuArgs &a, const uint64_t *sk, hipStream_t s) {
   return hipGetLastError();
 }
 
+hipError_t nu_windows(const NuArgs &a, int cur, hipStream_t s) {
+  k_gather_word<<<nblk(a.n), kB, 0, s>>>(a, cur ? a.sv1 : a.sv0, cur ? a.sk1 : a.sk0, 0);
+  return hipGetLastError();
+}
+
 hipError_t nu_sort(NuArgs &a, int full, uint32_t trie_bits, void *temp, hipStream_t s, uint64_t **sk,
                    uint32_t **sv, bool win_all_bits, int *cur_io, uint64_t vmask, uint64_t *sk_mask) {
   uint64_t *k[2] = {a.sk0, a.sk1};
@@ -2017,6 +2050,10 @@ hipError_t nu_sort(NuArgs &a, int full, uint32_t trie_bits, void *temp, hipStrea
                         (const uint64_t *)(a.scal + SC_WVAR));
     if (e != hipSuccess) return e;
     cur ^= which;
+    if (a.tbits) {
+      k_fix_runs<<<nblk(a.n), kB, 0, s>>>(a, k[cur], v[cur], 64);
+      GMPT_LAUNCH_CHECK();
+    }
   } else if (!full && !win_all_bits) {
     // top bits, then each run of equal top bits by the whole key.  Above the
     // trie id, enough window bits that a run holds 8 entries on average when
@@ -2043,6 +2080,10 @@ hipError_t nu_sort(NuArgs &a, int full, uint32_t trie_bits, void *temp, hipStrea
     e = radix_sort_u64(k[cur], v[cur], k[cur ^ 1], v[cur ^ 1], a.n, lo, 64, &which, temp, s);
     if (e != hipSuccess) return e;
     cur ^= which;
+    if (a.tbits) {
+      k_fix_runs<<<nblk(a.n), kB, 0, s>>>(a, k[cur], v[cur], 64);
+      GMPT_LAUNCH_CHECK();
+    }
   } else {
     // LSD over (words..., length): length first, then the words from last to first
     int nwords = full;
@@ -2055,14 +2096,19 @@ hipError_t nu_sort(NuArgs &a, int full, uint32_t trie_bits, void *temp, hipStrea
       cur ^= which;
     }
   }
-  if (full && trie_bits > 0) {
-    // stable sort of the current permutation by trie id
+  if (trie_bits > 0 && a.tbits == 0) {
+    // sorted by window or whole key: stable sort of the order by trie id
     uint32_t *t[2] = {a.tk0, a.tk1};
     k_gather_trie<<<nblk(a.n), kB, 0, s>>>(a, v[cur], t[0]);
     GMPT_LAUNCH_CHECK();
     e = radix_sort_u32(t[0], v[cur], t[1], v[cur ^ 1], a.n, 0, (int)((trie_bits + 7) & ~7u), &which, temp, s);
     if (e != hipSuccess) return e;
     if (which) cur ^= 1;
+    if (!full) {  // the windows in the new order, as they are
+      k_gather_word<<<nblk(a.n), kB, 0, s>>>(a, v[cur], k[cur], 0);
+      GMPT_LAUNCH_CHECK();
+      vmask = 0;
+    }
   }
   *sk = k[cur];
   *sv = v[cur];

@@ -198,3 +198,55 @@ def test_autotune_keeps_what_its_sample_cannot_tell_apart(gmpt, workloads, mode)
             t.set_option("hc_spread_max", value)
         assert t.autotune(sample, mode)[0] == value == t.get_option("hc_spread_max")
     t.close()
+
+
+@pytest.mark.parametrize("tries,n", [(7, 5000), (7, 30_000), (200, 5000), (200, 30_000), (3000, 30_000)])
+@pytest.mark.parametrize("shape,fallbacks", [("digits", 0), ("short", 0), ("wide", 0), ("long", 1), ("past", 0), ("past-long", 1)])
+def test_keys_of_a_trie_that_tie_beside_the_trie_id(gmpt, workloads, oracle, tries, n, shape, fallbacks):
+    # A multi-trie batch's first sort sees the trie id and the leading bits of
+    # the 16-nibble window (15, 14 or 13 nibbles for 7, 200 and 3,000 tries), in
+    # one workgroup, by buckets and by leading bits.  Keys of one trie that
+    # differ only in the window's last nibble or further on, in runs of a few
+    # and of hundreds, with repeated keys and keys that end in the run; only
+    # long runs whose keys agree in the whole window (all that differ in its last
+    # nibble alone do) take the sort by whole keys
+    rng = np.random.default_rng(tries + n + len(shape))
+    per = 6 if shape in ("digits", "short", "past") else 200
+    groups = n // per
+    keys, tid = [], []
+    for g in range(groups):
+        t = int(rng.integers(tries)) if per == 6 else g % 3
+        if shape == "digits":  # eight digits that vary
+            stem = b"user%018d" % int(rng.integers(10**7))
+            some = [stem + b"%d" % c for c in rng.integers(0, 10, per)]
+        elif shape == "wide":  # each another value of the window's last two nibbles
+            stem = [1] * 10 + [int(x) for x in rng.integers(0, 16, 12)] + [3, 4]
+            some = [bytes(stem + [int(x) // 16, int(x) % 16, 9, 16]) for x in rng.permutation(256)[:per]]
+        else:
+            stem = [1] * 10 + [int(x) for x in rng.integers(0, 16, 12)] + [3, 4, 5]
+            more = 1 if shape in ("short", "long") else 9  # 15 or more nibbles of the window in common
+            stem = stem + [2] * (more - 1)
+            some = [bytes(stem + [int(x) for x in rng.integers(0, 16, int(rng.integers(3, 20)))] + [16]) for _ in range(per)]
+            if shape.startswith("past"):
+                some[0] = bytes(stem + [16])
+        keys += some
+        tid += [t] * per
+    order = rng.permutation(len(keys))
+    vals = [b"%d" % i * (1 + i % 5) for i in range(len(keys))]
+    keys = [keys[i] for i in order]
+    b = (workloads.batch_from_bytes if shape == "digits" else workloads.batch_from_hex)(keys, vals)
+    b.trie_ids = np.array(tid, np.int32)[order]
+    f = gmpt.MPT(device=0, num_tries=tries)
+    _put(f, b)
+    roots = f.get_root_hashes()
+    assert f.stats()["fallback_sorts"] == fallbacks
+    for t in sorted(set(tid))[:: 1 + len(set(tid)) // 12]:
+        assert roots[t] == oracle.root_of(b.subset(np.flatnonzero(b.trie_ids == t))), t
+    again = b.subset(range(0, b.n, 2))  # over the loaded tries, from position order and latched
+    assert _put(f, again, "latching") == _put(f, again)
+    db = gmpt.DeviceBatch(b, adopt_values=True)
+    assert f.rebuild_graph(db) is False and f.get_root_hashes() == roots
+    # (a capture holds the first sort only; seven tries' 15 nibbles leave runs of 16)
+    assert f.rebuild_graph(db) is (per == 6 or (shape == "wide" and tries == 7)) and f.get_root_hashes() == roots
+    f.close()
+    db.free()
