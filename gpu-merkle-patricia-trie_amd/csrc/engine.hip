@@ -1269,7 +1269,10 @@ int Forest::gets(const BatchDesc &keys, uint64_t *hps, int32_t *sizes) {
   uint64_t *d_addr = c.take<uint64_t>(n);
   uint64_t *d_hp = c.take<uint64_t>(n);
   int32_t *d_size = c.take<int32_t>(n);
-  if (c.off > ws2_.cap && (r = ensure_ws(ws2_, c.off))) return r;
+  if (c.off > ws2_.cap) {  // (growing it here would free what was carved)
+    set_error("workspace carve overflow");
+    return -4;
+  }
   // the kernel writes a small batch's results to pinned memory itself, past
   // what is packed there of the batch
   const size_t bytes = 12ull * n;
