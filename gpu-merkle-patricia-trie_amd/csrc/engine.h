@@ -162,7 +162,7 @@ class Forest {
   int arena_exhausted();
   // hash()'s two forms: a short dirty list as one climb after `passes` row
   // launches (*done: every node was hashed), any list by levels.
-  int hash_tree(uint32_t n, int passes, bool *done);
+  int hash_tree(uint32_t n, int passes, bool longs, bool *done);
   int hash_by_level(uint32_t n);
   int hash_levels(const Pools &P, const uint32_t *hist, bool direct_leaves, bool captured, uint32_t *n_leaf_out);
   // rebuild_graph's parts (graph.hip)
@@ -195,6 +195,7 @@ class Forest {
   int build_sorted(NuArgs &a, void *temp, bool empty);
   int merge_groups(NuArgs &a, void *temp);
   bool bulk_fits(const BatchDesc &b) const;
+  void count_dirty(const NuArgs &a);
   uint8_t *value_space(uint64_t bytes);
 
   int device_ = 0;
@@ -233,6 +234,7 @@ class Forest {
   // since the last hash pass: distinct keys written (about a dirty leaf each)
   // and null entries the builds left in the dirty list
   uint64_t dirty_keys_ = 0, dirty_holes_ = 0;
+  bool dirty_long_ = false;      // and whether they may have made many leaves that the word builder does not take
   bool by_level_ = false;        // the next hash pass is to classify its nodes (rebuild_graph captures their bins)
   DevBuf hc_sorted_, hc_meta_, hc_cursor_, hc_slot_, hc_enc_, hc_scratch_, hc_lmeta_, hc_lmeta_tmp_;
   void *h_meta_ = nullptr;       // pinned HcMeta mirror

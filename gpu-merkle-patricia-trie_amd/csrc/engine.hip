@@ -10,6 +10,7 @@
 #include <new>
 
 #include "get.h"
+#include "hc_leaf.h"
 #include "locknu.h"
 #include "phasehc.h"
 #include "phasenu.h"
@@ -731,8 +732,17 @@ void Forest::finish_build(const NuArgs &a) {
   rec_.bdesc = a.bdesc;
   rec_.blo = rec_.lo + rec_.n;
   rec_.bn = cnt_.scal[SC_NREP_TOT];
-  dirty_keys_ += cnt_.scal[SC_M_UNIQ];
+  count_dirty(a);
   dirty_holes_ += cnt_.scal[SC_NREP_TOT] - cnt_.scal[SC_NEXT];
+}
+
+// What the next hash pass may expect of an insert's keys: a leaf each, with a
+// long remainder only where keys reach far past their common prefix, and a long
+// value only as often as the values' bytes allow (pairs that overlap aside).
+void Forest::count_dirty(const NuArgs &a) {
+  dirty_keys_ += cnt_.scal[SC_M_UNIQ];
+  dirty_long_ |= cnt_.scal[SC_MAXLEN] > (uint64_t)cnt_.scal[SC_W] + kLeafFastNibbles + 1 ||
+                 a.v_bytes > (uint64_t)kTreeLongLanes * kLeafDirectMaxValue;
 }
 
 // The sorted, deduplicated keys into the tries: descent (or, into empty tries,
@@ -852,21 +862,23 @@ int Forest::hash(void *targets, int n_targets) {
   // that write the same keys before one pass count them each time, so a long
   // list is taken to hold a sixth of them at least (uniform keys: a quarter).
   const uint64_t others = dirty_keys_ + dirty_holes_, inner = std::max<uint64_t>(n > others ? n - others : 0, n / 6);
+  const bool longs = dirty_long_ && n > kTreeLongLanes;
   dirty_keys_ = dirty_holes_ = 0;
+  dirty_long_ = false;
   if (n > 0 && n <= kTreeMax && inner <= kTreeRowsMaxInner && !by_level_ && hc_fuse_leaves_ && hc_fuse_inner_ &&
       hc_spread_max_ > 0 && !branch_.host && !shrt_.host) {
     const int passes = inner <= kTreeMaxInner ? 0 : kTreeRowPasses;
     bool done = false;
-    if ((r = hash_tree(n, passes, &done)) || done) return r;
+    if ((r = hash_tree(n, passes, longs, &done)) || done) return r;
   }
   return hash_by_level(n);
 }
 
-int Forest::hash_tree(uint32_t n, int passes, bool *done) {
+int Forest::hash_tree(uint32_t n, int passes, bool longs, bool *done) {
   int r;
   if ((r = ensure_ws(hc_sorted_, sizeof(ref_t) * (size_t)n))) return r;
   if ((r = ensure_ws(hc_enc_, sizeof(uint32_t) * (size_t)n))) return r;
-  if (passes && (r = ensure_ws(hc_slot_, sizeof(ref_t) * (size_t)n))) return r;
+  if ((passes || longs) && (r = ensure_ws(hc_slot_, sizeof(ref_t) * (size_t)n))) return r;
   if (!hc_tree_.p) tree_zero_ = false;
   if ((r = ensure_ws(hc_tree_, sizeof(TreeState)))) return r;
   TreeState *tree = (TreeState *)hc_tree_.p;
@@ -874,7 +886,7 @@ int Forest::hash_tree(uint32_t n, int passes, bool *done) {
   tree_zero_ = false;
   if (ev0_) HIP_TRY(hipEventRecord(ev0_, stream_));
   HIP_TRY(hc_tree(pools(), (const ref_t *)dirty_.p, n, (ref_t *)hc_sorted_.p, (ref_t *)hc_slot_.p, (ref_t *)hc_enc_.p,
-                  tree, passes, stream_));
+                  tree, passes, longs, stream_));
   const Publish pub = next_publish();
   HIP_TRY(hc_roots(pools(), ntries_, nullptr, stream_, tree, pub));
   if (ev0_) HIP_TRY(hipEventRecord(ev1_, stream_));
@@ -1126,6 +1138,7 @@ int Forest::clear() {
   HIP_TRY(hc_clear(d_cnt_, (TrieHdr *)tries_.p, ntries_, stream_));
   memset(&cnt_, 0, sizeof(cnt_));
   dirty_keys_ = dirty_holes_ = 0;
+  dirty_long_ = false;
   scal_zero_ = true;
   all_empty_ = true;
   key_used_ = 0;
@@ -1570,7 +1583,7 @@ int Forest::puts_latching(const BatchDesc &b, void **targets, int *n_targets) {
     if (cnt_.n_value != values_before) key_used_ = align_up(key_used_ + ktot, 8);
     stats_.restarts = cnt_.n_restarts;
     stats_.lock_fails = cnt_.n_lock_fail;
-    dirty_keys_ += m;
+    count_dirty(a);
   }
   if (targets) *targets = dirty_.p;
   if (n_targets) *n_targets = (int)cnt_.n_dirty;

@@ -218,6 +218,7 @@ bool Forest::graph_ok() {
   stats_.last_hash_ms = stats_.leaf_perm_ms = 0;
   hash_from_ = leaf_from_ = nullptr;  // the events of an earlier, eager pass
   dirty_keys_ = dirty_holes_ = 0;     // inserts the replay's clear undid
+  dirty_long_ = false;
   return true;
 }
 

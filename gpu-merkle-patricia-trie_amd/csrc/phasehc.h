@@ -113,17 +113,19 @@ constexpr int kTreeRowPasses = 2;
 struct TreeState {
   unsigned long long lists;     // ready, leaf and listed nodes (21 bits each)
   unsigned long long tall;      // leaves of more than one block
+  unsigned long long longs;     // leaves the word builder does not take
   unsigned long long rows[kTreeRowPasses];  // nodes ready after each row launch
-  unsigned long long pad[12];
+  unsigned long long pad[11];
   unsigned long long parts[kTreeParts][8];  // permutations, bytes, those of the leaves, nodes, leaves, extensions
 };
 // Hashes the dirty list list[0 .. n) (n <= kTreeMax) without classifying it:
 // every node is hashed by the wave that hashed its last dirty child, after up
 // to `passes` launches that hash ready nodes a lane each while they are many.
-// ready, ready1 (with passes) and leaves hold n entries each; hc_roots with the
-// same state folds the counts and clears it.  A pass whose hc_nodes differ from
-// its hc_listed left nodes out (a dirty node that no dirty path reaches) and is
-// to be repeated by levels.
+// longs: the list may hold more than kTreeLongLanes long leaves (k_tree_long).
+// ready, ready1 (with passes or longs) and leaves hold n entries each; hc_roots
+// with the same state folds the counts and clears it.  A
+// pass whose hc_nodes differ from its hc_listed left nodes out (a dirty node
+// that no dirty path reaches) and is to be repeated by levels.
 constexpr uint32_t kTreeMax = 1u << 20;
 // A row launch takes a ready list of at least this many nodes (the size up to
 // which a wave per node is as fast, kHcSpreadMaxDefault).
@@ -143,8 +145,10 @@ constexpr uint32_t kTreeRowsMaxInner = 57344;
 // SIMDs and lanes do more per cycle (whole builds, leaves by wave / by lane, of
 // 8,200 entries: 181 / 197 us, 13,600: 206 / 209, 19,000: 229 / 217).
 constexpr uint32_t kTreeSpreadLeaves = 16384;
+// More long leaves than this go by lanes too (measured at k_tree_long).
+constexpr uint32_t kTreeLongLanes = 7000;
 hipError_t hc_tree(const Pools &P, const ref_t *list, uint32_t n, ref_t *ready, ref_t *ready1, ref_t *leaves,
-                   TreeState *tree, int passes, hipStream_t s);
+                   TreeState *tree, int passes, bool longs, hipStream_t s);
 // Copies every trie's root hash into its header and empties the dirty list;
 // with parts (from hc_count), adds the pass's work counts to the counters;
 // with tree (from hc_tree), sets them from it, and keeps the dirty list, and

@@ -1586,7 +1586,10 @@ __global__ __launch_bounds__(256) void k_hc_small(Pools P, const ref_t *__restri
 //   k_tree_link    every dirty node gets its dirty parent (in its own dirty
 //                  word) and a branch the number of its dirty children; the
 //                  nodes without one are ready
-//   k_tree_leaves  (longer lists only) the leaves, one per lane
+//   k_tree_leaves  (longer lists only) the leaves the word builder takes, one
+//                  per lane
+//   k_tree_long    (lists that may hold many only) the other leaves, one per
+//                  lane while they are many, else ready
 //   k_tree_rows    (lists of many inner nodes only, a few launches) while many
 //                  nodes are ready, one per lane; those without a row of a few
 //                  blocks, and parents that became ready, make the next list
@@ -1633,17 +1636,18 @@ __device__ __forceinline__ uint32_t tree_ready(const TreeState *T, int k) {
 
 // One thread per dirty-list entry (W waves per block: one, to spread the loads
 // of a few thousand nodes over the CUs, or four, since blocks take their places
-// in the lists by an atomic on one address each).  With leaf_lanes the leaves
+// in the lists by an atomic on one address each).  With kLeafLanes the leaves
 // the word builder takes go to the leaf list, those of one block from its front
 // and the others from its back (a wave of both would take the longer's time),
-// otherwise every leaf is ready.
+// with kLongLeaves the long ones to a list of their own; other leaves are ready.
+constexpr int kLeafLanes = 1, kLongLeaves = 2;
 template <int W>
 __global__ __launch_bounds__(64 * W) void k_tree_link(Pools P, const ref_t *__restrict__ list, uint32_t n,
                                                   ref_t *__restrict__ ready, ref_t *__restrict__ leaves,
-                                                  TreeState *T, int leaf_lanes) {
+                                                  ref_t *__restrict__ longs, TreeState *T, int mode) {
   const uint32_t lane = __lane_id(), i = grid_tid();
   const ref_t r = i < n ? list[i] : REF_NULL;  // builds leave null holes
-  bool rdy = false, leaf = false, tall = false, listed = false;
+  bool rdy = false, leaf = false, tall = false, lng = false, listed = false;
   if (ref_type(r) == T_BRANCH) {
     Branch &B = P.branch[ref_idx(r)];
     ref_t c[16];
@@ -1678,11 +1682,15 @@ __global__ __launch_bounds__(64 * W) void k_tree_link(Pools P, const ref_t *__re
     const ref_t c = S.child;
     if (ref_type(c) == T_VALUE) {
       listed = true;
-      leaf = leaf_lanes && (uint32_t)S.key_len - S.term <= kLeafFastNibbles &&
-             P.value[ref_idx(c)].size <= kLeafDirectMaxValue;
-      rdy = !leaf;
-      tall = leaf && leaf_blocks((uint32_t)S.key_len - S.term, P.value[ref_idx(c)].size) > 1;
-      leaf = leaf && !tall;
+      if (mode) {
+        const uint32_t cnt = (uint32_t)S.key_len - S.term, vsz = P.value[ref_idx(c)].size;
+        leaf = cnt <= kLeafFastNibbles && vsz <= kLeafDirectMaxValue;
+        lng = !leaf && (mode & kLongLeaves);
+        leaf = leaf && (mode & kLeafLanes);
+        tall = leaf && leaf_blocks(cnt, vsz) > 1;
+        leaf = leaf && !tall;
+      }
+      rdy = !leaf && !tall && !lng;
     } else if (S.lock & 1) {
       S.dirty = 0;  // replaced by a split since it was listed: no node's child any more, and its child another's
     } else {
@@ -1693,38 +1701,45 @@ __global__ __launch_bounds__(64 * W) void k_tree_link(Pools P, const ref_t *__re
     }
   }
   const uint64_t mr = __ballot(rdy), ml = __ballot(leaf), mt = __ballot(tall), ma = __ballot(listed);
+  const uint64_t mo = __ballot(lng);
   const unsigned long long mine = (unsigned long long)__popcll(mr) | (unsigned long long)__popcll(ml) << kTreeListBits |
                                   (unsigned long long)__popcll(ma) << (2 * kTreeListBits);
-  unsigned long long base, tbase = 0;
+  unsigned long long base, tbase = 0, obase = 0;
   if (W == 1) {
     if (ma == 0) return;
     base = tree_reserve(&T->lists, mine, lane);
     if (mt) tbase = tree_reserve(&T->tall, (unsigned long long)__popcll(mt), lane);
+    if (mo) obase = tree_reserve(&T->longs, (unsigned long long)__popcll(mo), lane);
   } else {
-    __shared__ unsigned long long sums[W][2], place[2];
+    __shared__ unsigned long long sums[W][3], place[3];
     const uint32_t g = threadIdx.x / 64;
     if (lane == 0) {
       sums[g][0] = mine;
       sums[g][1] = (unsigned long long)__popcll(mt);
+      sums[g][2] = (unsigned long long)__popcll(mo);
     }
     __syncthreads();
-    if (threadIdx.x < 2) {
+    if (threadIdx.x < 3) {
       unsigned long long all = 0;
       for (int q = 0; q < W; q++) all += sums[q][threadIdx.x];
-      place[threadIdx.x] = all ? atomicAdd(threadIdx.x ? &T->tall : &T->lists, all) : 0ull;
+      unsigned long long *at = threadIdx.x == 0 ? &T->lists : threadIdx.x == 1 ? &T->tall : &T->longs;
+      place[threadIdx.x] = all ? atomicAdd(at, all) : 0ull;
     }
     __syncthreads();
     base = place[0];
     tbase = place[1];
+    obase = place[2];
     for (uint32_t q = 0; q < g; q++) {
       base += sums[q][0];
       tbase += sums[q][1];
+      obase += sums[q][2];
     }
   }
   const uint64_t below = (1ull << lane) - 1;
   if (rdy) ready[(uint32_t)(base & kTreeListMask) + (uint32_t)__popcll(mr & below)] = r;
   if (leaf) leaves[(uint32_t)(base >> kTreeListBits & kTreeListMask) + (uint32_t)__popcll(ml & below)] = r;
   if (tall) leaves[n - 1 - ((uint32_t)tbase + (uint32_t)__popcll(mt & below))] = r;
+  if (lng) longs[(uint32_t)obase + (uint32_t)__popcll(mo & below)] = r;
 }
 
 // Adds the wave's work counts (v on lanes 0 .. 6 as TreeState::parts' words).
@@ -2004,6 +2019,94 @@ __device__ __forceinline__ uint64_t tree_word(const uint64_t *b, const TreeMsg &
   return v;
 }
 
+// The long leaves (a key remainder past 64 nibbles or a value past 16 KB: the
+// word builder takes neither), one per lane: the bytes before the value in LDS,
+// the value's words from where they are, 8 to 9 us a block.  Few of them are
+// left to the climb, where a wave each costs 3 ns a leaf and 1.14 a block: both
+// take as long for about 7,000, whatever their blocks (whole builds, by lane /
+// in the climb: 10,000 leaves of 1 block 231 / 244 us, 4,000 233 / 229; 9,000 of
+// 16 416 / 460, 4,000 414 / 364; 8,000 of 126 1,423 / 1,534, 6,000 1,420 / 1,273).
+// Insert and hash of 150,000 36-byte keys: 1,268 us with all in the climb, 437 so,
+// 441 by levels; of 17,000 values of 17,000 bytes 2,897, 1,420 and 1,820.
+constexpr uint32_t kLongHead = 19;  // words: headers and a compact key of 128 bytes; odd, so that lanes' rows spread
+__global__ __launch_bounds__(64) void k_tree_long(Pools P, const ref_t *__restrict__ longs, ref_t *ready, TreeState *T) {
+  const uint32_t n = (uint32_t)T->longs, lane = threadIdx.x;
+  if (n == 0) return;
+  __shared__ uint64_t heads[64][kLongHead];
+  uint64_t *head = heads[lane];
+  const bool lanes = n > kTreeLongLanes;
+  uint32_t perms = 0, nodes = 0;
+  unsigned long long bytes = 0;
+  for (uint32_t b = blockIdx.x * 64; b < n; b += gridDim.x * 64) {
+    const bool act = b + lane < n;
+    const ref_t r = act ? longs[b + lane] : REF_NULL;
+    if (!lanes) {
+      tree_append(&T->lists, ready, r, lane);
+      continue;
+    }
+    ref_t up = REF_NULL;
+    if (act) {
+      const Short &S = P.shrt[ref_idx(r)];
+      const uint32_t par = S.dirty, term = S.term, cnt = (uint32_t)S.key_len - term;
+      TreeStr v;
+      v.load(P, S.child);
+      const uint32_t payload = rlp_item_len(cnt / 2 + 1, 0) + (v.raw() ? 1u : rlp_hdr_len(v.vsz) + v.vsz);
+      uint32_t hn, sn = 1;
+      const uint64_t hdr = rlp_hdr(payload, 0xC0, 0xF7, &hn);
+      const uint64_t sh = v.raw() ? (uint64_t)v.b0 : rlp_hdr(v.vsz, 0x80, 0xB7, &sn);
+      WordWriter w(head);
+      w.inline_bytes(hdr, hn);
+      w.rlp_compact(P.keys + S.key_off, S.key_start, cnt, term);
+      w.inline_bytes(sh, sn);
+      head[w.nw] = w.acc;
+      TreeMsg m;
+      m.plen = 8 * w.nw + w.accn;
+      m.va = v.va;
+      m.vsz = v.raw() ? 0u : v.vsz;
+      m.enc = hn + payload;
+      const uint32_t nb = keccak_blocks(m.enc);
+      uint64_t st[25];
+#pragma unroll
+      for (int q = 0; q < 25; q++) st[q] = 0;
+      // A block of value bytes only is loaded (its aligned words) before the
+      // permutation ahead of it, which hides the loads.
+      uint64_t word[18];
+      uint32_t off = 0;  // of the block's first byte in word[0]
+      bool loaded = false;
+      for (uint32_t k = 0; k < nb; k++) {
+        if (loaded) {
+#pragma unroll
+          for (uint32_t q = 0; q < 17; q++) st[q] ^= funnel8(word[q], word[q + 1], off);
+        } else {
+#pragma unroll
+          for (uint32_t q = 0; q < 17; q++) st[q] ^= tree_word(head, m, nb, 17 * k + q);
+        }
+        const uint32_t x = 136 * (k + 1);
+        loaded = x >= m.plen && m.vsz >= 136 && x - m.plen <= m.vsz - 136;
+        if (loaded) {
+          const uint64_t at = m.va + (x - m.plen);
+          const uint64_t *src = (const uint64_t *)(at & ~7ull);
+          off = (uint32_t)(at & 7);
+#pragma unroll
+          for (uint32_t q = 0; q < 17; q++) word[q] = src[q];
+          word[17] = src[off ? 17 : 16];  // no word past the value's last byte
+        }
+        keccak_f1600(st);
+      }
+      store_digest(P, r, st);
+      up = tree_up(P, par);
+      perms += nb;
+      bytes += m.enc;
+      nodes++;
+    }
+    tree_append(&T->lists, ready, up, lane);
+  }
+  perms = wave_sum(perms);
+  nodes = wave_sum(nodes);
+  for (int off = 32; off > 0; off >>= 1) bytes += (unsigned long long)__shfl_xor((long long)bytes, off);
+  tree_count(T, blockIdx.x, lane, lane == 0 || lane == 2 ? perms : lane == 1 || lane == 3 ? bytes : lane < 6 ? nodes : 0ull);
+}
+
 // One wave per ready node; the wave climbs as long as it hashed its node's
 // parent's last dirty child.  Its stores of a node (digest, then the word with
 // the size) are written through and complete before the parent's count goes
@@ -2192,7 +2295,7 @@ __device__ __forceinline__ void roots_body(const Pools &P, uint32_t ntries, cons
       P.cnt->hc_exts = (uint32_t)v[6];
       P.cnt->hc_listed = (uint32_t)(tree->lists >> (2 * kTreeListBits));
       if (P.cnt->hc_nodes == P.cnt->hc_listed) P.cnt->n_dirty = 0;  // otherwise the list stands for the levels
-      tree->lists = tree->tall = 0;
+      tree->lists = tree->tall = tree->longs = 0;
       for (uint32_t q = 0; q < kTreeRowPasses; q++) tree->rows[q] = 0;
     }
   }
@@ -2497,16 +2600,21 @@ hipError_t publish_counters(const Counters *cnt, Publish pub, hipStream_t s) {
 }
 
 hipError_t hc_tree(const Pools &P, const ref_t *list, uint32_t n, ref_t *ready, ref_t *ready1, ref_t *leaves,
-                   TreeState *tree, int passes, hipStream_t s) {
+                   TreeState *tree, int passes, bool longs, hipStream_t s) {
   if (n == 0 || n > kTreeMax) return hipErrorInvalidValue;
   const bool lanes = n > kTreeSpreadLeaves;
+  const int mode = (lanes ? kLeafLanes : 0) | (longs ? kLongLeaves : 0);
   if (passes)
-    k_tree_link<4><<<nblk(n), kB, 0, s>>>(P, list, n, ready, leaves, tree, lanes ? 1 : 0);
+    k_tree_link<4><<<nblk(n), kB, 0, s>>>(P, list, n, ready, leaves, ready1, tree, mode);
   else
-    k_tree_link<1><<<(n + 63) / 64, 64, 0, s>>>(P, list, n, ready, leaves, tree, lanes ? 1 : 0);
+    k_tree_link<1><<<(n + 63) / 64, 64, 0, s>>>(P, list, n, ready, leaves, ready1, tree, mode);
   GMPT_LAUNCH_CHECK();
   if (lanes) {
     k_tree_leaves<<<nblk(n + 63), kB, 0, s>>>(P, leaves, n, ready, tree);
+    GMPT_LAUNCH_CHECK();
+  }
+  if (longs) {
+    k_tree_long<<<std::min<uint32_t>((n + 63) / 64, 2048), 64, 0, s>>>(P, ready1, ready, tree);
     GMPT_LAUNCH_CHECK();
   }
   // (one more block than the CUs hold at a time gains nothing: blocks loop)

@@ -250,3 +250,51 @@ def test_keys_of_a_trie_that_tie_beside_the_trie_id(gmpt, workloads, oracle, tri
     assert f.rebuild_graph(db) is (per == 6 or (shape == "wide" and tries == 7)) and f.get_root_hashes() == roots
     f.close()
     db.free()
+
+
+@pytest.mark.parametrize("mode", list(PUTS))
+@pytest.mark.parametrize("n_long,n,klen", [(6990, 7200, 36), (7010, 7200, 36), (7010, 12_000, 126), (6990, 30_000, 60),
+                                           (7300, 30_000, 126), (45_000, 45_000, 40)])
+def test_long_leaves_around_the_line_to_lanes(gmpt, workloads, oracle, mode, n_long, n, klen):
+    # leaves the word builder does not take (remainders past 64 nibbles up to the
+    # longest key, odd and even): left to the climb up to 7,000 of them, one per
+    # lane above, in lists with row launches and without; values of no byte, one
+    # (raw and not), and around the ends of one to three blocks, at odd addresses
+    rng = np.random.default_rng(n_long + n)
+    keys = rng.integers(0, 256, (n, 32), dtype=np.uint8)
+    hexes = [b"".join(bytes((x >> 4, x & 15)) for x in k.tobytes()) for k in keys]
+    tails = rng.integers(0, 16, (n_long, 2 * klen - 64), dtype=np.uint8)
+    hexes = [h + (tails[i].tobytes()[i % 2 and 1:] if i < n_long else b"") + b"\x10" for i, h in enumerate(hexes)]
+    lens = rng.choice([0, 1, 1, 2, 31, 55, 56, 70, 90, 100, 135, 136, 137, 200, 272, 273, 400], n)
+    b = workloads.batch_from_hex(hexes, [bytes(rng.integers(0, 256, int(k), dtype=np.uint8)) for k in lens])
+    t, by_level = gmpt.MPT(device=0), gmpt.MPT(device=0)
+    by_level.set_option("hc_fuse_leaves", 0)
+    for part in (b, b.subset(range(0, n, 1 if n < 20_000 else 2))):  # new, then over the clean trie
+        assert _put(t, part, mode) == oracle.root_of(b) == _put(by_level, part, mode)
+        assert t.stats()["hash_launches"] in (1, 3)
+        for k in ("perms", "enc_bytes", "leaf_perms", "leaf_bytes", "leaf_nodes", "hashed_nodes"):
+            assert t.stats()[k] == by_level.stats()[k], k
+
+
+def test_long_values_around_the_line_to_lanes(gmpt, workloads, oracle):
+    # values past 16 KB, some of them at addresses that are no multiple of 8, of
+    # every remainder by a block: from an adopted buffer whose pairs overlap (the
+    # host does not expect so many), then from one that holds each
+    rng = np.random.default_rng(16)
+    n = 7100
+    b = _random_batch(workloads, rng, n)
+    lens = 16_383 + np.arange(n) % 200
+    at = rng.integers(0, 1 << 20, n)
+    b.values_bytes = rng.integers(0, 256, (1 << 20) + 20_000, dtype=np.uint8)
+    b.values_indexs = np.stack([at, at + lens - 1], 1).astype(np.int64).ravel()
+    b.values_indexs[-2:] = len(b.values_bytes) - 16_400, len(b.values_bytes) - 1
+    want = oracle.root_of(b)
+    db = gmpt.DeviceBatch(b, adopt_values=True)
+    db.struct.values_bytes_total = len(b.values_bytes)
+    t = gmpt.MPT(device=0)
+    assert _put(t, db) == want
+    t.clear()
+    flat = workloads.batch_from_hex([b.key(i) for i in range(n)], [b.value(i) for i in range(n)])
+    assert _put(t, flat) == want and t.stats()["leaf_nodes"] == n
+    t.close()
+    db.free()
