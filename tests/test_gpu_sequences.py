@@ -1,4 +1,4 @@
-"""Calls whose buffers, counters or routes an earlier call of the same forest left behind."""
+"""Sequences of calls on one forest, and the forms a hash pass or sort takes for them, against the CPU oracle."""
 import numpy as np
 import pytest
 
@@ -298,3 +298,91 @@ def test_long_values_around_the_line_to_lanes(gmpt, workloads, oracle):
     assert _put(t, flat) == want and t.stats()["leaf_nodes"] == n
     t.close()
     db.free()
+
+
+@pytest.mark.parametrize("seed", [61, 62, 63])
+def test_latched_inserts_into_larger_tries_split_fresh_nodes(gmpt, workloads, oracle, seed):
+    # clusters of keys that share prefixes of random lengths; half of them are in
+    # the trie, so the rest is latched, and lanes of a wave split the same fresh
+    # short nodes at many depths; keys that end inside others among them
+    rng = np.random.default_rng(seed)
+    keys = {}
+    for _ in range(500):
+        base = rng.integers(0, 16, 64)
+        for _ in range(int(rng.integers(2, 30))):
+            k = base.copy()
+            cut = int(rng.integers(1, 64))
+            k[cut:] = rng.integers(0, 16, 64 - cut)
+            keys[bytes(int(x) for x in k[:int(rng.integers(40, 65))]) + b"\x10"] = None
+    keys = list(keys)
+    keys = [keys[i] for i in rng.permutation(len(keys))]
+    cuts = [0, len(keys) // 2, 3 * len(keys) // 4, len(keys)]
+    t, o = gmpt.MPT(device=0), oracle.OracleMPT()
+    for k, (lo, hi) in enumerate(zip(cuts, cuts[1:])):
+        part = keys[lo:hi] + keys[:lo // 5]
+        b = workloads.batch_from_hex(part, [bytes(rng.integers(0, 256, int(rng.integers(0, 90)), dtype=np.uint8)) for _ in part])
+        before = t.stats()["pool_bytes_used"]
+        _put(t, b, "latching")
+        o.puts(b)
+        o.hash()
+        assert t.get_root_hash() == o.root()
+        # a latched key takes one branch, two short nodes and one value (288 bytes), used or not
+        if k:
+            assert t.stats()["pool_bytes_used"] - before >= 288 * (hi - lo)
+    assert t.get_values(b) == o.gets(b)
+
+
+@pytest.mark.parametrize("spread_max", [0, 8192, 1 << 30])
+@pytest.mark.parametrize("fuse_leaves", [0, 1])
+@pytest.mark.parametrize("case", ["plain", "block-edge", "tiny-values", "long-keys", "short-keys", "mixed"])
+def test_short_lists_by_levels(gmpt, workloads, oracle, spread_max, fuse_leaves, case):
+    # "hc_fuse_inner" 0 keeps a short list out of the climb: its levels by the
+    # spread and the lane kernels, leaves fused and not
+    rng = np.random.default_rng(len(case) + fuse_leaves)
+    n, klen, vlo, vhi = {"plain": (5000, 32, 70, 110), "block-edge": (129, 32, 70, 110), "tiny-values": (3000, 32, 0, 2),
+                         "long-keys": (2000, 44, 10, 60), "short-keys": (2500, 2, 0, 40), "mixed": (8000, 32, 20, 600)}[case]
+    flat, lens = workloads.random_values(rng, n, vlo, vhi)
+    b = workloads.batch_from_fixed(workloads.unique_random_keys(rng, n, klen), flat, lens)
+    t, climb = gmpt.MPT(device=0), gmpt.MPT(device=0)
+    t.set_option("hc_spread_max", spread_max)
+    t.set_option("hc_fuse_leaves", fuse_leaves)
+    t.set_option("hc_fuse_inner", 0)
+    want = oracle.root_of(b)
+    for part in (b, b.subset(range(0, n, 3))):
+        assert _put(t, part) == want == _put(climb, part)
+        assert climb.stats()["hash_launches"] == 1 < t.stats()["hash_launches"]
+        for k in ("perms", "enc_bytes", "leaf_perms", "leaf_bytes", "leaf_nodes", "hashed_nodes"):
+            assert t.stats()[k] == climb.stats()[k], k
+
+
+@pytest.mark.parametrize("mode", list(PUTS))
+def test_levels_beside_a_clean_long_leaf(gmpt, workloads, oracle, mode):
+    # by levels, the deepest small ones on the second stream: a new key beside a
+    # clean leaf that the leaf word builder does not take
+    rng = np.random.default_rng(81)
+
+    def key(*head):
+        return bytes(head) + bytes(rng.integers(0, 256, 32 - len(head), dtype=np.uint8))
+
+    keys = [key(0, 0), key(0, 1)] + [key(int(x)) for x in rng.integers(16, 256, 40)]
+    first = workloads.batch_from_bytes(keys, [b"long" * 5000] + [b"w%d" % i for i in range(len(keys) - 1)])
+    second = workloads.batch_from_bytes([key(0, 2)], [b"v3"])
+    t = gmpt.MPT(device=0)
+    t.set_option("hc_fuse_inner", 0)
+    assert _put(t, first, mode) == oracle.root_of(first)
+    assert _put(t, second, mode) == oracle.root_of(workloads.concat_batches([first, second]))
+    assert t.stats()["hash_launches"] > 1
+
+
+def test_leaves_by_wave_and_by_lane_around_their_line(gmpt, workloads, oracle):
+    # dirty lists either side of 16,384 entries
+    rng = np.random.default_rng(16384)
+    listed = []
+    for n in (9200, 9350, 9500, 9650, 9800, 12_000):
+        b = _random_batch(workloads, rng, n)
+        t = gmpt.MPT(device=0)
+        targets, m = t.puts_2phase_with_valuehp(b)
+        t.hash_onepass_v2(targets, m)
+        assert t.get_root_hash() == oracle.root_of(b) and t.stats()["hash_launches"] == 1
+        listed.append(m)
+    assert listed[0] <= 16_384 < listed[-1]
