@@ -200,7 +200,7 @@ __device__ __forceinline__ uint32_t *node_dirty_flag(const Pools &P, ref_t r) {
   return t == T_BRANCH ? &P.branch[i].dirty : &P.shrt[i].dirty;
 }
 
-// Block-staged dirty-list appends: lanes stage the nodes they flip in LDS
+// Block-staged dirty-list appends: lanes stage the nodes they mark in LDS
 // (an LDS atomic each) and the block appends them to the global list with one
 // global atomic in dirty_flush().  Appending straight to the list costs a
 // global atomic on one counter per wave and mark, which serialises when many
@@ -220,12 +220,6 @@ struct DirtyStage {
       P.dirty[slot] = r;
     else
       raise_error(P.cnt, ERR_POOL, 4);
-  }
-  // marks an existing node: the lane that flips its flag stages it
-  __device__ __forceinline__ void mark(const Pools &P, ref_t r) {
-    uint32_t *f = node_dirty_flag(P, r);
-    if (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0 && atomicExch(f, 1u) == 0u)
-      push(P, r);
   }
 };
 
