@@ -1,11 +1,14 @@
 // graph.hip -- a bulk rebuild pass (clear + PhaseNU + PhaseHC) captured once
 // as a HIP graph and replayed per batch.
 //
-// An eager pass synchronises with the host four times: after the sort (to
-// see whether a fallback sort is needed), after the build (counters), after
-// the hash classification (the host reads the level sizes to launch one
+// An eager pass hashed by levels waits for the device three times: after the
+// build (its counters, which also tell whether a fallback sort is needed),
+// after the hash classification (the host reads the level sizes to launch one
 // range per level) and at the end.  A replay runs the same launches with
 // the level sizes of the captured pass and one synchronisation at the end.
+// Insert + hash, plain calls / replayed: 20,000 keys 231 / 255 us (plain calls
+// hash short lists in one climb, a capture always by levels), 100,000 327 /
+// 342, 150,000 408 / 374, 400,000 504 / 496.
 // It is valid only when the batch behaves like the captured one, which the
 // device checks itself right after the classification (k_graph_check): no
 // sort fallback, no error, the same dirty-list length, element count and

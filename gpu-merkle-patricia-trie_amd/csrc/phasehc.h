@@ -8,8 +8,8 @@ constexpr uint32_t kHcClasses = 8;     // Keccak block-count classes per level
 constexpr uint32_t kHcMaxDepth = 255;  // levels: 0 = leaves, 1 + (255 - depth) otherwise
 constexpr uint32_t kHcLevels = kHcMaxDepth + 2;
 constexpr uint32_t kHcBins = kHcLevels * kHcClasses;
-// Levels with at most this many nodes spread each Keccak state over 25 lanes:
-// four waves on every SIMD take 4,096 nodes' permutation in 5.2 us, one state
+// Levels with at most this many nodes spread each Keccak state over one wave
+// (40 lanes): four waves on every SIMD take 4,096 nodes' permutation in 5.2 us, one state
 // per lane takes 7.2 however few there are, and its messages take longer to
 // lay out.  Builds of 100,000 / 250,000 / 400,000 / 1,000,000 keys with the
 // line at 1,024: 399 / 459 / 506 / 788 us, 8,192: 374 / 438 / 487 / 780.
@@ -29,15 +29,6 @@ struct HcMeta {
 };
 
 size_t hc_temp_bytes(uint32_t n);
-// Bins dirty nodes by (level, block class): out = the list ordered by bin,
-// slot[i] = byte offset of sorted node i's message slot in the scratch buffer
-// (for slot_lo <= i < nvalid; other entries are not written);
-// packed (n entries) is workspace.  With lmeta (2n words, lmeta_tmp 2n words
-// of workspace) the leaves whose key remainder has at most 64 nibbles and
-// whose value is under 16,383 bytes -- level 0, the first hist[0 .. 8)
-// sorted entries -- get no scratch slot but a metadata record lmeta[2i],
-// lmeta[2i + 1] for hc_hash_leaves_direct; other leaves are binned at
-// level 1 (no inner node can be there).
 // Bins and leaf metadata recorded by a build for dirty-list entries
 // [lo, lo + n): pk[k] = bin | blocks << 12 or kLeafPackedNone, meta[2k..] as
 // leaf_meta_words.  Valid only while nothing has changed those nodes since.
@@ -50,6 +41,15 @@ struct LeafRecords {
   const uint32_t *bdesc = nullptr;
   uint32_t blo = 0, bn = 0;
 };
+// Bins dirty nodes by (level, block class): out = the list ordered by bin,
+// slot[i] = byte offset of sorted node i's message slot in the scratch buffer
+// (for slot_lo <= i < nvalid; other entries are not written);
+// packed (n entries) is workspace.  With lmeta (2n words, lmeta_tmp 2n words
+// of workspace) the leaves whose key remainder has at most 64 nibbles and
+// whose value is under 16,383 bytes -- level 0, the first hist[0 .. 8)
+// sorted entries -- get no scratch slot but a metadata record lmeta[2i],
+// lmeta[2i + 1] for hc_hash_leaves_direct; other leaves are binned at
+// level 1 (no inner node can be there).
 hipError_t hc_classify(const Pools &P, const ref_t *list, uint32_t n, HcMeta *meta, uint32_t *cursor, ref_t *out,
                        uint64_t *slot, uint32_t *packed, void *temp, hipStream_t s, uint64_t *lmeta_tmp = nullptr,
                        uint64_t *lmeta = nullptr, LeafRecords rec = LeafRecords());
@@ -162,11 +162,11 @@ struct Publish {
 };
 hipError_t hc_roots(const Pools &P, uint32_t ntries, const unsigned long long *parts, hipStream_t s,
                     TreeState *tree = nullptr, Publish pub = Publish());
-// (publish_counters) Copies the counters to pinned host memory and then stores val at seq, which
-// the host waits for: a launch of ours in place of a copy's blit kernel, and
-// no wait for the stream's completion signal.
 // Root hashes (32-byte slots) and sizes of count tries, to pinned host memory.
 hipError_t gather_roots(const TrieHdr *tries, uint32_t count, uint8_t *hash, int32_t *size, hipStream_t s);
+// Copies the counters to pinned host memory and then stores val at seq, which
+// the host waits for: a launch of ours in place of a copy's blit kernel, and
+// no wait for the stream's completion signal.
 hipError_t publish_counters(const Counters *cnt, Publish pub, hipStream_t s);
 // Node export: encoding lengths; then, with their exclusive sums offs, the
 // encodings, 32-byte hash slots and inclusive [start, end] pairs.
@@ -175,7 +175,7 @@ hipError_t hc_enc_write(const Pools &P, const ref_t *refs, uint32_t m, const uin
                         uint64_t *hashes, uint64_t *pairs, hipStream_t s);
 // Keccak-256 of n messages (test hook for the sponge): scratch holds
 // keccak_scratch_bytes(len, n) bytes, slot n entries, temp scan workspace.
-// spread = 1 runs the 25-lane layout, 0 one state per lane.
+// spread = 1 runs the layout of one state per wave, 0 one state per lane.
 uint64_t keccak_scratch_bytes(const uint32_t *len, uint32_t n);
 hipError_t keccak_batch(const uint8_t *data, const uint64_t *off, const uint32_t *len, uint32_t n, uint8_t *out,
                         uint64_t *slot, uint64_t *scratch, void *temp, int spread, hipStream_t s);

@@ -17,8 +17,8 @@
 //    waves overlap the pointer chasing to children and values.
 //  - permute: Keccak-f[1600] over the slots.  Large levels keep one 25-word
 //    state per GPU lane (VGPRs, no communication); small levels are latency
-//    bound, so there one state is spread over 25 lanes of a 32-lane group
-//    and theta, pi and chi exchange words with cross-lane permutes.
+//    bound, so there one state is spread over a wave (40 lanes, a plane per
+//    8-lane half-row) and theta, pi and chi exchange words across lanes.
 //
 // Node encoding follows the reference's encoders exactly
 // (FullNode::encode node.cuh:414-452, ShortNode::encode node.cuh:526-559,
@@ -2027,7 +2027,7 @@ __device__ __forceinline__ uint64_t tree_word(const uint64_t *b, const TreeMsg &
 // in the climb: 10,000 leaves of 1 block 231 / 244 us, 4,000 233 / 229; 9,000 of
 // 16 416 / 460, 4,000 414 / 364; 8,000 of 126 1,423 / 1,534, 6,000 1,420 / 1,273).
 // Insert and hash of 150,000 36-byte keys: 1,268 us with all in the climb, 437 so,
-// 441 by levels; of 17,000 values of 17,000 bytes 2,897, 1,420 and 1,820.
+// 441 by levels; of 17,000 values of 17,000 bytes 2,897, 1,395 and 1,819.
 constexpr uint32_t kLongHead = 19;  // words: headers and a compact key of 128 bytes; odd, so that lanes' rows spread
 __global__ __launch_bounds__(64) void k_tree_long(Pools P, const ref_t *__restrict__ longs, ref_t *ready, TreeState *T) {
   const uint32_t n = (uint32_t)T->longs, lane = threadIdx.x;

@@ -325,7 +325,8 @@ class MPT:
     def rebuild_graph(self, batch):
         """Empties the forest and bulk-builds `batch` (a DeviceBatch made with
         adopt_values=True) as one replay of a captured HIP graph; the first
-        call for a batch's buffers captures.  Returns True when a replay stood
+        call for a batch's buffers, and the first after a call that replaced a
+        device buffer, captures.  Returns True when a replay stood
         (False: the pass ran eagerly, and was captured for the next call)."""
         if not isinstance(batch, DeviceBatch) or not batch.struct.adopt_values:
             raise GmptError("rebuild_graph takes a DeviceBatch with adopt_values=True")
@@ -518,7 +519,7 @@ class Server:
 
 def keccak256_batch(messages, mode=0):
     """Keccak-256 of each message, computed on the GPU (mode 0: one state per
-    lane, mode 1: one state spread over 25 lanes)."""
+    lane, mode 1: one state spread over a wave)."""
     n = len(messages)
     lens = np.array([len(m) for m in messages], np.uint32)
     offs = np.zeros(n, np.uint64)

@@ -80,7 +80,10 @@ const char *gmpt_last_error(void);
  * pass to gmpt_hash_onepass.
  * Replaces: MPT::puts_2phase_with_valuehp (gpu_mpt.cuh:95-97, 1262-1399). */
 int gmpt_puts_2phase(gmpt_forest *f, const gmpt_batch *b, void **targets, int *n_targets);
-/* LockNU batch insert.
+/* LockNU batch insert.  A batch into a forest of empty tries, or of more
+ * distinct keys than the forest's tries hold on average, is inserted as
+ * gmpt_puts_2phase does (the same tries result, and its lanes would wait for
+ * one another's latches); gmpt_stats' restarts and lock_fails are 0 then.
  * Replaces: MPT::puts_latching_with_valuehp_v2 (gpu_mpt.cuh:69-71, 554-615). */
 int gmpt_puts_latching(gmpt_forest *f, const gmpt_batch *b, void **targets, int *n_targets);
 /* Mixed read/write batch: rw_flags[i] = 0 reads key i, 1 writes it (a host
@@ -103,7 +106,7 @@ int gmpt_hash_onepass(gmpt_forest *f, void *targets, int n_targets);
  * is shorter than 32 bytes, or 0 for an empty trie.
  * Replaces: MPT::get_root_hash (gpu_mpt.cuh:151-152, 1217-1247). */
 int gmpt_get_root_hash(gmpt_forest *f, uint32_t trie, uint8_t out[32], int *size);
-/* Root hashes of tries [first, first + count) with one device copy: out holds
+/* Root hashes of tries [first, first + count), read at once: out holds
  * 32 bytes per trie (zero padded), sizes[i] as for gmpt_get_root_hash.
  * Replaces: MPT::get_root_hash called once per trie (gpu_mpt.cuh:1217-1247). */
 int gmpt_get_root_hashes(gmpt_forest *f, uint32_t first, uint32_t count, uint8_t *out, int *sizes);
@@ -129,9 +132,11 @@ int gmpt_reset_trie(gmpt_forest *f, uint32_t trie);
 int gmpt_forest_clear(gmpt_forest *f);
 int gmpt_synchronize(gmpt_forest *f);
 /* Tunables by name.  "hc_spread_max": PhaseHC levels with at most this many
- * dirty nodes run Keccak with one state spread over 25 lanes (latency), larger
- * levels one state per lane (throughput).  Default 1024, or the
- * GMPT_HC_SPREAD_MAX environment variable.  "hc_fuse_leaves" (0 or 1,
+ * dirty nodes run Keccak with one state spread over one wave (40 lanes;
+ * latency), larger levels one state per lane (throughput).  Default 8192, or
+ * the GMPT_HC_SPREAD_MAX environment variable.  Short dirty lists are hashed in
+ * one climb and not by levels: the value does not matter to them, except that
+ * 0 turns the climb off, as a 0 of either option below and "pool_memory" 1 do.  "hc_fuse_leaves" (0 or 1,
  * default 1): leaves whose key remainder has at most 64 nibbles and whose
  * value is under 16,383 bytes are encoded and hashed by one kernel, the
  * message built in registers, instead of an encode kernel, an HBM scratch
@@ -157,7 +162,9 @@ int gmpt_get_stats(gmpt_forest *f, gmpt_stats *out);
  * for a batch -- its device buffers and sizes -- runs the pass eagerly,
  * captures it and replays it once; later calls with the same buffers (new
  * contents of the same shape) replay it with one host synchronisation
- * instead of four.  The device checks each replay against the captured pass
+ * instead of three; a call in between that replaces a device buffer of the
+ * forest (a larger batch, read or export) drops the capture, and the next call
+ * makes it again.  The device checks each replay against the captured pass
  * (no fallback sort, the same dirty-node count and hash levels); a batch that
  * differs is redone eagerly and captured again, so results are always those
  * of the plain calls.  *replayed = 1 when the replay stood.  Roots are then
@@ -183,8 +190,8 @@ int gmpt_timer_stop(gmpt_forest *f, float *ms);
 int gmpt_keccak256_batch(const uint8_t *data, const uint64_t *offsets, const uint32_t *lengths, uint32_t n,
                          uint8_t *out);
 /* As gmpt_keccak256_batch with the permutation layout chosen: mode 0 keeps one
- * state per GPU lane (PhaseHC's large levels), mode 1 spreads one state over 25
- * lanes (PhaseHC's small levels).  No reference counterpart (test hook). */
+ * state per GPU lane (PhaseHC's large levels), mode 1 spreads one state over a
+ * wave, 40 lanes (PhaseHC's small levels).  No reference counterpart (test hook). */
 int gmpt_keccak256_batch_mode(const uint8_t *data, const uint64_t *offsets, const uint32_t *lengths, uint32_t n,
                               uint8_t *out, int mode);
 
