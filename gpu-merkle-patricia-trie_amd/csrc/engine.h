@@ -48,8 +48,11 @@ struct Arena {
   uint8_t *base = nullptr;
   size_t cap = 0;
   size_t used = 0;
+  size_t next() const { return (used + 255) & ~(size_t)255; }
+  // bytes as a buffer takes them: rounded up to 256
+  bool fits(size_t bytes) const { return next() <= cap && ((bytes + 255) & ~(size_t)255) <= cap - next(); }
   void *take(size_t bytes) {
-    size_t off = (used + 255) & ~(size_t)255;
+    size_t off = next();
     if (off > cap || bytes > cap - off) return nullptr;
     used = off + bytes;
     return base + off;

@@ -878,9 +878,12 @@ int Forest::hash_tree(uint32_t n, int passes, bool longs, bool *done) {
   int r;
   if ((r = ensure_ws(hc_sorted_, sizeof(ref_t) * (size_t)n))) return r;
   if ((r = ensure_ws(hc_enc_, sizeof(uint32_t) * (size_t)n))) return r;
-  if ((passes || longs) && (r = ensure_ws(hc_slot_, sizeof(ref_t) * (size_t)n))) return r;
   if (!hc_tree_.p) tree_zero_ = false;
   if ((r = ensure_ws(hc_tree_, sizeof(TreeState)))) return r;
+  // (a region that holds the batch but not a list of its long leaves leaves them to the climb)
+  const size_t list = sizeof(ref_t) * (size_t)n;
+  if (arena_ && !passes && hc_slot_.cap < list && !arena_->fits(list)) longs = false;
+  if ((passes || longs) && (r = ensure_ws(hc_slot_, list))) return r;
   TreeState *tree = (TreeState *)hc_tree_.p;
   if (!tree_zero_) HIP_TRY(hipMemsetAsync(tree, 0, sizeof(TreeState), stream_));
   tree_zero_ = false;

@@ -80,3 +80,33 @@ def test_noalloc_rejects_batches_above_its_limit(gmpt, workloads):
         gmpt.build_root_noalloc(big, 0)
     ok = _rand_batch(workloads, 702, 100, 10, 20)
     assert len(gmpt.build_root_noalloc(ok, 1)) == 32
+
+
+def test_noalloc_takes_long_leaves_to_the_end_of_its_region(gmpt, workloads, oracle):
+    # The largest values the region takes beside 8,000 keys: one key of 36 bytes
+    # (its leaf is a long one, and the list of such leaves would take 43 KB)
+    # costs the region the key's own few bytes, in arrays rounded to 256.
+    rng = np.random.default_rng(91)
+    n = 8000
+    keys = [bytes(k) for k in workloads.unique_random_keys(rng, n, 32)]
+    keys[0] = keys[0][:31]
+
+    def batch(ks, total):
+        sizes = np.full(n, total // n, np.int64)
+        sizes[:total % n] += 1
+        b = workloads.batch_from_bytes(ks, [b"v"] * n)
+        ends = np.cumsum(sizes)
+        b.values_bytes = np.full(total, 0x5a, np.uint8)
+        b.values_indexs = np.stack([ends - sizes, ends - 1], 1).reshape(-1).astype(b.values_indexs.dtype)
+        return b
+
+    lo, hi = 1 << 20, 64 << 20  # taken, refused
+    while hi - lo > 256:
+        mid = (lo + hi) // 2
+        try:
+            gmpt.build_root_noalloc(batch(keys, mid), 0)
+            lo = mid
+        except gmpt.GmptError:
+            hi = mid
+    b = batch(keys[:-1] + [keys[-1] + b"tail"], lo - 4096)
+    assert gmpt.build_root_noalloc(b, 0) == oracle.root_of(b)
