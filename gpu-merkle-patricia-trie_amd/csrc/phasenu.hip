@@ -571,7 +571,6 @@ __device__ __forceinline__ T block_offset(const T *cnt, bool pre, T *sh) {
   return tot;
 }
 
-// Adjacent keys of the sorted order: LCP, duplicate and new-trie flags.
 // Whether key ia of a trie comes after key ib of it in path order, given that
 // they agree up to the batch's common prefix: the order k_gather_word's words
 // (then lengths) sort in.
@@ -585,6 +584,7 @@ __device__ bool key_after(const NuArgs &a, uint32_t ia, uint32_t ib) {
   return x.len > y.len;
 }
 
+// Adjacent keys of the sorted order: LCP, duplicate and new-trie flags.
 // With cmask != 0 the keys are windows compressed to the bits of cmask
 // (k_compress_windows): the XOR of two is scattered back to window bits
 // before its leading zeros give the first differing nibble.
